@@ -34,39 +34,44 @@ FLAGS = [
     "-I", INCLUDE,
 ]
 
-# The grouped GEMM kernels keep 256 accumulators in AGPRs next to an almost full VGPR file and hand-placed waits around
-# asynchronous inline-assembly loads: a register that the compiler spills inside the MFMA loop, behind those waits,
-# could be stored before its load has arrived and corrupt data silently.  The build therefore reads the generated ISA of
-# those kernels and fails if a scratch STORE sits between the first and the last MFMA of one of them (spills in front of
-# the first MFMA, where nothing asynchronous is live, are harmless, and so is reloading such a value later), and says so
-# if the compiler is not the version the kernels were written and measured with.
-LOOP_NO_SCRATCH = {"grouped_gemm.hip": re.compile(r"grouped_gemm")}
+# The grouped GEMM kernels read their fragments from LDS with inline assembly and wait for them by hand: between a read and
+# its wait the compiler takes the destination registers for ordinary values, and a spill or a copy of one of them would move
+# data that has not arrived.  The build therefore reads the generated ISA of those kernels and fails if any instruction
+# touches the destination of such a read before the next s_waitcnt lgkmcnt(0), and says so if the compiler is not the
+# version the kernels were written and measured with.
+CHECK_LDS_READS = {"grouped_gemm.hip": re.compile(r"grouped_gemm")}
 TESTED_HIPCC = "7.2"
 USAGE_REPORT = os.path.join(HERE, "build", "kernel_resource_usage.txt")
 
 
-def _scratch_inside_mfma_loop(asm_path: str, which: re.Pattern) -> list[str]:
-    """kernels matching `which` whose ISA has a scratch store between their first and last MFMA"""
-    bad, name, first, last, scratch = [], None, None, None, []
+def _registers(operands: str) -> set[str]:
+    regs = set()
+    for kind, lo, hi, kind1, n in re.findall(r"\b([va])\[(\d+):(\d+)\]|\b([va])(\d+)\b", operands):
+        regs |= {f"{kind}{i}" for i in range(int(lo), int(hi) + 1)} if kind else {kind1 + n}
+    return regs
 
-    def close():
-        if name and first is not None and any(first < n < last for n in scratch):
-            bad.append(name)
 
+def _touched_in_flight(asm_path: str, which: re.Pattern) -> list[str]:
+    """instructions of the kernels matching `which` that touch the destination of an inline-assembly ds_read before the wait
+    behind it (followed in program order; a block that is only jumped to starts with nothing in flight)"""
+    bad, name, in_asm, flight = [], None, False, set()
     with open(asm_path) as f:
-        for n, line in enumerate(f):
-            m = re.match(r"^(_Z\w+):\s*(;.*)?$", line)
+        for n, line in enumerate(f, 1):
+            m = re.match(r"^(_Z\w+):", line)
             if m:
-                close()
-                name = m.group(1) if which.search(m.group(1)) else None
-                first, last, scratch = None, None, []
-            elif name:
-                if "v_mfma" in line:
-                    first = n if first is None else first
-                    last = n
-                elif "scratch_store" in line:
-                    scratch.append(n)
-    close()
+                name, flight = (m.group(1) if which.search(m.group(1)) else None), set()
+            text = line.strip()
+            if text.startswith(";;#ASM"):
+                in_asm = text.startswith(";;#ASMSTART")
+            if not name or not text or text[0] in ";." or text.endswith(":"):
+                continue
+            op, _, operands = text.split(";")[0].partition(" " if " " in text.split("\t")[0] else "\t")
+            if op == "s_waitcnt" and "lgkmcnt(0)" in operands or op in ("s_branch", "s_endpgm", "s_setpc_b64"):
+                flight.clear()
+            elif in_asm and op.startswith("ds_read"):
+                flight |= _registers(operands.split(",")[0])
+            elif flight & _registers(operands):
+                bad.append(f"{name} line {n}: {text}")
     return bad
 
 
@@ -125,7 +130,7 @@ def _check_compiler(verbose: bool) -> None:
 def _compile(src: str, verbose: bool, defines: tuple[str, ...] = (), tag: str = "") -> str:
     obj = os.path.join(HERE, "build", src.replace(".hip", tag + ".o"))
     # keeps the device ISA next to the object (named after the source, so only the untagged build of a file may do this)
-    extra = ["-save-temps=obj"] if src in LOOP_NO_SCRATCH and not tag else []
+    extra = ["-save-temps=obj"] if src in CHECK_LDS_READS and not tag else []
     cmd = [HIPCC, *FLAGS, *extra, *defines, "-c", os.path.join(CSRC, src), "-o", obj]
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -140,9 +145,9 @@ def _compile(src: str, verbose: bool, defines: tuple[str, ...] = (), tag: str = 
         print(err, file=sys.stderr)
     if extra:
         asm = os.path.join(HERE, "build", src.replace(".hip", "-hip-amdgcn-amd-amdhsa-gfx950.s"))
-        bad = _scratch_inside_mfma_loop(asm, LOOP_NO_SCRATCH[src])
+        bad = _touched_in_flight(asm, CHECK_LDS_READS[src])
         if bad:
-            raise RuntimeError(f"{src}: scratch stores inside the MFMA loop of:\n  " + "\n  ".join(bad))
+            raise RuntimeError(f"{src}: registers touched while an LDS read into them is in flight:\n  " + "\n  ".join(bad[:10]))
         usage = _resource_usage_from_asm(asm)
     return obj, usage
 

@@ -56,7 +56,7 @@ constexpr int GEMM_SMEM_BYTES = NSTAGE * STAGE_CHUNKS * 16; // 128 KB
 // 1 KB of zeros: the source of every chunk that lies beyond the K extent of an operand
 __device__ __attribute__((aligned(16))) uint32_t g_zero_page[256];
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void lds_dma16(const uint16_t *src, u32x4 *lds_wave_base) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
@@ -233,6 +233,138 @@ __device__ __forceinline__ uint32_t lds_addr_of(const void *p) {
 #define XMA_WAIT_LOADS_AND_BARRIER() asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory")
 #define XMA_WAIT_ALL_LOADS() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 
+// ------------------------------------------------------------------------------------------------
+// K loop by quadrants.  A wave's 128 x 128 corner is four quadrants of 64 x 64 (2 x 2 accumulator tiles); a K step of 64
+// is four phases, one quadrant each over all 64 k: (Q0,P0) (Q0,P1) (Q1,P1) (Q1,P0), where Q0 / Q1 are the two 64-row
+// halves of the wave's Q rows and P0 / P1 those of its P rows.  A half of an operand tile is read from LDS completely in
+// one phase - P1 in the first, Q1 in the second, Q0 and P0 of the next step in the third and fourth - and its LDS is free
+// from then on, while the other half of the same step is still to be read.  So the loads of step kt + 2 go out in two
+// groups, {Q0, P0} in phases 1 and 2 and {P1, Q1} in phases 3 and 4 of step kt, each into the place that was read two
+// phases before, and are needed five to six phases later: about one and a half K steps of lead from two LDS stages, where
+// a loop that reads a step k16 by k16 frees a stage only when the step is over and gets half of that.
+//
+//   phase      multiplies    reads from LDS      loads (into the LDS just freed)
+//   1          Q0 P0         P1(kt)              Q0(kt+2)
+//   2          Q0 P1         Q1(kt)              P0(kt+2)
+//   barrier B  all waves have read P1, Q1 of kt; {Q0, P0}(kt+1) have landed
+//   3          Q1 P1         Q0(kt+1)            P1(kt+2)
+//   4          Q1 P0         P0(kt+1)            Q1(kt+2)
+//   barrier A  all waves have read Q0, P0 of kt+1; {P1, Q1}(kt+1) have landed
+//
+// The fragments of a half are 8 x 4 registers; P0(kt+1) goes to the registers of P1(kt), so the two P sets change roles
+// every step.  Sums run over k in the same order as in a k16 by k16 walk: results are bit-identical.
+//
+// Measured against the k16 by k16 walk (timing build, cycles per steady step; 2048 = the MFMAs back to back): 2375 -> 2224
+// (x @ W^T, 8 experts of H = 4096, I = 14336, 16384 rows), 2594 -> 2266 (dy @ W, same), and the two or three steps behind a
+// tile's first, which wait for panels that are not in L2 yet, 2800 - 4400 -> 2180 - 2300.  Launches 3 to 12 % shorter; the
+// board's power limit takes back part of what the cycles give (the clock drops from 1.6 to 1.45 GHz).
+//
+// LDS layouts, 32 KB per operand tile as above.  Row-major: [256 rows][8 chunks], a wave loads rows
+// half_row(wave, piece): 8 rows per LDS-DMA piece, four pieces per half.  Transposed source: two halves of
+// [64 k-rows][16 chunks] (the 64-column groups 0, 2 and 1, 3 of the tile), chunk c of k-row kr at slot c ^ ((kr & 3) << 2):
+// a piece covers four k-rows, two whole 128-byte lines each.
+// ------------------------------------------------------------------------------------------------
+struct Half {
+    u32x4 f[4][2]; // [k16 step][32-row block]
+};
+
+// first of the 8 rows of row-major piece i (0..3: half 0, 4..7: half 1)
+__device__ __forceinline__ int half_row(int wave, int i) { return (wave & 1) * 32 + (wave >> 1) * 128 + (i >> 2) * 64 + (i & 3) * 8; }
+// transposed piece i: first of its 4 k-rows; the lane's k-row is + (lane >> 4)
+__device__ __forceinline__ int half_krow(int wave, int i) { return wave * 16 + (i & 3) * 4; }
+// the 16-byte column chunk (of the tile's 32) that this lane fetches for transposed piece i
+__device__ __forceinline__ int half_col_chunk(int i, int lane) {
+    const int c = (lane & 15) ^ (((lane >> 4) & 3) << 2);
+    return (c >> 3) * 16 + (i >> 2) * 8 + (c & 7);
+}
+// LDS byte offset of piece i inside its operand tile
+template <int TR> __device__ __forceinline__ int half_piece_lds(int wave, int i) {
+    return TR == 0 ? half_row(wave, i) * 128 : (i >> 2) * 16384 + half_krow(wave, i) * 256;
+}
+
+template <int TR> struct HalfBase {
+    uint32_t b[TR == 0 ? 4 : 2]; // row-major: one per k16 step; transposed: one per block of a half
+};
+template <int TR> __device__ __forceinline__ void make_half_base(HalfBase<TR> &f, uint32_t tile_lds_addr, int R0, int lane) {
+    if constexpr (TR == 0) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) f.b[kk] = tile_lds_addr + rowmajor_frag_offset(R0, kk, lane);
+    } else {
+        const int p = lane & 15, G = lane >> 4;
+        const int kr = ((G >> 1) << 3) + (p >> 2);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int c = (R0 >> 7) * 8 + b * 4 + ((G & 1) << 1) + ((p & 3) >> 1);
+            f.b[b] = tile_lds_addr + (uint32_t)(kr * 256 + ((c ^ ((kr & 3) << 2)) << 4) + ((p & 1) << 3));
+        }
+    }
+}
+template <int TR> __device__ __forceinline__ void flip_half_base(HalfBase<TR> &f) {
+#pragma unroll
+    for (int q = 0; q < (TR == 0 ? 4 : 2); ++q) f.b[q] ^= (uint32_t)(STAGE_CHUNKS * 16);
+}
+template <int TR, int HALF, int KK, int B> __device__ __forceinline__ u32x4 read_half_frag(const HalfBase<TR> &f) {
+    if constexpr (TR == 0) {
+        u32x4 r;
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(f.b[KK]), "n"((HALF * 2 + B) * 4096));
+        return r;
+    } else {
+        u32x2 lo, hi;
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo) : "v"(f.b[B]), "n"(HALF * 16384 + KK * 4096));
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi) : "v"(f.b[B]), "n"(HALF * 16384 + KK * 4096 + 1024));
+        u32x4 r = {lo[0], lo[1], hi[0], hi[1]};
+        return r;
+    }
+}
+// the eight fragments tied to this point: no MFMA that uses them moves above it (the wait itself stands in front)
+__device__ __forceinline__ void tie_half(Half &h) {
+    asm volatile("" : "+v"(h.f[0][0]), "+v"(h.f[0][1]), "+v"(h.f[1][0]), "+v"(h.f[1][1]), "+v"(h.f[2][0]), "+v"(h.f[2][1]),
+                      "+v"(h.f[3][0]), "+v"(h.f[3][1]));
+}
+#define XMA_WAIT_READS() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
+// all but the N youngest loads of this wave have landed and its LDS reads have returned; then meet the other waves
+#define XMA_WAIT_AND_BARRIER(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory")
+
+// The 16 MFMAs of a quadrant in eight slots of two.  Behind each slot: its share of the eight fragment reads (two, one,
+// one, two, one, one: the LDS serves four waves, and the last read still has a slot and a half to return) and one call of
+// the hook, which the callers use for a load every other slot.  NB < 2: only the first NB 32-row blocks of the Q half
+// hold valid rows.
+template <typename T, int J0, int I0, int NB, typename Read, typename Hook>
+__device__ __forceinline__ void quadrant(const Half &p, const Half &q, f32x16 (&acc)[4][4], Read read, Hook hook) {
+    static_for<8>([&](auto S) {
+        constexpr int t = S.value;
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<2>([&](auto M) {
+            // (0,0) (0,1) (1,1) (1,0): consecutive MFMAs differ in one operand only
+            constexpr int m = 2 * t + M.value, kk = m >> 2, j = (m >> 1) & 1, i = (m & 1) ^ j;
+            if constexpr (i < NB) acc[J0 + j][I0 + i] = Elem<T>::mfma(p.f[kk][j], q.f[kk][i], acc[J0 + j][I0 + i]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (t == 0) read(IC<0>{}), read(IC<1>{});
+        if constexpr (t == 1) read(IC<2>{});
+        if constexpr (t == 2) read(IC<3>{});
+        if constexpr (t == 3) read(IC<4>{}), read(IC<5>{});
+        if constexpr (t == 4) read(IC<6>{});
+        if constexpr (t == 5) read(IC<7>{});
+        hook(S);
+    });
+    __builtin_amdgcn_sched_barrier(0);
+}
+struct NoRead {
+    template <typename R> __device__ __forceinline__ void operator()(R) const {}
+};
+template <int TR, int HALF, int NB> struct ReadHalf {
+    Half &h;
+    const HalfBase<TR> &base;
+    template <typename R> __device__ __forceinline__ void operator()(R) const {
+        constexpr int r = R::value, kk = r >> 1, b = r & 1;
+        if constexpr (b < NB) h.f[kk][b] = read_half_frag<TR, HALF, kk, b>(base);
+    }
+};
+template <int TR, int HALF, int NB> __device__ __forceinline__ ReadHalf<TR, HALF, NB> reader(Half &h, const HalfBase<TR> &base) {
+    return ReadHalf<TR, HALF, NB>{h, base};
+}
+
 // Epilogue staging in LDS, private to a wave: one 32-row block of its 128 x 128 corner as 16-bit values (rows padded
 // by 16 bytes against bank conflicts), followed by the 32 x 64 block of SwiGLU activations.
 constexpr int EPI_Z_STRIDE = 128 * 2 + 16, EPI_H_STRIDE = 64 * 2 + 16;
@@ -291,8 +423,8 @@ __device__ __forceinline__ void add_bias(const FwdArgs &a, f32x16 (&acc)[4][4], 
 
 // The accumulators of a tile set to its expert's bias, or to zero without one, by sixteen MFMAs of that rank-one product
 // onto a constant zero: the matrix pipe clears the 256 registers in half the cycles that 256 register writes take.
-template <typename T>
-__device__ __forceinline__ void init_acc(const FwdArgs &a, f32x16 (&acc)[4][4], int e, int n0, int wp, int lane) {
+template <typename T, typename Hook>
+__device__ __forceinline__ void init_acc(const FwdArgs &a, f32x16 (&acc)[4][4], int e, int n0, int wp, int lane, Hook hook) {
     const bool k0 = lane < 32;
     const u32x4 q = {k0 ? one_bits<T>() : 0u, 0u, 0u, 0u};
     uint32_t v[4] = {0u, 0u, 0u, 0u};
@@ -308,12 +440,14 @@ __device__ __forceinline__ void init_acc(const FwdArgs &a, f32x16 (&acc)[4][4], 
     f32x16 zero;
 #pragma unroll
     for (int c = 0; c < 16; ++c) zero[c] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    static_for<16>([&](auto S) {
+        constexpr int j = S.value >> 2, i = S.value & 3;
         const u32x4 p = {k0 ? v[j] : 0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[j][i] = Elem<T>::mfma(p, q, zero);
-    }
+        __builtin_amdgcn_sched_barrier(0);
+        acc[j][i] = Elem<T>::mfma(p, q, zero);
+        __builtin_amdgcn_sched_barrier(0);
+        hook(S);
+    });
 }
 
 // Which tile a workgroup works on.
@@ -497,54 +631,44 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
         // A store instruction of the accumulator layout would touch 32 rows with 16 bytes each.  Instead every
         // 32-row block goes through a wave-private LDS area and leaves as whole rows: 16 lanes x 16 bytes per row of
         // 128 columns (8 lanes per row of the 64 activation columns), i.e. full 128-byte lines.
+        // Stores are unconditional: a lane whose row or column lies outside the tile's valid part repeats the store of a
+        // lane inside it (same address, same data, read from the same place of the staging area).  Under a per-lane
+        // condition every store sits in a branch of its own, with its addresses spilled and reloaded around it.
+        if (__builtin_amdgcn_readfirstlane(n0 + wp) >= a.N) return; // this wave's columns all lie past N
         unsigned char *stage = smem + wave * EPI_WAVE_BYTES;
         unsigned char *z_w = stage + lrow * EPI_Z_STRIDE + lhalf * 8;
         unsigned char *h_w = stage + 32 * EPI_Z_STRIDE + lrow * EPI_H_STRIDE + lhalf * 4;
-        const unsigned char *z_r = stage + (lane >> 4) * EPI_Z_STRIDE + (lane & 15) * 16;
-        const unsigned char *h_r = stage + 32 * EPI_Z_STRIDE + (lane >> 3) * EPI_H_STRIDE + (lane & 7) * 16;
-        const int cz = n0 + wp + (lane & 15) * 8;        // this lane's 8 output columns on the way out
-        const int ch = ((n0 + wp) >> 1) + (lane & 7) * 8; // and its 8 activation columns
+        const int z_piece = (n0 + wp + (lane & 15) * 8 < a.N) ? (lane & 15) : 0; // this lane's 8 output columns on the way out
+        const int h_piece = (n0 + wp + (lane & 7) * 16 < a.N) ? (lane & 7) : 0;  // and its 8 activation columns
+        const int cz = n0 + wp + z_piece * 8, ch = ((n0 + wp) >> 1) + h_piece * 8;
         const bool write_z = (EPI == XMA_ROCM_EPI_STORE) || a.out != nullptr;
-        // destination row and scale of this lane's row in each of the four blocks, fetched before the first store:
+        // scattered row and scale of this lane's row in each of the four blocks, fetched before the first store:
         // loads and stores retire in order, so a load between the blocks would wait for the stores before it
-        int dst_i[4];
-        float sc_i[4];
-        const bool need_idx = !a.y_grouped || a.scale != nullptr;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            int r = wq + i * 32 + lrow;
-            if (r >= rows_valid) r = rows_valid - 1; // duplicates are computed and never stored
-            const int64_t n = row0 + r;
-            dst_i[i] = need_idx ? (pre ? pre->idx[i] : (int)a.idx[n]) : (int)n;
-        }
-        if (a.scale && pre) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc_i[i] = pre->sc[i];
-        } else if (a.scale) {
-            uint16_t raw[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) raw[i] = a.scale[dst_i[i]];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc_i[i] = Elem<T>::lo((uint32_t)raw[i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc_i[i] = 1.f;
-        }
-        if (a.y_grouped) {
+        int idx_i[4] = {0, 0, 0, 0};
+        float sc_i[4] = {1.f, 1.f, 1.f, 1.f};
+        if (!a.y_grouped || a.scale != nullptr) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 int r = wq + i * 32 + lrow;
-                if (r >= rows_valid) r = rows_valid - 1;
-                dst_i[i] = (int)(row0 + r);
+                if (r >= rows_valid) r = rows_valid - 1; // duplicates are computed and stored again
+                idx_i[i] = pre ? pre->idx[i] : (int)a.idx[row0 + r];
             }
         }
-        // two copies of the loop: without a row scale the 256 multiplications by one are left out
-        auto blocks = [&](auto SCALED) {
+        if (a.scale) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sc_i[i] = pre ? pre->sc[i] : Elem<T>::lo((uint32_t)a.scale[idx_i[i]]);
+        }
+        // copies of the loop: without a row scale the 256 multiplications by one are left out; rows in grouped order
+        // need no exchange of row indices between lanes
+        auto blocks = [&](auto SCALED, auto GROUPED) {
+        const int last = rows_valid - 1;
+        uint16_t *out0 = a.out + (GROUPED.value ? row0 * a.ldo : 0) + cz;
+        uint16_t *aux0 = a.aux + (GROUPED.value ? row0 * a.ldaux : 0) + ch;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            if (wq + i * 32 >= rows_valid) break; // wave-uniform
+            const int rbase = wq + i * 32;
+            if (rbase >= rows_valid) break; // wave-uniform
             if (only_i >= 0 && i != only_i) continue;
-            const int dst = dst_i[i];
             const float sc = sc_i[i];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -567,32 +691,43 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                 }
             }
             wave_lds_sync();
-            const int rbase = wq + i * 32;
             if (write_z) {
 #pragma unroll
                 for (int it = 0; it < 8; ++it) {
-                    const int rr = 4 * it + (lane >> 4);
-                    const u32x4 v = *(const u32x4 *)(z_r + it * 4 * EPI_Z_STRIDE);
-                    const int d = __shfl(dst, rr);
-                    if (rbase + rr < rows_valid && cz < a.N) *(u32x4 *)(a.out + (int64_t)d * a.ldo + cz) = v;
+                    int r = rbase + 4 * it + (lane >> 4);
+                    if (r > last) r = last;
+                    const u32x4 v = *(const u32x4 *)(stage + (r - rbase) * EPI_Z_STRIDE + z_piece * 16);
+                    const int64_t d = GROUPED.value ? r : __shfl(idx_i[i], r - rbase);
+                    *(u32x4 *)(out0 + d * a.ldo) = v;
                 }
             }
             if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) {
 #pragma unroll
                 for (int it = 0; it < 4; ++it) {
-                    const int rr = 8 * it + (lane >> 3);
-                    const u32x4 v = *(const u32x4 *)(h_r + it * 8 * EPI_H_STRIDE);
-                    const int d = __shfl(dst, rr);
-                    if (rbase + rr < rows_valid && 2 * ch < a.N) *(u32x4 *)(a.aux + (int64_t)d * a.ldaux + ch) = v;
+                    int r = rbase + 8 * it + (lane >> 3);
+                    if (r > last) r = last;
+                    const u32x4 v = *(const u32x4 *)(stage + 32 * EPI_Z_STRIDE + (r - rbase) * EPI_H_STRIDE + h_piece * 16);
+                    const int64_t d = GROUPED.value ? r : __shfl(idx_i[i], r - rbase);
+                    *(u32x4 *)(aux0 + d * a.ldaux) = v;
                 }
             }
             wave_lds_sync(); // the next block overwrites the area
         }
         };
-        if (a.scale)
-            blocks(IC<1>{});
-        else
-            blocks(IC<0>{});
+        if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) { // the layer's form: grouped rows, no scale
+            if (a.y_grouped && !a.scale)
+                blocks(IC<0>{}, IC<1>{});
+            else if (a.y_grouped)
+                blocks(IC<1>{}, IC<1>{});
+            else
+                blocks(IC<1>{}, IC<0>{});
+        } else {
+            if (a.scale) {
+                if (a.y_grouped) blocks(IC<1>{}, IC<1>{}); else blocks(IC<1>{}, IC<0>{});
+            } else {
+                if (a.y_grouped) blocks(IC<0>{}, IC<1>{}); else blocks(IC<0>{}, IC<0>{});
+            }
+        }
     } else {
         // SwiGLU backward: the accumulators are d h for the wave's 128 columns; z and dz have twice as many (gate, up
         // interleaved).  Each 32-row block of z comes in as whole rows (2 rows of 512 bytes per instruction) through
@@ -961,10 +1096,11 @@ constexpr int PST_STAGING_OFF = STAGE_CHUNKS * 16; // the epilogue's staging are
 // across the main loop: 8 gathered rows of the next tile, 2 x 4 rows of the epilogue (next tile's arrive while this
 // tile's are still needed), 4 row scales of this tile.
 constexpr int PST_ROWS_OFF = PST_STAGING_OFF + 4 * EPI_BWD_WAVE_BYTES;
-constexpr int PST_QR = 0, PST_ER = 8, PST_SC = 16, PST_ROW_ITEMS = 20;
+constexpr int PST_QR = 0, PST_ER = 1, PST_SC = 5, PST_ROW_ITEMS = 7;
 constexpr int PST_TABLE_OFF = PST_SMEM_BYTES - 2 * (PST_MAX_E + 1) * (int)sizeof(int);
+constexpr int PST_WALK = GEMM_THREADS, PST_WALK_OFF = PST_TABLE_OFF - PST_WALK * 16 - 16; // entries; counts of the waves behind them
 constexpr int PST_STEP_LDS_OFF = PST_ROWS_OFF + PST_ROW_ITEMS * 1024; // timing build: 8 bytes per K step, up to the tables
-static_assert(EPI_BWD_WAVE_BYTES >= EPI_WAVE_BYTES && PST_ROWS_OFF + PST_ROW_ITEMS * 1024 <= PST_TABLE_OFF,
+static_assert(EPI_BWD_WAVE_BYTES >= EPI_WAVE_BYTES && PST_ROWS_OFF + PST_ROW_ITEMS * 1024 <= PST_WALK_OFF,
               "epilogue staging and the prefetched rows must fit between stage 0 and the schedule tables");
 
 __device__ __forceinline__ void lds_dma16_raw(const void *src, uint32_t lds_wave_base) {
@@ -975,6 +1111,36 @@ __device__ __forceinline__ void lds_dma16_raw(const void *src, uint32_t lds_wave
 __device__ __forceinline__ void lds_dma4_raw(const void *src, uint32_t lds_wave_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_wave_base), "v"(src)
                  : "memory", "m0");
+}
+
+// The same through a buffer descriptor: uniform 48-bit base, 32-bit byte offset per lane.  An offset at or past the size in
+// the descriptor (BUF_OUTSIDE) reads zeros.
+constexpr uint32_t BUF_OUTSIDE = 0xffffffffu;
+__device__ __forceinline__ i32x4 buf_desc(const void *base, uint32_t bytes = 0xfffffff0u) {
+    // the base is uniform by construction; where the register allocation keeps it in vector registers all the same, the two
+    // readfirstlane bring it back (they fold away where it already is scalar)
+    const uint64_t b = (uint64_t)base;
+    i32x4 d;
+    d[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    d[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32) & 0xffff);
+    d[2] = __builtin_amdgcn_readfirstlane((int)bytes);
+    d[3] = 0x00020000;       // raw 32-bit data
+    return d;
+}
+// a * b + c in two 32-bit instructions (the compiler's 64-bit multiply-add would take a register pair for the result)
+__device__ __forceinline__ uint32_t mul_add_u32(uint32_t a, uint32_t b, uint32_t c) {
+    uint32_t m = a * b;
+    asm("" : "+v"(m));
+    return m + c;
+}
+__device__ __forceinline__ void lds_dma4_buf(i32x4 desc, uint32_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_base), "v"(off), "s"(desc)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ void lds_dma16_buf(i32x4 desc, uint32_t off, uint32_t lds_base, uint32_t stage) {
+    asm volatile("s_add_i32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds" ::"s"(lds_base), "s"(stage), "v"(off),
+                 "s"(desc)
+                 : "memory", "m0", "scc");
 }
 
 // Optional phase stamps of the persistent kernel (builds with -DXMA_PST_TIMING only): workgroup b writes the 100 MHz
@@ -1010,7 +1176,7 @@ __device__ uint64_t g_pst_steps[256][PST_MAX_STEPS];
 #endif
 
 struct PstTile {
-    int valid, t, e, n0, rows_valid, row0; // t: position in the workgroup's walk (linear tile id before the XCD remap)
+    int valid, n, e, n0, rows_valid, row0; // n: index in the table of the workgroup's walk
 };
 
 template <typename T, int WT, int EPI>
@@ -1020,9 +1186,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
     int *s_hi = s_pre + (PST_MAX_E + 1);        // [E] inclusive row offsets
     const int NT = (a.N + BN - 1) / BN;
     const int KT = (a.K + BK - 1) / BK;
-    const int KT_full = a.K / BK;                // end of the steps without a chunk past K
     const bool k_tail = (a.K & (BK - 1)) != 0;
-    const uint16_t *zero = (const uint16_t *)g_zero_page;
     const uint32_t lds0 = lds_addr_of(smem);
 
     // ---- schedule tables, once per workgroup
@@ -1062,180 +1226,175 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
         if (parts < 2) full = total;
     }
 
-    // first tile at or behind position t of this workgroup's walk (every wave computes the same, from LDS only)
-    auto lookup = [&](int t, int lane) -> PstTile {
-        PstTile r = {0, 0, 0, 0, 0, 0};
-        for (; t < a.grid_main; t += gridDim.x) {
-            const int L = xcd_remap(t, a.grid_main);
-            if (L >= full) continue;
-            int e;
-            if (a.E <= WAVE) {
-                const int x = lane < a.E ? lane : a.E;
-                const int lo = s_pre[x], hi = s_pre[x < a.E ? x + 1 : a.E];
-                e = __builtin_ctzll(__ballot(lo <= L && L < hi));
-            } else { // two levels of 64-way search
-                const int seg = (a.E + WAVE - 1) / WAVE;
-                const int x1 = lane * seg < a.E ? lane * seg : a.E;
-                const int b0 = (63 - __builtin_clzll(__ballot(s_pre[x1] <= L))) * seg;
-                const int x = b0 + lane < a.E ? b0 + lane : a.E;
-                const int lo = s_pre[x], hi = s_pre[x < a.E ? x + 1 : a.E];
-                e = b0 + __builtin_ctzll(__ballot(lane < seg && lo <= L && L < hi));
+    // The workgroup's walk: the tiles blockIdx.x + i * gridDim.x of the launch that exist, PST_WALK of them at a time as
+    // table entries in LDS (expert, first column, valid rows, first row), found by one binary search per thread.  The next
+    // tile of the walk is then one 16-byte LDS read, which the main loop of the tile before it can afford anywhere.
+    i32x4 *s_walk = (i32x4 *)(smem + PST_WALK_OFF);
+    int *s_cnt = (int *)(s_walk + PST_WALK);
+    int walk_pos = 0; // candidates i looked at so far
+    // fills the table from candidate walk_pos on; returns the number of entries (0: the walk is over).  All waves meet here.
+    auto fill_walk = [&](int tid) -> int {
+        const int lane = tid & 63, wave = tid >> 6;
+        for (;;) {
+            const int64_t t = (int64_t)blockIdx.x + (int64_t)(walk_pos + tid) * gridDim.x;
+            if ((int64_t)blockIdx.x + (int64_t)walk_pos * gridDim.x >= a.grid_main) return 0;
+            const int L = t < a.grid_main ? xcd_remap((int)t, a.grid_main) : full;
+            const uint64_t have = __ballot(L < full);
+            if (lane == 0) s_cnt[wave] = __popcll(have);
+            __syncthreads();
+            int before = __popcll(have & ((1ull << lane) - 1)), total = 0;
+            for (int w = 0; w < 4; ++w) {
+                if (w < wave) before += s_cnt[w];
+                total += s_cnt[w];
             }
-            e = __builtin_amdgcn_readfirstlane(e);
-            const int local = L - __builtin_amdgcn_readfirstlane(s_pre[e]);
-            const int row_hi = __builtin_amdgcn_readfirstlane(s_hi[e]);
-            const int row_lo = e ? __builtin_amdgcn_readfirstlane(s_hi[e - 1]) : 0;
-            const int tiles_m = (row_hi - row_lo + BM - 1) / BM;
-            int m_tile, n_tile;
-            tile_of_expert(local, tiles_m, NT, m_tile, n_tile);
-            r.valid = 1;
-            r.t = t;
-            r.e = e;
-            r.row0 = row_lo + m_tile * BM;
-            r.rows_valid = (row_hi - r.row0 < BM) ? row_hi - r.row0 : BM;
-            r.n0 = n_tile * BN;
-            break;
+            if (L < full) {
+                int lo = 0, hi = a.E; // s_pre[lo] <= L < s_pre[hi]
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (s_pre[mid] <= L)
+                        lo = mid;
+                    else
+                        hi = mid;
+                }
+                const int row_hi = s_hi[lo], row_lo = lo ? s_hi[lo - 1] : 0;
+                int m_tile, n_tile;
+                tile_of_expert(L - s_pre[lo], (row_hi - row_lo + BM - 1) / BM, NT, m_tile, n_tile);
+                const int row0 = row_lo + m_tile * BM;
+                s_walk[before] = i32x4{lo, n_tile * BN, (row_hi - row0 < BM) ? row_hi - row0 : BM, row0};
+            }
+            __syncthreads();
+            walk_pos += PST_WALK;
+            if (total) return __builtin_amdgcn_readfirstlane(total);
         }
+    };
+    int walk_len = 0; // entries of the table
+    auto entry = [&](int n) -> PstTile {
+        const i32x4 w = s_walk[n < walk_len ? n : 0];
+        PstTile r;
+        r.valid = __builtin_amdgcn_readfirstlane(n < walk_len ? 1 : 0);
+        r.n = n;
+        r.e = __builtin_amdgcn_readfirstlane(w[0]);
+        r.n0 = __builtin_amdgcn_readfirstlane(w[1]);
+        r.rows_valid = __builtin_amdgcn_readfirstlane(w[2]);
+        r.row0 = __builtin_amdgcn_readfirstlane(w[3]);
         return r;
     };
-    // Rows of a lane: the 8 rows of its LDS-DMA pieces (q) and the 4 rows of its epilogue (e), clamped to the tile's last
-    // valid row (duplicates are computed and never stored).  Where a row's scattered index is needed, its low dword is
-    // fetched by a 4-byte LDS-DMA load into the lane's slot of an item of the row area and read back behind the main loop.
+    // Rows of a wave whose scattered indices are needed: the 64 rows of its LDS-DMA pieces (one item: lane l holds row
+    // l % 8 of piece l / 8) and the 128 rows of its epilogue (two items: lane l of item m holds row 64 m + l), clamped to
+    // the tile's last valid row (duplicates are computed and never stored).  An item is one 4-byte LDS-DMA load (the low
+    // dword of the index) into the wave's part of the row area.
     const uint32_t *idx32 = (const uint32_t *)a.idx;
     const bool need_q_idx = !a.x_grouped, need_e_idx = !a.y_grouped || a.scale != nullptr;
-    auto q_row = [&](const PstTile &t, int i, int lane, int wave) {
-        const int r = wave * 64 + i * 8 + (lane >> 3);
-        return t.row0 + (r < t.rows_valid ? r : t.rows_valid - 1);
-    };
-    auto e_row = [&](const PstTile &t, int i, int lane, int wave) {
-        const int r = (wave & 1) * 128 + i * 32 + (lane & 31);
-        return t.row0 + (r < t.rows_valid ? r : t.rows_valid - 1);
-    };
+    auto clamp_row = [&](const PstTile &t, int r) { return r < t.rows_valid ? r : t.rows_valid - 1; };
     auto row_item_lds = [&](int item, int wave) { return lds0 + (uint32_t)(PST_ROWS_OFF + item * 1024 + wave * 256); };
-    auto row_item = [&](int item, int tid) { return ((const uint32_t *)(smem + PST_ROWS_OFF + item * 1024))[tid]; };
-    auto prefetch_rows = [&](const PstTile &t, int lane, int wave, bool q, int e_buf) {
-        if (q && need_q_idx) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) lds_dma4_raw(idx32 + 2 * (int64_t)q_row(t, i, lane, wave), row_item_lds(PST_QR + i, wave));
-        }
-        if (need_e_idx) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                lds_dma4_raw(idx32 + 2 * (int64_t)e_row(t, i, lane, wave), row_item_lds(PST_ER + 4 * e_buf + i, wave));
-        }
+    auto row_item = [&](int item, int wave, int slot) {
+        return ((const uint32_t *)(smem + PST_ROWS_OFF + item * 1024 + wave * 256))[slot];
     };
-
-    // The same fetches as 16 items of one LDS-DMA load each, for the first K step of a tile to issue one by one between
-    // its MFMAs: 0..7 the gathered rows of the next tile, 8..11 the rows of its epilogue, 12..15 the row scales of this
-    // tile.  An item that is not needed loads from the zero page instead, so that their number is always 16 and the wait
-    // in front of that step's barrier can leave exactly these loads in flight.
-    auto prefetch_item = [&](auto ITEM, const PstTile &t, int lane, int wave, int tid, int e_buf) {
+    // The five items of a tile's main loop: 0 the gathered rows of the next tile, 1, 2 the rows of its epilogue, 3, 4 the
+    // row scales of this tile (the aligned dword that holds the 16-bit scale; the host checks that the vector starts on 4
+    // bytes).  One that is not needed is a load from an empty buffer, so that their number is always five.
+    constexpr int ROW_LOADS = 5;
+    auto prefetch_item = [&](auto ITEM, const PstTile &t, int lane, int wave, int e_buf) {
         constexpr int it = ITEM.value;
-        const void *src = zero;
-        uint32_t dst;
-        if constexpr (it < 8) {
-            dst = row_item_lds(PST_QR + it, wave);
-            if (t.valid && need_q_idx) src = idx32 + 2 * (int64_t)q_row(t, it, lane, wave);
-        } else if constexpr (it < 12) {
-            dst = row_item_lds(PST_ER + 4 * (e_buf ^ 1) + (it - 8), wave);
-            if (t.valid && need_e_idx) src = idx32 + 2 * (int64_t)e_row(t, it - 8, lane, wave);
+        if constexpr (it < 3) {
+            const bool need = t.valid && (it == 0 ? need_q_idx : need_e_idx);
+            const int r = clamp_row(t, it == 0 ? half_row(wave, 0) + (lane >> 5) * 64 + (lane & 31) : (wave & 1) * 128 + (it - 1) * 64 + lane);
+            lds_dma4_buf(buf_desc(idx32 + 2 * (int64_t)t.row0, need ? 0xfffffff0u : 0u), (uint32_t)r * 8,
+                         row_item_lds(it == 0 ? PST_QR : PST_ER + 2 * (e_buf ^ 1) + (it - 1), wave));
         } else {
-            dst = row_item_lds(PST_SC + (it - 12), wave);
-            if (a.scale) src = (const uint32_t *)a.scale + (row_item(PST_ER + 4 * e_buf + (it - 12), tid) >> 1);
+            const uint32_t s_idx = row_item(PST_ER + 2 * e_buf + (it - 3), wave, lane);
+            lds_dma4_buf(buf_desc(a.scale, a.scale ? 0xfffffff0u : 0u), (s_idx >> 1) * 4, row_item_lds(PST_SC + (it - 3), wave));
         }
-        lds_dma4_raw(src, dst);
     };
 
-    // Addresses of the 16 LDS-DMA pieces of a tile: a uniform base per operand (SGPRs: the tile's corner of the weight
-    // matrix; the activations' first row for a gathered operand, the tile's first row for a grouped one) and one 32-bit
-    // byte offset per piece and lane.  A K step adds a uniform amount to the bases, so a piece in the loop is the M0
-    // update and the load, without any vector address arithmetic.  The host has checked that the offsets fit 32 bits.
+    // Addresses of the 16 LDS-DMA pieces of a tile (0..3 Q0, 4..7 Q1, 8..11 P0, 12..15 P1): a uniform base per operand
+    // (SGPRs: the tile's corner of the weight matrix; the activations' first row for a gathered operand, the tile's first
+    // row for a grouped one) and one 32-bit byte offset per piece and lane.  A K step adds a uniform amount to the bases,
+    // so a piece in the loop is the M0 update and the load, without any vector address arithmetic.  The host has checked
+    // that the offsets fit 32 bits.
     uint32_t q_off[8], p_off[8];
     const char *q_base = nullptr, *p_base = nullptr;
+    uint32_t tile_bytes = 0xfffffff0u; // size in the buffer descriptors: 0 for a tile that does not exist
     const int64_t p_step_b = (WT == 0) ? 2 * BK : (int64_t)2 * BK * a.ldw; // bytes per K step along the weights
-    // offsets of pieces i (activations) and 8 + i (weights); i == 0 also sets the two bases; raw: the row of piece i (its
-    // scattered index for a gathered operand)
-    auto make_pointer = [&](const PstTile &t, auto I_, int lane, int wave, uint32_t raw) {
+    auto make_bases = [&](const PstTile &t) {
+        const uint16_t *We = a.W + (int64_t)t.e * a.w_es;
+        p_base = (WT == 0) ? (const char *)(We + (int64_t)t.n0 * a.ldw) : (const char *)(We + t.n0);
+        q_base = (const char *)(need_q_idx ? a.X : a.X + (int64_t)t.row0 * a.ldx);
+        tile_bytes = t.valid ? 0xfffffff0u : 0u;
+    };
+    auto make_p_off = [&](const PstTile &t, auto I_, int lane, int wave) {
         constexpr int i = I_.value;
-        if constexpr (i == 0) {
-            const uint16_t *We = a.W + (int64_t)t.e * a.w_es;
-            p_base = (WT == 0) ? (const char *)(We + (int64_t)t.n0 * a.ldw) : (const char *)(We + t.n0);
-            q_base = (const char *)(need_q_idx ? a.X : a.X + (int64_t)t.row0 * a.ldx);
-        }
         if (WT == 0) {
-            int r = wave * 64 + i * 8 + (lane >> 3);
+            int r = half_row(wave, i) + (lane >> 3);
             if (t.n0 + r >= a.N) r = a.N - 1 - t.n0;
-            p_off[i] = (uint32_t)r * (uint32_t)(2 * a.ldw) + rowmajor_lane_chunk(i, lane) * 16;
+            p_off[i] = mul_add_u32((uint32_t)r, (uint32_t)(2 * a.ldw), (uint32_t)rowmajor_lane_chunk(i, lane) * 16);
         } else {
             const int max_chunk = ((a.N - t.n0) >> 3) - 1;
-            int cj = transposed_lane_chunk(i, lane);
+            int cj = half_col_chunk(i, lane);
             if (cj > max_chunk) cj = max_chunk;
-            p_off[i] = (uint32_t)(wave * 16 + 2 * i + (lane >> 5)) * (uint32_t)(2 * a.ldw) + cj * 16;
+            p_off[i] = mul_add_u32((uint32_t)(half_krow(wave, i) + (lane >> 4)), (uint32_t)(2 * a.ldw), (uint32_t)cj * 16);
         }
-        const uint32_t src = need_q_idx ? fastdiv(raw, a.fan_div) : raw - (uint32_t)t.row0;
-        q_off[i] = src * (uint32_t)(2 * a.ldx) + rowmajor_lane_chunk(i, lane) * 16;
     };
-    auto make_pointers = [&](const PstTile &t, int lane, int wave, const uint32_t (&raw)[8]) {
-        static_for<8>([&](auto I) { make_pointer(t, I, lane, wave, raw[I.value]); });
+    // The row of piece i of a lane is the scattered index that the row item holds, divided by fan_out, for a gathered operand
+    // and the row inside the tile for a grouped one (where the launch has set the divisor to one).
+    const uint32_t gather_mask = need_q_idx ? 0xffffffffu : 0u;
+    auto make_q_off = [&](const PstTile &t, auto I_, int lane, int wave, uint32_t idx) {
+        constexpr int i = I_.value;
+        const uint32_t local = (uint32_t)clamp_row(t, half_row(wave, i) + (lane >> 3));
+        const uint32_t src = fastdiv((idx & gather_mask) | (local & ~gather_mask), a.fan_div);
+        q_off[i] = mul_add_u32(src, (uint32_t)(2 * a.ldx), (uint32_t)rowmajor_lane_chunk(i, lane) * 16);
     };
-    // piece 0..15 of K step kt of the tile the bases and offsets describe -> stage kt & 1; FULL: the step exists and has
-    // no chunk past K
     int wave_u = 0; // this wave's index, set per tile (uniform)
     int lane_v = 0;
+    // one piece of K step kt of the tile the bases and offsets describe -> stage kt & 1.  FULL: the step exists and has no
+    // chunk past K; otherwise every lane whose chunk lies past K (all of them in a step past the last one) asks for an
+    // address outside the buffer, which the load answers with zeros, so that every step of a tile issues the same number
+    // of loads: the waits count on that
     auto issue_piece = [&](int kt, auto PIECE, auto FULL) {
         constexpr int piece = PIECE.value;
-        if constexpr (!FULL.value) {
-            if (kt >= KT) return; // uniform
-        }
+        constexpr int tr = (piece < 8) ? 0 : WT;
         // LDS destination = the piece's place in stage 0 (loop invariant) + the stage; both uniform
-        const uint32_t dst0 = lds0 + (uint32_t)(((piece >> 3) * OP_CHUNKS + (piece & 7) * 64 + wave_u * 512) * 16);
+        const uint32_t dst0 = lds0 + (uint32_t)((piece >> 3) * OP_CHUNKS * 16 + half_piece_lds<tr>(wave_u, piece & 7));
         const uint32_t stage = (uint32_t)((kt & 1) * STAGE_CHUNKS * 16);
-        const uint32_t dst = dst0 + stage;
         const char *base = (piece < 8) ? q_base + (int64_t)kt * (2 * BK) : p_base + (int64_t)kt * p_step_b; // uniform
-        const uint32_t off = (piece < 8) ? q_off[piece] : p_off[piece - 8];
-        if constexpr (FULL.value) {
-            // the base is uniform by construction; where the register allocation keeps it in vector registers all the
-            // same, the two readfirstlane bring it back (they fold away where it already is scalar)
-            const uint64_t b64 = (uint64_t)base;
-            const char *ubase = (const char *)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b64 >> 32)) << 32) |
-                                               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b64));
-            asm volatile("s_add_i32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" ::"s"(dst0), "s"(stage), "v"(off),
-                         "s"(ubase)
-                         : "memory", "m0", "scc");
-        } else {
-            const char *src = base + off;
-            if (k_tail && kt == KT - 1) {
-                asm volatile("" ::: "memory");
-                if (piece < 8 || WT == 0) {
-                    if (kt * BK + rowmajor_lane_chunk(piece & 7, lane_v) * 8 >= a.K) src = (const char *)zero;
-                } else {
-                    if (kt * BK + wave_u * 16 + 2 * (piece - 8) + (lane_v >> 5) >= a.K) src = (const char *)zero;
-                }
-            }
-            lds_dma16_raw(src, dst);
+        uint32_t off = (piece < 8) ? q_off[piece & 7] : p_off[piece & 7];
+        if constexpr (!FULL.value) {
+            const int k = (tr == 0) ? rowmajor_lane_chunk(piece & 7, lane_v) * 8 : half_krow(wave_u, piece & 7) + (lane_v >> 4);
+            off = (k < a.K - kt * BK) ? off : BUF_OUTSIDE;
         }
+        lds_dma16_buf(buf_desc(base, tile_bytes), off, dst0, stage);
+    };
+    // pieces in the order in which the halves are needed: Q0, P0, P1, Q1
+    auto ordered = [](auto P) {
+        constexpr int p = P.value;
+        return IC<(p < 4) ? p : (p < 12) ? p + 4 : p - 8>{};
     };
 
     // ---- first tile: its gathered rows are fetched on the spot, the rows of its epilogue go the way of all later ones
     PstTile cur;
     int e_buf = 0; // which of the two epilogue-row buffers holds the current tile's
-    {
+    auto first_tile = [&]() {
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
         const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        cur = lookup((int)blockIdx.x, lane);
-        if (!cur.valid) return;
+        cur = entry(0);
         uint32_t q_raw[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int n = q_row(cur, i, lane, wave);
-            q_raw[i] = need_q_idx ? idx32[2 * (int64_t)n] : (uint32_t)n;
-        }
-        make_pointers(cur, lane, wave, q_raw);
+        for (int i = 0; i < 8; ++i)
+            q_raw[i] = need_q_idx ? idx32[2 * ((int64_t)cur.row0 + clamp_row(cur, half_row(wave, i) + (lane >> 3)))] : 0u;
+        make_bases(cur);
+        static_for<8>([&](auto I) { make_q_off(cur, I, lane, wave, q_raw[I.value]), make_p_off(cur, I, lane, wave); });
         wave_u = wave, lane_v = lane;
-        static_for<16>([&](auto P) { issue_piece(0, P, IC<0>{}); });
-        prefetch_rows(cur, lane, wave, false, e_buf);
-    }
+        static_for<16>([&](auto P) { issue_piece(0, ordered(P), IC<0>{}); });
+        e_buf = 0;
+        if (need_e_idx)
+            static_for<2>([&](auto M) {
+                lds_dma4_raw(idx32 + 2 * ((int64_t)cur.row0 + clamp_row(cur, (wave & 1) * 128 + M.value * 64 + lane)), row_item_lds(PST_ER + M.value, wave));
+            });
+    };
+    walk_len = fill_walk((int)threadIdx.x);
+    if (walk_len == 0) return;
+    first_tile();
 
 #ifdef XMA_PST_TIMING
     const bool ovl_allowed = !g_pst_no_ovl;
@@ -1255,174 +1414,196 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
         // epilogue have been handed over and its staging area is dead
         asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         PST_STAMP(1);
-        if (KT_full >= 2) // the second K step exists and is complete: the short form of the loads
-            static_for<DMA_N0>([&](auto P) { issue_piece(1, P, IC<1>{}); });
-        else
-            static_for<DMA_N0>([&](auto P) { issue_piece(1, P, IC<0>{}); });
 
         // One tile ahead: the next tile's schedule entry and rows, and this tile's row scales (their addresses are the
-        // epilogue's row indices, fetched a tile ago); all of it lands in LDS during the main loop.  A full tile with an
-        // even number of at least four K steps does this between the MFMAs of its first K step, and sets up and issues
-        // the first K step of the next tile between the MFMAs of its last one (`ovl`); any other tile does it here and
-        // behind the loop, with idle matrix pipes.
+        // epilogue's row indices, fetched a tile ago); all of it lands in LDS during the main loop.  A tile of more than
+        // 192 rows with an even number of at least four complete K steps does this between the MFMAs of its first K step,
+        // sets up and loads the first K step of the next tile in its last one
+        // (`ovl`); any other tile does it here and behind the loop, with idle matrix pipes.
         const int wq = (wave & 1) * 128, wp = (wave >> 1) * 128;
         const int q_blocks = (cur.rows_valid > wq) ? (cur.rows_valid - wq + 31) >> 5 : 0;
         // uniform over the workgroup: the waves of a tile's lower half (wq == 0) and upper half disagree on q_blocks, so
         // the decision is taken on the tile's row count
-        const bool ovl = cur.rows_valid > 128 + 64 && (KT & 1) == 0 && KT >= 4 && ovl_allowed;
+        const bool ovl = cur.rows_valid > 128 + 64 && (KT & 1) == 0 && KT >= 4 && !k_tail && ovl_allowed;
         PstTile nxt = {0, 0, 0, 0, 0, 0};
         if (!ovl) {
-            nxt = lookup(cur.t + (int)gridDim.x, lane);
-            if (nxt.valid) prefetch_rows(nxt, lane, wave, true, e_buf ^ 1);
-            if (a.scale) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    // the aligned dword that holds the 16-bit scale (the host checks that the vector starts on 4 bytes)
-                    const uint32_t s_idx = row_item(PST_ER + 4 * e_buf + i, tid);
-                    lds_dma4_raw((const uint32_t *)a.scale + (s_idx >> 1), row_item_lds(PST_SC + i, wave));
-                }
-            }
+            nxt = entry(cur.n + 1);
+            static_for<ROW_LOADS>([&](auto IT) { prefetch_item(IT, nxt, lane, wave, e_buf); });
         }
-
+        // Two copies of the rest of the tile: the accumulators of the one that overlaps do not have to meet those of the
+        // other in the same registers.
+        auto rest_of_tile = [&](auto OVL) {
+        HalfBase<0> qb;
+        HalfBase<WT> pb;
+        make_half_base<0>(qb, lds0, wq, lane);
+        make_half_base<WT>(pb, lds0 + OP_CHUNKS * 16, wp, lane);
+        Half q0, q1, pA, pB;
+        static_for<8>([&](auto R) { reader<0, 0, 2>(q0, qb)(R), reader<WT, 0, 2>(pA, pb)(R); });
         PST_STAMP(2);
+        // The first half of the second K step's loads goes out between the MFMAs that produce the accumulators, the second
+        // half in the first phase of the loop: sixteen in a row would hold up the first MFMAs until the texture unit has
+        // taken them all.
         f32x16 acc[4][4];
-        init_acc<T>(a, acc, cur.e, cur.n0, wp, lane);
-        FragBase<0> qb;
-        FragBase<WT> pb;
-        make_frag_base<0>(qb, lds0, wq, lane);
-        make_frag_base<WT>(pb, lds0 + OP_CHUNKS * 16, wp, lane);
+        init_acc<T>(a, acc, cur.e, cur.n0, wp, lane, [&](auto S) {
+            if constexpr (S.value < 8) issue_piece(1, ordered(S), OVL);
+        });
+        XMA_WAIT_READS();
+        tie_half(q0), tie_half(pA);
         auto main_loop = [&](auto NI_) {
-            constexpr int NI = NI_.value;
-            Frags f0, f1;
-            if constexpr (NI > 0) {
-                static_for<4>([&](auto I) { f0.p[I.value] = read_frag<WT, I.value, 0>(pb); });
-                static_for<NI>([&](auto I) { f0.q[I.value] = read_frag<0, I.value, 0>(qb); });
-            }
-            // One K step.  FULL = 1: steps kt + 1 and kt + 2 exist and are complete; FULL = 2: step kt + 1 exists and is
-            // complete and is the tile's last (nothing is loaded for kt + 2); FULL = 0: every piece checks.  MODE 1, the first step of a tile that
-            // overlaps (`ovl`): the free slots of its second half take the next tile's schedule entry and the 16 row
-            // items; they are the youngest loads at the step's barrier, which leaves exactly them in flight.  MODE 2, the
-            // last step of such a tile (it lives in stage 1, stage 0 has been free since the barrier before): its slots
-            // take the operand addresses of the next tile and the 16 pieces of that tile's first K step, which stay in
-            // flight through the epilogue.  The loads of this tile have all been issued by then.
-            auto k_step = [&](int kt, auto FULL, auto MODE) {
+            constexpr int NI = NI_.value, NB0 = NI < 2 ? NI : 2, NB1 = NI > 2 ? 2 : 0;
+            // One K step; on entry q0 and p0 hold Q0 and P0 of step kt, on exit q0 and p1 those of step kt + 1.
+            //   MODE 0  the loads of step kt + 2 go out in its slots (complete steps)
+            //   MODE 1  the same, first step of a tile that overlaps: phase 2 finds the next tile, phase 4 also loads its rows
+            //   MODE 2  the same, the step behind that one: the waits leave the row loads in flight, too
+            //   MODE 3  second-last step of such a tile: nothing is loaded
+            //   MODE 4  its last step (stage 1; stage 0 is free): addresses and loads of the next tile's first K step, which
+            //           lands during the epilogue; no fragments are read ahead
+            //   MODE 5  any step of any other tile (every piece checks), MODE 6 its first
+            auto k_step = [&](int kt, Half &p0, Half &p1, auto MODE) {
                 constexpr int mode = MODE.value;
-                int kt_a = kt + 1, kt_b = kt + 2;
-                asm volatile("" : "+s"(kt_a), "+s"(kt_b));
-                // MODE 2: the next tile's eight gathered rows, read from the row area in one go in front of the step's MFMAs
-                // (one wait for all of them; read inside the slots, each would stall the MFMA stream for an LDS round trip)
+                constexpr int extra = (mode == 2) ? ROW_LOADS : 0;
+                int kt_b = kt + 2;
+                asm volatile("" : "+s"(kt_b)); // one address per step, not sixteen running pointers
                 [[maybe_unused]] uint32_t nxt_rows[8];
-                if constexpr (mode == 2) {
+                if constexpr (mode == 4) {
+                    // the next tile's eight gathered rows, read in one go in front of the step's MFMAs; also when there is
+                    // no next tile (nothing is loaded from the addresses then: its buffers are empty)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        nxt_rows[i] = need_q_idx ? row_item(PST_QR + i, tid) : (uint32_t)q_row(nxt, i, lane, wave);
+                    for (int i = 0; i < 8; ++i) nxt_rows[i] = row_item(PST_QR, wave, 8 * i + (lane >> 3));
+                    make_bases(nxt);
                 }
-                mma_step<T, WT, 0, 1, NI>(f0, f1, pb, qb, acc, [&](auto G) {
-                    if constexpr (mode == 2) {
-                        // also when there is no next tile (all fields zero then: addresses that nothing is loaded from):
-                        // a branch here would only add a join of sixteen registers to the loop
-                        make_pointer(nxt, G, lane, wave, nxt_rows[G.value]);
-                    } else if constexpr (G.value < DMA_N1) {
-                        issue_piece(kt_a, IC<DMA_N0 + G.value>{}, IC<(FULL.value != 0) ? 1 : 0>{});
+                auto load = [&](auto S, auto GROUP) {
+                    if constexpr ((mode == 1 || mode == 6) && GROUP.value < 2) {
+                        // phase 1: the second half of step 1; phase 2: the first half of step 2
+                        issue_piece(GROUP.value == 0 ? kt_b - 1 : kt_b, ordered(IC<(GROUP.value == 0 ? 8 : 0) + S.value>{}), IC<(mode != 6) ? 1 : 0>{});
+                    } else if constexpr (mode == 0 || mode == 1 || mode == 2 || mode == 5 || mode == 6) {
+                        if constexpr ((S.value & 1) == 1)
+                            issue_piece(kt_b, ordered(IC<GROUP.value * 4 + S.value / 2>{}), IC<(mode < 5) ? 1 : 0>{});
+                    } else if constexpr (mode == 4) { // addresses of the weights; their loads and the rows; the loads of the rows
+                        if constexpr (GROUP.value == 0) make_p_off(nxt, S, lane, wave);
+                        if constexpr (GROUP.value == 1) issue_piece(0, IC<8 + S.value>{}, IC<1>{}), make_q_off(nxt, S, lane, wave, nxt_rows[S.value]);
+                        if constexpr (GROUP.value == 2) issue_piece(0, S, IC<1>{});
                     }
+                };
+                quadrant<T, 0, 0, NB0>(p0, q0, acc, reader<WT, 1, (NI > 0) ? 2 : 0>(p1, pb), [&](auto S) {
+                    load(S, IC<0>{});
                 });
-                mma_step<T, WT, 0, 2, NI>(f1, f0, pb, qb, acc, [&](auto G) {
-                    if constexpr (mode == 1) {
-                        if constexpr (G.value == 0) nxt = lookup(cur.t + (int)gridDim.x, lane);
-                    } else if constexpr (mode == 2) {
-                        if (nxt.valid) issue_piece(0, G, IC<1>{});
-                    } else if constexpr (G.value < DMA_N2) {
-                        issue_piece(kt_a, IC<DMA_N0 + DMA_N1 + G.value>{}, IC<(FULL.value != 0) ? 1 : 0>{});
-                    }
+                XMA_WAIT_READS();
+                tie_half(p1);
+                quadrant<T, 2, 0, NB0>(p1, q0, acc, reader<0, 1, NB1>(q1, qb), [&](auto S) {
+                    load(S, IC<1>{});
+                    if constexpr (mode == 1 && S.value == 7) nxt = entry(cur.n + 1);
                 });
-                mma_step<T, WT, 0, 3, NI>(f0, f1, pb, qb, acc, [&](auto G) {
-                    if constexpr (mode == 1) {
-                        prefetch_item(IC<2 * G.value>{}, nxt, lane, wave, tid, e_buf);
-                        prefetch_item(IC<2 * G.value + 1>{}, nxt, lane, wave, tid, e_buf);
-                    } else if constexpr (mode == 2) {
-                        if (nxt.valid) issue_piece(0, IC<8 + G.value>{}, IC<1>{});
-                    }
-                });
-                if constexpr (mode == 0)
-                    XMA_WAIT_LOADS_AND_BARRIER(); // step kt + 1 has landed; nobody reads this stage any more
+                // {Q0, P0} of step kt + 1 have landed, everybody has read {P1, Q1} of this step
+                if constexpr (mode == 4)
+                    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                else if constexpr (mode == 3)
+                    XMA_WAIT_AND_BARRIER(8);
                 else
-                    asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" ::: "memory"); // all but the 16 youngest
-                flip_stage(pb);
-                flip_stage(qb);
-                mma_step<T, WT, 0, 0, NI, (mode == 2 ? 0 : 1)>(f1, f0, pb, qb, acc, [&](auto G) {
-                    if constexpr (mode != 2 && FULL.value != 2) {
-                        if constexpr (G.value < DMA_N0) issue_piece(kt_b, G, FULL);
-                        if constexpr (G.value + 8 < DMA_N0) issue_piece(kt_b, IC<G.value + 8>{}, FULL);
-                    }
-                });
+                    XMA_WAIT_AND_BARRIER(16 + extra);
+                tie_half(q1);
+                flip_half_base(qb), flip_half_base(pb);
+                if constexpr (mode == 4) {
+                    quadrant<T, 2, 2, NB1>(p1, q1, acc, NoRead(), [&](auto S) { load(S, IC<2>{}); });
+                    quadrant<T, 0, 2, NB1>(p0, q1, acc, NoRead(), [&](auto S) { load(S, IC<3>{}); });
+                } else {
+                    quadrant<T, 2, 2, NB1>(p1, q1, acc, reader<0, 0, NB0>(q0, qb), [&](auto S) { load(S, IC<2>{}); });
+                    quadrant<T, 0, 2, NB1>(p0, q1, acc, reader<WT, 0, (NI > 0) ? 2 : 0>(p1, pb), [&](auto S) {
+                        load(S, IC<3>{});
+                        if constexpr (mode == 1 && S.value >= 3) prefetch_item(IC<S.value - 3>{}, nxt, lane, wave, e_buf);
+                    });
+                    // {P1, Q1} of step kt + 1 have landed, everybody has read {Q0, P0} of it
+                    if constexpr (mode == 3)
+                        XMA_WAIT_AND_BARRIER(0);
+                    else if constexpr (mode == 1)
+                        XMA_WAIT_AND_BARRIER(16 + ROW_LOADS);
+                    else
+                        XMA_WAIT_AND_BARRIER(16);
+                    tie_half(q0), tie_half(p1);
+                }
                 PST_STEP_STAMP(kt);
             };
-            int kt = 0, kt_end = KT;
-            if constexpr (NI == 4) {
-                if (ovl) { // KT >= 4, so the first step is followed by two complete ones
-                    k_step(0, IC<1>{}, IC<1>{});
-                    kt = 1, kt_end = KT - 1;
+            if constexpr (OVL.value != 0) {
+                k_step(0, pA, pB, IC<1>{});
+                k_step(1, pB, pA, IC<2>{});
+                for (int kt = 2; kt < KT - 2; kt += 2) {
+                    k_step(kt, pA, pB, IC<0>{});
+                    k_step(kt + 1, pB, pA, IC<0>{});
                 }
-                for (; kt + 2 < KT_full && kt < kt_end; ++kt) k_step(kt, IC<1>{}, IC<0>{});
-                if (kt + 2 == KT && kt + 1 < KT_full && kt < kt_end) { // the step in front of a complete last step
-                    k_step(kt, IC<2>{}, IC<0>{});
-                    ++kt;
+                k_step(KT - 2, pA, pB, IC<3>{});
+                k_step(KT - 1, pB, pA, IC<4>{});
+            } else {
+                k_step(0, pA, pB, IC<6>{});
+                int kt = 1;
+                for (; kt + 1 < KT; kt += 2) {
+                    k_step(kt, pB, pA, IC<5>{});
+                    k_step(kt + 1, pA, pB, IC<5>{});
                 }
-            }
-            for (; kt < kt_end; ++kt) k_step(kt, IC<0>{}, IC<0>{});
-            if constexpr (NI == 4) {
-                if (ovl) k_step(KT - 1, IC<0>{}, IC<2>{});
+                if (kt < KT) k_step(kt, pB, pA, IC<5>{});
             }
         };
-        if (q_blocks > 2)
+        if constexpr (OVL.value != 0) {
+            // the waves meet behind their last reads of stage 1; only the next tile's first K step is in flight, into stage 0
             main_loop(IC<4>{});
-        else if (q_blocks == 2)
-            main_loop(IC<2>{});
-        else if (q_blocks == 1)
-            main_loop(IC<1>{});
-        else
-            main_loop(IC<0>{});
-        if (ovl) {
-            // The waves met at the last step's barrier with their reads of stage 1 done (the last sub-step reads no
-            // fragments ahead); only the next tile's first K step is in flight, into stage 0.
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         } else {
-            // every load has landed (the index loads above as well), no wave touches the operand tiles any more
-            XMA_WAIT_LOADS_AND_BARRIER();
+            if (q_blocks > 2)
+                main_loop(IC<4>{});
+            else if (q_blocks == 2)
+                main_loop(IC<2>{});
+            else if (q_blocks == 1)
+                main_loop(IC<1>{});
+            else
+                main_loop(IC<0>{});
+            XMA_WAIT_LOADS_AND_BARRIER(); // every load has landed, no wave touches the operand tiles any more
         }
         PST_STAMP(3);
 
         int tid_e = threadIdx.x;
         asm volatile("" : "+v"(tid_e));
         const int lane_e = tid_e & 63, wave_e = __builtin_amdgcn_readfirstlane(tid_e >> 6);
-        if (!ovl && nxt.valid) { // first K step of the next tile: in flight during the epilogue
-            uint32_t q_raw[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                q_raw[i] = need_q_idx ? row_item(PST_QR + i, tid_e) : (uint32_t)q_row(nxt, i, lane_e, wave_e);
-            make_pointers(nxt, lane_e, wave_e, q_raw);
+        if constexpr (OVL.value == 0) { // first K step of the next tile: in flight during the epilogue
             wave_u = wave_e, lane_v = lane_e;
-            static_for<16>([&](auto P) { issue_piece(0, P, IC<0>{}); });
+            make_bases(nxt);
+            static_for<8>([&](auto I) {
+                make_q_off(nxt, I, lane_e, wave_e, row_item(PST_QR, wave_e, 8 * I.value + (lane_e >> 3)));
+                make_p_off(nxt, I, lane_e, wave_e);
+            });
+            static_for<16>([&](auto P) { issue_piece(0, ordered(P), IC<0>{}); });
         }
         PST_STAMP(4);
         EpiRows er;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t s_idx = need_e_idx ? row_item(PST_ER + 4 * e_buf + i, tid_e) : 0u;
+            const int slot = (i & 1) * 32 + (lane_e & 31);
+            const uint32_t s_idx = need_e_idx ? row_item(PST_ER + 2 * e_buf + (i >> 1), wave_e, slot) : 0u;
             er.idx[i] = (int)s_idx;
             er.sc[i] = 1.f;
             if (a.scale) {
-                const uint32_t w = row_item(PST_SC + i, tid_e);
+                const uint32_t w = row_item(PST_SC + (i >> 1), wave_e, slot);
                 er.sc[i] = (s_idx & 1) ? Elem<T>::hi(w) : Elem<T>::lo(w);
             }
         }
         tile_epilogue<T, EPI>(a, acc, smem + PST_STAGING_OFF, cur.row0, cur.rows_valid, cur.n0, tid_e, -1, &er);
+        };
+        if (ovl)
+            rest_of_tile(IC<1>{});
+        else
+            rest_of_tile(IC<0>{});
         PST_STAMP(5);
 #ifdef XMA_PST_TIMING
         if (tile_no == PST_STEP_TILE && threadIdx.x == 0 && blockIdx.x < 256)
             for (int q = 0; q < KT && q < PST_MAX_STEPS; ++q) g_pst_steps[blockIdx.x][q] = ((uint64_t *)(smem + PST_STEP_LDS_OFF))[q];
 #endif
-        if (!nxt.valid) break;
+        if (!nxt.valid) {
+            // the end of the table: usually of the walk; a launch of more than PST_WALK tiles per workgroup refills it and
+            // starts over as at the top of the kernel
+            XMA_WAIT_LOADS_AND_BARRIER(); // (no load into LDS is in flight when the workgroup ends)
+            if ((int64_t)blockIdx.x + (int64_t)walk_pos * gridDim.x >= a.grid_main) break;
+            walk_len = fill_walk((int)threadIdx.x);
+            if (walk_len == 0) break;
+            first_tile();
+            continue;
+        }
         cur = nxt;
         e_buf ^= 1;
     }
@@ -1812,7 +1993,7 @@ static int scatter2scatter_impl(const void *X, int64_t ldx, const void *W, int64
     a.K = K;
     a.E = E;
     a.fan_out = fan_out;
-    a.fan_div = make_fastdiv((uint32_t)fan_out);
+    a.fan_div = make_fastdiv((uint32_t)(x_grouped ? 1 : fan_out));
     a.x_grouped = x_grouped;
     a.y_grouped = y_grouped;
     a.partial = nullptr;
