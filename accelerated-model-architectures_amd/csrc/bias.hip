@@ -4,9 +4,8 @@
 
 namespace {
 
-constexpr int CS_THREADS = 256;
 constexpr int CS_COLS = 128;                   // columns per workgroup: a wave reads 256 (fp32: 512) contiguous bytes of a row
-constexpr int CS_PHASES = CS_THREADS / WAVE;   // rows a workgroup has in flight per step (times the unroll)
+constexpr int CS_UNROLL = 8;                   // rows a wave has in flight
 
 template <typename T> struct Pair; // two neighbouring elements of a row as floats
 template <> struct Pair<float> {
@@ -36,11 +35,17 @@ template <> struct Pair<_Float16> {
 };
 
 // out[e, c] = sum over the grouped rows n of expert e of A[src(n), c] * scale[idx[n]], src(n) = n (idx == NULL) or
-// idx[n] / fan_out.  Workgroup (column block, expert); the rows are dealt to the four waves round-robin and added in a
+// idx[n] / fan_out.  Workgroup (column block, expert); the rows are dealt to the waves round-robin and added in a
 // fixed order (per wave in row order, then the waves in order), so the result does not depend on timing.  Experts
 // without rows get zeros.
-template <typename T>
-__global__ __launch_bounds__(CS_THREADS) void expert_column_sums_kernel(const void *__restrict__ A, int64_t lda,
+// A workgroup walks its expert's rows in steps of one round trip to memory each.  Launches of few workgroups are bound by
+// these, so they get 16 waves with 8 rows in flight, 128 rows a step (measured against 4 waves with 4 rows: 16 experts,
+// 8198 rows of 1024 / 4096 columns 18.3 -> 7.0 / 37.5 -> 14.5 us; 8 experts, 16384 rows of 4096: 131 -> 44 us).  From four
+// workgroups per CU on, 4 waves each fill the chip, and the larger workgroups only wait for their own last waves (128
+// experts, 1000 rows of 4096 columns: 5.6 us with 4 waves, 10.1 with 16; 8 experts, 16384 rows of 28672: 241 and 260).
+constexpr int CS_FEW_BLOCKS = 1024;
+template <typename T, int CS_PHASES>
+__global__ __launch_bounds__(CS_PHASES * WAVE) void expert_column_sums_kernel(const void *__restrict__ A, int64_t lda,
                                                                         const int64_t *__restrict__ idx, FastDiv fan_div,
                                                                         const void *__restrict__ scale,
                                                                         const int64_t *__restrict__ offs, void *__restrict__ out,
@@ -53,11 +58,11 @@ __global__ __launch_bounds__(CS_THREADS) void expert_column_sums_kernel(const vo
     if (!col_ok) c = N - 2; // clamped, never stored
     const int64_t lo = e ? offs[e - 1] : 0, hi = offs[e];
     float s0 = 0.f, s1 = 0.f;
-    for (int64_t r0 = lo + phase; r0 < hi; r0 += 4 * CS_PHASES) {
-        float2 v[4];
-        float w[4];
+    for (int64_t r0 = lo + phase; r0 < hi; r0 += CS_UNROLL * CS_PHASES) {
+        float2 v[CS_UNROLL];
+        float w[CS_UNROLL];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < CS_UNROLL; ++u) {
             const int64_t r = r0 + u * CS_PHASES;
             v[u] = make_float2(0.f, 0.f);
             w[u] = 1.f;
@@ -72,7 +77,7 @@ __global__ __launch_bounds__(CS_THREADS) void expert_column_sums_kernel(const vo
             }
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) s0 += v[u].x * w[u], s1 += v[u].y * w[u];
+        for (int u = 0; u < CS_UNROLL; ++u) s0 += v[u].x * w[u], s1 += v[u].y * w[u];
     }
     s_part[phase][lane] = make_float2(s0, s1);
     __syncthreads();
@@ -101,11 +106,18 @@ extern "C" int xma_rocm_expert_column_sums(const void *A, int64_t lda, const int
     const dim3 grid((N + CS_COLS - 1) / CS_COLS, E);
     hipStream_t st = (hipStream_t)stream;
     const FastDiv fd = make_fastdiv((uint32_t)fan_out);
+#define CS_LAUNCH(T, PHASES)                                                                                       \
+    expert_column_sums_kernel<T, PHASES><<<grid, PHASES * WAVE, 0, st>>>(A, lda, sorted_scattered_idxs, fd, row_scale, \
+                                                                         expert_offsets, out, ldo, N)
+#define CS_LAUNCH_T(T) few ? CS_LAUNCH(T, 16) : CS_LAUNCH(T, 4)
+    const bool few = (int64_t)grid.x * grid.y < CS_FEW_BLOCKS;
     if (dtype == XMA_ROCM_BF16)
-        expert_column_sums_kernel<__bf16><<<grid, CS_THREADS, 0, st>>>(A, lda, sorted_scattered_idxs, fd, row_scale, expert_offsets, out, ldo, N);
+        CS_LAUNCH_T(__bf16);
     else if (dtype == XMA_ROCM_F16)
-        expert_column_sums_kernel<_Float16><<<grid, CS_THREADS, 0, st>>>(A, lda, sorted_scattered_idxs, fd, row_scale, expert_offsets, out, ldo, N);
+        CS_LAUNCH_T(_Float16);
     else
-        expert_column_sums_kernel<float><<<grid, CS_THREADS, 0, st>>>(A, lda, sorted_scattered_idxs, fd, row_scale, expert_offsets, out, ldo, N);
+        CS_LAUNCH_T(float);
+#undef CS_LAUNCH_T
+#undef CS_LAUNCH
     return xma_check_launch("expert_column_sums_kernel");
 }

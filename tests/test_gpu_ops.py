@@ -203,6 +203,20 @@ def test_scatter2scatter_bias_and_expert_column_sums(dtype):
             assert torch.count_nonzero(got[e]) == 0 and torch.count_nonzero(got2[e]) == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts,N", [((0, 1, 127, 128, 129, 700), 130), ((3,) * 511 + (40,), 256), ((3,) * 512, 254)])
+def test_expert_column_sums_block_sizes(dtype, counts, N):
+    """both workgroup sizes (below and from 1024 workgroups on), experts around the rows of one step, a partial column block"""
+    from xma.rocm import ops
+
+    print(f"column sums E={len(counts)} N={N} {dtype}", flush=True)
+    A = torch.randn(sum(counts), N, generator=torch.Generator().manual_seed(5)).to(dtype)
+    got = torch.full((len(counts), N), float("nan"), dtype=dtype, device="cuda")
+    ops.expert_column_sums_rocm(A.cuda(), None, torch.tensor(counts).cumsum(0).cuda(), got, None, 1)
+    want = torch.stack([a.double().sum(0) for a in A.split(counts)])
+    assert nerr(got, want) <= _tol(dtype)
+
+
 def _routing_with_counts(counts, k, seed):
     """a routing whose experts own exactly `counts` rows (sum divisible by k): the slots are dealt out at random"""
     g = torch.Generator().manual_seed(seed)
