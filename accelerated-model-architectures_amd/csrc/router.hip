@@ -564,6 +564,111 @@ __global__ __launch_bounds__(128 * KS) void router_gate_topk_lds_kernel(const ui
             logits, ldl, weights, ids, ids_i64);
 }
 
+// Few tokens: the kernels above put 32 or 64 tokens on a workgroup whose waves walk H one dependent load after the other, which
+// leaves all of a decoding batch to one or two CUs.  Here a workgroup takes 16 tokens (v_mfma_f32_16x16x32, NT tiles of
+// 16 experts) and 16 waves share out the K steps of 64, so every wave has one to four of them at H = 1024 .. 4096 and the
+// whole of Wg is in flight at once.  A step's 64 k go to the four 16-lane groups of a wave as 16 + 16 + 16 + 16, the same
+// permutation of k for both operands.  The 16 partial sums meet in LDS and are added in a fixed order; eight waves
+// finish two tokens each.  Every workgroup reads all of Wg, so its share of the L2 traffic grows with T: up to
+// RF_MAX_TOKENS, one workgroup per CU (at E = 128, H = 2048 twice as many take as long as the kernel above).
+// Measured against the kernels above, us: E = 128, H = 576, 7 tokens 14.3 -> 7.8; E = 64, H = 2048, 64 tokens 22.6 -> 11.9;
+// E = 8, H = 4096, 1 / 3001 tokens 7.7 -> 5.2 / 13.7 -> 8.7; 4096 tokens 14.4 -> 8.9 (E = 8), 23.1 -> 13.0 (64), 28.8 -> 20.7 (128).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int RF_TOKENS = 16, RF_WAVES = 16;
+constexpr int64_t RF_MAX_TOKENS = 4096;
+template <int NT> constexpr int rf_row() { return NT * 16 + 4; } // floats; the four row groups of an accumulator 16 banks apart
+template <int NT> constexpr int rf_lds_bytes() { return RF_WAVES * RF_TOKENS * rf_row<NT>() * 4; }
+
+template <typename T> __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+    if constexpr (__is_same(T, __bf16))
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+template <typename T, int DT, int NT>
+__global__ __launch_bounds__(RF_WAVES * 64) void router_gate_topk_few_kernel(const uint16_t *__restrict__ x, int64_t ldx,
+                                                                             const uint16_t *__restrict__ wg, int64_t ldw,
+                                                                             int64_t n_tokens, int H, int E, int k,
+                                                                             uint16_t *__restrict__ logits, int64_t ldl,
+                                                                             void *__restrict__ weights,
+                                                                             void *__restrict__ ids, int ids_i64) {
+    constexpr int NB = (NT + 1) / 2, ROW = rf_row<NT>();
+    constexpr int AHEAD = NT <= 4 ? 2 : 1; // steps loaded together: what 128 registers hold
+    extern __shared__ __attribute__((aligned(16))) float s_sum[]; // [wave][token][expert]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int64_t t0 = (int64_t)blockIdx.x * RF_TOKENS;
+    const int64_t my_t = (t0 + r < n_tokens) ? t0 + r : n_tokens - 1; // clamped: rows past the end are never stored
+    const uint16_t *xrow = x + my_t * ldx + g * 16;
+    const uint16_t *wrow[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) { // columns past E take row E - 1 and are never looked at
+        const int e = n * 16 + r;
+        wrow[n] = wg + (int64_t)(e < E ? e : E - 1) * ldw + g * 16;
+    }
+    f32x4 acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 xa[AHEAD][2], wb[AHEAD][NT][2];
+    auto multiply = [&](int s) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = mfma16<T>(xa[s][q], wb[s][n][q], acc[n]);
+    };
+    const int steps_full = H / 64;
+    for (int step = wave; step < steps_full; step += AHEAD * RF_WAVES) {
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) {
+            const int st = step + s * RF_WAVES, k0 = (st < steps_full ? st : step) * 64; // past the end: loaded, not used
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                xa[s][q] = *(const u32x4 *)(xrow + k0 + 8 * q);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) wb[s][n][q] = *(const u32x4 *)(wrow[n] + k0 + 8 * q);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s)
+            if (step + s * RF_WAVES < steps_full) multiply(s);
+    }
+    if (steps_full * 64 < H && wave == steps_full % RF_WAVES) { // H is a multiple of 8: a chunk lies inside the row or outside
+        const u32x4 zero4 = {0u, 0u, 0u, 0u};
+        const int k0 = steps_full * 64;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const bool in = k0 + g * 16 + 8 * q < H;
+            xa[0][q] = in ? *(const u32x4 *)(xrow + k0 + 8 * q) : zero4;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) wb[0][n][q] = in ? *(const u32x4 *)(wrow[n] + k0 + 8 * q) : zero4;
+        }
+        multiply(0);
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) s_sum[(wave * RF_TOKENS + 4 * g + v) * ROW + n * 16 + r] = acc[n][v];
+    __syncthreads();
+    if (wave >= RF_TOKENS / 2) return;
+    const int token = 2 * wave + (lane >> 5);
+    gate_finish_slots<T, DT, NB, 1>(
+        n_tokens, lane & 31, lane, E, k, [&](int) { return t0 + token; },
+        [&](int, int b) {
+            const int e = b * 32 + (lane & 31);
+            const float *p = s_sum + token * ROW + (e < NT * 16 ? e : NT * 16 - 1);
+            float part[RF_WAVES];
+#pragma unroll
+            for (int w = 0; w < RF_WAVES; ++w) part[w] = p[w * RF_TOKENS * ROW];
+#pragma unroll
+            for (int d = RF_WAVES / 2; d > 0; d >>= 1)
+#pragma unroll
+                for (int w = 0; w < d; ++w) part[w] += part[w + d];
+            return part[0];
+        },
+        logits, ldl, weights, ids, ids_i64);
+}
+
 template <typename T, int DT>
 int router_gate_launch(const void *x, int64_t ldx, const void *wg, int64_t ldw, int64_t n_tokens, int H, int E, int k,
                        void *logits, int64_t ldl, void *weights, void *ids, int ids_i64, hipStream_t st) {
@@ -580,8 +685,25 @@ int router_gate_launch(const void *x, int64_t ldx, const void *wg, int64_t ldw, 
         RL_LAUNCH(NB, 2)          \
     else                          \
         RL_LAUNCH(NB, 1)
+#define RF_LAUNCH(NT)                                                                                              \
+    {                                                                                                              \
+        auto kernel = router_gate_topk_few_kernel<T, DT, NT>;                                                      \
+        if (int rc = xma_set_max_lds_once((const void *)kernel, rf_lds_bytes<NT>())) return rc;                    \
+        kernel<<<(unsigned)((n_tokens + RF_TOKENS - 1) / RF_TOKENS), RF_WAVES * 64, rf_lds_bytes<NT>(), st>>>(RG_ARGS); \
+    }
     const bool split_k = n_tokens < RL_SPLIT_K_BELOW;
-    if (E <= 32)
+    if (n_tokens <= RF_MAX_TOKENS) {
+        if (E <= 16)
+            RF_LAUNCH(1)
+        else if (E <= 32)
+            RF_LAUNCH(2)
+        else if (E <= 64)
+            RF_LAUNCH(4)
+        else if (E <= 96)
+            RF_LAUNCH(6)
+        else
+            RF_LAUNCH(8)
+    } else if (E <= 32)
         router_gate_topk_kernel<T, DT, 1><<<(unsigned)((n_tokens + RG_TOKENS - 1) / RG_TOKENS), RG_THREADS, 0, st>>>(RG_ARGS);
     else if (E <= 64)
         RL_LAUNCH_NB(2)
@@ -591,6 +713,7 @@ int router_gate_launch(const void *x, int64_t ldx, const void *wg, int64_t ldw, 
         RL_LAUNCH_NB(4)
 #undef RL_LAUNCH_NB
 #undef RL_LAUNCH
+#undef RF_LAUNCH
 #undef RG_ARGS
     return xma_check_launch("router_gate_topk_kernel");
 }

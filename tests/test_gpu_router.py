@@ -254,3 +254,23 @@ def test_router_gate_backward_with_a_loss_on_the_logits():
             ref = ref + (lg * dl.float()).sum()
         ref.backward()
         assert nerr(xd.grad, xf.grad) <= 2e-2 and nerr(wd.grad, wf.grad) <= 2e-2, with_logits
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (16, 2), (17, 4), (33, 3), (64, 6), (65, 8), (97, 32), (128, 8)])
+@pytest.mark.parametrize("T,H", [(1, 8), (7, 576), (15, 64), (16, 1024), (17, 1032), (33, 2120), (4096, 72), (4097, 72)])
+def test_router_gate_few_tokens(T, H, E, k):
+    """Edges of the few-token kernel: its 16-token workgroups and 16-expert tiles, fewer and more K steps than waves with and
+    without a remainder, and the last T that it takes and the first that it does not; same bounds as above."""
+    from xma.layers.moe import rocm_implementation as R
+
+    print(f"router few tokens T={T} H={H} E={E} k={k}", flush=True)
+    g = torch.Generator().manual_seed(T + H + E)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    wg = (torch.randn(E, H, generator=g) * (H**-0.5)).to(torch.bfloat16)
+    with torch.no_grad():
+        logits, w, ids = (t.cpu() for t in R.router_gate_topk(x.cuda(), wg.cuda(), k))
+    want = x.float() @ wg.float().t()
+    assert (want - logits.float()).abs().max().item() <= 2 * ULP[torch.bfloat16] * max(1.0, want.abs().max().item())
+    want_w, want_ids = oracle.routing_topk(logits, k, torch.bfloat16)
+    assert torch.equal(ids.long(), want_ids)
+    assert (w.float() - want_w.float()).abs().max().item() <= ULP[torch.bfloat16]
