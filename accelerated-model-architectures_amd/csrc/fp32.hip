@@ -2,8 +2,8 @@
 //
 // The MoE layer is meant to run in bf16/fp16; fp32 is the dtype of parity runs against the CPU path and of the
 // reference's own test grid.  These kernels are therefore written for exactness and simplicity, not for the roofline:
-// v_mfma_f32_32x32x2_f32 with fp32 operands and accumulators (no reduced-precision pass anywhere), 128 x 128 output
-// tiles, K steps of 16, operands staged through registers into k-major LDS tiles.  Schedule, operand roles, gather /
+// v_mfma_f32_32x32x2_f32 with fp32 operands and accumulators (no reduced-precision pass anywhere), 64 x 64 or 128 x 128
+// output tiles, operands staged through registers into k-major LDS tiles.  Schedule, operand roles, gather /
 // scatter semantics and epilogues are those of the 16-bit kernels in grouped_gemm.hip:
 //   forward / dX :  Q = activation rows (tokens),  P = weight rows (output features)
 //   dW           :  Q = dY columns (out features), P = X columns (in features), K = tokens of the expert
@@ -13,92 +13,111 @@
 
 namespace {
 
-constexpr int FBM = 128, FBN = 128, FBK = 16;
-constexpr int FLD = 132; // floats per k-row of an LDS tile [16 k][128 + 4]: 16-byte aligned rows, conflict-free columns
 constexpr int FTHREADS = 256;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Output tile of a workgroup: 64 TB x 64 TB, a quarter per wave (TB x TB blocks of 32 x 32).  A K step of the large tile
+// is 2048 cycles of matrix pipe behind one step's loads.  The small one has 1024 and keeps the loads of two steps in
+// flight: its launches have one or two workgroups per compute unit, so nothing else covers the latency.
+template <int TB> struct Tile {
+    static constexpr int DIM = 64 * TB, BK = 32 / TB, SETS = 3 - TB;
+    static constexpr int LD = DIM + 4; // floats per k-row of an LDS tile [BK][DIM + 4]: 16-byte aligned rows, conflict-free columns
+    // K-contiguous source ([row][k]): 2 or 4 neighbouring threads share a row, two float4 per thread
+    static __device__ __forceinline__ int row(int tid) { return TB == 2 ? tid >> 1 : tid >> 2; }
+    static __device__ __forceinline__ int kc(int tid, int h) { return TB == 2 ? (tid & 1) * 8 + 4 * h : (tid & 3) * 4 + 16 * h; }
+    // K-strided source ([k][row], rows contiguous): DIM / 4 neighbouring threads share a k
+    static __device__ __forceinline__ int ks(int tid, int h) { return tid / (DIM / 4) + (BK / 2) * h; }
+    static __device__ __forceinline__ int col(int tid) { return (tid % (DIM / 4)) * 4; }
+};
 
 struct TileRegs {
     f32x4 v[2];
 };
 
-// ---- operand tile loaders: 128 "rows" x 16 k per tile, two float4 per thread
-// K-contiguous source ([row][k]): thread t -> row t / 2, k = 8 (t & 1) + {0..7}
-__device__ __forceinline__ void load_kcontig(TileRegs &r, const float *row_ptr, int k0, int K, int tid) {
-    const int kb = k0 + (tid & 1) * 8;
+// ---- operand tile loaders: DIM "rows" x BK k per tile, two float4 per thread
+template <int TB> __device__ __forceinline__ void load_kcontig(TileRegs &r, const float *row_ptr, int k0, int K, int tid) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int k = kb + 4 * h;
+        const int k = k0 + Tile<TB>::kc(tid, h);
         r.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (k < K) r.v[h] = *(const f32x4 *)(row_ptr + k); // K % 4 == 0: a float4 is inside or outside as a whole
     }
 }
-__device__ __forceinline__ void store_kcontig(float *tile, const TileRegs &r, int tid) {
-    const int row = tid >> 1, kb = (tid & 1) * 8;
+template <int TB> __device__ __forceinline__ void store_kcontig(float *tile, const TileRegs &r, int tid) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) tile[(kb + 4 * h + q) * FLD + row] = r.v[h][q];
+        for (int q = 0; q < 4; ++q) tile[(Tile<TB>::kc(tid, h) + q) * Tile<TB>::LD + Tile<TB>::row(tid)] = r.v[h][q];
 }
-// K-strided source ([k][row], rows contiguous): thread t -> k = t / 32 + 8 pass, rows 4 (t & 31) + {0..3}
-__device__ __forceinline__ void store_kstrided(float *tile, const TileRegs &r, int tid) {
+template <int TB> __device__ __forceinline__ void store_kstrided(float *tile, const TileRegs &r, int tid) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) *(f32x4 *)(tile + ((tid >> 5) + 8 * h) * FLD + (tid & 31) * 4) = r.v[h];
+    for (int h = 0; h < 2; ++h) *(f32x4 *)(tile + Tile<TB>::ks(tid, h) * Tile<TB>::LD + Tile<TB>::col(tid)) = r.v[h];
 }
 
-__device__ __forceinline__ void zero_acc(f32x16 (&acc)[2][2]) {
+template <int TB> __device__ __forceinline__ void zero_acc(f32x16 (&acc)[TB][TB]) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TB; ++j)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < TB; ++i)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[j][i][v] = 0.f;
 }
 
-// the 16 k of the LDS tiles: 8 MFMA steps of k = 2
-__device__ __forceinline__ void mma_tiles(const float *sP, const float *sQ, f32x16 (&acc)[2][2], int wp, int wq, int lane) {
+// the BK k of the LDS tiles, MFMA steps of k = 2; the order of a sum over k does not depend on the tile
+template <int TB>
+__device__ __forceinline__ void mma_tiles(const float *sP, const float *sQ, f32x16 (&acc)[TB][TB], int wp, int wq, int lane) {
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
+    for (int kk = 0; kk < Tile<TB>::BK / 2; ++kk) {
         const int k = 2 * kk + (lane >> 5);
-        float p[2], q[2];
+        float p[TB], q[TB];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            p[b] = sP[k * FLD + wp + b * 32 + (lane & 31)];
-            q[b] = sQ[k * FLD + wq + b * 32 + (lane & 31)];
+        for (int b = 0; b < TB; ++b) {
+            p[b] = sP[k * Tile<TB>::LD + wp + b * 32 + (lane & 31)];
+            q[b] = sQ[k * Tile<TB>::LD + wq + b * 32 + (lane & 31)];
         }
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < TB; ++j)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(p[j], q[i], acc[j][i], 0, 0, 0);
+            for (int i = 0; i < TB; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(p[j], q[i], acc[j][i], 0, 0, 0);
     }
 }
 
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
 // ------------------------------------------------------------------------------------------------ forward / dX
-template <int WT, int EPI>
+template <int WT, int EPI, int TB>
 __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
+    typedef Tile<TB> T;
     extern __shared__ int s_pre[]; // [E + 1]
-    __shared__ __attribute__((aligned(16))) float sQ[FBK * FLD];
-    __shared__ __attribute__((aligned(16))) float sP[FBK * FLD];
+    __shared__ __attribute__((aligned(16))) float sQ[T::BK * T::LD];
+    __shared__ __attribute__((aligned(16))) float sP[T::BK * T::LD];
     __shared__ int s_sched[2];
     const float *X = (const float *)a.X, *W = (const float *)a.W, *scale = (const float *)a.scale;
     float *out = (float *)a.out, *aux = (float *)a.aux;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int NT = (a.N + FBN - 1) / FBN;
+    const int NT = (a.N + T::DIM - 1) / T::DIM;
 
-    // expert-major schedule from the inclusive offsets (one prefix entry per expert, serial scan by thread 0: E is small
-    // next to the work of a tile)
-    if (tid == 0) {
+    // expert-major schedule from the inclusive offsets: prefix sum of the experts' tiles by wave 0, 64 experts a step
+    if (wave == 0) {
         int run = 0;
-        for (int e = 0; e < a.E; ++e) {
-            s_pre[e] = run;
-            const int64_t cnt = a.offs[e] - (e ? a.offs[e - 1] : 0);
-            run += (int)((cnt + FBM - 1) / FBM) * NT;
+        for (int e0 = 0; e0 < a.E; e0 += WAVE) {
+            const int e = e0 + lane;
+            int tiles = 0;
+            if (e < a.E) tiles = (int)((a.offs[e] - (e ? a.offs[e - 1] : 0) + T::DIM - 1) / T::DIM) * NT;
+            int incl = tiles;
+#pragma unroll
+            for (int d = 1; d < WAVE; d <<= 1) {
+                const int t = __shfl_up(incl, d);
+                if (lane >= d) incl += t;
+            }
+            if (e < a.E) s_pre[e] = run + incl - tiles;
+            run += __shfl(incl, WAVE - 1);
         }
-        s_pre[a.E] = run;
-        s_sched[0] = -1;
+        if (lane == 0) {
+            s_pre[a.E] = run;
+            s_sched[0] = -1;
+        }
     }
     __syncthreads();
     const int L = blockIdx.x;
@@ -111,85 +130,93 @@ __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
     const int e = s_sched[0];
     if (e < 0) return; // the grid is an upper bound
     const int64_t row_lo = e ? a.offs[e - 1] : 0, row_hi = a.offs[e];
-    const int tiles_m = (int)((row_hi - row_lo + FBM - 1) / FBM);
-    const int64_t row0 = row_lo + (int64_t)(s_sched[1] % tiles_m) * FBM;
-    const int n0 = (s_sched[1] / tiles_m) * FBN;
-    const int rows_valid = (int)((row_hi - row0 < FBM) ? row_hi - row0 : FBM);
+    const int tiles_m = (int)((row_hi - row_lo + T::DIM - 1) / T::DIM);
+    const int64_t row0 = row_lo + (int64_t)(s_sched[1] % tiles_m) * T::DIM;
+    const int n0 = (s_sched[1] / tiles_m) * T::DIM;
+    const int rows_valid = (int)((row_hi - row0 < T::DIM) ? row_hi - row0 : T::DIM);
 
     // loader set-up
     const float *q_row; // this thread's activation row (K-contiguous source)
     {
-        int r = tid >> 1;
+        int r = T::row(tid);
         if (r >= rows_valid) r = rows_valid - 1; // duplicates, masked at the store
         const int64_t n = row0 + r;
-        const int64_t src = a.x_grouped ? n : a.idx[n] / a.fan_out;
+        const int64_t src = a.x_grouped ? n : (int64_t)fastdiv((uint32_t)a.idx[n], a.fan_div);
         q_row = X + src * a.ldx;
     }
     const float *We = W + (int64_t)e * a.w_es;
-    const float *p_row = nullptr; // WT == 0: weight row n0 + tid / 2
+    const float *p_row = nullptr; // WT == 0: this thread's weight row
     int p_col = 0;                // WT == 1: first of this thread's 4 columns
     if (WT == 0) {
-        int r = n0 + (tid >> 1);
+        int r = n0 + T::row(tid);
         if (r >= a.N) r = a.N - 1;
         p_row = We + (int64_t)r * a.ldw;
     } else {
-        p_col = n0 + (tid & 31) * 4;
+        p_col = n0 + T::col(tid);
         if (p_col >= a.N) p_col = a.N - 4; // masked at the store
     }
     auto load_p = [&](TileRegs &r, int k0) {
         if (WT == 0) {
-            load_kcontig(r, p_row, k0, a.K, tid);
+            load_kcontig<TB>(r, p_row, k0, a.K, tid);
         } else {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int k = k0 + (tid >> 5) + 8 * h;
+                const int k = k0 + T::ks(tid, h);
                 r.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
                 if (k < a.K) r.v[h] = *(const f32x4 *)(We + (int64_t)k * a.ldw + p_col);
             }
         }
     };
 
-    f32x16 acc[2][2];
-    zero_acc(acc);
-    const int wq = (wave & 1) * 64, wp = (wave >> 1) * 64;
+    f32x16 acc[TB][TB];
+    zero_acc<TB>(acc);
+    const int wq = (wave & 1) * 32 * TB, wp = (wave >> 1) * 32 * TB;
     if (a.bias) { // the expert's bias is the first term of every sum (see the epilogue for a lane's columns)
         const float *b = (const float *)a.bias + (int64_t)e * a.bias_es;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < TB; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 int col = n0 + wp + j * 32 + g * 8 + (lane >> 5) * 4;
                 if (col > a.N - 4) col = a.N - 4;
                 const f32x4 v = *(const f32x4 *)(b + col);
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < TB; ++i)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) acc[j][i][4 * g + q] = v[q];
             }
     }
-    const int KT = (a.K + FBK - 1) / FBK;
-    TileRegs rq, rp;
-    load_kcontig(rq, q_row, 0, a.K, tid);
-    load_p(rp, 0);
-    for (int kt = 0; kt < KT; ++kt) {
-        __syncthreads(); // the previous step's fragments have been read
-        store_kcontig(sQ, rq, tid);
-        if (WT == 0)
-            store_kcontig(sP, rp, tid);
-        else
-            store_kstrided(sP, rp, tid);
-        __syncthreads();
-        if (kt + 1 < KT) { // next step's loads fly while this one multiplies
-            load_kcontig(rq, q_row, (kt + 1) * FBK, a.K, tid);
-            load_p(rp, (kt + 1) * FBK);
+    const int KT = (a.K + T::BK - 1) / T::BK;
+    TileRegs rq[T::SETS], rp[T::SETS]; // the next SETS steps
+#pragma unroll
+    for (int s = 0; s < T::SETS; ++s) {
+        load_kcontig<TB>(rq[s], q_row, s * T::BK, a.K, tid); // zeros past K
+        load_p(rp[s], s * T::BK);
+    }
+    for (int kt0 = 0; kt0 < KT; kt0 += T::SETS) {
+#pragma unroll
+        for (int s = 0; s < T::SETS; ++s) {
+            const int kt = kt0 + s;
+            if (kt >= KT) break; // uniform
+            __syncthreads();     // the previous step's fragments have been read
+            store_kcontig<TB>(sQ, rq[s], tid);
+            if (WT == 0)
+                store_kcontig<TB>(sP, rp[s], tid);
+            else
+                store_kstrided<TB>(sP, rp[s], tid);
+            __syncthreads();
+            if (kt + T::SETS < KT) { // these loads fly while this step (and the next) multiplies
+                load_kcontig<TB>(rq[s], q_row, (kt + T::SETS) * T::BK, a.K, tid);
+                load_p(rp[s], (kt + T::SETS) * T::BK);
+            }
+            mma_tiles<TB>(sP, sQ, acc, wp, wq, lane);
         }
-        mma_tiles(sP, sQ, acc, wp, wq, lane);
     }
 
     // epilogue: lane owns row (lane & 31) of each 32-row block, 4 consecutive columns per quad
     const int lrow = lane & 31, lhalf = lane >> 5;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < TB; ++i) {
         const int r = wq + i * 32 + lrow;
         if (r >= rows_valid) continue;
         const int64_t n = row0 + r;
@@ -198,7 +225,7 @@ __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
         const int64_t dst = a.y_grouped ? n : sidx;
         const float sc = scale ? scale[sidx] : 1.f;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < TB; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int col = n0 + wp + j * 32 + g * 8 + lhalf * 4;
@@ -232,36 +259,37 @@ __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------ dW
-__global__ __launch_bounds__(FTHREADS) void dw_f32_kernel(const DwArgs a) {
-    __shared__ __attribute__((aligned(16))) float sQ[FBK * FLD];
-    __shared__ __attribute__((aligned(16))) float sP[FBK * FLD];
+template <int TB> __global__ __launch_bounds__(FTHREADS) void dw_f32_kernel(const DwArgs a) {
+    typedef Tile<TB> T;
+    __shared__ __attribute__((aligned(16))) float sQ[T::BK * T::LD];
+    __shared__ __attribute__((aligned(16))) float sP[T::BK * T::LD];
     const float *DY = (const float *)a.DY, *X = (const float *)a.X, *scale = (const float *)a.scale;
     float *DW = (float *)a.DW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int OT = (a.N_out + FBM - 1) / FBM, IT = (a.K_in + FBN - 1) / FBN;
+    const int OT = (a.N_out + T::DIM - 1) / T::DIM, IT = (a.K_in + T::DIM - 1) / T::DIM;
     const int e = blockIdx.x / (OT * IT), rem = blockIdx.x % (OT * IT);
-    const int o0 = (rem / IT) * FBM, i0 = (rem % IT) * FBN;
+    const int o0 = (rem / IT) * T::DIM, i0 = (rem % IT) * T::DIM;
     const int64_t row_lo = e ? a.offs[e - 1] : 0, row_hi = a.offs[e];
     const int rows = (int)(row_hi - row_lo);
-    const int KT = (rows + FBK - 1) / FBK;
-    int q_col = o0 + (tid & 31) * 4, p_col = i0 + (tid & 31) * 4;
+    const int KT = (rows + T::BK - 1) / T::BK;
+    int q_col = o0 + T::col(tid), p_col = i0 + T::col(tid);
     if (q_col >= a.N_out) q_col = a.N_out - 4; // masked at the store
     if (p_col >= a.K_in) p_col = a.K_in - 4;
 
-    // k-rows are tokens of the expert: thread t takes rows t / 32 and t / 32 + 8 of a step, through the index if the
+    // k-rows are tokens of the expert: a thread takes two rows of a step, through the index if the
     // operand is in scattered order; dY may carry a per-token scale
     auto load_tiles = [&](TileRegs &rq, TileRegs &rp, int k0) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int k = k0 + (tid >> 5) + 8 * h;
+            const int k = k0 + T::ks(tid, h);
             rq.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
             rp.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
             if (k < rows) {
                 const int64_t n = row_lo + k;
                 int64_t sidx = 0;
                 if (!a.dy_grouped || !a.x_grouped || scale) sidx = a.idx[n];
-                const int64_t dsrc = a.dy_grouped ? n : sidx / a.dy_fan_out;
-                const int64_t xsrc = a.x_grouped ? n : sidx / a.x_fan_out;
+                const int64_t dsrc = a.dy_grouped ? n : (int64_t)fastdiv((uint32_t)sidx, a.dy_div);
+                const int64_t xsrc = a.x_grouped ? n : (int64_t)fastdiv((uint32_t)sidx, a.x_div);
                 rq.v[h] = *(const f32x4 *)(DY + dsrc * a.lddy + q_col);
                 if (scale) rq.v[h] *= scale[sidx];
                 rp.v[h] = *(const f32x4 *)(X + xsrc * a.ldx + p_col);
@@ -269,28 +297,34 @@ __global__ __launch_bounds__(FTHREADS) void dw_f32_kernel(const DwArgs a) {
         }
     };
 
-    f32x16 acc[2][2];
-    zero_acc(acc);
-    const int wq = (wave & 1) * 64, wp = (wave >> 1) * 64;
-    TileRegs rq, rp;
-    if (KT > 0) load_tiles(rq, rp, 0);
-    for (int kt = 0; kt < KT; ++kt) {
-        __syncthreads();
-        store_kstrided(sQ, rq, tid);
-        store_kstrided(sP, rp, tid);
-        __syncthreads();
-        if (kt + 1 < KT) load_tiles(rq, rp, (kt + 1) * FBK);
-        mma_tiles(sP, sQ, acc, wp, wq, lane);
+    f32x16 acc[TB][TB];
+    zero_acc<TB>(acc);
+    const int wq = (wave & 1) * 32 * TB, wp = (wave >> 1) * 32 * TB;
+    TileRegs rq[T::SETS], rp[T::SETS];
+#pragma unroll
+    for (int s = 0; s < T::SETS; ++s) load_tiles(rq[s], rp[s], s * T::BK); // zeros past the expert's rows
+    for (int kt0 = 0; kt0 < KT; kt0 += T::SETS) {
+#pragma unroll
+        for (int s = 0; s < T::SETS; ++s) {
+            const int kt = kt0 + s;
+            if (kt >= KT) break; // uniform
+            __syncthreads();
+            store_kstrided<TB>(sQ, rq[s], tid);
+            store_kstrided<TB>(sP, rp[s], tid);
+            __syncthreads();
+            if (kt + T::SETS < KT) load_tiles(rq[s], rp[s], (kt + T::SETS) * T::BK);
+            mma_tiles<TB>(sP, sQ, acc, wp, wq, lane);
+        }
     }
     // every element of DW[e] is written, zeros for an expert without tokens
     const int lrow = lane & 31, lhalf = lane >> 5;
     float *DWe = DW + (int64_t)e * a.dw_es;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < TB; ++i) {
         const int o = o0 + wq + i * 32 + lrow;
         if (o >= a.N_out) continue;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < TB; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int col = i0 + wp + j * 32 + g * 8 + lhalf * 4;
@@ -382,30 +416,50 @@ __global__ __launch_bounds__(FTHREADS) void swiglu_bwd_f32_kernel(const float *x
 
 inline int blocks_for(int64_t work) { return (int)((work + FTHREADS - 1) / FTHREADS); }
 
-template <int WT> int launch_gemm(const FwdArgs &a, int epi, int grid, size_t lds, hipStream_t st) {
+template <int WT, int TB> int launch_gemm(const FwdArgs &a, int epi, int grid, size_t lds, hipStream_t st) {
     if (epi == XMA_ROCM_EPI_STORE)
-        gemm_f32_kernel<WT, XMA_ROCM_EPI_STORE><<<grid, FTHREADS, lds, st>>>(a);
+        gemm_f32_kernel<WT, XMA_ROCM_EPI_STORE, TB><<<grid, FTHREADS, lds, st>>>(a);
     else if (epi == XMA_ROCM_EPI_SWIGLU)
-        gemm_f32_kernel<WT, XMA_ROCM_EPI_SWIGLU><<<grid, FTHREADS, lds, st>>>(a);
+        gemm_f32_kernel<WT, XMA_ROCM_EPI_SWIGLU, TB><<<grid, FTHREADS, lds, st>>>(a);
     else
-        gemm_f32_kernel<WT, XMA_ROCM_EPI_SWIGLU_BWD><<<grid, FTHREADS, lds, st>>>(a);
+        gemm_f32_kernel<WT, XMA_ROCM_EPI_SWIGLU_BWD, TB><<<grid, FTHREADS, lds, st>>>(a);
     return xma_check_launch("gemm_f32_kernel");
 }
+
+// Which tile: a launch is bound by the matrix pipes of the compute units that have a tile, so it takes the small one until
+// the large one fills the chip several times over, and with up to 64 rows per expert on average, where the large one is
+// mostly padding.  Results are bit-identical.  Measured, large / small tile in us (x @ W^T; dy @ W; both of the forward and
+// dX GEMMs of H x I experts):  8 experts of 256 x 512, 1024 rows 29 / 18; 83 / 30, 32768 rows (2048 large tiles) 213 / 224;
+// 221 / 185;  8 of 512 x 1024, 4096 rows 129 / 125; 163 / 129, 16384 rows (2048 tiles) 364 / 381; 420 / 359;  128 of
+// 576 x 256, 56 rows 52 / 32; 45 / 27, 65536 rows (2048 and 2560 tiles) 418 / 450; 433 / 424.
+constexpr int F32_SMALL_TILES = 2048;
+// dW: the reduction is the expert's rows, so the small tile pays only where the large ones leave compute units idle.  128
+// tiles: 8 experts of 256 x 512, dW1, 1024 / 32768 rows 18.5 -> 12.3 / 464 -> 233 us; 256 tiles: dW2 of 512 x 1024, 16384
+// rows 202 -> 167; 512 tiles: dW1 337 -> 365, so not there.
+constexpr int F32_SMALL_TILES_DW = 512;
+inline int64_t f32_tiles(int64_t m, int64_t n, int dim) { return ((m + dim - 1) / dim) * ((n + dim - 1) / dim); }
 
 } // namespace
 
 int f32_scatter2scatter(const FwdArgs &a, int w_is_kn, int epilogue, hipStream_t st) {
-    const int64_t grid = (a.M / FBM + a.E) * ((a.N + FBN - 1) / FBN); // sum_e ceil(c_e / 128) <= floor(M / 128) + E
+    const bool small = a.M <= (int64_t)64 * a.E || f32_tiles(a.M, a.N, 128) < F32_SMALL_TILES;
+    const int dim = small ? 64 : 128;
+    const int64_t grid = (a.M / dim + a.E) * ((a.N + dim - 1) / dim); // sum_e ceil(c_e / dim) <= floor(M / dim) + E
     XMA_REQUIRE(grid < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "scatter2scatter (fp32): grid too large");
     XMA_REQUIRE(a.E <= 8192, XMA_ROCM_EUNSUPPORTED, "scatter2scatter (fp32): E=%d > 8192", a.E);
     const size_t lds = (size_t)(a.E + 1) * sizeof(int);
-    return w_is_kn ? launch_gemm<1>(a, epilogue, (int)grid, lds, st) : launch_gemm<0>(a, epilogue, (int)grid, lds, st);
+    if (small) return w_is_kn ? launch_gemm<1, 1>(a, epilogue, (int)grid, lds, st) : launch_gemm<0, 1>(a, epilogue, (int)grid, lds, st);
+    return w_is_kn ? launch_gemm<1, 2>(a, epilogue, (int)grid, lds, st) : launch_gemm<0, 2>(a, epilogue, (int)grid, lds, st);
 }
 
 int f32_group_bwd_W(const DwArgs &a, hipStream_t st) {
-    const int64_t grid = (int64_t)a.E * ((a.N_out + FBM - 1) / FBM) * ((a.K_in + FBN - 1) / FBN);
+    const bool small = a.E * f32_tiles(a.N_out, a.K_in, 128) < F32_SMALL_TILES_DW;
+    const int64_t grid = a.E * f32_tiles(a.N_out, a.K_in, small ? 64 : 128);
     XMA_REQUIRE(grid < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "group_bwd_W (fp32): grid too large");
-    dw_f32_kernel<<<(int)grid, FTHREADS, 0, st>>>(a);
+    if (small)
+        dw_f32_kernel<1><<<(int)grid, FTHREADS, 0, st>>>(a);
+    else
+        dw_f32_kernel<2><<<(int)grid, FTHREADS, 0, st>>>(a);
     return xma_check_launch("dw_f32_kernel");
 }
 

@@ -750,3 +750,35 @@ def test_scatter2scatter_with_and_without_workspace():
     assert rc == -3 and b"workspace" in lib.xma_rocm_last_error()
     # launches of many rounds of tiles never split: no scratch asked for
     assert lib.xma_rocm_scatter2scatter_workspace_bytes(16384, 28672, 4096, 8) == 0
+
+
+@pytest.mark.parametrize("counts,K,N", [
+    ((63, 0, 64, 65, 129, 1), 40, 72),  # 64 x 64 tiles, dW 64 x 64: edges of both, K and N with remainders
+    ((1, 3, 0, 2), 1032, 136),  # few rows, long K: an odd and an even number of K steps in flight
+    ((2047, 127, 0, 1), 40, 15368),  # 128 x 128 tiles; dW by 64 x 64
+    ((70, 0, 17, 128, 5, 64, 33, 300), 1000, 1032),  # dW from 512 tiles of 128 x 128 on
+])
+def test_fp32_tiles(counts, K, N):
+    """Both output tiles of the fp32 GEMMs, in the three forms, with rows in scattered and in grouped order; the bound is
+    that of the other fp32 tests (operands and sums in fp32, only the order of a sum differs from the oracle's)."""
+    from xma.rocm import ops
+
+    g = torch.Generator().manual_seed(17)
+    E, M = len(counts), sum(counts)
+    se = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ss = torch.randperm(M, generator=g)
+    offs = torch.tensor(counts).cumsum(0)
+    X, DY = torch.randn(M, K, generator=g), torch.randn(M, N, generator=g)
+    W = torch.randn(E, N, K, generator=g) * 0.1
+    Wd, ssd, offsd = W.cuda(), ss.cuda(), offs.cuda()
+    print(f"case counts={counts} K={K} N={N}", flush=True)
+    for x_grouped, y_grouped in ((False, True), (True, False)):
+        out = torch.full((M, N), float("nan"), device="cuda")
+        ops.scatter2scatter_rocm(X.cuda(), Wd.permute(0, 2, 1), ssd, offsd, out, None, 1, x_grouped, y_grouped)
+        assert nerr(out, oracle.scatter2scatter(X, W.permute(0, 2, 1), se, ss, 1, x_grouped, y_grouped, None)) <= TOL_F32
+        out = torch.full((M, K), float("nan"), device="cuda")
+        ops.scatter2scatter_rocm(DY.cuda(), Wd, ssd, offsd, out, None, 1, x_grouped, y_grouped)
+        assert nerr(out, oracle.scatter2scatter(DY, W, se, ss, 1, x_grouped, y_grouped, None)) <= TOL_F32
+    dw = torch.full((E, N, K), float("nan"), device="cuda")
+    ops.group_bwd_W_rocm(DY.cuda(), X.cuda(), ssd, offsd, dw.permute(0, 2, 1), None, 0, 1)
+    assert nerr(dw.permute(0, 2, 1), oracle.group_bwd_W(DY, X[ss], offs, E)) <= TOL_F32
