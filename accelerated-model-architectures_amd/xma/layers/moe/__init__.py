@@ -140,7 +140,6 @@ class MoE(nn.Module):
         if kernel_backend == KernelBackend.rocm:
             from . import rocm_implementation as R
 
-            _, expert_offsets, _, sorted_expert_idxs, sorted_scattered_idxs = R.route(selected_experts, self.num_experts)
             x = x.contiguous()
             w_fc, w_proj = self.c_fc.weight.permute(0, 2, 1), self.c_proj.weight.permute(0, 2, 1)
             # the experts' biases (the reference applies them on its torch path only, :96-100; its Triton path asserts
@@ -148,9 +147,11 @@ class MoE(nn.Module):
             b_fc, b_proj = self.c_fc.bias, self.c_proj.bias
 
             if self.is_glu and getattr(self.act, "_xma_fused_activation", None) == "swiglu_packed":
+                expert_offsets, sorted_scattered_idxs = R.route_offsets(selected_experts, self.num_experts)
                 x = R.fused_swiglu_experts(x, w_fc, w_proj, router_weights, sorted_scattered_idxs, expert_offsets, b_fc,
                                            b_proj, self.save_activations)
             else:
+                _, expert_offsets, _, sorted_expert_idxs, sorted_scattered_idxs = R.route(selected_experts, self.num_experts)
                 x = R.up_projection_experts(x, w_fc, self.top_k, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets,
                                             b_fc)
                 x = self.act(x)

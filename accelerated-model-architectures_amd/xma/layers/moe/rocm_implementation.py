@@ -42,6 +42,17 @@ def route(selected_experts: torch.Tensor, num_experts: int):
     return counts, incl, excl, sorted_expert_idxs, sorted_scattered_idxs
 
 
+def route_offsets(selected_experts: torch.Tensor, num_experts: int):
+    """(inclusive offsets int64 (E,), sorted_scattered_idxs int64): the two of `route` that the fused experts read"""
+    ids = selected_experts.flatten().contiguous()
+    n, dev = ids.numel(), ids.device
+    counts = torch.empty(num_experts, dtype=torch.uint32, device=dev)
+    incl = torch.empty(num_experts, dtype=torch.int64, device=dev)
+    sorted_scattered_idxs = torch.empty(n, dtype=torch.int64, device=dev)
+    ops.route_rocm(ids, counts, incl, None, None, sorted_scattered_idxs, None)
+    return incl, sorted_scattered_idxs
+
+
 class _RouterTopK(torch.autograd.Function):
     """top-k + fp32 softmax over the selected logits + cast, and the gradient of the logits
     (xma/layers/moe/__init__.py:186-193, 256-262)"""
