@@ -14,7 +14,8 @@
 //       LDS [64 k][32 chunks] exactly as in memory, chunk c of k-row kr at slot c ^ ((kr & 3) << 1);
 //       MFMA fragments are two ds_read_b64_tr_b16 per lane, which hand each lane 4 consecutive k of one column.
 //
-// Pipeline: two stages (128 KB of the 160 KB LDS), one barrier per K step.  A K step is four k16 sub-steps of 16 MFMAs;
+// Pipeline: two stages (128 KB of the 160 KB LDS).  The persistent forward / dX kernel walks a K step by quadrants of the
+// tile (below, at "K loop by quadrants").  The others have one barrier per K step, which is four k16 sub-steps of 16 MFMAs;
 // the fragments of sub-step kk + 1 are read while sub-step kk multiplies.  The barrier sits between sub-steps 2 and 3:
 // by then a wave holds the last fragments of the step in registers, so behind the barrier the other stage (step s + 1,
 // waited for with vmcnt(0) just before) is readable and this stage is free.  The loads of step s + 2 are issued one per
