@@ -132,66 +132,95 @@ __global__ __launch_bounds__(EW_THREADS) void group_kernel(const uint16_t *__res
     }
 }
 
-// y[r, c..c+7] from x[r, 2c..2c+15]
-template <typename ET>
-__global__ __launch_bounds__(EW_THREADS) void swiglu_packed_fwd_kernel(const uint16_t *__restrict__ x, int64_t ldx,
-                                                                       uint16_t *__restrict__ y, int64_t ldy,
-                                                                       int64_t rows, int chunks_per_row, FastDiv cpr_div) {
-    const int64_t g = (int64_t)blockIdx.x * EW_THREADS + threadIdx.x;
-    if (g >= rows * chunks_per_row) return;
-    int64_t r;
-    int c;
-    split_row(g, chunks_per_row, cpr_div, r, c);
-    c *= 8;
-    const u32x4 a = *(const u32x4 *)(x + r * ldx + 2 * c);
-    const u32x4 b = *(const u32x4 *)(x + r * ldx + 2 * c + 8);
-    float h[8];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        float g0 = Elem<ET>::lo(a[q]), u0 = Elem<ET>::hi(a[q]);
-        float g1 = Elem<ET>::lo(b[q]), u1 = Elem<ET>::hi(b[q]);
-        h[q] = u0 * g0 * sigmoidf_fast(g0);
-        h[4 + q] = u1 * g1 * sigmoidf_fast(g1);
-    }
-    u32x4 o;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = Elem<ET>::pack(h[2 * q], h[2 * q + 1]);
-    *(u32x4 *)(y + r * ldy + c) = o;
+// Packed SwiGLU, y[r, 4c..4c+3] from x[r, 8c..8c+7].  HBM-bound: a thread takes 16 bytes of x and 8 of y at a time, so that the
+// lanes of every load and store are neighbours in memory (pieces of 32 and 16 bytes leave every other 16 bytes of x to a
+// second instruction), and two such pieces.  Non-temporal (NT) where a launch moves more than the 256 MB Infinity Cache, which
+// keeps nothing for the next kernel then; below that the plain accesses find what the kernel before has left there.
+// Forward + backward in us, 32-byte pieces / two of 16, plain / the same, NT:  65536 x 4096 730 / 742 / 687 (4.7 TB/s);
+// 4099 x 4096 (101 and 168 MB) 39.8 / 39.7 / 44.7;  16384 x 1408 53.8 / 54.7 / 59.7;  1024 x 1024 7.7 / 6.8 / 7.1.
+constexpr int SWP_ITEMS = 2, SWP_OUT = 4; // pieces per thread, outputs per piece
+
+constexpr int64_t SWP_NT_BYTES = 256 << 20;    // traffic of a launch from which it is non-temporal
+template <int NT, typename V> __device__ __forceinline__ V packed_load(const uint16_t *p) {
+    return NT ? __builtin_nontemporal_load((const V *)p) : *(const V *)p;
+}
+template <int NT, typename V> __device__ __forceinline__ void packed_store(uint16_t *p, V v) {
+    if (NT)
+        __builtin_nontemporal_store(v, (V *)p);
+    else
+        *(V *)p = v;
 }
 
-template <typename ET>
+// the pieces of a thread lie EW_THREADS apart; one past the end repeats the last and is not stored
+struct PackedPieces {
+    int64_t row[SWP_ITEMS];
+    int piece[SWP_ITEMS];
+    bool in[SWP_ITEMS];
+};
+__device__ __forceinline__ PackedPieces packed_pieces(int64_t rows, int per_row, FastDiv per_row_div) {
+    PackedPieces p;
+    const int64_t n = rows * per_row, g0 = (int64_t)blockIdx.x * (EW_THREADS * SWP_ITEMS) + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < SWP_ITEMS; ++i) {
+        const int64_t g = g0 + i * EW_THREADS;
+        p.in[i] = g < n;
+        split_row(p.in[i] ? g : n - 1, per_row, per_row_div, p.row[i], p.piece[i]);
+    }
+    return p;
+}
+
+template <typename ET, int NT>
+__global__ __launch_bounds__(EW_THREADS) void swiglu_packed_fwd_kernel(const uint16_t *__restrict__ x, int64_t ldx,
+                                                                       uint16_t *__restrict__ y, int64_t ldy,
+                                                                       int64_t rows, int pieces_per_row, FastDiv ppr_div) {
+    const PackedPieces p = packed_pieces(rows, pieces_per_row, ppr_div);
+    u32x4 a[SWP_ITEMS];
+#pragma unroll
+    for (int i = 0; i < SWP_ITEMS; ++i) a[i] = packed_load<NT, u32x4>(x + p.row[i] * ldx + 2 * SWP_OUT * p.piece[i]);
+#pragma unroll
+    for (int i = 0; i < SWP_ITEMS; ++i) {
+        if (!p.in[i]) return;
+        float h[SWP_OUT];
+#pragma unroll
+        for (int q = 0; q < SWP_OUT; ++q) {
+            const float g = Elem<ET>::lo(a[i][q]), u = Elem<ET>::hi(a[i][q]);
+            h[q] = u * g * sigmoidf_fast(g);
+        }
+        const u32x2 o = {Elem<ET>::pack(h[0], h[1]), Elem<ET>::pack(h[2], h[3])};
+        packed_store<NT>(y + p.row[i] * ldy + SWP_OUT * p.piece[i], o);
+    }
+}
+
+template <typename ET, int NT>
 __global__ __launch_bounds__(EW_THREADS) void swiglu_packed_bwd_kernel(const uint16_t *__restrict__ x, int64_t ldx,
                                                                        const uint16_t *__restrict__ dy, int64_t lddy,
                                                                        uint16_t *__restrict__ dx, int64_t lddx,
-                                                                       int64_t rows, int chunks_per_row, FastDiv cpr_div) {
-    const int64_t g = (int64_t)blockIdx.x * EW_THREADS + threadIdx.x;
-    if (g >= rows * chunks_per_row) return;
-    int64_t r;
-    int c;
-    split_row(g, chunks_per_row, cpr_div, r, c);
-    c *= 8;
-    const u32x4 d = *(const u32x4 *)(dy + r * lddy + c);
-    float dv[8];
+                                                                       int64_t rows, int pieces_per_row, FastDiv ppr_div) {
+    const PackedPieces p = packed_pieces(rows, pieces_per_row, ppr_div);
+    u32x4 a[SWP_ITEMS];
+    u32x2 d[SWP_ITEMS];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        dv[2 * q] = Elem<ET>::lo(d[q]);
-        dv[2 * q + 1] = Elem<ET>::hi(d[q]);
+    for (int i = 0; i < SWP_ITEMS; ++i) {
+        a[i] = packed_load<NT, u32x4>(x + p.row[i] * ldx + 2 * SWP_OUT * p.piece[i]);
+        d[i] = packed_load<NT, u32x2>(dy + p.row[i] * lddy + SWP_OUT * p.piece[i]);
     }
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const u32x4 a = *(const u32x4 *)(x + r * ldx + 2 * c + 8 * half);
+    for (int i = 0; i < SWP_ITEMS; ++i) {
+        if (!p.in[i]) return;
         u32x4 o;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float gg = Elem<ET>::lo(a[q]), uu = Elem<ET>::hi(a[q]), dd = dv[4 * half + q];
+        for (int q = 0; q < SWP_OUT; ++q) {
+            const float gg = Elem<ET>::lo(a[i][q]), uu = Elem<ET>::hi(a[i][q]);
+            const float dd = (q & 1) ? Elem<ET>::hi(d[i][q >> 1]) : Elem<ET>::lo(d[i][q >> 1]);
             const float s = sigmoidf_fast(gg), silu = gg * s;
             o[q] = Elem<ET>::pack(dd * uu * (s + silu * (1.f - s)), dd * silu);
         }
-        *(u32x4 *)(dx + r * lddx + 2 * c + 8 * half) = o;
+        packed_store<NT>(dx + p.row[i] * lddx + 2 * SWP_OUT * p.piece[i], o);
     }
 }
 
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
+inline int packed_grid(int64_t pieces) { return (int)((pieces + EW_THREADS * SWP_ITEMS - 1) / (EW_THREADS * SWP_ITEMS)); }
 inline int grid_for(int64_t work) { return (int)((work + EW_THREADS - 1) / EW_THREADS); }
 
 } // namespace
@@ -294,9 +323,12 @@ extern "C" int xma_rocm_swiglu_packed_forward(const void *x, int64_t ldx, void *
             int rc = f32_swiglu_packed_forward(x, ldx, y, ldy, rows, vcols, st);
             if (rc) return rc;
         } else {
-            const int cpr = vcols / 8;
-            DISPATCH_T(dtype, (swiglu_packed_fwd_kernel<ET><<<grid_for(rows * cpr), EW_THREADS, 0, st>>>(
-                                  (const uint16_t *)x, ldx, (uint16_t *)y, ldy, rows, cpr, make_fastdiv((uint32_t)cpr))));
+            const int ppr = vcols / SWP_OUT;
+            const bool nt = 6 * rows * vcols > SWP_NT_BYTES;
+            DISPATCH_T(dtype, auto kernel = nt ? swiglu_packed_fwd_kernel<ET, 1> : swiglu_packed_fwd_kernel<ET, 0>;
+                       kernel<<<packed_grid(rows * ppr), EW_THREADS, 0, st>>>(
+                           (const uint16_t *)x, ldx, (uint16_t *)y, ldy, rows, ppr,
+                           make_fastdiv((uint32_t)ppr)));
             int rc = xma_check_launch("swiglu_packed_fwd_kernel");
             if (rc) return rc;
         }
@@ -322,10 +354,12 @@ extern "C" int xma_rocm_swiglu_packed_backward(const void *x, int64_t ldx, const
             int rc = f32_swiglu_packed_backward(x, ldx, dy, lddy, dx, lddx, rows, vcols, st);
             if (rc) return rc;
         } else {
-            const int cpr = vcols / 8;
-            DISPATCH_T(dtype, (swiglu_packed_bwd_kernel<ET><<<grid_for(rows * cpr), EW_THREADS, 0, st>>>(
-                                  (const uint16_t *)x, ldx, (const uint16_t *)dy, lddy, (uint16_t *)dx, lddx, rows, cpr,
-                                  make_fastdiv((uint32_t)cpr))));
+            const int ppr = vcols / SWP_OUT;
+            const bool nt = 10 * rows * vcols > SWP_NT_BYTES;
+            DISPATCH_T(dtype, auto kernel = nt ? swiglu_packed_bwd_kernel<ET, 1> : swiglu_packed_bwd_kernel<ET, 0>;
+                       kernel<<<packed_grid(rows * ppr), EW_THREADS, 0, st>>>(
+                           (const uint16_t *)x, ldx, (const uint16_t *)dy, lddy, (uint16_t *)dx, lddx, rows, ppr,
+                           make_fastdiv((uint32_t)ppr)));
             int rc = xma_check_launch("swiglu_packed_bwd_kernel");
             if (rc) return rc;
         }

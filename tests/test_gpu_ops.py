@@ -558,6 +558,33 @@ def test_swiglu_packed_standalone(dtype):
         assert nerr(xd.grad, want) <= _tol(dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols", [(1, 1024), (1, 2048), (1, 2056), (3, 1000), (33, 1003), (11003, 4104)])
+def test_swiglu_packed_pieces(dtype, rows, cols):
+    """Edges of the 16-byte kernels (a workgroup takes 2048 outputs; columns that no 16-byte piece divides; a launch above 256
+    MB, non-temporal): bit-identical to the same rows one by one or in parts, and the first rows against the oracle."""
+    from xma import KernelBackend
+    from xma.functional import swiglu_packed
+
+    print(f"swiglu_packed {rows}x{cols} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x = torch.randn(rows, 2 * cols, generator=g, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(rows, cols, generator=g, device="cuda").to(dtype)
+    y = swiglu_packed(x, kernel_backend=KernelBackend.rocm)
+    y.backward(dy)
+    for part in torch.arange(rows).chunk(3):
+        lo, hi = int(part[0]), int(part[-1]) + 1
+        xp = x.detach()[lo:hi].clone().requires_grad_()
+        yp = swiglu_packed(xp, kernel_backend=KernelBackend.rocm)
+        yp.backward(dy[lo:hi].clone())
+        assert torch.equal(yp, y[lo:hi]) and torch.equal(xp.grad, x.grad[lo:hi])
+    n = min(rows, 40)
+    x32, dy32 = x.detach()[:n].float().cpu(), dy[:n].float().cpu()
+    assert nerr(y[:n], oracle.swiglu_packed(x32)) <= _tol(dtype)
+    dg, du = oracle.swiglu_backward(x32[..., 0::2], x32[..., 1::2], dy32)
+    assert nerr(x.grad[:n], torch.stack([dg, du], dim=-1).flatten(-2)) <= _tol(dtype)
+
+
 def _2d_sizes():
     """the reference's 2-D size rule (tests/utils.py:31-42: squares 2^i + j, and ragged sizes around 3000), thinned so
     that the CPU oracle stays within seconds"""
