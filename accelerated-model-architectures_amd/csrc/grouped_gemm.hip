@@ -41,6 +41,7 @@
 
 #include "fp32.hpp"
 #include "gemm_common.hpp"
+#include "k_schedule.hpp"
 
 namespace xma_rocm {
 
@@ -252,6 +253,9 @@ __device__ __forceinline__ uint32_t lds_addr_of(const void *p) {
 //   4          Q1 P0         P0(kt+1)            Q1(kt+2)
 //   barrier A  all waves have read Q0, P0 of kt+1; {P1, Q1}(kt+1) have landed
 //
+// Q0 and P0 of a tile's first step are read in front of the loop, so a barrier of their own stands there for the loads that
+// phase 2 of that step puts into their place.  Loads, reads and waits are those of k_schedule.hpp, which is checked on the host.
+//
 // The fragments of a half are 8 x 4 registers; P0(kt+1) goes to the registers of P1(kt), so the two P sets change roles
 // every step.  Sums run over k in the same order as in a k16 by k16 walk: results are bit-identical.
 //
@@ -323,7 +327,8 @@ __device__ __forceinline__ void tie_half(Half &h) {
                       "+v"(h.f[3][0]), "+v"(h.f[3][1]));
 }
 #define XMA_WAIT_READS() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
-// all but the N youngest loads of this wave have landed and its LDS reads have returned; then meet the other waves
+// its LDS reads have returned (and all but the N youngest loads of this wave have landed); then meet the other waves
+#define XMA_WAIT_READS_AND_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 #define XMA_WAIT_AND_BARRIER(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory")
 
 // The 16 MFMAs of a quadrant in eight slots of two.  Behind each slot: its share of the eight fragment reads (two, one,
@@ -1294,7 +1299,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
     // The five items of a tile's main loop: 0 the gathered rows of the next tile, 1, 2 the rows of its epilogue, 3, 4 the
     // row scales of this tile (the aligned dword that holds the 16-bit scale; the host checks that the vector starts on 4
     // bytes).  One that is not needed is a load from an empty buffer, so that their number is always five.
-    constexpr int ROW_LOADS = 5;
+    constexpr int ROW_LOADS = k_schedule::ROW_LOADS;
     auto prefetch_item = [&](auto ITEM, const PstTile &t, int lane, int wave, int e_buf) {
         constexpr int it = ITEM.value;
         if constexpr (it < 3) {
@@ -1365,11 +1370,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
         }
         lds_dma16_buf(buf_desc(base, tile_bytes), off, dst0, stage);
     };
-    // pieces in the order in which the halves are needed: Q0, P0, P1, Q1
-    auto ordered = [](auto P) {
-        constexpr int p = P.value;
-        return IC<(p < 4) ? p : (p < 12) ? p + 4 : p - 8>{};
-    };
+    auto ordered = [](auto P) { return IC<k_schedule::ordered(P.value)>{}; };
 
     // ---- first tile: its gathered rows are fetched on the spot, the rows of its epilogue go the way of all later ones
     PstTile cur;
@@ -1446,45 +1447,41 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
         // taken them all.
         f32x16 acc[4][4];
         init_acc<T>(a, acc, cur.e, cur.n0, wp, lane, [&](auto S) {
-            if constexpr (S.value < 8) issue_piece(1, ordered(S), OVL);
+            constexpr k_schedule::Load l = k_schedule::load_before_loop(S.value);
+            if constexpr (l.piece >= 0) issue_piece(l.ahead, IC<l.piece>{}, OVL);
         });
-        XMA_WAIT_READS();
+        if constexpr (k_schedule::BARRIER_BEFORE_LOOP)
+            XMA_WAIT_READS_AND_BARRIER();
+        else
+            XMA_WAIT_READS();
         tie_half(q0), tie_half(pA);
         auto main_loop = [&](auto NI_) {
             constexpr int NI = NI_.value, NB0 = NI < 2 ? NI : 2, NB1 = NI > 2 ? 2 : 0;
-            // One K step; on entry q0 and p0 hold Q0 and P0 of step kt, on exit q0 and p1 those of step kt + 1.
-            //   MODE 0  the loads of step kt + 2 go out in its slots (complete steps)
-            //   MODE 1  the same, first step of a tile that overlaps: phase 2 finds the next tile, phase 4 also loads its rows
-            //   MODE 2  the same, the step behind that one: the waits leave the row loads in flight, too
-            //   MODE 3  second-last step of such a tile: nothing is loaded
-            //   MODE 4  its last step (stage 1; stage 0 is free): addresses and loads of the next tile's first K step, which
-            //           lands during the epilogue; no fragments are read ahead
-            //   MODE 5  any step of any other tile (every piece checks), MODE 6 its first
+            // One K step; on entry q0 and p0 hold Q0 and P0 of step kt, on exit q0 and p1 those of step kt + 1.  MODE: what
+            // it loads and waits for.
             auto k_step = [&](int kt, Half &p0, Half &p1, auto MODE) {
                 constexpr int mode = MODE.value;
-                constexpr int extra = (mode == 2) ? ROW_LOADS : 0;
                 int kt_b = kt + 2;
                 asm volatile("" : "+s"(kt_b)); // one address per step, not sixteen running pointers
                 [[maybe_unused]] uint32_t nxt_rows[8];
-                if constexpr (mode == 4) {
+                if constexpr (mode == k_schedule::OVL_LAST) {
                     // the next tile's eight gathered rows, read in one go in front of the step's MFMAs; also when there is
                     // no next tile (nothing is loaded from the addresses then: its buffers are empty)
 #pragma unroll
                     for (int i = 0; i < 8; ++i) nxt_rows[i] = row_item(PST_QR, wave, 8 * i + (lane >> 3));
                     make_bases(nxt);
                 }
-                auto load = [&](auto S, auto GROUP) {
-                    if constexpr ((mode == 1 || mode == 6) && GROUP.value < 2) {
-                        // phase 1: the second half of step 1; phase 2: the first half of step 2
-                        issue_piece(GROUP.value == 0 ? kt_b - 1 : kt_b, ordered(IC<(GROUP.value == 0 ? 8 : 0) + S.value>{}), IC<(mode != 6) ? 1 : 0>{});
-                    } else if constexpr (mode == 0 || mode == 1 || mode == 2 || mode == 5 || mode == 6) {
-                        if constexpr ((S.value & 1) == 1)
-                            issue_piece(kt_b, ordered(IC<GROUP.value * 4 + S.value / 2>{}), IC<(mode < 5) ? 1 : 0>{});
-                    } else if constexpr (mode == 4) { // addresses of the weights; their loads and the rows; the loads of the rows
-                        if constexpr (GROUP.value == 0) make_p_off(nxt, S, lane, wave);
-                        if constexpr (GROUP.value == 1) issue_piece(0, IC<8 + S.value>{}, IC<1>{}), make_q_off(nxt, S, lane, wave, nxt_rows[S.value]);
-                        if constexpr (GROUP.value == 2) issue_piece(0, S, IC<1>{});
+                auto load = [&](auto S, auto PHASE) {
+                    constexpr k_schedule::Load l = k_schedule::load_of(mode, PHASE.value, S.value);
+                    if constexpr (mode == k_schedule::OVL_LAST) { // addresses in the slots in front of the loads
+                        if constexpr (PHASE.value == 0) make_p_off(nxt, S, lane, wave);
+                        if constexpr (l.piece >= 0) issue_piece(0, IC<l.piece>{}, IC<1>{});
+                        if constexpr (PHASE.value == 1) make_q_off(nxt, S, lane, wave, nxt_rows[S.value]);
+                    } else if constexpr (l.piece >= 0) {
+                        issue_piece(kt_b - 2 + l.ahead, IC<l.piece>{}, IC<(mode < k_schedule::CHECKED) ? 1 : 0>{});
                     }
+                    constexpr int row = k_schedule::row_load_of(mode, PHASE.value, S.value);
+                    if constexpr (row >= 0) prefetch_item(IC<row>{}, nxt, lane, wave, e_buf);
                 };
                 quadrant<T, 0, 0, NB0>(p0, q0, acc, reader<WT, 1, (NI > 0) ? 2 : 0>(p1, pb), [&](auto S) {
                     load(S, IC<0>{});
@@ -1493,54 +1490,45 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
                 tie_half(p1);
                 quadrant<T, 2, 0, NB0>(p1, q0, acc, reader<0, 1, NB1>(q1, qb), [&](auto S) {
                     load(S, IC<1>{});
-                    if constexpr (mode == 1 && S.value == 7) nxt = entry(cur.n + 1);
+                    if constexpr (mode == k_schedule::OVL_FIRST && S.value == 7) nxt = entry(cur.n + 1);
                 });
                 // {Q0, P0} of step kt + 1 have landed, everybody has read {P1, Q1} of this step
-                if constexpr (mode == 4)
-                    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                else if constexpr (mode == 3)
-                    XMA_WAIT_AND_BARRIER(8);
+                constexpr int left_b = k_schedule::in_flight_b(mode), left_a = k_schedule::in_flight_a(mode);
+                if constexpr (left_b < 0)
+                    XMA_WAIT_READS_AND_BARRIER();
                 else
-                    XMA_WAIT_AND_BARRIER(16 + extra);
+                    XMA_WAIT_AND_BARRIER(left_b);
                 tie_half(q1);
                 flip_half_base(qb), flip_half_base(pb);
-                if constexpr (mode == 4) {
+                if constexpr (!k_schedule::reads_ahead(mode)) {
                     quadrant<T, 2, 2, NB1>(p1, q1, acc, NoRead(), [&](auto S) { load(S, IC<2>{}); });
                     quadrant<T, 0, 2, NB1>(p0, q1, acc, NoRead(), [&](auto S) { load(S, IC<3>{}); });
                 } else {
                     quadrant<T, 2, 2, NB1>(p1, q1, acc, reader<0, 0, NB0>(q0, qb), [&](auto S) { load(S, IC<2>{}); });
-                    quadrant<T, 0, 2, NB1>(p0, q1, acc, reader<WT, 0, (NI > 0) ? 2 : 0>(p1, pb), [&](auto S) {
-                        load(S, IC<3>{});
-                        if constexpr (mode == 1 && S.value >= 3) prefetch_item(IC<S.value - 3>{}, nxt, lane, wave, e_buf);
-                    });
+                    quadrant<T, 0, 2, NB1>(p0, q1, acc, reader<WT, 0, (NI > 0) ? 2 : 0>(p1, pb), [&](auto S) { load(S, IC<3>{}); });
                     // {P1, Q1} of step kt + 1 have landed, everybody has read {Q0, P0} of it
-                    if constexpr (mode == 3)
-                        XMA_WAIT_AND_BARRIER(0);
-                    else if constexpr (mode == 1)
-                        XMA_WAIT_AND_BARRIER(16 + ROW_LOADS);
-                    else
-                        XMA_WAIT_AND_BARRIER(16);
+                    XMA_WAIT_AND_BARRIER(left_a);
                     tie_half(q0), tie_half(p1);
                 }
                 PST_STEP_STAMP(kt);
             };
             if constexpr (OVL.value != 0) {
-                k_step(0, pA, pB, IC<1>{});
-                k_step(1, pB, pA, IC<2>{});
+                k_step(0, pA, pB, IC<k_schedule::OVL_FIRST>{});
+                k_step(1, pB, pA, IC<k_schedule::OVL_SECOND>{});
                 for (int kt = 2; kt < KT - 2; kt += 2) {
-                    k_step(kt, pA, pB, IC<0>{});
-                    k_step(kt + 1, pB, pA, IC<0>{});
+                    k_step(kt, pA, pB, IC<k_schedule::STEADY>{});
+                    k_step(kt + 1, pB, pA, IC<k_schedule::STEADY>{});
                 }
-                k_step(KT - 2, pA, pB, IC<3>{});
-                k_step(KT - 1, pB, pA, IC<4>{});
+                k_step(KT - 2, pA, pB, IC<k_schedule::OVL_DRAIN>{});
+                k_step(KT - 1, pB, pA, IC<k_schedule::OVL_LAST>{});
             } else {
-                k_step(0, pA, pB, IC<6>{});
+                k_step(0, pA, pB, IC<k_schedule::CHECKED_FIRST>{});
                 int kt = 1;
                 for (; kt + 1 < KT; kt += 2) {
-                    k_step(kt, pB, pA, IC<5>{});
-                    k_step(kt + 1, pA, pB, IC<5>{});
+                    k_step(kt, pB, pA, IC<k_schedule::CHECKED>{});
+                    k_step(kt + 1, pA, pB, IC<k_schedule::CHECKED>{});
                 }
-                if (kt < KT) k_step(kt, pB, pA, IC<5>{});
+                if (kt < KT) k_step(kt, pB, pA, IC<k_schedule::CHECKED>{});
             }
         };
         if constexpr (OVL.value != 0) {
