@@ -34,12 +34,14 @@ FLAGS = [
     "-I", INCLUDE,
 ]
 
-# The grouped GEMM kernels read their fragments from LDS with inline assembly and wait for them by hand: between a read and
-# its wait the compiler takes the destination registers for ordinary values, and a spill or a copy of one of them would move
-# data that has not arrived.  The build therefore reads the generated ISA of those kernels and fails if any instruction
-# touches the destination of such a read before the next s_waitcnt lgkmcnt(0), and says so if the compiler is not the
-# version the kernels were written and measured with.
-CHECK_LDS_READS = {"grouped_gemm.hip": re.compile(r"grouped_gemm")}
+# The grouped GEMM kernels read their fragments from LDS, and some of their row indices from memory, with inline assembly and
+# wait for them by hand: between such a load and its wait the compiler takes the destination registers for ordinary values
+# (or, if nothing uses them, for free ones), and whatever it does with them there meets data that arrives later.  The build
+# therefore reads the generated ISA of those kernels and fails if any instruction that a path of the program leads to touches
+# the destination of such a load before the wait, or if a loop of MFMAs without an inner loop accesses scratch memory (spills;
+# those outside such loops are reported with the kernel's registers).  It also says so if the compiler is not the version the
+# kernels were written and measured with.
+CHECK_ISA = {"grouped_gemm.hip": re.compile(r"grouped_gemm")}
 TESTED_HIPCC = "7.2"
 USAGE_REPORT = os.path.join(HERE, "build", "kernel_resource_usage.txt")
 
@@ -51,28 +53,107 @@ def _registers(operands: str) -> set[str]:
     return regs
 
 
-def _touched_in_flight(asm_path: str, which: re.Pattern) -> list[str]:
-    """instructions of the kernels matching `which` that touch the destination of an inline-assembly ds_read before the wait
-    behind it (followed in program order; a block that is only jumped to starts with nothing in flight)"""
-    bad, name, in_asm, flight = [], None, False, set()
+class _Block:
+    """basic block of a kernel: (line number, opcode, operands, inside inline assembly, text) per instruction, the indices of
+    its successors, and the registers with a load in flight at its entry"""
+
+    def __init__(self):
+        self.code, self.succ, self.flight = [], [], frozenset()
+
+
+def _kernels(asm_path: str, which: re.Pattern):
+    """(name, basic blocks in program order) of the kernels of a device ISA listing whose names match `which`"""
+    name, blocks, labels, in_asm = None, [], {}, False
     with open(asm_path) as f:
         for n, line in enumerate(f, 1):
-            m = re.match(r"^(_Z\w+):", line)
-            if m:
-                name, flight = (m.group(1) if which.search(m.group(1)) else None), set()
+            label = re.match(r"^(_Z\w+|\.LBB\w+|\.Lfunc_end\w+):", line)
+            if label and not label.group(1).startswith(".LBB"):
+                if name:
+                    for i, b in enumerate(blocks):
+                        op, target = b.code[-1][1:3] if b.code else ("", "")
+                        b.succ = [labels[target.strip()]] if op.startswith(("s_branch", "s_cbranch")) else []
+                        if op not in ("s_branch", "s_endpgm", "s_setpc_b64") and i + 1 < len(blocks):
+                            b.succ.append(i + 1)
+                    yield name, blocks
+                name = label.group(1) if which.search(label.group(1)) else None
+                blocks, labels, in_asm = [_Block()], {}, False
+                continue
             text = line.strip()
             if text.startswith(";;#ASM"):
                 in_asm = text.startswith(";;#ASMSTART")
-            if not name or not text or text[0] in ";." or text.endswith(":"):
+            if label and name:
+                if blocks[-1].code:
+                    blocks.append(_Block())
+                labels[label.group(1)] = len(blocks) - 1
+            elif name and text and text[0] not in ";.":
+                op, _, operands = re.sub(r"\s+", " ", text.split(";")[0]).partition(" ")
+                blocks[-1].code.append((n, op, operands, in_asm, text))
+                if op.startswith(("s_branch", "s_cbranch", "s_endpgm", "s_setpc")):
+                    blocks.append(_Block())
+
+
+def _touched_in_flight(blocks: list[_Block]) -> list[str]:
+    """instructions that touch the destination of an inline-assembly load from LDS or memory on some path before the wait
+    behind it (s_waitcnt lgkmcnt(0) or vmcnt(0)); fills in the blocks' `flight`"""
+
+    def walk(block, bad):
+        flight = set(block.flight)
+        for n, op, operands, in_asm, text in block.code:
+            if op == "s_waitcnt":
+                done = [c for c, wait in (("ds", "lgkmcnt(0)"), ("global", "vmcnt(0)")) if wait in operands]
+                flight = {f for f in flight if f[0] not in done}
                 continue
-            op, _, operands = text.split(";")[0].partition(" " if " " in text.split("\t")[0] else "\t")
-            if op == "s_waitcnt" and "lgkmcnt(0)" in operands or op in ("s_branch", "s_endpgm", "s_setpc_b64"):
-                flight.clear()
-            elif in_asm and op.startswith("ds_read"):
-                flight |= _registers(operands.split(",")[0])
-            elif flight & _registers(operands):
-                bad.append(f"{name} line {n}: {text}")
+            regs = _registers(operands) if flight or in_asm else ()
+            if any((c, r) in flight for r in regs for c in ("ds", "global")):
+                bad.append((n, text))
+            if in_asm and (op.startswith("ds_read") or op.startswith("global_load") and "_lds" not in op):
+                flight |= {(op.split("_")[0], r) for r in _registers(operands.split(",")[0])}
+        return frozenset(flight)
+
+    todo = list(range(len(blocks)))
+    while todo:
+        block = blocks[todo.pop()]
+        out = walk(block, [])
+        for s in block.succ:
+            if not out <= blocks[s].flight:
+                blocks[s].flight |= out
+                todo.append(s)
+    bad: list[tuple[int, str]] = []
+    for block in blocks:
+        walk(block, bad)
+    return [f"line {n}: {text}" for n, text in sorted(bad)]
+
+
+def _scratch_in_mfma_loops(blocks: list[_Block]) -> list[str]:
+    """scratch accesses in the loops that contain MFMAs and no inner loop"""
+    pred: list[list[int]] = [[] for _ in blocks]
+    for i, block in enumerate(blocks):
+        for s in block.succ:
+            pred[s].append(i)
+    loops: dict[int, set[int]] = {}
+    for tail, block in enumerate(blocks):
+        for head in block.succ:
+            if head <= tail:
+                body, todo = loops.setdefault(head, {head}), [tail]
+                while todo:
+                    i = todo.pop()
+                    if i not in body:
+                        body.add(i)
+                        todo += pred[i]
+    bad = []
+    for head, body in loops.items():
+        code = [c for i in sorted(body) for c in blocks[i].code]
+        if not any(h != head and h in body for h in loops) and any(c[1].startswith("v_mfma") for c in code):
+            bad += [f"line {c[0]}: {c[4]}" for c in code if c[1].startswith("scratch_")]
     return bad
+
+
+def _check_isa(asm_path: str, which: re.Pattern) -> None:
+    for name, blocks in _kernels(asm_path, which):
+        for what, bad in (("registers touched while a load into them is in flight", _touched_in_flight(blocks)),
+                          ("scratch accesses inside an MFMA loop", _scratch_in_mfma_loops(blocks))):
+            if bad:
+                raise RuntimeError(f"{what}, {name}:\n  " + "\n  ".join(bad[:10]))
 
 
 def _resource_usage_from_asm(asm_path: str) -> dict[str, dict[str, str]]:
@@ -130,7 +211,7 @@ def _check_compiler(verbose: bool) -> None:
 def _compile(src: str, verbose: bool, defines: tuple[str, ...] = (), tag: str = "") -> str:
     obj = os.path.join(HERE, "build", src.replace(".hip", tag + ".o"))
     # keeps the device ISA next to the object (named after the source, so only the untagged build of a file may do this)
-    extra = ["-save-temps=obj"] if src in CHECK_LDS_READS and not tag else []
+    extra = ["-save-temps=obj"] if src in CHECK_ISA and not tag else []
     cmd = [HIPCC, *FLAGS, *extra, *defines, "-c", os.path.join(CSRC, src), "-o", obj]
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -145,9 +226,7 @@ def _compile(src: str, verbose: bool, defines: tuple[str, ...] = (), tag: str = 
         print(err, file=sys.stderr)
     if extra:
         asm = os.path.join(HERE, "build", src.replace(".hip", "-hip-amdgcn-amd-amdhsa-gfx950.s"))
-        bad = _touched_in_flight(asm, CHECK_LDS_READS[src])
-        if bad:
-            raise RuntimeError(f"{src}: registers touched while an LDS read into them is in flight:\n  " + "\n  ".join(bad[:10]))
+        _check_isa(asm, CHECK_ISA[src])
         usage = _resource_usage_from_asm(asm)
     return obj, usage
 

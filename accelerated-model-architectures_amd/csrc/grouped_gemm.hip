@@ -1010,6 +1010,9 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_kernel(const Fwd
         if constexpr (NI == 4)
             for (; kt + 2 < KT_full; ++kt) k_step(kt, IC<1>{});
         for (; kt < kt1; ++kt) k_step(kt, IC<0>{});
+        // The last sub-step reads ahead for a step that does not exist.  Nobody uses these fragments, so the compiler would
+        // take their registers, to move the accumulators where the four loops meet, while the reads are in flight.
+        wait_frags(f0);
     };
     if (q_blocks > 2)
         main_loop(IC<4>{});
@@ -1019,8 +1022,8 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_kernel(const Fwd
         main_loop(IC<1>{});
     else
         main_loop(IC<0>{});
-    // every load has landed, every fragment read has returned (the last sub-step reads ahead into registers nobody
-    // uses), and no wave touches the operand tiles any more: LDS becomes the staging area of the epilogue
+    // every load has landed, every fragment read has returned, and no wave touches the operand tiles any more: LDS becomes
+    // the staging area of the epilogue
     XMA_WAIT_LOADS_AND_BARRIER();
 
     if constexpr (ROLE == ROLE_SLICES) {
@@ -1787,6 +1790,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_dw_kernel(const 
         int kt = 0;
         for (; kt + 2 < KT_full; ++kt) k_step(kt, IC<1>{});
         for (; kt < KT; ++kt) k_step(kt, IC<0>{});
+        wait_frags(f0); // read ahead and not used: see the forward kernel
         XMA_WAIT_ALL_LOADS();
         DW_STAMP(2);
     }
