@@ -5,7 +5,7 @@
 namespace {
 
 constexpr int CS_COLS = 128;                   // columns per workgroup: a wave reads 256 (fp32: 512) contiguous bytes of a row
-constexpr int CS_UNROLL = 8;                   // rows a wave has in flight
+constexpr int CS_UNROLL = 4;                   // rows a wave has in flight
 
 template <typename T> struct Pair; // two neighbouring elements of a row as floats
 template <> struct Pair<float> {
@@ -39,10 +39,13 @@ template <> struct Pair<_Float16> {
 // fixed order (per wave in row order, then the waves in order), so the result does not depend on timing.  Experts
 // without rows get zeros.
 // A workgroup walks its expert's rows in steps of one round trip to memory each.  Launches of few workgroups are bound by
-// these, so they get 16 waves with 8 rows in flight, 128 rows a step (measured against 4 waves with 4 rows: 16 experts,
-// 8198 rows of 1024 / 4096 columns 18.3 -> 7.0 / 37.5 -> 14.5 us; 8 experts, 16384 rows of 4096: 131 -> 44 us).  From four
-// workgroups per CU on, 4 waves each fill the chip, and the larger workgroups only wait for their own last waves (128
-// experts, 1000 rows of 4096 columns: 5.6 us with 4 waves, 10.1 with 16; 8 experts, 16384 rows of 28672: 241 and 260).
+// these, so they get 16 waves with 4 rows in flight, 64 rows a step (measured against 4 waves with 4 rows: 16 experts of 300
+// rows, 1024 / 4096 columns 11.3 -> 4.5 / 22.9 -> 8.8 us; of 4096 rows, 4096 columns 384 -> 127).  From four workgroups per CU
+// on, 4 waves each fill the chip, and the larger workgroups only wait for their own last waves (2048 workgroups of 16 / 300
+// rows: 3.0 / 26.4 us with 4 waves, 5.7 / 28.3 with 16; of 1024 rows 126 / 129).  With up to 16 rows per expert, one step or
+// less, the larger workgroups cost 0.1 to 0.3 us of 2 to 2.4; the host does not know the number of rows.  8 rows in flight
+// instead of 4 are slower on both sides (16 waves, 512 workgroups of 4096 rows 140 against 127 us; 4 waves, 2048 workgroups
+// of 1024 rows 139 against 126).
 constexpr int CS_FEW_BLOCKS = 1024;
 template <typename T, int CS_PHASES>
 __global__ __launch_bounds__(CS_PHASES * WAVE) void expert_column_sums_kernel(const void *__restrict__ A, int64_t lda,

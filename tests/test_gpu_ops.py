@@ -204,7 +204,7 @@ def test_scatter2scatter_bias_and_expert_column_sums(dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("counts,N", [((0, 1, 127, 128, 129, 700), 130), ((3,) * 511 + (40,), 256), ((3,) * 512, 254)])
+@pytest.mark.parametrize("counts,N", [((0, 1, 127, 128, 129, 700), 130), ((15, 17, 63, 0, 64, 65), 258), ((3,) * 511 + (40,), 256), ((3,) * 512, 254)])
 def test_expert_column_sums_block_sizes(dtype, counts, N):
     """both workgroup sizes (below and from 1024 workgroups on), experts around the rows of one step, a partial column block"""
     from xma.rocm import ops
