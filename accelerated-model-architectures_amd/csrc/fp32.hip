@@ -426,23 +426,22 @@ template <int WT, int TB> int launch_gemm(const FwdArgs &a, int epi, int grid, s
     return xma_check_launch("gemm_f32_kernel");
 }
 
-// Which tile: a launch is bound by the matrix pipes of the compute units that have a tile, so it takes the small one until
-// the large one fills the chip several times over, and with up to 64 rows per expert on average, where the large one is
-// mostly padding.  Results are bit-identical.  Measured, large / small tile in us (x @ W^T; dy @ W; both of the forward and
-// dX GEMMs of H x I experts):  8 experts of 256 x 512, 1024 rows 29 / 18; 83 / 30, 32768 rows (2048 large tiles) 213 / 224;
-// 221 / 185;  8 of 512 x 1024, 4096 rows 129 / 125; 163 / 129, 16384 rows (2048 tiles) 364 / 381; 420 / 359;  128 of
-// 576 x 256, 56 rows 52 / 32; 45 / 27, 65536 rows (2048 and 2560 tiles) 418 / 450; 433 / 424.
-constexpr int F32_SMALL_TILES = 2048;
-// dW: the reduction is the expert's rows, so the small tile pays only where the large ones leave compute units idle.  128
-// tiles: 8 experts of 256 x 512, dW1, 1024 / 32768 rows 18.5 -> 12.3 / 464 -> 233 us; 256 tiles: dW2 of 512 x 1024, 16384
-// rows 202 -> 167; 512 tiles: dW1 337 -> 365, so not there.
+// Which tile: a launch is bound by the matrix pipes of the compute units that have a tile.  The small one pays where the large
+// one is mostly padding, up to 64 rows per expert on average, and where the large ones leave compute units idle, below two
+// per unit.  Results are bit-identical.  Measured, large / small tile in us (x @ W^T; dy @ W).  Padding: 64 experts of
+// K = 1024, N = 2048, 30 rows each 302 / 184; 285 / 178, 64 rows 287 / 188; 288 / 186, 70 rows 292 / 291; 288 / 288.  Tiles:
+// 128 of them 45 / 30; 45 / 28, 256 48 / 49; 47 / 46, 384 78 / 69; 80 / 69, 512 80 / 85; 81 / 85 (K = 512) and 163 / 184;
+// 157 / 179 (64 experts of 128 rows, K = 1024), 1024 156 / 170; 150 / 164, 2048 297 / 322; 290 / 322.
+constexpr int64_t F32_SMALL_ROWS = 64, F32_SMALL_TILES = 512;
+// dW: the reduction is the expert's rows.  64 large tiles 476 / 194, 256 125 / 97, 384 655 / 553, 2560 72 / 80, 4096 1150 / 1378.
 constexpr int F32_SMALL_TILES_DW = 512;
 inline int64_t f32_tiles(int64_t m, int64_t n, int dim) { return ((m + dim - 1) / dim) * ((n + dim - 1) / dim); }
 
 } // namespace
 
 int f32_scatter2scatter(const FwdArgs &a, int w_is_kn, int epilogue, hipStream_t st) {
-    const bool small = a.M <= (int64_t)64 * a.E || f32_tiles(a.M, a.N, 128) < F32_SMALL_TILES;
+    const int64_t rows = (a.M + a.E - 1) / a.E; // of an expert, on average
+    const bool small = rows <= F32_SMALL_ROWS || a.E * f32_tiles(rows, a.N, 128) < F32_SMALL_TILES;
     const int dim = small ? 64 : 128;
     const int64_t grid = (a.M / dim + a.E) * ((a.N + dim - 1) / dim); // sum_e ceil(c_e / dim) <= floor(M / dim) + E
     XMA_REQUIRE(grid < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "scatter2scatter (fp32): grid too large");
