@@ -427,28 +427,40 @@ __device__ __forceinline__ void add_bias(const FwdArgs &a, f32x16 (&acc)[4][4], 
         for (int i = 0; i < 4; ++i) acc[j][i] = Elem<T>::mfma(p[j], q, acc[j][i]);
 }
 
-// The accumulators of a tile set to its expert's bias, or to zero without one, by sixteen MFMAs of that rank-one product
-// onto a constant zero: the matrix pipe clears the 256 registers in half the cycles that 256 register writes take.
-template <typename T, typename Hook>
-__device__ __forceinline__ void init_acc(const FwdArgs &a, f32x16 (&acc)[4][4], int e, int n0, int wp, int lane, Hook hook) {
-    const bool k0 = lane < 32;
-    const u32x4 q = {k0 ? one_bits<T>() : 0u, 0u, 0u, 0u};
-    uint32_t v[4] = {0u, 0u, 0u, 0u};
+// The bias of this lane's four columns, zeros without one.  The values are used inside the branch, so that the wait for them
+// stands there and covers loads that are older; behind it the compiler knows of no load to wait for.
+struct Bias {
+    uint32_t v[4];
+};
+__device__ __forceinline__ Bias load_bias(const FwdArgs &a, int e, int n0, int wp, int lane) {
+    Bias r = {{0u, 0u, 0u, 0u}};
     if (a.bias != nullptr) { // uniform
         const uint16_t *b = a.bias + (int64_t)e * a.bias_es;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             int col = n0 + wp + 32 * j + (lane & 31);
             if (col >= a.N) col = a.N - 1;
-            v[j] = b[col];
+            r.v[j] = b[col];
         }
+        asm volatile("" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]));
     }
+    return r;
+}
+
+// The accumulators of a tile set to its expert's bias, or to zero without one, by MFMAs of that rank-one product onto a
+// constant zero.  The blocks of a column block j have the same operands, so four MFMAs are left of the sixteen, and the first
+// MFMA of each block reads one of their results as its addend: no register is written on its own.  The hook's loads are
+// placed between them.
+template <typename T, typename Hook>
+__device__ __forceinline__ void init_acc(const Bias &bias, f32x16 (&acc)[4][4], int lane, Hook hook) {
+    const bool k0 = lane < 32;
+    const u32x4 q = {k0 ? one_bits<T>() : 0u, 0u, 0u, 0u};
     f32x16 zero;
 #pragma unroll
     for (int c = 0; c < 16; ++c) zero[c] = 0.f;
     static_for<16>([&](auto S) {
         constexpr int j = S.value >> 2, i = S.value & 3;
-        const u32x4 p = {k0 ? v[j] : 0u, 0u, 0u, 0u};
+        const u32x4 p = {k0 ? bias.v[j] : 0u, 0u, 0u, 0u};
         __builtin_amdgcn_sched_barrier(0);
         acc[j][i] = Elem<T>::mfma(p, q, zero);
         __builtin_amdgcn_sched_barrier(0);
@@ -1415,6 +1427,8 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
         asm volatile("" : "+v"(tid));
         const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         wave_u = wave, lane_v = lane;
+        const int wq = (wave & 1) * 128, wp = (wave >> 1) * 128;
+        const Bias bias = load_bias(a, cur.e, cur.n0, wp, lane); // behind the first K step: the wait is one for both
         // the first K step and the rows of this tile's epilogue have landed in every wave, the stores of the last
         // epilogue have been handed over and its staging area is dead
         asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
@@ -1425,7 +1439,6 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
         // 192 rows with an even number of at least four complete K steps does this between the MFMAs of its first K step,
         // sets up and loads the first K step of the next tile in its last one
         // (`ovl`); any other tile does it here and behind the loop, with idle matrix pipes.
-        const int wq = (wave & 1) * 128, wp = (wave >> 1) * 128;
         const int q_blocks = (cur.rows_valid > wq) ? (cur.rows_valid - wq + 31) >> 5 : 0;
         // uniform over the workgroup: the waves of a tile's lower half (wq == 0) and upper half disagree on q_blocks, so
         // the decision is taken on the tile's row count
@@ -1449,7 +1462,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
         // half in the first phase of the loop: sixteen in a row would hold up the first MFMAs until the texture unit has
         // taken them all.
         f32x16 acc[4][4];
-        init_acc<T>(a, acc, cur.e, cur.n0, wp, lane, [&](auto S) {
+        init_acc<T>(bias, acc, lane, [&](auto S) {
             constexpr k_schedule::Load l = k_schedule::load_before_loop(S.value);
             if constexpr (l.piece >= 0) issue_piece(l.ahead, IC<l.piece>{}, OVL);
         });
