@@ -1387,6 +1387,19 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
     };
     auto ordered = [](auto P) { return IC<k_schedule::ordered(P.value)>{}; };
 
+    // From here on the offsets are those of the last K step of a tile that overlaps: chunks past K lie outside the buffers.
+    // (The loads of such a tile do not check; the next tile's offsets are made in that step.)
+    auto cut_tail = [&]() {
+        if (!k_tail) return;
+        const int k_left = a.K - (KT - 1) * BK;
+        static_for<8>([&](auto I) {
+            constexpr int i = I.value;
+            const bool in_row = rowmajor_lane_chunk(i, lane_v) * 8 < k_left;
+            q_off[i] = in_row ? q_off[i] : BUF_OUTSIDE;
+            p_off[i] = (WT == 0 ? in_row : half_krow(wave_u, i) + (lane_v >> 4) < k_left) ? p_off[i] : BUF_OUTSIDE;
+        });
+    };
+
     // ---- first tile: its gathered rows are fetched on the spot, the rows of its epilogue go the way of all later ones
     PstTile cur;
     int e_buf = 0; // which of the two epilogue-row buffers holds the current tile's
@@ -1436,13 +1449,13 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
 
         // One tile ahead: the next tile's schedule entry and rows, and this tile's row scales (their addresses are the
         // epilogue's row indices, fetched a tile ago); all of it lands in LDS during the main loop.  A tile of more than
-        // 192 rows with an even number of at least four complete K steps does this between the MFMAs of its first K step,
+        // 192 rows with an even number of at least four K steps does this between the MFMAs of its first K step,
         // sets up and loads the first K step of the next tile in its last one
         // (`ovl`); any other tile does it here and behind the loop, with idle matrix pipes.
         const int q_blocks = (cur.rows_valid > wq) ? (cur.rows_valid - wq + 31) >> 5 : 0;
         // uniform over the workgroup: the waves of a tile's lower half (wq == 0) and upper half disagree on q_blocks, so
         // the decision is taken on the tile's row count
-        const bool ovl = cur.rows_valid > 128 + 64 && (KT & 1) == 0 && KT >= 4 && !k_tail && ovl_allowed;
+        const bool ovl = cur.rows_valid > 128 + 64 && (KT & 1) == 0 && KT >= 4 && ovl_allowed;
         PstTile nxt = {0, 0, 0, 0, 0, 0};
         if (!ovl) {
             nxt = entry(cur.n + 1);
@@ -1530,9 +1543,11 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
             };
             if constexpr (OVL.value != 0) {
                 k_step(0, pA, pB, IC<k_schedule::OVL_FIRST>{});
+                if (KT == 4) cut_tail();
                 k_step(1, pB, pA, IC<k_schedule::OVL_SECOND>{});
                 for (int kt = 2; kt < KT - 2; kt += 2) {
                     k_step(kt, pA, pB, IC<k_schedule::STEADY>{});
+                    if (kt == KT - 4) cut_tail(); // the next step loads the last one
                     k_step(kt + 1, pB, pA, IC<k_schedule::STEADY>{});
                 }
                 k_step(KT - 2, pA, pB, IC<k_schedule::OVL_DRAIN>{});

@@ -809,3 +809,30 @@ def test_fp32_tiles(counts, K, N):
     dw = torch.full((E, N, K), float("nan"), device="cuda")
     ops.group_bwd_W_rocm(DY.cuda(), X.cuda(), ssd, offsd, dw.permute(0, 2, 1), None, 0, 1)
     assert nerr(dw.permute(0, 2, 1), oracle.group_bwd_W(DY, X[ss], offs, E)) <= TOL_F32
+
+
+@pytest.mark.parametrize("K", [200, 232, 328, 456, 1000])
+@pytest.mark.parametrize("w_kn", [False, True])
+def test_scatter2scatter_k_tail_of_overlapping_tiles(K, w_kn):
+    """Four to sixteen K steps with a partial last one, tiles of more than 192 rows one after another on a workgroup (which load
+    the next tile's first step inside their last one) and a smaller one among them: whatever lies past K in memory is NaN."""
+    from xma.rocm import ops
+
+    counts, N, pad = (2300, 150, 2305, 2048), 2568, 64
+    E, M = len(counts), sum(counts)
+    print(f"K tail K={K} w_kn={w_kn}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    X = torch.full((M, K + pad), float("nan"), device="cuda", dtype=torch.bfloat16)
+    X[:, :K] = torch.randn(M, K, generator=g, device="cuda")
+    W = torch.full((E, K + pad, N) if w_kn else (E, N, K + pad), float("nan"), device="cuda", dtype=torch.bfloat16)
+    Wv = W[:, :K] if w_kn else W[..., :K].permute(0, 2, 1)
+    Wv.copy_(torch.randn(E, K, N, generator=g, device="cuda") * 0.1)
+    out = torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+    idx = torch.randperm(M, generator=g, device="cuda")
+    ops.scatter2scatter_rocm(X[:, :K], Wv, idx, torch.tensor(counts).cumsum(0).cuda(), out, None, 1, False, True)
+    row = 0
+    for e, c in enumerate(counts):
+        want = X[idx[row : row + c], :K].float() @ Wv[e].float()
+        err = (out[row : row + c].float() - want).abs().max() / want.abs().max()
+        assert err <= 2.0**-8, e  # rounding to bf16: half a unit in the last place, 2^-9 of the value
+        row += c
