@@ -836,3 +836,30 @@ def test_scatter2scatter_k_tail_of_overlapping_tiles(K, w_kn):
         err = (out[row : row + c].float() - want).abs().max() / want.abs().max()
         assert err <= 2.0**-8, e  # rounding to bf16: half a unit in the last place, 2^-9 of the value
         row += c
+
+
+@pytest.mark.parametrize("counts", [(17,) * 1000, (0,) * 400 + (16990,) + (0,) * 598 + (10,)])
+@pytest.mark.parametrize("w_kn", [False, True])
+def test_scatter2scatter_walk_refills_its_table(counts, w_kn):
+    """Launches of more than 256 candidate tiles for each of 256 workgroups, (M / 256 + E) column blocks in all: a workgroup
+    looks for its tiles 256 candidates at a time, and the second table holds tiles (even counts) or none (two experts with
+    rows).  bf16 products of 64 terms, so the result is the rounded fp32 sum."""
+    from xma.rocm import ops
+
+    E, M, K, N = len(counts), sum(counts), 64, 67 * 256 - 8
+    assert (M // 256 + E) * 67 > 256 * 256 and M > ops.FEW_ROWS_MAX
+    print(f"walk refill E={E} M={M} N={N} w_kn={w_kn}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    X = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    W = torch.randn(E, *((K, N) if w_kn else (N, K)), generator=g, device="cuda", dtype=torch.bfloat16)
+    out = torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+    idx = torch.randperm(M, generator=g, device="cuda")
+    Wv = W if w_kn else W.permute(0, 2, 1)
+    ops.scatter2scatter_rocm(X, Wv, idx, torch.tensor(counts).cumsum(0).cuda(), out, None, 1, False, True)
+    row = 0
+    for e, c in enumerate(counts):
+        if c:
+            want = X[idx[row : row + c]].float() @ Wv[e].float()
+            err = (out[row : row + c].float() - want).abs().max() / want.abs().max()
+            assert err <= 2.0**-8, e  # rounding to bf16: half a unit in the last place, 2^-9 of the value
+        row += c
