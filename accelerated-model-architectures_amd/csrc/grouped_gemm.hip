@@ -1861,9 +1861,11 @@ template <typename T, int WT, int EPI> int launch_fwd(const FwdArgs &a, hipStrea
     int rc;
     const int cus = device_cus();
     // The persistent kernel fetches a row scale as the aligned dword around it and addresses the operands of a tile with
-    // 32-bit byte offsets from a uniform base: 256 rows of W or of a grouped X, any row of a gathered X.
+    // 32-bit byte offsets from a uniform base: 256 rows of W or of a grouped X, any row of a gathered X, any row scale (the
+    // dword of the last one has to end within the 2^32 - 16 bytes of a buffer, or it reads zeros).
     const int64_t x_rows = a.x_grouped ? 256 : (a.M + a.fan_out - 1) / a.fan_out;
-    const bool offsets_fit = x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)256 * a.ldw * 2 < ((int64_t)1 << 32);
+    const bool offsets_fit = x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)256 * a.ldw * 2 < ((int64_t)1 << 32) &&
+                             (!a.scale || 2 * a.M <= (int64_t)0xfffffff0);
     // The persistent kernel exists for the operand layouts the layer launches: x @ W^T with any epilogue, dy @ W with a
     // plain store or the SwiGLU backward.  (dy @ W with the SwiGLU forward epilogue, reachable through the C ABI only,
     // would be the one instantiation whose register allocation spills inside the K loop.)
