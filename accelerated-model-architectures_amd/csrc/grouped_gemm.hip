@@ -180,9 +180,7 @@ __device__ __forceinline__ void load_frags(Frags &f, const FragBase<PTR> &pb, co
 // slower, although an isolated instruction-mix benchmark prefers them).  NI < 4: only the first NI of the wave's four
 // 32-wide Q blocks hold valid rows; the MFMAs and fragment reads of the others are left out.
 constexpr int MMA_GROUP = 2;
-// READ_NEXT = 0: no fragment reads (the last sub-step of a tile whose hooks hold compiler-generated code: fragments read
-// ahead there would never be used, so the compiler would treat their registers as free while the reads are in flight).
-template <typename T, int PTR, int QTR, int KK, int NI = 4, int READ_NEXT = 1, typename Hook>
+template <typename T, int PTR, int QTR, int KK, int NI = 4, typename Hook>
 __device__ __forceinline__ void mma_step(Frags &cur, Frags &nxt, const FragBase<PTR> &pb, const FragBase<QTR> &qb,
                                          f32x16 (&acc)[4][4], Hook hook) {
     wait_frags(cur); // issued at least 8 MFMAs ago
@@ -199,7 +197,7 @@ __device__ __forceinline__ void mma_step(Frags &cur, Frags &nxt, const FragBase<
         __builtin_amdgcn_sched_barrier(0);
         // fragment reads: 8 (4 P, 4 Q) over the first SLOTS / 2 slots
         constexpr int RPS = 16 / SLOTS; // reads per slot of the first half
-        if constexpr (t < SLOTS / 2 && READ_NEXT != 0) {
+        if constexpr (t < SLOTS / 2) {
             static_for<RPS>([&](auto R) {
                 constexpr int r = t * RPS + R.value, f = r >> 1;
                 if constexpr ((r & 1) == 0) {
@@ -1113,9 +1111,9 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_fixup_kernel(con
 constexpr int PST_MAX_E = 1023;
 constexpr int PST_SMEM_BYTES = 160 * 1024 - 64;
 constexpr int PST_STAGING_OFF = STAGE_CHUNKS * 16; // the epilogue's staging area starts above stage 0
-// Rows fetched one tile ahead wait in LDS, one dword per lane and item (1 KB per item), so that no register is held
-// across the main loop: 8 gathered rows of the next tile, 2 x 4 rows of the epilogue (next tile's arrive while this
-// tile's are still needed), 4 row scales of this tile.
+// Rows fetched one tile ahead wait in LDS, one dword per row and wave, so that no register is held across the main loop.
+// An item is 64 rows of each wave (1 KB): one of gathered rows of the next tile, 2 x 2 of rows of the epilogue (the next
+// tile's arrive while this tile's are still needed), two of row scales of this tile.
 constexpr int PST_ROWS_OFF = PST_STAGING_OFF + 4 * EPI_BWD_WAVE_BYTES;
 constexpr int PST_QR = 0, PST_ER = 1, PST_SC = 5, PST_ROW_ITEMS = 7;
 constexpr int PST_TABLE_OFF = PST_SMEM_BYTES - 2 * (PST_MAX_E + 1) * (int)sizeof(int);
@@ -1867,8 +1865,8 @@ template <typename T, int WT, int EPI> int launch_fwd(const FwdArgs &a, hipStrea
     const bool offsets_fit = x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)256 * a.ldw * 2 < ((int64_t)1 << 32) &&
                              (!a.scale || 2 * a.M <= (int64_t)0xfffffff0);
     // The persistent kernel exists for the operand layouts the layer launches: x @ W^T with any epilogue, dy @ W with a
-    // plain store or the SwiGLU backward.  (dy @ W with the SwiGLU forward epilogue, reachable through the C ABI only,
-    // would be the one instantiation whose register allocation spills inside the K loop.)
+    // plain store or the SwiGLU backward.  (dy @ W with the SwiGLU forward epilogue is reachable through the C ABI only: not
+    // worth another 120 KB of code per type.)
     constexpr bool persistent_variant = !(WT == 1 && EPI == XMA_ROCM_EPI_SWIGLU);
     bool persistent = false;
     if constexpr (persistent_variant) {

@@ -573,6 +573,8 @@ __global__ __launch_bounds__(128 * KS) void router_gate_topk_lds_kernel(const ui
 // RF_MAX_TOKENS, one workgroup per CU (at E = 128, H = 2048 twice as many take as long as the kernel above).
 // Measured against the kernels above, us: E = 128, H = 576, 7 tokens 14.3 -> 7.8; E = 64, H = 2048, 64 tokens 22.6 -> 11.9;
 // E = 8, H = 4096, 1 / 3001 tokens 7.7 -> 5.2 / 13.7 -> 8.7; 4096 tokens 14.4 -> 8.9 (E = 8), 23.1 -> 13.0 (64), 28.8 -> 20.7 (128).
+// Also where most waves have no step, 4096 tokens of H = 64 / 512: E = 8 3.9 -> 2.8 / 4.9 -> 3.4, E = 32 4.2 -> 3.1 / 5.7 -> 4.2,
+// E = 64 11.9 -> 4.0 / 14.3 -> 5.7, E = 128 13.6 -> 4.9 / 16.8 -> 8.2.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int RF_TOKENS = 16, RF_WAVES = 16;
 constexpr int64_t RF_MAX_TOKENS = 4096;

@@ -17,6 +17,7 @@
  *   - leading dimensions (ld*) and expert strides are in ELEMENTS;
  *   - "grouped" order = position n in the expert-sorted list; "scattered" order
  *     = row sorted_scattered_idxs[n] of the flattened (T, k) selection.
+ *     Indices and ids number fewer than 2^31 (xma_rocm_route refuses more): the kernels divide indices by fan_out in 31 bits.
  *
  * Citations are to the reference tree (xma/...), which each entry point replaces.
  */
