@@ -1093,9 +1093,9 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_fixup_kernel(con
 //
 // Between two main loops a workgroup has to find its next tile, fetch the scattered row indices, and wait for the first
 // K step to arrive from HBM: three dependent round trips with idle matrix pipes, as long as the epilogue itself.  Here
-// everything a tile needs is fetched one tile ahead: while tile i is in its main loop the schedule entry, the gathered
-// row indices and the epilogue's indices of tile i + 1 are loaded into registers, and the 16 LDS-DMA pieces of the first
-// K step of tile i + 1 go out right behind the last barrier of tile i's main loop, before its epilogue starts.  They land
+// everything a tile needs is fetched one tile ahead: while tile i is in its main loop the entry of tile i + 1 is read from
+// the table of the workgroup's tiles and its row indices go into LDS, and the 16 LDS-DMA pieces of its first K step go out
+// in the last step of tile i or right behind its main loop, before its epilogue starts.  They land
 // in stage 0 while the epilogue stages its rows in the LDS above it (stage 1 and the 32 KB that the two stages leave
 // free), so the next main loop starts as soon as the epilogue's stores have been handed over.
 //

@@ -49,12 +49,12 @@ WORKLOADS = {
 # run; the roofline block carries the one of the kernel it names.
 MEASURED_TRAFFIC_BYTES = {
     "c3": {
-        "up_swiglu": 8.79e9,  # 7.38 GB fetched + 1.41 GB written (3.42 GB algorithmic)
-        "down": 3.74e9,  # three launches: whole tiles, K slices of the last round, their sum
-        "dx2_swiglu_bwd": 6.51e9,
+        "up_swiglu": 15.04e9,  # 13.54 GB fetched + 1.51 GB written (3.42 GB algorithmic)
+        "down": 5.03e9,  # three launches: whole tiles, K slices of the last round, their sum
+        "dx2_swiglu_bwd": 8.74e9,
         "dw2": 3.76e9,
         "dw1": 7.52e9,  # 5.64 GB fetched + 1.88 GB written (2.95 GB algorithmic)
-        "dx1": 7.59e9,  # three launches
+        "dx1": 10.80e9,  # three launches
     },
     "c2": 92.2e6,  # route: unit histogram 18.9 MB + scan 0.6 MB + scatter 72.7 MB (36.1 MB fetched + 56.1 MB written)
 }
