@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT_DIR = os.path.join(HERE, "xma", "rocm")
 LIB = os.path.join(OUT_DIR, "libxma_rocm.so")
-SOURCES = ["api.hip", "routing.hip", "elementwise.hip", "grouped_gemm.hip", "grouped_gemm_staged.hip", "fp32.hip", "router.hip", "swiglu.hip", "bias.hip", "few_rows.hip", "diagnostics.hip"]
+SOURCES = ["api.hip", "routing.hip", "elementwise.hip", "grouped_gemm.hip", "mid_rows.hip", "grouped_gemm_staged.hip", "fp32.hip", "router.hip", "swiglu.hip", "bias.hip", "few_rows.hip", "diagnostics.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -41,7 +41,7 @@ FLAGS = [
 # the destination of such a load before the wait, or if a loop of MFMAs without an inner loop accesses scratch memory (spills;
 # those outside such loops are reported with the kernel's registers).  It also says so if the compiler is not the version the
 # kernels were written and measured with.
-CHECK_ISA = {"grouped_gemm.hip": re.compile(r"grouped_gemm")}
+CHECK_ISA = {"grouped_gemm.hip": re.compile(r"grouped_gemm"), "mid_rows.hip": re.compile(r"mid_\w+_kernel")}
 TESTED_HIPCC = "7.2"
 USAGE_REPORT = os.path.join(HERE, "build", "kernel_resource_usage.txt")
 
@@ -58,7 +58,7 @@ class _Block:
     its successors, and the registers with a load in flight at its entry"""
 
     def __init__(self):
-        self.code, self.succ, self.flight = [], [], frozenset()
+        self.code, self.succ, self.flight = [], [], {}
 
 
 def _kernels(asm_path: str, which: re.Pattern):
@@ -94,29 +94,35 @@ def _kernels(asm_path: str, which: re.Pattern):
 
 def _touched_in_flight(blocks: list[_Block]) -> list[str]:
     """instructions that touch the destination of an inline-assembly load from LDS or memory on some path before the wait
-    behind it (s_waitcnt lgkmcnt(0) or vmcnt(0)); fills in the blocks' `flight`"""
+    behind it: s_waitcnt lgkmcnt(0) for LDS; for memory, where loads and stores retire in order, vmcnt(n) with at least n
+    memory instructions behind the load on every path.  Fills in the blocks' `flight`: {(class, register): memory
+    instructions behind the load, at least}"""
 
     def walk(block, bad):
-        flight = set(block.flight)
+        flight = dict(block.flight)
         for n, op, operands, in_asm, text in block.code:
             if op == "s_waitcnt":
-                done = [c for c, wait in (("ds", "lgkmcnt(0)"), ("global", "vmcnt(0)")) if wait in operands]
-                flight = {f for f in flight if f[0] not in done}
+                vm = re.search(r"vmcnt\((\d+)\)", operands)
+                younger = int(vm.group(1)) if vm else 1 << 30
+                flight = {f: c for f, c in flight.items() if ("lgkmcnt(0)" not in operands if f[0] == "ds" else c < younger)}
                 continue
             regs = _registers(operands) if flight or in_asm else ()
             if any((c, r) in flight for r in regs for c in ("ds", "global")):
                 bad.append((n, text))
+            if op.startswith(("global_", "buffer_load", "buffer_store", "buffer_atomic", "scratch_", "flat_")):
+                flight = {f: c if f[0] == "ds" else min(c + 1, 64) for f, c in flight.items()}
             if in_asm and (op.startswith("ds_read") or op.startswith("global_load") and "_lds" not in op):
-                flight |= {(op.split("_")[0], r) for r in _registers(operands.split(",")[0])}
-        return frozenset(flight)
+                flight |= {(op.split("_")[0], r): 0 for r in _registers(operands.split(",")[0])}
+        return flight
 
     todo = list(range(len(blocks)))
     while todo:
         block = blocks[todo.pop()]
         out = walk(block, [])
         for s in block.succ:
-            if not out <= blocks[s].flight:
-                blocks[s].flight |= out
+            merged = {f: min(c, blocks[s].flight.get(f, c)) for f, c in out.items()}
+            if any(blocks[s].flight.get(f) != c for f, c in merged.items()):
+                blocks[s].flight = blocks[s].flight | merged
                 todo.append(s)
     bad: list[tuple[int, str]] = []
     for block in blocks:

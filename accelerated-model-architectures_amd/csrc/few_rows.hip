@@ -5,7 +5,7 @@
 // load instruction, many short workgroups per compute unit; vector FMAs for one or two rows per expert, small MFMA tiles
 // beyond.  Correct for any number of rows, but the forward-type kernels stream the weights once per 32 rows of an expert:
 // the caller picks these entry points by the number of rows per expert.
-#include "gemm_common.hpp"
+#include "mid_rows.hpp"
 
 namespace {
 
@@ -176,6 +176,7 @@ extern "C" int xma_rocm_group_bwd_W_few_rows(const void *DY, int64_t lddy, int d
     a.dy_div = make_fastdiv((uint32_t)dy_fan_out);
     a.x_div = make_fastdiv((uint32_t)x_fan_out);
     hipStream_t st = (hipStream_t)stream;
+    if (M > (int64_t)MID_ROWS_DW_FROM * E && xma_rocm::mid_dw_takes(a, M)) return xma_rocm::mid_dw(a, dtype, st);
     const bool wide = M > 0 && M <= (int64_t)DW_WIDE_ROWS_PER_EXPERT * E;
     const int TN = wide ? 64 : 128, TK = 16384 / TN;
     const dim3 grid((K_in + TK - 1) / TK, (N_out + TN - 1) / TN, E);
@@ -389,12 +390,12 @@ __global__ __launch_bounds__(FR_THREADS) void fr_epilogue_kernel(const FwdArgs a
 }
 
 // ------------------------------------------------------------------------------------------------
-// 3 to 128 rows per expert: too many for vector FMAs (one pass over the weights per 4 or 8 rows), too few for the
-// 256 x 256 tiles (one 32 KB stage of weights in flight per compute unit).  A small MFMA tile instead: 32 (or 128) rows of
-// the expert x 128 output columns, operands through registers into 40 (64) KB of LDS, so that four (two) workgroups
-// share a compute unit and keep 80 (128) KB of loads in flight.  One v_mfma_f32_32x32x16 block per wave; lane l holds 16 sums of row l % 32 in
+// 3 to 24 rows per expert: too many for vector FMAs (one pass over the weights per 4 or 8 rows), too few for the larger
+// tiles (64 KB or less of weights in flight per compute unit, two or three times the columns).  A small MFMA tile instead: 32
+// rows of the expert x 128 output columns, operands through registers into 40 KB of LDS, so that four workgroups
+// share a compute unit and keep 80 KB of loads in flight.  One v_mfma_f32_32x32x16 block per wave; lane l holds 16 sums of row l % 32 in
 // quads of 4 consecutive columns, so bias, row scale and the epilogues are lane-local, with the arithmetic of
-// tile_epilogue in grouped_gemm.hip.  An expert's rows are taken 32 or 128 at a time.  Every load instruction of a workgroup
+// tile_epilogue in grouped_gemm.hip.  An expert's rows are taken 32 at a time.  Every load instruction of a workgroup
 // asks for 256 contiguous bytes per row of memory (128-byte pieces of 128 rows of W measured 4.4 TB/s, 256-byte pieces
 // the 5.6 TB/s of a copy):
 //   WT = 0, W[e] as (N, K): K in steps of 128; the W tile is [128 n][128 k] in one LDS stage, read back with ds_read_b128
@@ -416,11 +417,9 @@ __device__ __forceinline__ int st_slot_nt(int row, int chunk) { return row * 256
 
 // EPI = -1: the launch is cut along K (blockIdx.z takes `steps_per` steps) because N alone gives too few workgroups; the
 // fp32 sums go to part[blockIdx.z][M][N] and fr_epilogue_kernel finishes.
-// MB = 32-row blocks of the expert per pass (1 or 4): the weights are streamed once per pass.
-template <typename T, int WT, int EPI, int MB>
-__global__ __launch_bounds__(FR_THREADS, MB == 1 ? 4 : 2) void fr_tile_kernel(const FwdArgs a, float *__restrict__ part, int steps_per) {
-    constexpr int X_BYTES = MB * ST_X_BYTES, STAGE = ST_W_BYTES + X_BYTES; // WT = 1, per stage
-    __shared__ __attribute__((aligned(16))) unsigned char s_t[WT == 0 ? ST_W_BYTES_NT + 2 * X_BYTES : 2 * STAGE];
+template <typename T, int WT, int EPI>
+__global__ __launch_bounds__(FR_THREADS, 4) void fr_tile_kernel(const FwdArgs a, float *__restrict__ part, int steps_per) {
+    __shared__ __attribute__((aligned(16))) unsigned char s_t[WT == 0 ? ST_W_BYTES_NT + 2 * ST_X_BYTES : 2 * ST_STAGE];
     typedef short v4s __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) v4s *lds_v4s;
     const int e = blockIdx.y;
@@ -457,26 +456,24 @@ __global__ __launch_bounds__(FR_THREADS, MB == 1 ? 4 : 2) void fr_tile_kernel(co
         const int m = wave * 32 + ((G & 1) << 4) + ((p & 3) << 2), kr = ((G >> 1) << 3) + (p >> 2);
         w_frag = kr * 256 + ((((m >> 3) ^ ((kr & 3) << 2))) << 4) + ((m & 7) << 1);
     }
-    for (int64_t r0 = lo; r0 < hi; r0 += MB * ST_M) {
-        f32x16 acc[MB];
+    for (int64_t r0 = lo; r0 < hi; r0 += ST_M) {
+        f32x16 acc;
 #pragma unroll
-        for (int b = 0; b < MB; ++b)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
         const u32x4 zero = {0u, 0u, 0u, 0u};
         if constexpr (WT == 0) {
-            const uint16_t *x_src[2 * MB];
+            const uint16_t *x_src[2];
 #pragma unroll
-            for (int i = 0; i < 2 * MB; ++i) {
+            for (int i = 0; i < 2; ++i) {
                 int64_t xr = r0 + kn_row + 16 * i;
                 if (xr >= hi) xr = hi - 1;
                 x_src[i] = a.X + fr_src_row(a, xr) * a.ldx + 8 * kn_chunk;
             }
-            u32x4 wv[8], xv[2 * MB];
+            u32x4 wv[8], xv[2];
             auto fetch = [&](int s) {
                 const bool ok = s * ST_K_NT + 8 * kn_chunk < a.K; // chunks past K are zeros
 #pragma unroll
-                for (int i = 0; i < 2 * MB; ++i) xv[i] = ok ? *(const u32x4 *)(x_src[i] + s * ST_K_NT) : zero;
+                for (int i = 0; i < 2; ++i) xv[i] = ok ? *(const u32x4 *)(x_src[i] + s * ST_K_NT) : zero;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) wv[i] = ok ? __builtin_nontemporal_load((const u32x4 *)(w_base + (size_t)s * (ST_K_NT * 2) + w_off[i])) : zero;
             };
@@ -497,7 +494,7 @@ __global__ __launch_bounds__(FR_THREADS, MB == 1 ? 4 : 2) void fr_tile_kernel(co
 #pragma unroll
                 for (int i = 0; i < 8; ++i) *(u32x4 *)(s_t + slot_st + 16 * 256 * i) = wv[i]; // rows + 16 i: the same rotation
 #pragma unroll
-                for (int i = 0; i < 2 * MB; ++i) *(u32x4 *)(s_t + ST_W_BYTES_NT + slot_st + 16 * 256 * i) = xv[i];
+                for (int i = 0; i < 2; ++i) *(u32x4 *)(s_t + ST_W_BYTES_NT + slot_st + 16 * 256 * i) = xv[i];
                 __syncthreads();
                 s_at = next_step(s_at);
                 if (done + 1 < n_steps) fetch(s_at); // in flight while this step is multiplied
@@ -505,22 +502,15 @@ __global__ __launch_bounds__(FR_THREADS, MB == 1 ? 4 : 2) void fr_tile_kernel(co
                 for (int kk = 0; kk < 8; ++kk) {
                     const int slot = st_slot_nt(row_rd, 2 * kk + half);
                     const u32x4 wa = *(const u32x4 *)(s_t + wave * (32 * 256) + slot);
-#pragma unroll
-                    for (int b = 0; b < MB; ++b) acc[b] = Elem<T>::mfma(wa, *(const u32x4 *)(s_t + ST_W_BYTES_NT + b * (32 * 256) + slot), acc[b]);
+                    acc = Elem<T>::mfma(wa, *(const u32x4 *)(s_t + ST_W_BYTES_NT + slot), acc);
                 }
             }
         } else {
-            const uint16_t *x_src[MB];
-#pragma unroll
-            for (int b = 0; b < MB; ++b) {
-                int64_t xr = r0 + ld_row + 32 * b;
-                if (xr >= hi) xr = hi - 1;
-                x_src[b] = a.X + fr_src_row(a, xr) * a.ldx + 8 * ld_chunk;
-            }
-            u32x4 wv[4], xv[MB];
+            const int64_t xr = r0 + ld_row < hi ? r0 + ld_row : hi - 1;
+            const uint16_t *x_src = a.X + fr_src_row(a, xr) * a.ldx + 8 * ld_chunk;
+            u32x4 wv[4], xv;
             auto fetch = [&](int s) {
-#pragma unroll
-                for (int b = 0; b < MB; ++b) xv[b] = (s * ST_K + 8 * ld_chunk < a.K) ? *(const u32x4 *)(x_src[b] + s * ST_K) : zero; // chunks past K are zeros
+                xv = (s * ST_K + 8 * ld_chunk < a.K) ? *(const u32x4 *)(x_src + s * ST_K) : zero; // chunks past K are zeros
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const bool ok = kn_ok && s * ST_K + kn_row + 16 * i < a.K;
@@ -528,11 +518,10 @@ __global__ __launch_bounds__(FR_THREADS, MB == 1 ? 4 : 2) void fr_tile_kernel(co
                 }
             };
             auto stash = [&](int stage) {
-                unsigned char *base = s_t + stage * STAGE;
+                unsigned char *base = s_t + stage * ST_STAGE;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) *(u32x4 *)(base + st_slot_kn(kn_row + 16 * i, kn_chunk)) = wv[i];
-#pragma unroll
-                for (int b = 0; b < MB; ++b) *(u32x4 *)(base + ST_W_BYTES + st_slot(ld_row + 32 * b, ld_chunk)) = xv[b];
+                *(u32x4 *)(base + ST_W_BYTES + st_slot(ld_row, ld_chunk)) = xv;
             };
             __syncthreads(); // the pass before no longer reads the stages
             fetch(s_begin);
@@ -540,49 +529,45 @@ __global__ __launch_bounds__(FR_THREADS, MB == 1 ? 4 : 2) void fr_tile_kernel(co
             __syncthreads();
             for (int s = s_begin; s < s_end; ++s) {
                 if (s + 1 < s_end) fetch(s + 1); // in flight while this step computes
-                unsigned char *base = s_t + (s & 1) * STAGE;
+                unsigned char *base = s_t + (s & 1) * ST_STAGE;
 #pragma unroll
                 for (int kk = 0; kk < 4; ++kk) { // k-rows 16 kk + ..: the swizzle depends on kr & 3 only, so kk adds 16 rows = 4096 bytes
                     const v4s k03 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(base + w_frag + kk * 4096));
                     const v4s k47 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(base + w_frag + kk * 4096 + 1024));
                     const u32x2 a01 = __builtin_bit_cast(u32x2, k03), a23 = __builtin_bit_cast(u32x2, k47);
                     const u32x4 wa = u32x4{a01[0], a01[1], a23[0], a23[1]};
-#pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        acc[b] = Elem<T>::mfma(wa, *(const u32x4 *)(base + ST_W_BYTES + st_slot(l32 + 32 * b, 2 * kk + half)), acc[b]);
+                    acc = Elem<T>::mfma(wa, *(const u32x4 *)(base + ST_W_BYTES + st_slot(l32, 2 * kk + half)), acc);
                 }
                 if (s + 1 < s_end) stash((s + 1) & 1); // that stage was last read in step s - 1, behind a barrier
                 __syncthreads();
             }
         }
-#pragma unroll
-        for (int b = 0; b < MB; ++b) {
-            const int64_t r = r0 + 32 * b + l32;
-            if (r >= hi) continue;
+        const int64_t r = r0 + l32;
+        if (r < hi) {
             if constexpr (EPI < 0) {
                 float *mine = part + ((int64_t)blockIdx.z * a.M + r) * a.N;
-    #pragma unroll
+#pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const int n = n0 + wave * 32 + 8 * g + 4 * half;
-                    if (n < a.N) *(float4 *)(mine + n) = make_float4(acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]);
+                    if (n < a.N) *(float4 *)(mine + n) = make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
                 }
                 continue;
             }
             const int64_t s_idx = a.idx ? a.idx[r] : r;
             const float sc = a.scale ? fr_scalar<T>(a.scale, s_idx) : 1.f;
             const int64_t dst = a.y_grouped ? r : s_idx;
-    #pragma unroll
+#pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int n = n0 + wave * 32 + 8 * g + 4 * half; // acc[b][4 g + q] is column n + q of row r
+                const int n = n0 + wave * 32 + 8 * g + 4 * half; // acc[4 g + q] is column n + q of row r
                 if (n >= a.N) continue;
                 if constexpr (EPI == XMA_ROCM_EPI_SWIGLU_BWD) {
                     // d h of 4 columns -> (d gate, d up) of their 4 pairs; rows are grouped on both sides
                     const u32x4 z = *(const u32x4 *)(a.aux + r * a.ldaux + 2 * n);
                     u32x4 o;
                     float hv[4];
-    #pragma unroll
+#pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        const float dh = acc[b][4 * g + q] * sc;
+                        const float dh = acc[4 * g + q] * sc;
                         const float gg = Elem<T>::lo(z[q]), uu = Elem<T>::hi(z[q]);
                         const float sg = sigmoidf_fast(gg), silu = gg * sg;
                         o[q] = Elem<T>::pack(dh * uu * (sg + silu * (1.f - sg)), dh * silu);
@@ -592,9 +577,9 @@ __global__ __launch_bounds__(FR_THREADS, MB == 1 ? 4 : 2) void fr_tile_kernel(co
                     if (a.aux2) *(u32x2 *)(a.aux2 + r * a.ldaux2 + n) = u32x2{Elem<T>::pack(hv[0], hv[1]), Elem<T>::pack(hv[2], hv[3])};
                 } else {
                     float v[4];
-    #pragma unroll
+#pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        v[q] = acc[b][4 * g + q];
+                        v[q] = acc[4 * g + q];
                         if (a.bias) v[q] += fr_scalar<T>(a.bias, (int64_t)e * a.bias_es + n + q);
                         v[q] *= sc;
                     }
@@ -617,10 +602,12 @@ inline bool fr_takes_tile(int64_t M, int K, int E, int w_is_kn) {
     return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE;
 }
 
-// passes of 128 rows once many experts have more than 32: two workgroups per compute unit instead of four (registers
-// and 64 KB of LDS), 3-10 % slower than passes of 32 rows where those suffice; passes of 64 rows and three workgroups were
-// no faster than these anywhere
-inline int fr_tile_row_blocks(int64_t M, int E) { return M > (int64_t)24 * E ? 4 : 1; }
+// More rows than the small tile takes in one pass go to the 128 x 256 tiles of mid_rows.hip, where those have the variant.  8
+// experts of H = 2048, I = 8192, 32 rows each, up- / down-projection: 132 -> 102 / 61 -> 55 us against a small tile of 128 rows that
+// stood here; 128 experts of H = 2048, I = 768, 64 rows: 190 -> 166 / 103 -> 90.
+inline bool fr_takes_mid(const FwdArgs &a, int w_is_kn, int epilogue) {
+    return a.M > (int64_t)MID_ROWS_FWD_FROM * a.E && xma_rocm::mid_fwd_takes(a, w_is_kn, epilogue);
+}
 
 // K ranges of the small MFMA tile: enough workgroups for two per compute unit of a 256-CU device, ranges of at least 512
 // columns of K.  Measured (8 experts, 16 rows each, down-projection / dX1 / dX2): 1024 workgroups 61 / 99 / 57 us, 512
@@ -640,23 +627,19 @@ template <typename T, int EPI> int fr_launch_epilogue(const FwdArgs &a, const fl
     return xma_check_launch("fr_epilogue_kernel");
 }
 
-template <typename T, int WT, int EPI, int MB> int fr_launch_tile_mb(const FwdArgs &a, float *part, hipStream_t st) {
+template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, float *part, hipStream_t st) {
     const int S_max = fr_tile_splits(a.N, a.K, a.E, WT);
     const int steps_all = (a.K + st_k(WT) - 1) / st_k(WT), steps_per = (steps_all + S_max - 1) / S_max;
     const int S = (steps_all + steps_per - 1) / steps_per; // ranges that hold a step (25 steps in 6 ranges of 5: only 5 do)
     const dim3 grid((a.N + ST_N - 1) / ST_N, a.E, S);
     if (S == 1) {
-        fr_tile_kernel<T, WT, EPI, MB><<<grid, FR_THREADS, 0, st>>>(a, nullptr, steps_all);
+        fr_tile_kernel<T, WT, EPI><<<grid, FR_THREADS, 0, st>>>(a, nullptr, steps_all);
         return xma_check_launch("fr_tile_kernel");
     }
-    fr_tile_kernel<T, WT, -1, MB><<<grid, FR_THREADS, 0, st>>>(a, part, steps_per);
+    fr_tile_kernel<T, WT, -1><<<grid, FR_THREADS, 0, st>>>(a, part, steps_per);
     int rc = xma_check_launch("fr_tile_kernel");
     if (rc) return rc;
     return fr_launch_epilogue<T, EPI>(a, part, S, st);
-}
-
-template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, float *part, hipStream_t st) {
-    return fr_tile_row_blocks(a.M, a.E) == 4 ? fr_launch_tile_mb<T, WT, EPI, 4>(a, part, st) : fr_launch_tile_mb<T, WT, EPI, 1>(a, part, st);
 }
 
 template <typename T, int EPI> int fr_launch_epi(const FwdArgs &a, int w_is_kn, float *part, hipStream_t st) {
@@ -683,19 +666,32 @@ template <typename T> int fr_launch(const FwdArgs &a, int w_is_kn, int epilogue,
 
 } // namespace
 
+int split_sums_epilogue(const FwdArgs &a, const float *part, int S, int epilogue, int dtype, hipStream_t st) {
+    auto run = [&](auto elem) {
+        using T = decltype(elem);
+        if (epilogue == XMA_ROCM_EPI_STORE) return fr_launch_epilogue<T, XMA_ROCM_EPI_STORE>(a, part, S, st);
+        if (epilogue == XMA_ROCM_EPI_SWIGLU) return fr_launch_epilogue<T, XMA_ROCM_EPI_SWIGLU>(a, part, S, st);
+        return fr_launch_epilogue<T, XMA_ROCM_EPI_SWIGLU_BWD>(a, part, S, st);
+    };
+    return dtype == XMA_ROCM_BF16 ? run(__bf16{}) : run(_Float16{});
+}
+
 extern "C" size_t xma_rocm_scatter2scatter_few_rows_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E, int w_is_kn,
                                                                     int epilogue) {
     if (M <= 0 || N <= 0 || K <= 0 || E <= 0) return 0;
+    // (the 128 x 256 tiles may turn out not to take the launch: then it runs through the small tile, so the larger of the two)
+    const size_t mid = M > (int64_t)MID_ROWS_FWD_FROM * E ? xma_rocm::mid_fwd_workspace_bytes(M, N, K, E) : 0;
     int S;
     if (fr_takes_tile(M, K, E, w_is_kn)) { // the small MFMA tile, cut along K or not
         S = fr_tile_splits(N, K, E, w_is_kn);
-        if (S == 1) return 0;
+        if (S == 1) return mid;
     } else if (epilogue == XMA_ROCM_EPI_SWIGLU_BWD) {
         S = 1; // the vector kernel's sums go to the epilogue kernel
     } else {
-        return 0; // the vector kernel finishes the job itself
+        return mid; // the vector kernel finishes the job itself
     }
-    return (size_t)S * (size_t)M * (size_t)N * sizeof(float);
+    const size_t few = (size_t)S * (size_t)M * (size_t)N * sizeof(float);
+    return few > mid ? few : mid;
 }
 
 extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, const void *W, int64_t w_expert_stride,
@@ -765,6 +761,7 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
     a.split_cus = 0;
     a.grid_main = 0;
     hipStream_t st = (hipStream_t)stream;
+    if (fr_takes_mid(a, w_is_kn ? 1 : 0, epilogue)) return xma_rocm::mid_fwd(a, w_is_kn ? 1 : 0, epilogue, dtype, (float *)workspace, st);
     if (dtype == XMA_ROCM_BF16) return fr_launch<__bf16>(a, w_is_kn ? 1 : 0, epilogue, (float *)workspace, st);
     return fr_launch<_Float16>(a, w_is_kn ? 1 : 0, epilogue, (float *)workspace, st);
 }

@@ -1,0 +1,22 @@
+// Grouped GEMMs of 128 x 256 tiles (mid_rows.hip): argument checks are the callers'.
+#pragma once
+
+#include "gemm_common.hpp"
+
+// Rows per expert on average beyond which the few-row entry points take these kernels (measured in few_rows.hip).
+constexpr int MID_ROWS_FWD_FROM = 24, MID_ROWS_DW_FROM = 40;
+
+namespace xma_rocm {
+
+// whether the kernels have the variant and can address the operands
+bool mid_fwd_takes(const FwdArgs &a, int w_is_kn, int epilogue);
+bool mid_dw_takes(const DwArgs &a, int64_t M);
+// fp32 sums of the K ranges of a launch with few tiles; 0: not cut
+size_t mid_fwd_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E);
+int mid_fwd(const FwdArgs &a, int w_is_kn, int epilogue, int dtype, float *part, hipStream_t st);
+int mid_dw(const DwArgs &a, int dtype, hipStream_t st);
+
+} // namespace xma_rocm
+
+// few_rows.hip: adds the S parts part[S][M][N] in order and applies bias, scale and the epilogue of `a`
+int split_sums_epilogue(const FwdArgs &a, const float *part, int S, int epilogue, int dtype, hipStream_t st);

@@ -357,7 +357,7 @@ class _FusedSwiGLUExperts(torch.autograd.Function):
             ops.down_projection_dx_swiglu_rocm(
                 grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, flat_w, top_k
             )
-            if b_proj is None and ops._few_rows(z.size(0), w_proj.size(0), z.dtype, "dW"):
+            if b_proj is None and ops._dw_loader_scales(z.size(0), w_proj.size(0), z.dtype):
                 # a handful of rows per expert: the weight gradient's loader gathers and scales the rows of dy itself (and
                 # rounds them like the copy would), one launch less
                 ops.group_bwd_W_rocm(grad_out, h, sorted_scattered_idxs, expert_offsets, d_w_proj, flat_w, top_k, 0)

@@ -102,6 +102,17 @@ CONTINUOUS_COUNT_SET_MAX_BINS = 8192
 FEW_ROWS_PER_EXPERT = {"x @ W^T": 96, "dy @ W": 96, "dW": 128}
 FEW_ROWS_MAX = 16384  # rows in all, every form (beyond the measured range; 0 switches the few-token entry points off)
 FEW_ROWS_MAX_WORKSPACE = 256 << 20  # bytes of fp32 partial sums a forward-type launch may ask for
+# Beyond these limits the same entry points lead a while longer with 128 x 256 tiles, two workgroups per compute unit, where the
+# 256 x 256 tiles spend their time at the tiles' edges.  Forward-type GEMMs up to 352 rows per expert (64 experts of H = 2048, I =
+# 1408, 256 rows, dX2 208 -> 170 us; 400 rows: equal), 112 where K is long (8 experts of H = 4096, I = 14336, 176 rows, dX1, K =
+# 28672: 470 us with 256 x 256 tiles, 544 without), and where even those tiles are at most two per compute unit and K is short
+# (8 experts of H = 512, I = 1024, 512 rows: down-projection 37 -> 19 us, dX1 50 -> 31).  dW up to 640 rows per expert (64 experts, 256
+# rows, dW1 403 -> 269; 512 rows 557 -> 440), or where it has at most one 256 x 256 tile per compute unit (2048 rows of the
+# small layer: 49 -> 42).
+MID_ROWS_PER_EXPERT, MID_ROWS_PER_EXPERT_LONG_K, MID_ROWS_LONG_K = 352, 112, 8192
+MID_ROWS_FEW_TILES, MID_ROWS_FEW_TILES_K = 512, 2048
+MID_ROWS_MAX = 65535  # rows in all, limit of the forward-type entry point
+MID_ROWS_PER_EXPERT_DW, MID_ROWS_FEW_TILES_DW = 640, 256
 
 
 @torch.library.custom_op("xma_rocm::continuous_count_set", mutates_args={"y"})
@@ -187,9 +198,43 @@ def _few_rows(M: int, E: int, dtype: torch.dtype, form: str) -> bool:
     return 0 < M <= min(FEW_ROWS_MAX, FEW_ROWS_PER_EXPERT[form] * E) and dtype in (torch.bfloat16, torch.float16)
 
 
-def _few_rows_fwd(M: int, N: int, K: int, E: int, w_is_kn: int, ldw: int, dtype: torch.dtype, epilogue: int) -> bool:
+MID_ROWS_MAX_EXPERTS, MID_ROWS_OFFSETS = 1024, 1 << 31  # 32-bit byte offsets: elements from a base to the end of an operand
+
+
+def _mid_rows_fwd(M: int, N: int, K: int, E: int, w_is_kn: int, ldw: int, x_span: int, dtype: torch.dtype, epilogue: int) -> bool:
+    """whether a forward-type GEMM of more rows than `_few_rows` allows takes the same entry point, for its 128 x 256 tiles (x_span:
+    elements from X's first row to the end of its last)"""
+    if not 0 < M <= MID_ROWS_MAX or FEW_ROWS_MAX == 0 or dtype not in (torch.bfloat16, torch.float16):
+        return False
+    # what the tiles cover: the layouts that the layer launches, offsets that fit
+    if epilogue != EPI_STORE and w_is_kn != (epilogue == EPI_SWIGLU_BWD):
+        return False
+    if E > MID_ROWS_MAX_EXPERTS or x_span >= MID_ROWS_OFFSETS or 256 * ldw >= MID_ROWS_OFFSETS:
+        return False
+    if M <= (MID_ROWS_PER_EXPERT if K <= MID_ROWS_LONG_K else MID_ROWS_PER_EXPERT_LONG_K) * E:
+        return True
+    return K <= MID_ROWS_FEW_TILES_K and (M // 256 + E // 2) * -(-N // 256) <= MID_ROWS_FEW_TILES
+
+
+def _mid_rows_dw(M: int, N_out: int, K_in: int, E: int, dtype: torch.dtype) -> bool:
+    """the same for the weight gradient (of operands that are not both gathered, unscaled)"""
+    if M <= 0 or FEW_ROWS_MAX == 0 or dtype not in (torch.bfloat16, torch.float16) or max(E, -(-N_out // 32)) > 65535:
+        return False
+    return M <= MID_ROWS_PER_EXPERT_DW * E or E * -(-N_out // 256) * -(-K_in // 256) <= MID_ROWS_FEW_TILES_DW
+
+
+def _dw_loader_scales(M: int, E: int, dtype: torch.dtype) -> bool:
+    """whether dW2 gathers and scales the rows of dy in its loader, which the small tile of dW does and the larger ones do not;
+    the scaled grouped copy costs a launch and pays from about 64 rows per expert on (8 experts of H = 2048, I = 8192: 64 rows 61
+    against 57 + 4 us, 96 rows 76 against 63 + 4)"""
+    return _few_rows(M, E, dtype, "dW") and M <= 64 * E
+
+
+def _few_rows_fwd(M: int, N: int, K: int, E: int, w_is_kn: int, ldw: int, x_span: int, dtype: torch.dtype, epilogue: int) -> bool:
     """the same for a forward-type GEMM, whose few-token entry point has limits of its own"""
-    if not _few_rows(M, E, dtype, "dy @ W" if w_is_kn else "x @ W^T"):
+    if not _few_rows(M, E, dtype, "dy @ W" if w_is_kn else "x @ W^T") and not _mid_rows_fwd(
+        M, N, K, E, w_is_kn, ldw, x_span, dtype, epilogue
+    ):
         return False
     if not w_is_kn and N * ldw >= FEW_ROWS_NT_MAX_ELEMENTS:  # it addresses the rows of W[e] with 32-bit byte offsets
         return False
@@ -225,7 +270,7 @@ def _scatter2scatter(X, W, idx, offs, out, aux, scale, fan_out, x_grouped, y_gro
     if scale is not None:
         assert scale.dtype == X.dtype and scale.is_contiguous()
     lib = get_library()
-    if _few_rows_fwd(M, N, K, W.size(0), w_is_kn, ldw, X.dtype, epilogue):
+    if _few_rows_fwd(M, N, K, W.size(0), w_is_kn, ldw, X.size(0) * X.stride(0), X.dtype, epilogue):
         _scatter2scatter_few_rows(lib, X, W, w_is_kn, w_es, ldw, idx, offs, out, aux, None, scale, bias, fan_out, x_grouped,
                                   y_grouped, epilogue, M, N, K)
         return
@@ -330,7 +375,7 @@ def down_projection_dx_swiglu_scaled_act_rocm(
     w_is_kn, w_es, ldw = _weight_layout(W)
     assert w_is_kn == 1, "W should be the down-projection parameter as stored, (E, H, I) with I contiguous"
     lib = get_library()
-    if _few_rows_fwd(M, N, K, E, 1, ldw, dY.dtype, EPI_SWIGLU_BWD):
+    if _few_rows_fwd(M, N, K, E, 1, ldw, dY.size(0) * dY.stride(0), dY.dtype, EPI_SWIGLU_BWD):
         _scatter2scatter_few_rows(lib, dY, W, 1, w_es, ldw, sorted_scattered_idxs, expert_offsets, dz, z, scaled_act,
                                   row_scale, None, FAN_OUT, False, True, EPI_SWIGLU_BWD, M, N, K)
         return
@@ -368,9 +413,13 @@ def group_bwd_W_rocm(
     if dy_scale is not None:
         assert dy_scale.dtype == DY.dtype and dy_scale.is_contiguous()
     lib = get_library()
-    # a handful of rows per expert (the index has one entry per row): the launch is a stream of stores, not arithmetic
+    # a handful of rows per expert (the index has one entry per row): the launch is a stream of stores, not arithmetic; some
+    # hundreds: the same entry point, for its 128 x 256 tiles where they cover the operands
     M = sorted_scattered_idxs.numel()
-    few = _few_rows(M, E, DW.dtype, "dW")
+    few = _few_rows(M, E, DW.dtype, "dW") or (
+        dy_scale is None and 0 in (dy_fan_out, x_fan_out) and _mid_rows_dw(M, N_out, K_in, E, DW.dtype)
+        and max(DY.size(0) * DY.stride(0), X.size(0) * X.stride(0)) < MID_ROWS_OFFSETS
+    )
     name = "xma_rocm_group_bwd_W_few_rows" if few else "xma_rocm_group_bwd_W"
     operands = (
         _ptr(DY), _rows(DY, "DY"), int(dy_fan_out == 0), max(dy_fan_out, 1), _ptr(dy_scale),

@@ -201,16 +201,18 @@ XMA_API int xma_rocm_down_projection_dx_swiglu(const void *dY, int64_t lddy, con
  * (aux2 = the scaled activations of the latter, or NULL), the same results up to the order of the fp32 sums, bf16 / fp16
  * only.  With a handful of rows per expert the product is a stream over the weights.  W[e] as (N, K), up to 2 rows per
  * expert on average (and 64 in all), K at least 2048: vector FMAs, a wave reads two rows of W with its lanes along K.
- * Everything else: a small MFMA tile (32 rows of the expert x 128 output columns and four workgroups per compute unit,
- * or 128 rows and two from 24 rows per expert on average), cut along K where N alone gives too few workgroups.
+ * Everything else: a small MFMA tile (32 rows of the expert x 128 output columns, four workgroups per compute unit), and
+ * from 24 rows per expert on average 128 x 256 tiles, two workgroups per compute unit (x @ W^T with a plain store or SwiGLU,
+ * dy @ W with a plain store or the SwiGLU backward, E at most 1024, operands within 32-bit byte offsets; the small tile
+ * otherwise), both cut along K where N alone gives too few workgroups.
  * Whatever does not finish in one kernel sums through the workspace (xma_rocm_scatter2scatter_few_rows_workspace_bytes
  * bytes for the same M, N, K, num_experts, w_is_kn and epilogue; 0 = none needed, pass NULL) to a small kernel that
  * applies the bias and the epilogue with the arithmetic of the MFMA kernels.  Limits: M and E at most 65535, N * ldw
  * below 2^31 - 128 elements for W as (N, K) (32-bit byte offsets inside an expert).
- * Correct for any M, but an expert's rows are walked 4 (vector kernel), 32 or 128 (small tile) at a time, each pass
- * streaming its weights again: meant for launches of a few rows per expert (the torch ops of this package take it up to
- * 96 on average, 48 with the SwiGLU backward, and 16384 in all).  No counterpart in the reference (its kernel is the
- * same for every size).
+ * Correct for any M, but an expert's rows are walked 4 (vector kernel), 32 (small tile) or 128 at a time, each pass
+ * streaming its weights again: meant for launches of up to some hundreds of rows per expert (the torch ops of this package
+ * take it up to 352 on average, 112 where K is beyond 8192, and beyond that where a launch has few tiles).  No counterpart
+ * in the reference (its kernel is the same for every size).
  */
 XMA_API size_t xma_rocm_scatter2scatter_few_rows_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t num_experts,
                                                          int w_is_kn, int epilogue);
@@ -244,12 +246,13 @@ XMA_API int xma_rocm_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped, i
  * xma_rocm_group_bwd_W for the few-token regime (same arguments and limits plus M, same result up to the order of the
  * fp32 sums; bf16 / fp16 only; a scaled row of DY is rounded to the operand type before it is multiplied, as a scaled
  * grouped copy would hold it).  M = rows in all (the length of the grouped order), which picks the shape of a
- * workgroup's tile of DW[e]: 64 x 256 up to 24 rows per expert on average, 128 x 128 beyond or when M <= 0 (not known).
- * The expert's rows are the K dimension of the tile's MFMAs, 32 at a time: with a handful of rows per expert the launch
+ * workgroup's tile of DW[e]: 64 x 256 up to 24 rows per expert on average, 128 x 128 beyond or when M <= 0 (not known), and from
+ * 40 rows on 128 x 256, two workgroups per compute unit, where nothing is scaled and at most one operand is gathered.  In the
+ * first two the expert's rows are the K dimension of the tile's MFMAs, 32 at a time: with a handful of rows per expert the launch
  * runs at the rate of a fill of DW, where xma_rocm_group_bwd_W spends a prologue, one K step and an epilogue per
- * 256 x 256 tile.  Correct for any number of rows; more rows are more passes over two small operand tiles, so it leads
- * until the loads outweigh the stores (the torch ops take it up to 128 rows per expert on average).  No counterpart in
- * the reference (its kernel is the same for every size).
+ * 256 x 256 tile.  Correct for any number of rows; more rows are more passes over small operand tiles, so it leads
+ * until the loads outweigh the stores (the torch ops take it up to 128 rows per expert on average, 640 with the larger tiles, and
+ * beyond that where DW has few tiles).  No counterpart in the reference (its kernel is the same for every size).
  */
 XMA_API int xma_rocm_group_bwd_W_few_rows(const void *DY, int64_t lddy, int dy_grouped, int32_t dy_fan_out,
                                   const void *dy_scale, const void *X, int64_t ldx, int x_grouped, int32_t x_fan_out,

@@ -1,0 +1,94 @@
+"""The 128 x 256 tiles that the few-row entry points take beyond 24 (forward-type) and 40 (dW) rows per expert, at the edges of
+their tiles, K steps and ranges, each against the CPU oracle and the 256 x 256 kernels on the same operands."""
+
+import pytest
+import torch
+
+from oracle import moe as oracle
+
+from .test_gpu_ops import _few_rows_limit, _tol
+from .utils import nerr
+
+
+pytestmark = pytest.mark.gpu
+
+# rows per expert, K, N: one tile and one row more, 32- and 64-row blocks of the waves, empty experts, a K step and its tail, K ranges
+# (few tiles, long K), one and several column tiles with clamped columns, more experts than lanes, and more than two chunks of them
+CASES = [
+    ([25], 8, 8),
+    ([128, 129, 0, 32, 33, 127], 72, 264),
+    ([64, 65, 0, 97], 64, 256),
+    ([300, 0, 1], 200, 136),
+    ([260] * 8, 1024, 512),
+    ([90, 31], 4096, 256),
+    ([40 + e for e in range(70)], 136, 24),
+    ([e % 37 * 7 for e in range(140)], 192, 256),
+]
+
+
+def _both(fn, outs):
+    """fn() with the 256 x 256 kernels and through the few-row entry points, all outputs poisoned in between"""
+    res = []
+    for limit in (0, 65535):
+        for o in outs:
+            o.fill_(float("nan"))
+        with _few_rows_limit(limit):
+            fn()
+        torch.cuda.synchronize()
+        res.append([o.clone() for o in outs])
+    return zip(*res)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"E{len(c[0])}-M{sum(c[0])}-K{c[1]}-N{c[2]}")
+def test_mid_rows_tiles(dtype, case):
+    from xma.rocm import ops
+
+    rows, K, N = case
+    E, M = len(rows), sum(rows)
+    assert M > 24 * E
+    g = torch.Generator().manual_seed(M + K)
+    se = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))
+    ss = torch.randperm(M, generator=g)
+    offs = torch.tensor(rows).cumsum(0).cuda()
+    idx = ss.cuda()
+    wide = torch.randn(M, K + 16, generator=g).to(dtype)
+    x = wide[:, 8 : 8 + K]  # rows further apart than they are long
+    Wn = (torch.randn(E, N, K, generator=g) * K**-0.5).to(dtype)
+    Wk = (torch.randn(E, K, N, generator=g) * K**-0.5).to(dtype)
+    bias = torch.randn(E, N, generator=g).to(dtype)
+    w = torch.rand(M, generator=g).to(dtype)
+    z = torch.randn(M, 2 * N, generator=g).to(dtype)
+    dy = torch.randn(M, N, generator=g).to(dtype)
+    xd, Wnd, Wkd, bd, wd, zd, dyd = wide.cuda()[:, 8 : 8 + K], Wn.cuda(), Wk.cuda(), bias.cuda(), w.cuda(), z.cuda(), dy.cuda()
+    out, h, dz, dW = (torch.empty(s, dtype=dtype, device="cuda") for s in ((M, N), (M, N // 2), (M, 2 * N), (E, N, K)))
+    tol = _tol(dtype)
+
+    def agree(fn, outs, want):
+        for (tiles256, got), ref in zip(_both(fn, outs), want):
+            assert torch.isfinite(got).all()
+            assert nerr(got, ref) <= tol and nerr(got, tiles256) <= tol
+
+    for x_grouped in (False, True):
+        for y_grouped in (False, True):
+            for scale in (None, w):
+                sd = None if scale is None else wd
+                args = (se, ss, 1, x_grouped, y_grouped)
+                agree(lambda: ops.scatter2scatter_rocm(xd, Wnd.permute(0, 2, 1), idx, offs, out, sd, 1, x_grouped, y_grouped, bd), [out],
+                      [oracle.scatter2scatter(x, Wn.permute(0, 2, 1), *args, scale, bias=bias)])
+                agree(lambda: ops.scatter2scatter_rocm(xd, Wkd, idx, offs, out, sd, 1, x_grouped, y_grouped), [out],
+                      [oracle.scatter2scatter(x, Wk, *args, scale)])
+    if N % 16 == 0:
+        want = oracle.scatter2scatter(x, Wn.permute(0, 2, 1), se, ss, 1, False, True, None, bias=bias)
+        agree(lambda: ops.up_projection_swiglu_rocm(xd, Wnd.permute(0, 2, 1), idx, offs, out, h, 1, bd), [out, h],
+              [want, oracle.swiglu_packed(want)])
+    # SwiGLU backward, its second output, and the three forms of dW: agreement with the 256 x 256 kernels, which other tests hold
+    # against the oracle
+    def same(fn, outs):
+        for tiles256, got in _both(fn, outs):
+            assert torch.isfinite(got).all() and nerr(got, tiles256) <= tol
+
+    same(lambda: ops.down_projection_dx_swiglu_rocm(xd, Wkd, idx, offs, zd, dz, wd, 1), [dz])
+    same(lambda: ops.down_projection_dx_swiglu_scaled_act_rocm(xd, Wkd, idx, offs, zd, dz, out, wd, 1), [dz, out])
+    for dy_fan, x_fan in ((0, 0), (1, 0), (0, 1)):
+        same(lambda: ops.group_bwd_W_rocm(dyd, xd, idx, offs, dW.permute(0, 2, 1), None, dy_fan, x_fan), [dW])

@@ -114,6 +114,27 @@ def test_few_token_dispatch_rule():
     assert ops._few_rows(14, 8, torch.float16, "dy @ W")
 
 
+def test_mid_rows_dispatch_rule():
+    """which launches beyond the few-token limits take the few-row entry points for their 128 x 256 tiles"""
+    from xma.rocm import ops
+
+    bf, store, glu, bwd = torch.bfloat16, ops.EPI_STORE, ops.EPI_SWIGLU, ops.EPI_SWIGLU_BWD
+    fwd = lambda M, N, K, E, kn=0, ldw=4096, span=1 << 20, dt=bf, epi=store: ops._mid_rows_fwd(M, N, K, E, kn, ldw, span, dt, epi)
+    assert fwd(352 * 64, 2816, 2048, 64) and not fwd(352 * 64 + 1, 2816, 2048, 64)
+    assert fwd(112 * 8, 4096, 28672, 8) and not fwd(112 * 8 + 1, 4096, 28672, 8)
+    assert fwd(16384, 512, 1024, 8) and not fwd(16384, 512, 4096, 8)  # few tiles and a short K
+    assert not fwd(65536, 512, 64, 1024) and not fwd(2000, 64, 64, 1025) and not fwd(0, 64, 64, 8)
+    assert fwd(999, 64, 64, 8, kn=0, epi=glu) and not fwd(999, 64, 64, 8, kn=1, epi=glu)
+    assert fwd(999, 64, 64, 8, kn=1, epi=bwd) and not fwd(999, 64, 64, 8, kn=0, epi=bwd)
+    assert not fwd(999, 64, 64, 8, span=1 << 31) and not fwd(999, 64, 64, 8, ldw=1 << 23) and not fwd(999, 64, 64, 8, dt=torch.float32)
+    dw = ops._mid_rows_dw
+    assert dw(640 * 64, 4096, 4096, 64, bf) and not dw(640 * 64 + 1, 4096, 4096, 64, bf)
+    assert dw(1 << 20, 1024, 512, 8, bf) and not dw(1 << 20, 4096, 4096, 8, bf)
+    assert not dw(999, 64, 64, 65536, bf) and not dw(999, 64, 64, 8, torch.float32)
+    assert ops._dw_loader_scales(64 * 8, 8, bf) and not ops._dw_loader_scales(64 * 8 + 1, 8, bf)
+
+
+
 def test_fused_router_shape_rule_matches_the_library():
     """the Python restatement of the fused gate + router kernel's coverage (evaluated under torch.compile, where a ctypes
     call cannot be traced) against the library's own answer"""
