@@ -97,9 +97,32 @@ class MoE(nn.Module):
     def forward(self, x: torch.Tensor, *, kernel_backend: KernelBackend | None = None) -> tuple[torch.Tensor, torch.Tensor]:
         original_shape = x.shape
         x = x.view(-1, self.hidden_size)
+        if x.is_cuda and not torch.compiler.is_compiling() and self._runs_as_one_call(kernel_backend):
+            from .rocm_implementation import layer
+
+            out = layer(self, x)
+            if out is not None:
+                return out[0].view(original_shape), out[1]
         router_logits, router_weights, selected_experts = self._compute_routing_weights(x, kernel_backend=kernel_backend)
         x = self._compute_experts(x, router_weights, selected_experts, kernel_backend=kernel_backend)
         return x.view(original_shape), router_logits
+
+    def _runs_as_one_call(self, kernel_backend: KernelBackend | None) -> bool:
+        """rocm backend, packed SwiGLU, and the two parts below as they are written here"""
+        if kernel_backend is None:
+            kernel_backend = Accelerator.get_kernel_backend()
+        elif kernel_backend == KernelBackend.rocm:
+            assert kernel_backend.verify_accelerator()
+        cls, own = type(self), self.__dict__
+        return (
+            kernel_backend == KernelBackend.rocm
+            and self.is_glu
+            and getattr(self.act, "_xma_fused_activation", None) == "swiglu_packed"
+            and cls._compute_experts is MoE._compute_experts
+            and cls._compute_routing_weights is MoE._compute_routing_weights
+            and "_compute_experts" not in own
+            and "_compute_routing_weights" not in own
+        )
 
     def _compute_routing_weights(
         self, x: torch.Tensor, *, kernel_backend: KernelBackend | None = None

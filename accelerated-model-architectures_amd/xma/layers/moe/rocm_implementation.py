@@ -21,9 +21,13 @@ Differences from the reference's data flow, all of which remove HBM passes:
 
 from __future__ import annotations
 
+import struct
+from functools import lru_cache
+
 import torch
 
 from ...rocm import ops
+from ...rocm.loader import check, get_library
 
 
 # ----------------------------------------------------------------------------------------- routing
@@ -211,7 +215,11 @@ def _scale_activations_for_dw2(top_k: int, grad_out: torch.Tensor) -> bool:
     costs more than the extra output of the epilogue (measured on the whole forward + backward step, two boxes: -2.4 / -3.1 % at
     top-8 with H = 2048, I = 768; -1.0 / -1.4 % at top-6 with I = 1408; +0.7 / +1.0 % at top-2 with H = 4096, I = 14336).  h then is not kept for
     the backward.  16-bit only: the fp32 kernels have no such epilogue."""
-    return top_k >= 4 and grad_out.dtype in (torch.bfloat16, torch.float16)
+    return _scale_by_top_k(top_k) and grad_out.dtype in (torch.bfloat16, torch.float16)
+
+
+def _scale_by_top_k(top_k: int) -> bool:
+    return top_k >= 4
 
 
 # ----------------------------------------------------------------------------------------- autograd
@@ -395,3 +403,185 @@ def fused_swiglu_experts(x, w_fc, w_proj, router_weights, sorted_scattered_idxs,
     down-projection GEMM."""
     return _FusedSwiGLUExperts.apply(x, w_fc, w_proj, router_weights, sorted_scattered_idxs, expert_offsets, b_fc, b_proj,
                                      save_activations)
+
+
+# ----------------------------------------------------------------------------------------- the layer as one call
+# A pass of a handful of tokens is as long as its host work, so the layer with packed SwiGLU runs as one autograd node, whose
+# forward and backward are one library call each (two around the gate's own products), on scratch that is laid out once per shape:
+# the same launches as the ops above, bit for bit.  Everything else (other activations, tracing, transforms, tensors that the
+# entry point does not describe) goes through the ops.
+_BLOCK_POINTERS = struct.Struct("28Q")
+_BLOCK_SIZES = struct.Struct("16q")
+
+
+class _Plan:
+    """sizes, choices and scratch layout of a layer call; a function of the shape, the options and the dispatch limits only"""
+
+    __slots__ = ("sizes_forward", "sizes_backward", "keep", "temp", "back", "keep_bytes", "temp_bytes", "back_bytes", "recompute")
+
+
+def _layout(sizes: dict[str, int]) -> tuple[dict[str, int], int]:
+    offsets, end = {}, 0
+    for name, size in sizes.items():
+        offsets[name] = end
+        end += (size + 255) // 256 * 256
+    return offsets, max(end, 256)
+
+
+@lru_cache(maxsize=4096)
+def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, b_proj: bool, save: bool, device_index: int, _limits) -> _Plan:
+    M, s = T * k, dtype.itemsize
+    few16 = dtype != torch.float32
+
+    def gemm(N, K, w_is_kn, ldw, x_span, epilogue):
+        """(which entry point, bytes of its workspace)"""
+        if few16 and ops._few_rows_fwd(M, N, K, E, w_is_kn, ldw, x_span, dtype, epilogue):
+            return 1, ops._few_rows_workspace_bytes(M, N, K, E, w_is_kn, epilogue)
+        return 0, ops.scatter2scatter_workspace_bytes(M, N, K, E, device_index)
+
+    def dw(N_out, K_in, scaled):
+        return int(ops._few_rows(M, E, dtype, "dW") or (
+            not scaled and ops._mid_rows_dw(M, N_out, K_in, E, dtype) and M * max(N_out, K_in) < ops.MID_ROWS_OFFSETS))
+
+    up, down = gemm(2 * I, H, 0, H, T * H, ops.EPI_SWIGLU), gemm(H, I, 0, I, M * I, ops.EPI_STORE)
+    dx2, dx1 = gemm(I, H, 1, I, T * H, ops.EPI_SWIGLU_BWD), gemm(H, 2 * I, 1, H, M * 2 * I, ops.EPI_STORE)
+    # the operand of dW2: see xma_rocm_moe in the library's header
+    if few16 and _scale_by_top_k(k):
+        dw2_form, dw2_operand = 1, M * I * s
+    elif not b_proj and ops._dw_loader_scales(M, E, dtype):
+        dw2_form, dw2_operand = 0, 0
+    else:
+        dw2_form, dw2_operand = 2, M * H * s
+    keep_h = save and dw2_form != 1
+    sizes = dict(weights=M * s, ids=M * 4, offsets=E * 8, idx=M * 8, z=M * 2 * I * s)
+    temp = dict(counts=E * 4, workspace=max(ops.route_workspace_elements(M, E) * 4, up[1], down[1]))
+    (sizes if keep_h else temp)["h"] = M * I * s
+    (sizes if save else temp)["out"] = M * H * s
+    # the scattered rows of dX1 take the place of dW2's operand
+    back = dict(d_weights=M * s, dz=M * 2 * I * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], 256))
+    if not save:
+        back |= dict(h=M * I * s, out=M * H * s)
+    p = _Plan()
+    p.keep, p.keep_bytes = _layout(sizes)
+    p.temp, p.temp_bytes = _layout(temp)
+    p.back, p.back_bytes = _layout(back)
+    p.recompute = not save
+    few = (up[0], down[0], dx2[0], dw(H, I, dw2_form == 0), dw(2 * I, H, False), dx1[0], dw2_form, int(not save))
+    block = _BLOCK_SIZES.size + _BLOCK_POINTERS.size
+    p.sizes_forward = _BLOCK_SIZES.pack(block, T, H, I, E, k, ops._DTYPE_CODE[dtype], *few, temp["workspace"])
+    p.sizes_backward = _BLOCK_SIZES.pack(block, T, H, I, E, k, ops._DTYPE_CODE[dtype], *few, back["workspace"])
+    return p
+
+
+def _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, save, grad):
+    """(y, logits, kept buffer, plan); gate_weight None: the logits are given"""
+    T, H = x.shape
+    E, I = w_proj.size(0), w_proj.size(2)
+    device = x.device
+    p = _plan(T, H, I, E, k, x.dtype, b_proj is not None, save, device.index, (ops.FEW_ROWS_MAX, *ops.FEW_ROWS_PER_EXPERT.values()))
+    y = torch.empty_like(x)
+    if gate_weight is not None:
+        logits = torch.empty(T, E, dtype=x.dtype, device=device)
+    if grad:
+        kept = torch.empty(p.keep_bytes, dtype=torch.uint8, device=device)
+        scratch = torch.empty(p.temp_bytes, dtype=torch.uint8, device=device)
+        a, b = kept.data_ptr(), scratch.data_ptr()
+    else:
+        kept = torch.empty(p.keep_bytes + p.temp_bytes, dtype=torch.uint8, device=device)
+        a = kept.data_ptr()
+        b = a + p.keep_bytes
+    keep, temp = p.keep, p.temp
+    check(
+        get_library().xma_rocm_moe_forward(p.sizes_forward + _BLOCK_POINTERS.pack(
+            x.data_ptr(), 0 if gate_weight is None else gate_weight.data_ptr(), w_fc.data_ptr(), w_proj.data_ptr(),
+            0 if b_fc is None else b_fc.data_ptr(), 0 if b_proj is None else b_proj.data_ptr(), logits.data_ptr(),
+            a + keep["weights"], a + keep["ids"], b + temp["counts"], a + keep["offsets"], a + keep["idx"], a + keep["z"],
+            a + keep["h"] if "h" in keep else b + temp["h"], a + keep["out"] if "out" in keep else b + temp["out"], y.data_ptr(),
+            b + temp["workspace"], 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0,
+        ), ops._stream(x)),
+        "xma_rocm_moe_forward",
+    )
+    return y, logits, kept, p
+
+
+class _Layer(torch.autograd.Function):
+    """the whole layer: with gate_weight (logits None) -> (y, logits), with given logits -> y"""
+
+    @staticmethod
+    def forward(ctx, x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, save):
+        y, logits, kept, ctx.plan = _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, save, True)
+        ctx.save_for_backward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, kept)
+        ctx.set_materialize_grads(False)
+        return y if gate_weight is None else (y, logits)
+
+    @staticmethod
+    def backward(ctx, dy, d_logits_out=None):
+        x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, kept = ctx.saved_tensors
+        need_x, need_gate, need_logits = ctx.needs_input_grad[:3]
+        if dy is None:  # nothing but the logits was used
+            if d_logits_out is None:
+                return (None,) * 9
+            d_x = d_logits_out @ gate_weight if need_x else None
+            return d_x, _gate_weight_grad(d_logits_out, x) if need_gate else None, None, None, None, None, None, None, None
+        dy = dy.contiguous()
+        p = ctx.plan
+        scratch = torch.empty(p.back_bytes, dtype=torch.uint8, device=x.device)
+        d_logits = torch.empty_like(logits, memory_format=torch.contiguous_format)
+        d_x, d_w_fc, d_w_proj = torch.empty_like(x), torch.empty_like(w_fc), torch.empty_like(w_proj)
+        d_b_fc, d_b_proj = (None if b is None else torch.empty_like(b) for b in (b_fc, b_proj))
+        a, b, keep, back = kept.data_ptr(), scratch.data_ptr(), p.keep, p.back
+        block = p.sizes_backward + _BLOCK_POINTERS.pack(
+            x.data_ptr(), 0, w_fc.data_ptr(), w_proj.data_ptr(), 0 if b_fc is None else b_fc.data_ptr(),
+            0 if b_proj is None else b_proj.data_ptr(), logits.data_ptr(), a + keep["weights"], a + keep["ids"], 0, a + keep["offsets"],
+            a + keep["idx"], a + keep["z"], b + back["h"] if "h" in back else a + keep["h"] if "h" in keep else 0,
+            b + back["out"] if "out" in back else a + keep["out"], 0, b + back["workspace"], dy.data_ptr(), b + back["d_weights"],
+            d_logits.data_ptr(), b + back["dz"], b + back["scattered"], b + back["scattered"], d_w_fc.data_ptr(), d_w_proj.data_ptr(),
+            0 if d_b_fc is None else d_b_fc.data_ptr(), 0 if d_b_proj is None else d_b_proj.data_ptr(), d_x.data_ptr(),
+        )
+        lib, stream = get_library(), ops._stream(x)
+        check(lib.xma_rocm_moe_backward_router(block, stream), "xma_rocm_moe_backward_router")
+        check(lib.xma_rocm_moe_backward(block, stream), "xma_rocm_moe_backward")
+        d_gate = None
+        if gate_weight is not None:
+            if d_logits_out is not None:  # the caller also used the returned router logits (an auxiliary loss)
+                d_logits = d_logits + d_logits_out
+            if need_x:
+                d_x = d_x + d_logits @ gate_weight
+            if need_gate:
+                d_gate = _gate_weight_grad(d_logits, x)
+        return d_x, d_gate, d_logits if need_logits else None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None
+
+
+def _plain(t: torch.Tensor, like: torch.Tensor) -> bool:
+    return t.dtype == like.dtype and t.device == like.device and t.is_contiguous() and t.data_ptr() % 16 == 0 and \
+        type(t) in (torch.nn.Parameter, torch.Tensor)
+
+
+def layer(moe, x: torch.Tensor):
+    """(y, router logits) of a layer with packed SwiGLU whose tensors the library's layer entry point describes: contiguous, one
+    dtype and device, aligned; None for anything else, and under function transforms and forward-mode differentiation"""
+    w_fc, w_proj, b_fc, b_proj = moe.c_fc.weight, moe.c_proj.weight, moe.c_fc.bias, moe.c_proj.bias
+    gate, k = moe.gate, moe.top_k
+    T, H = x.shape
+    if T == 0 or x.dtype not in ops._DTYPE_CODE or type(x) not in (torch.Tensor, torch.nn.Parameter) or x.data_ptr() % 16 or not x.is_contiguous():
+        return None
+    if not (_plain(w_fc, x) and _plain(w_proj, x)) or (b_fc is not None and not _plain(b_fc, x)) or (b_proj is not None and not _plain(b_proj, x)):
+        return None
+    E, I2, _ = w_fc.shape
+    if H % 8 or I2 % 16 or w_fc.size(2) != H or w_proj.shape != (E, H, I2 // 2) or E > 16384 or T * k >= 1 << 31:
+        return None
+    if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
+        return None
+    gate_weight, logits = gate.weight, None
+    if gate.bias is None and router_gate_topk_supported(x, gate_weight, k) and _plain(gate_weight, x):
+        tensors = (x, gate_weight, w_fc, w_proj, b_fc, b_proj)
+    else:
+        gate_weight, logits = None, gate(x)
+        if logits.shape != (T, E) or not _plain(logits, x):  # a gate that casts, for one
+            return moe._compute_experts(x, *router_topk(logits, k)), logits
+        tensors = (x, logits, w_fc, w_proj, b_fc, b_proj)
+    save = moe.save_activations
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
+        out = _Layer.apply(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, bool(save))
+        return out if logits is None else (out, logits)
+    return _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, True, False)[:2]

@@ -339,6 +339,35 @@ XMA_API int xma_rocm_router_topk_bwd(const void *logits, int64_t ld, int64_t T, 
                              int ids_is_i64, const void *d_weights, void *d_logits, int64_t ldd, void *stream);
 
 /*
+ * The layer as one call: the launches of the entry points above in their order, on buffers that the caller has laid out
+ * (MoE.forward, xma/layers/moe/__init__.py:170-262, with packed SwiGLU, and its backward).  Everything is row-major without gaps
+ * and 16-byte aligned; every field is 8 bytes wide, so that the block can be packed without a compiler.  few_* pick the few-row
+ * entry point for a GEMM (1) or the 256 x 256 tiles (0).  gate_weight NULL: `logits` is an input.  dw2_form: the operand of dW2,
+ * 0: dy through the few-row loader, which scales it; 1: `dw2_operand` = scaled activations (M, I), written by dX2; 2:
+ * `dw2_operand` = scaled grouped copy of dy (M, H).  recompute: h and expert_out are rebuilt from z by
+ * xma_rocm_moe_backward_router.  d_b_fc / d_b_proj may be NULL.  M = T k.  `workspace`: the largest that any of the calls asks for
+ * (route, and per GEMM its entry point's).  Argument errors as in the single calls; launches before one that is refused stand.
+ */
+typedef struct xma_rocm_moe {
+    int64_t size; /* sizeof(xma_rocm_moe) */
+    int64_t T, H, I, E, k, dtype;
+    int64_t few_up, few_down, few_dx2, few_dw2, few_dw1, few_dx1, dw2_form, recompute, workspace_bytes;
+    const void *x, *gate_weight, *w_fc, *w_proj, *b_fc, *b_proj;       /* (T,H) (E,H) (E,2I,H) (E,H,I) (E,2I) (E,H) */
+    void *logits, *router_weights, *expert_ids, *counts;                /* (T,E) (T,k) int32 (T,k) uint32 (E) */
+    void *expert_offsets, *sorted_scattered_idxs, *z, *h, *expert_out;  /* int64 (E) int64 (M) (M,2I) (M,I) (M,H) */
+    void *y, *workspace;                                                /* (T,H) */
+    const void *dy;                                                     /* (T,H) */
+    void *d_router_weights, *d_logits, *dz, *dw2_operand, *scattered;   /* (T,k) (T,E) (M,2I) see dw2_form (M,H) */
+    void *d_w_fc, *d_w_proj, *d_b_fc, *d_b_proj, *d_x;                  /* like the weights; (T,H) */
+} xma_rocm_moe;
+/* router, route, up-projection + SwiGLU, down-projection, combine */
+XMA_API int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream);
+/* [h and expert_out again], combine backward, d_logits */
+XMA_API int xma_rocm_moe_backward_router(const xma_rocm_moe *m, void *stream);
+/* dX2, dW2, dW1, bias gradients, dX1, sum over the k slots; behind xma_rocm_moe_backward_router */
+XMA_API int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream);
+
+/*
  * Measurement aid with no counterpart in the reference: `workgroups` workgroups of 4 waves each issue iters x 64
  * independent v_mfma_f32_32x32x16_bf16 on operands read once from `operands` (16 x 256 x 16 bytes: 8 A and 8 B fragments
  * per lane), nothing else in the loop.  2 * 32 * 32 * 16 * 64 * 4 * workgroups * iters FLOP per call; out receives

@@ -1,0 +1,124 @@
+"""The layer as one autograd node against the same layer through the single ops: same launches, so bit for bit."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+from xma.functional import swiglu_packed
+from xma.layers import MoE
+
+
+pytestmark = pytest.mark.gpu
+
+
+class _ThroughOps(MoE):
+    def _compute_experts(self, *args, **kwargs):  # overridden: the layer does not run as one call
+        return super()._compute_experts(*args, **kwargs)
+
+
+def _layers(T, E, k, H, I, dtype, bias=False, save=True, seed=3):
+    torch.manual_seed(seed)
+    one = MoE(E, k, H, I, swiglu_packed, True, add_bias=bias, std=0.05)
+    if bias:
+        nn.init.normal_(one.c_fc.bias)
+        nn.init.normal_(one.c_proj.bias)
+    ops = _ThroughOps(E, k, H, I, swiglu_packed, True, add_bias=bias, std=0.05)
+    ops.load_state_dict(one.state_dict())
+    one, ops = one.to("cuda", dtype), ops.to("cuda", dtype)
+    one.save_activations = ops.save_activations = save
+    return one, ops, torch.randn(T, H, device="cuda", dtype=dtype), torch.randn(T, H, device="cuda", dtype=dtype)
+
+
+def _step(moe, x, dy, aux=0.0, use_y=True):
+    x = x.clone().requires_grad_()
+    y, logits = moe(x)
+    loss = (y * dy).sum() if use_y else 0.0
+    if aux:
+        loss = loss + aux * (logits.float() ** 2).sum()
+    grads = torch.autograd.grad(loss, [x, *moe.parameters()], allow_unused=True)
+    return [y, logits, *grads]
+
+
+def _same(a, b):
+    assert len(a) == len(b)
+    for u, v in zip(a, b):
+        assert (u is None) == (v is None)
+        assert u is None or (u.shape == v.shape and u.dtype == v.dtype and torch.equal(u, v))
+
+
+CASES = [
+    # T, E, k, H, I: vector kernel, small tile, 128 x 256 tiles (both forms of dW2's operand), 256 x 256 tiles
+    (1, 8, 2, 2048, 64),
+    (7, 16, 8, 64, 24),
+    (33, 8, 2, 64, 40),
+    (300, 8, 2, 136, 72),
+    (500, 8, 5, 128, 64),
+    (3100, 4, 2, 128, 2816),
+]
+
+
+@pytest.mark.parametrize("bias,save", [(False, True), (True, True), (False, False), (True, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", CASES)
+def test_one_call_matches_the_ops(case, dtype, bias, save):
+    T, E, k, H, I = case
+    one, ops, x, dy = _layers(T, E, k, H, I, dtype, bias, save)
+    with torch.no_grad():
+        _same(one(x), ops(x))
+    _same(_step(one, x, dy), _step(ops, x, dy))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_which_gradients_are_asked_for(dtype):
+    """an auxiliary loss on the logits, alone and beside the output; frozen gate; frozen experts; no gradient of x"""
+    one, ops, x, dy = _layers(65, 8, 2, 64, 32, dtype)
+    _same(_step(one, x, dy, aux=0.1), _step(ops, x, dy, aux=0.1))
+    _same(_step(one, x, dy, aux=0.1, use_y=False), _step(ops, x, dy, aux=0.1, use_y=False))
+    for frozen in (["gate.weight"], ["c_fc.weight", "c_proj.weight"], ["gate.weight", "c_fc.weight", "c_proj.weight"]):
+        got = []
+        for moe in (one, ops):
+            for n, p in moe.named_parameters():
+                p.requires_grad_(n not in frozen)
+                p.grad = None
+            xx = x.clone().requires_grad_(len(frozen) == 3)
+            moe(xx)[0].backward(dy)
+            got.append([xx.grad, *(p.grad for p in moe.parameters())])
+        _same(*got)
+
+
+def test_what_goes_through_the_ops():
+    """forms the layer entry point does not describe are accepted as before, with the same results"""
+    from xma.layers.moe import rocm_implementation as R
+
+    one, ops, x, dy = _layers(40, 8, 2, 64, 32, torch.bfloat16)
+    assert R.layer(one, x) is not None
+    wide = torch.randn(40, 80, device="cuda", dtype=torch.bfloat16)
+    assert R.layer(one, wide[:, 8:72]) is None and R.layer(one, x[:0]) is None
+    flat = torch.randn(40 * 64 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(40, 64)  # starts off a 16-byte boundary
+    assert R.layer(one, flat) is None
+    held = one.c_fc.weight
+    one.c_fc.weight = nn.Parameter(held.detach().transpose(1, 2).contiguous().transpose(1, 2))  # same values, (E, in, out) storage
+    assert R.layer(one, x) is None
+    one.c_fc.weight = held
+    with torch.autograd.forward_ad.dual_level():
+        assert R.layer(one, x) is None
+    y, logits = one(x.view(5, 8, 64))
+    assert y.shape == (5, 8, 64) and logits.shape == (40, 8)
+    torch.manual_seed(0)
+    with torch.autograd.graph.save_on_cpu():
+        a = _step(one, x, dy)
+    _same(a, _step(ops, x, dy))
+
+
+def test_two_passes_before_the_backward():
+    """each pass keeps its own buffers"""
+    one, ops, x, dy = _layers(50, 8, 2, 64, 32, torch.bfloat16)
+    got = []
+    for moe in (one, ops):
+        x1, x2 = x.clone().requires_grad_(), (x * 0.5).requires_grad_()
+        y1, y2 = moe(x1)[0], moe(x2)[0]
+        y1.backward(dy, retain_graph=True)
+        y2.backward(dy)
+        y1.backward(dy)
+        got.append([x1.grad, x2.grad, *(p.grad for p in moe.parameters())])
+    _same(*got)
