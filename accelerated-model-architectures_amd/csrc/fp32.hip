@@ -338,7 +338,7 @@ template <int TB> __global__ __launch_bounds__(FTHREADS) void dw_f32_kernel(cons
 // ------------------------------------------------------------------------------------------------ elementwise
 // one thread per float4 of the output
 __global__ __launch_bounds__(FTHREADS) void combine_f32_kernel(const float *in, int64_t ld_in, const float *w, float *y,
-                                                                int64_t ldy, int64_t T, int k, int cpr) {
+                                                                int64_t ldy, int64_t T, int k, int cpr, const float *addend, int64_t ld_add) {
     const int64_t id = (int64_t)blockIdx.x * FTHREADS + threadIdx.x;
     if (id >= T * cpr) return;
     const int64_t t = id / cpr;
@@ -348,6 +348,7 @@ __global__ __launch_bounds__(FTHREADS) void combine_f32_kernel(const float *in, 
         const float s = w ? w[t * k + j] : 1.f;
         acc += s * *(const f32x4 *)(in + (t * k + j) * ld_in + c);
     }
+    if (addend) acc += *(const f32x4 *)(addend + t * ld_add + c);
     *(f32x4 *)(y + t * ldy + c) = acc;
 }
 
@@ -462,10 +463,10 @@ int f32_group_bwd_W(const DwArgs &a, hipStream_t st) {
     return xma_check_launch("dw_f32_kernel");
 }
 
-int f32_combine(const void *in, int64_t ld_in, const void *w, void *y, int64_t ldy, int64_t T, int k, int H, hipStream_t st) {
+int f32_combine(const void *in, int64_t ld_in, const void *w, const void *addend, int64_t ld_add, void *y, int64_t ldy, int64_t T, int k, int H, hipStream_t st) {
     const int cpr = H / 4;
     combine_f32_kernel<<<blocks_for(T * cpr), FTHREADS, 0, st>>>((const float *)in, ld_in, (const float *)w, (float *)y, ldy,
-                                                                 T, k, cpr);
+                                                                 T, k, cpr, (const float *)addend, ld_add);
     return xma_check_launch("combine_f32_kernel");
 }
 

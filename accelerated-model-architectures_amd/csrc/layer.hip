@@ -123,5 +123,5 @@ extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
         RUN(xma_rocm_expert_column_sums(m->dz, 2 * I, nullptr, 1, nullptr, offs, m->d_b_fc, 2 * I, (int32_t)(2 * I), (int32_t)m->E, dtype, stream));
     RUN(gemm(m, m->few_dx1, m->dz, m->w_fc, 2 * I * H, H, 1, m->scattered, nullptr, 0, nullptr, nullptr, nullptr, H, 2 * I, 1, 1, 0,
              XMA_ROCM_EPI_STORE, stream));
-    return xma_rocm_combine(m->scattered, H, nullptr, m->d_x, H, m->T, (int32_t)m->k, (int32_t)H, dtype, stream);
+    return xma_rocm_combine_add(m->scattered, H, nullptr, m->d_x_addend, H, m->d_x, H, m->T, (int32_t)m->k, (int32_t)H, dtype, stream);
 }

@@ -410,7 +410,7 @@ def fused_swiglu_experts(x, w_fc, w_proj, router_weights, sorted_scattered_idxs,
 # forward and backward are one library call each (two around the gate's own products), on scratch that is laid out once per shape:
 # the same launches as the ops above, bit for bit.  Everything else (other activations, tracing, transforms, tensors that the
 # entry point does not describe) goes through the ops.
-_BLOCK_POINTERS = struct.Struct("28Q")
+_BLOCK_POINTERS = struct.Struct("29Q")
 _BLOCK_SIZES = struct.Struct("16q")
 
 
@@ -497,7 +497,7 @@ def _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, save, 
             0 if b_fc is None else b_fc.data_ptr(), 0 if b_proj is None else b_proj.data_ptr(), logits.data_ptr(),
             a + keep["weights"], a + keep["ids"], b + temp["counts"], a + keep["offsets"], a + keep["idx"], a + keep["z"],
             a + keep["h"] if "h" in keep else b + temp["h"], a + keep["out"] if "out" in keep else b + temp["out"], y.data_ptr(),
-            b + temp["workspace"], 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0,
+            b + temp["workspace"], 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0,
         ), ops._stream(x)),
         "xma_rocm_moe_forward",
     )
@@ -530,7 +530,7 @@ class _Layer(torch.autograd.Function):
         d_x, d_w_fc, d_w_proj = torch.empty_like(x), torch.empty_like(w_fc), torch.empty_like(w_proj)
         d_b_fc, d_b_proj = (None if b is None else torch.empty_like(b) for b in (b_fc, b_proj))
         a, b, keep, back = kept.data_ptr(), scratch.data_ptr(), p.keep, p.back
-        block = p.sizes_backward + _BLOCK_POINTERS.pack(
+        pointers = (
             x.data_ptr(), 0, w_fc.data_ptr(), w_proj.data_ptr(), 0 if b_fc is None else b_fc.data_ptr(),
             0 if b_proj is None else b_proj.data_ptr(), logits.data_ptr(), a + keep["weights"], a + keep["ids"], 0, a + keep["offsets"],
             a + keep["idx"], a + keep["z"], b + back["h"] if "h" in back else a + keep["h"] if "h" in keep else 0,
@@ -539,16 +539,17 @@ class _Layer(torch.autograd.Function):
             0 if d_b_fc is None else d_b_fc.data_ptr(), 0 if d_b_proj is None else d_b_proj.data_ptr(), d_x.data_ptr(),
         )
         lib, stream = get_library(), ops._stream(x)
-        check(lib.xma_rocm_moe_backward_router(block, stream), "xma_rocm_moe_backward_router")
-        check(lib.xma_rocm_moe_backward(block, stream), "xma_rocm_moe_backward")
-        d_gate = None
+        check(lib.xma_rocm_moe_backward_router(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0), stream), "xma_rocm_moe_backward_router")
+        d_gate = d_x_gate = None
         if gate_weight is not None:
             if d_logits_out is not None:  # the caller also used the returned router logits (an auxiliary loss)
                 d_logits = d_logits + d_logits_out
             if need_x:
-                d_x = d_x + d_logits @ gate_weight
+                d_x_gate = d_logits @ gate_weight
             if need_gate:
                 d_gate = _gate_weight_grad(d_logits, x)
+        check(lib.xma_rocm_moe_backward(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0 if d_x_gate is None else d_x_gate.data_ptr()),
+                                        stream), "xma_rocm_moe_backward")
         return d_x, d_gate, d_logits if need_logits else None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None
 
 

@@ -274,6 +274,9 @@ XMA_API int xma_rocm_group(const void *A, int64_t lda, const int64_t *idx, void 
  */
 XMA_API int xma_rocm_combine(const void *expert_out, int64_t ld_in, const void *w, void *y, int64_t ldy, int64_t T,
                      int32_t k, int32_t H, int dtype, void *stream);
+/* the same with addend (T, H) (row stride ld_add, 16-byte aligned, or NULL) added to the rounded sum */
+XMA_API int xma_rocm_combine_add(const void *expert_out, int64_t ld_in, const void *w, const void *addend, int64_t ld_add, void *y,
+                         int64_t ldy, int64_t T, int32_t k, int32_t H, int dtype, void *stream);
 
 /*
  * Combine backward w.r.t. the router weights:
@@ -359,6 +362,7 @@ typedef struct xma_rocm_moe {
     const void *dy;                                                     /* (T,H) */
     void *d_router_weights, *d_logits, *dz, *dw2_operand, *scattered;   /* (T,k) (T,E) (M,2I) see dw2_form (M,H) */
     void *d_w_fc, *d_w_proj, *d_b_fc, *d_b_proj, *d_x;                  /* like the weights; (T,H) */
+    const void *d_x_addend;                                             /* (T,H) or NULL: the gate's part of d_x */
 } xma_rocm_moe;
 /* router, route, up-projection + SwiGLU, down-projection, combine */
 XMA_API int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream);
