@@ -694,6 +694,10 @@ extern "C" size_t xma_rocm_scatter2scatter_few_rows_workspace_bytes(int64_t M, i
     return few > mid ? few : mid;
 }
 
+extern "C" int xma_rocm_scatter2scatter_few_rows_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
+    return M > 0 && N > 0 && K > 0 && E > 0 && xma_rocm::mid_fwd_leads(M, N, K, E, epilogue) ? 1 : 0;
+}
+
 extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, const void *W, int64_t w_expert_stride,
                                                  int64_t ldw, int w_is_kn, const int64_t *sorted_scattered_idxs,
                                                  const int64_t *expert_offsets, void *out, int64_t ldo, void *aux,

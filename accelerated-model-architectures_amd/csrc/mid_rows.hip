@@ -24,12 +24,15 @@
 // 2048, I = 1408, 96 rows 933 -> 715, 256 rows 1470 -> 1240; E = 128, H = 576, I = 256, 128 rows 197 -> 143; E = 8, H = 512, I =
 // 1024, 256 rows 169 -> 95.  What bounds them: up to some 100 rows the stream of the weights, or of the stores of dW (4.5 to 5
 // TB/s); beyond that the K loop, 2.1 us a step for the two workgroups of a compute unit (the products alone 0.9), part of it the
-// board's power (cleared operands: 10 - 15 % shorter).  From 350 to 650 rows per expert on the 256 x 256 tiles lead, which
-// move two thirds of the bytes per product through L2 and LDS.
+// board's power (cleared operands: 10 - 15 % shorter).  In launches of many rounds the 256 x 256 tiles, which move two thirds of the
+// bytes per product through L2 and LDS, lead from about 350 (forward types) and 650 (dW) rows per expert on; in launches of a few
+// rounds the smaller tiles stay ahead for longer, because they fill the last round better (mid_fwd_leads).
 //
 // Operand layouts in an item, as in grouped_gemm.hip with 16 KB instead of 32: K contiguous in memory [128 rows][8 chunks of
 // 16 B], chunk c of row r at slot c ^ ((r >> 1) & 7); K the row index in memory [64 k-rows][16 chunks], chunk c of k-row kr at
 // slot c ^ ((kr & 3) << 2), read with ds_read_b64_tr_b16.
+#include <math.h>
+
 #include "grouped_gemm_tile.hpp"
 #include "mid_rows.hpp"
 
@@ -549,31 +552,56 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void mid_dw_kernel(const DwArgs a)
     }
 }
 
-// about what the offsets will give: half a tile of an expert's last rows on average, where it has more than one
-inline double mid_tiles(int64_t M, int N, int E) {
+// Tiles of `height` rows x 256 columns that the offsets will give, about: one per expert while nearly all fit into it, half a tile
+// of an expert's last rows beyond that.
+inline double tiles_about(int64_t M, int N, int E, int height) {
     const double rows = (double)M / E;
-    return (rows <= 104 ? (M < E ? M : E) : E * (rows / MR_BM + 0.5)) * ((N + MR_BN - 1) / MR_BN);
+    return (rows + 2.5 * sqrt(rows) <= height ? (M < E ? M : E) : E * (rows / height + 0.5)) * ((N + MR_BN - 1) / MR_BN);
 }
 
-// K ranges of a forward-type launch, at least 4 steps each: as many as make the launch shortest by what is known of it here.  t
-// workgroups on 256 compute units stream their operands at 4.9 TB/s from about 185 busy units on; alone on its unit a workgroup
-// takes 1.1 us a step, two that share one 2.1 us each, in rounds of 512 of them; the sums of S > 1 ranges go through memory twice
-// (3.3 TB/s) behind one more launch.  Within 10 % of the best of 1 .. 8 wherever it was checked (8, 16 and 128 experts, 16 to 384 rows
-// each); the same launches with one range 1.2 to 2 times as long.
-inline int mid_fwd_splits(int64_t M, int N, int K, int E) {
-    const double tiles = mid_tiles(M, N, E), bytes = 2.0 * (M < E ? M : E) * N * K + 2.0 * M * (N + K);
+// The length of a forward-type launch of 128 x 256 tiles cut into S ranges of K, about, and the S (each at least 4 steps) that makes
+// it shortest.  t workgroups on 256 compute units stream their operands at 4.9 TB/s from about 185 busy units on; alone on its unit a
+// workgroup takes 1.1 us a step, two that share one 2.1 us each, with 512 at a time, 2.4 where more wait behind them (power); the
+// sums of S > 1 ranges go through memory twice (3.3 TB/s) behind one more launch.  This and tiles256_seconds were fitted together to 336
+// measured pairs of launches (the layers of the benchmark and six others, 100 to 4000 rows per expert): within 12 and 10 % on average.
+// On 504 pairs the launches that mid_fwd_leads chooses are 1.17 times as fast as the 256 x 256 ones, the worst of them 9 % slower.
+inline double mid_fwd_seconds(int64_t M, int N, int K, int E, int epilogue, int *best) {
+    const double tiles = tiles_about(M, N, E, MR_BM), bytes = 2.0 * (M < E ? M : E) * N * K + 2.0 * M * (N + K);
+    const double epi = epilogue == XMA_ROCM_EPI_SWIGLU_BWD ? 7.7e-6 : 0.;
     const int steps = (K + MR_K - 1) / MR_K;
-    int best = 1;
     double shortest = 1e30;
-    for (int S = 1; S <= 8 && (S == 1 || steps / S >= 4) && (double)S * M * N * 4 <= 256e6; ++S) {
-        const double t = tiles * S, busy = t <= MR_RUN / 2 ? t : t < MR_RUN ? t / 2 : MR_RUN / 2;
-        const double rounds = t <= MR_RUN ? 1. : t < 4 * MR_RUN ? (double)(int64_t)((t + MR_RUN - 1) / MR_RUN) : t / MR_RUN + 0.5;
+    *best = 1;
+    for (int S = 1; S <= 8 && (S == 1 || (steps / S >= 4 && (double)S * M * N * 4 <= 256e6)); ++S) {
+        const double t = tiles * S, rounds = t / MR_RUN, busy = t <= MR_RUN / 2 ? t : t < MR_RUN ? t / 2 : MR_RUN / 2;
         const double stream = bytes / 4.9e12 * (busy < 185 ? 185 / busy : 1.);
-        const double walk = rounds * ((steps + S - 1) / S) * (t <= MR_RUN / 2 ? 1.1e-6 : 2.1e-6);
-        const double time = (stream > walk ? stream : walk) + (S > 1 ? 8.0 * S * M * N / 3.3e12 + 4e-6 : 0.);
-        if (time < shortest * 0.98) shortest = time, best = S;
+        const double step = rounds <= 0.5 ? 1.1e-6 : rounds <= 1 ? 2.1e-6 * (0.5 + rounds / 2) : 2.4e-6 * rounds;
+        const double walk = ((steps + S - 1) / S) * step + (S == 1 ? epi * (rounds > 1 ? rounds : 1.) : 0.);
+        const double time = pow(pow(stream, 4.4) + pow(walk, 4.4), 1 / 4.4) + 7e-6 + (S > 1 ? 8.0 * S * M * N / 3.3e12 + 4e-6 : 0.);
+        if (time < shortest) shortest = time, *best = S;
     }
-    return best;
+    return shortest;
+}
+
+inline int mid_fwd_splits(int64_t M, int N, int K, int E) {
+    int S;
+    mid_fwd_seconds(M, N, K, E, XMA_ROCM_EPI_STORE, &S);
+    return S;
+}
+
+// The same for the 256 x 256 kernels: 1.6 us a step, 8 to 21 us at a tile's edges by its epilogue, in rounds of 256 tiles; a last round
+// is a round to itself in a launch of up to three, a third of one behind more; its tiles run as K slices where they are few enough
+// for two or more slices each (two more launches, sums through memory).
+inline double tiles256_seconds(int64_t M, int N, int K, int E, int epilogue) {
+    const double tiles = tiles_about(M, N, E, 256), n = tiles / 256, full = floor(n), rest = tiles - 256 * full;
+    const int steps = (K + MR_K - 1) / MR_K;
+    const double bytes = 2.0 * (M < E ? M : E) * N * K + 2.0 * M * (N + K);
+    const double edges = epilogue == XMA_ROCM_EPI_SWIGLU_BWD ? 20.8e-6 : epilogue == XMA_ROCM_EPI_SWIGLU ? 10.6e-6 : 7.6e-6;
+    const int parts = rest > 0 ? (int)(256 / rest < steps / 8 ? 256 / rest : steps / 8) : 0;
+    const bool split = parts >= 2 && tiles <= 12 * 256;
+    double rounds = full + (rest <= 0 ? 0. : split ? 1. / parts : 1.);
+    if (n > 3 && rounds > n + 0.34) rounds = n + 0.34;
+    const double walk = rounds * (steps * 1.6e-6 * (n < 1 ? 0.9 + 0.1 * n : 1.) + edges);
+    return pow(pow(walk, 3.2) + pow(bytes / 4.5e12, 3.2), 1 / 3.2) + (split ? rest * parts * 2 * 262144 / 3.5e12 : 0.) + (steps >= 16 ? 10e-6 : 0.);
 }
 
 template <typename T, int WT, int EPI> int mid_launch_fwd(const FwdArgs &a, float *sums, hipStream_t st) {
@@ -583,7 +611,7 @@ template <typename T, int WT, int EPI> int mid_launch_fwd(const FwdArgs &a, floa
     const int64_t grid = (a.M / MR_BM + a.E) * ((a.N + MR_BN - 1) / MR_BN) * S + 7; // at most
     // The dispatcher puts two neighbouring workgroups of an XCD on one compute unit while others have none.  A launch that leaves
     // compute units idle asks for more LDS than half a compute unit has, and gets one of its own for every workgroup.
-    const int smem = mid_tiles(a.M, a.N, a.E) * S <= MR_RUN / 2 ? MR_SMEM_ALONE : MR_SMEM_BYTES;
+    const int smem = tiles_about(a.M, a.N, a.E, MR_BM) * S <= MR_RUN / 2 ? MR_SMEM_ALONE : MR_SMEM_BYTES;
     int rc;
     if (S == 1) {
         if ((rc = gemm_set_smem(mid_fwd_kernel<T, WT, EPI>, MR_SMEM_ALONE))) return rc;
@@ -629,6 +657,14 @@ bool mid_fwd_takes(const FwdArgs &a, int wt, int epi) {
     if (a.E > MR_MAX_E || (wt == 0 ? epi == XMA_ROCM_EPI_SWIGLU_BWD : epi == XMA_ROCM_EPI_SWIGLU)) return false;
     const int64_t x_rows = a.x_grouped ? MR_BM : (a.M + a.fan_out - 1) / a.fan_out; // 32-bit byte offsets from a tile's base
     return a.M > 0 && a.M <= 65535 && x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)MR_BN * a.ldw * 2 < ((int64_t)1 << 32);
+}
+
+bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
+    // K beyond 8192 (few experts, wide layers): tiles of twice the products per byte lead as soon as experts need two of the smaller
+    // ones (8 experts of 176 rows, K = 28672: 470 against 516 us; K = 14336, 268 against 281; 320 rows 340 against 428)
+    if (K > 8192 && M > (int64_t)112 * E) return false;
+    int S;
+    return mid_fwd_seconds(M, N, K, E, epilogue, &S) < 0.96 * tiles256_seconds(M, N, K, E, epilogue); // even: as it was
 }
 
 int mid_fwd(const FwdArgs &a, int wt, int epi, int dtype, float *part, hipStream_t st) {

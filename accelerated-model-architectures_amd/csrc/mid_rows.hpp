@@ -11,6 +11,8 @@ namespace xma_rocm {
 // whether the kernels have the variant and can address the operands
 bool mid_fwd_takes(const FwdArgs &a, int w_is_kn, int epilogue);
 bool mid_dw_takes(const DwArgs &a, int64_t M);
+// whether a forward-type launch beyond the few-row regime is shorter with 128 x 256 than with 256 x 256 tiles, as far as its sizes tell
+bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue);
 // fp32 sums of the K ranges of a launch with few tiles; 0: not cut
 size_t mid_fwd_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E);
 int mid_fwd(const FwdArgs &a, int w_is_kn, int epilogue, int dtype, float *part, hipStream_t st);

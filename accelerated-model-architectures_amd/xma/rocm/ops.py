@@ -103,14 +103,10 @@ FEW_ROWS_PER_EXPERT = {"x @ W^T": 96, "dy @ W": 96, "dW": 128}
 FEW_ROWS_MAX = 16384  # rows in all, every form (beyond the measured range; 0 switches the few-token entry points off)
 FEW_ROWS_MAX_WORKSPACE = 256 << 20  # bytes of fp32 partial sums a forward-type launch may ask for
 # Beyond these limits the same entry points lead a while longer with 128 x 256 tiles, two workgroups per compute unit, where the
-# 256 x 256 tiles spend their time at the tiles' edges.  Forward-type GEMMs up to 352 rows per expert (64 experts of H = 2048, I =
-# 1408, 256 rows, dX2 208 -> 170 us; 400 rows: equal), 112 where K is long (8 experts of H = 4096, I = 14336, 176 rows, dX1, K =
-# 28672: 470 us with 256 x 256 tiles, 544 without), and where even those tiles are at most two per compute unit and K is short
-# (8 experts of H = 512, I = 1024, 512 rows: down-projection 37 -> 19 us, dX1 50 -> 31).  dW up to 640 rows per expert (64 experts, 256
-# rows, dW1 403 -> 269; 512 rows 557 -> 440), or where it has at most one 256 x 256 tile per compute unit (2048 rows of the
-# small layer: 49 -> 42).
-MID_ROWS_PER_EXPERT, MID_ROWS_PER_EXPERT_LONG_K, MID_ROWS_LONG_K = 352, 112, 8192
-MID_ROWS_FEW_TILES, MID_ROWS_FEW_TILES_K = 512, 2048
+# 256 x 256 tiles spend their time at the tiles' edges and in a last round that is nearly empty.  Forward-type GEMMs: the library
+# compares the two by the sizes (64 experts of H = 2048, I = 1408, 256 rows, dX2 208 -> 170 us; 400 rows: equal; 16 experts, K = N = 2048,
+# 1024 rows 175 -> 150, 768 rows 112, 116 with the smaller tiles).  dW up to 640 rows per expert (64 experts, 256 rows, dW1 403 -> 269;
+# 512 rows 557 -> 440), or where it has at most one 256 x 256 tile per compute unit (8 experts of H = 512, I = 1024, 2048 rows: 49 -> 42).
 MID_ROWS_MAX = 65535  # rows in all, limit of the forward-type entry point
 MID_ROWS_PER_EXPERT_DW, MID_ROWS_FEW_TILES_DW = 640, 256
 
@@ -198,6 +194,12 @@ def _few_rows(M: int, E: int, dtype: torch.dtype, form: str) -> bool:
     return 0 < M <= min(FEW_ROWS_MAX, FEW_ROWS_PER_EXPERT[form] * E) and dtype in (torch.bfloat16, torch.float16)
 
 
+@lru_cache(maxsize=4096)
+def _mid_rows_lead(M: int, N: int, K: int, E: int, epilogue: int) -> bool:
+    """the library's answer, a function of the sizes only"""
+    return bool(get_library().xma_rocm_scatter2scatter_few_rows_leads(M, N, K, E, epilogue))
+
+
 MID_ROWS_MAX_EXPERTS, MID_ROWS_OFFSETS = 1024, 1 << 31  # 32-bit byte offsets: elements from a base to the end of an operand
 
 
@@ -211,9 +213,7 @@ def _mid_rows_fwd(M: int, N: int, K: int, E: int, w_is_kn: int, ldw: int, x_span
         return False
     if E > MID_ROWS_MAX_EXPERTS or x_span >= MID_ROWS_OFFSETS or 256 * ldw >= MID_ROWS_OFFSETS:
         return False
-    if M <= (MID_ROWS_PER_EXPERT if K <= MID_ROWS_LONG_K else MID_ROWS_PER_EXPERT_LONG_K) * E:
-        return True
-    return K <= MID_ROWS_FEW_TILES_K and (M // 256 + E // 2) * -(-N // 256) <= MID_ROWS_FEW_TILES
+    return _mid_rows_lead(M, N, K, E, epilogue)
 
 
 def _mid_rows_dw(M: int, N_out: int, K_in: int, E: int, dtype: torch.dtype) -> bool:

@@ -211,11 +211,13 @@ XMA_API int xma_rocm_down_projection_dx_swiglu(const void *dY, int64_t lddy, con
  * below 2^31 - 128 elements for W as (N, K) (32-bit byte offsets inside an expert).
  * Correct for any M, but an expert's rows are walked 4 (vector kernel), 32 (small tile) or 128 at a time, each pass
  * streaming its weights again: meant for launches of up to some hundreds of rows per expert (the torch ops of this package
- * take it up to 352 on average, 112 where K is beyond 8192, and beyond that where a launch has few tiles).  No counterpart
+ * take it up to 96 on average, and beyond that by xma_rocm_scatter2scatter_few_rows_leads).  No counterpart
  * in the reference (its kernel is the same for every size).
  */
 XMA_API size_t xma_rocm_scatter2scatter_few_rows_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t num_experts,
                                                          int w_is_kn, int epilogue);
+/* whether a launch of more than some 100 rows per expert is shorter through this entry point (1) or with 256 x 256 tiles (0) */
+XMA_API int xma_rocm_scatter2scatter_few_rows_leads(int64_t M, int32_t N, int32_t K, int32_t num_experts, int epilogue);
 XMA_API int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, const void *W, int64_t w_expert_stride, int64_t ldw,
                                       int w_is_kn, const int64_t *sorted_scattered_idxs,
                                       const int64_t *expert_offsets, void *out, int64_t ldo, void *aux, int64_t ldaux,

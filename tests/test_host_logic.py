@@ -120,9 +120,9 @@ def test_mid_rows_dispatch_rule():
 
     bf, store, glu, bwd = torch.bfloat16, ops.EPI_STORE, ops.EPI_SWIGLU, ops.EPI_SWIGLU_BWD
     fwd = lambda M, N, K, E, kn=0, ldw=4096, span=1 << 20, dt=bf, epi=store: ops._mid_rows_fwd(M, N, K, E, kn, ldw, span, dt, epi)
-    assert fwd(352 * 64, 2816, 2048, 64) and not fwd(352 * 64 + 1, 2816, 2048, 64)
-    assert fwd(112 * 8, 4096, 28672, 8) and not fwd(112 * 8 + 1, 4096, 28672, 8)
-    assert fwd(16384, 512, 1024, 8) and not fwd(16384, 512, 4096, 8)  # few tiles and a short K
+    assert fwd(256 * 64, 2816, 2048, 64) and not fwd(1000 * 64, 2816, 2048, 64)  # many rounds: by the rows per expert
+    assert fwd(1024 * 16, 2048, 2048, 16) and not fwd(4000 * 16, 2048, 2048, 16)  # few rounds, the last one nearly empty
+    assert fwd(100 * 8, 4096, 28672, 8) and not fwd(176 * 8, 4096, 28672, 8)  # long K
     assert not fwd(65536, 512, 64, 1024) and not fwd(2000, 64, 64, 1025) and not fwd(0, 64, 64, 8)
     assert fwd(999, 64, 64, 8, kn=0, epi=glu) and not fwd(999, 64, 64, 8, kn=1, epi=glu)
     assert fwd(999, 64, 64, 8, kn=1, epi=bwd) and not fwd(999, 64, 64, 8, kn=0, epi=bwd)
