@@ -125,4 +125,18 @@ __device__ __forceinline__ void transpose8x8_b16(const u32x4 in[8], u32x4 out[8]
 }
 
 // v_exp_f32 and v_rcp_f32 (1 ulp each) instead of an IEEE division: the result is rounded to 16 bits anyway
+__device__ __forceinline__ float sigmoidf_fast(float x);
+
+// GELU and its derivative; erf_form 0: the tanh approximation x sigmoid(2 u), u = sqrt(2 / pi) (x + 0.044715 x^3), which is
+// x / 2 (1 + tanh u) without the cancellation for negative x; 1: x / 2 (1 + erf(x / sqrt 2)).
+template <typename Sigmoid> __device__ __forceinline__ float gelu(float x, int erf_form, Sigmoid sigmoid) {
+    if (erf_form) return 0.5f * x * (1.f + erff(x * 0.70710678f));
+    return x * sigmoid(1.5957691f * (x + 0.044715f * x * x * x));
+}
+template <typename Sigmoid> __device__ __forceinline__ float gelu_grad(float x, int erf_form, Sigmoid sigmoid) {
+    if (erf_form) return 0.5f * (1.f + erff(x * 0.70710678f)) + x * 0.39894228f * expf(-0.5f * x * x);
+    const float s = sigmoid(1.5957691f * (x + 0.044715f * x * x * x));
+    return s + x * s * (1.f - s) * 1.5957691f * (1.f + 0.134145f * x * x);
+}
+
 __device__ __forceinline__ float sigmoidf_fast(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }

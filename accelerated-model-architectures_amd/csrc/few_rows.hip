@@ -10,6 +10,7 @@
 namespace {
 
 constexpr int FR_THREADS = 256;
+constexpr int EPI_GELU = XMA_ROCM_EPI_GELU_TANH, EPI_GELU_BWD = XMA_ROCM_EPI_GELU_TANH_BWD; // FwdArgs::erf_form says which
 
 template <typename T> __device__ __forceinline__ float fr_scalar(const uint16_t *p, int64_t i) { return Elem<T>::lo(p[i]); }
 
@@ -305,6 +306,8 @@ __device__ __forceinline__ void fr_nt_rows(const FwdArgs &a, float *__restrict__
                             const float g = Elem<T>::lo(z), up = Elem<T>::hi(z);
                             a.aux[dst * a.ldaux + (n_a >> 1)] = (uint16_t)(Elem<T>::pack(up * g * sigmoidf_fast(g), 0.f) & 0xffffu);
                         }
+                        if constexpr (EPI == EPI_GELU)
+                            *(uint32_t *)(a.aux + dst * a.ldaux + n_a) = Elem<T>::pack(gelu(Elem<T>::lo(z), a.erf_form, sigmoidf_fast), gelu(Elem<T>::hi(z), a.erf_form, sigmoidf_fast));
                     }
                 }
             }
@@ -378,6 +381,10 @@ __global__ __launch_bounds__(FR_THREADS) void fr_epilogue_kernel(const FwdArgs a
             }
             *(u32x2 *)(a.out + r * a.ldo + 2 * n) = u32x2{o[0], o[1]};
             if (a.aux2) *(uint32_t *)(a.aux2 + r * a.ldaux2 + n) = Elem<T>::pack(hv[0], hv[1]);
+        } else if constexpr (EPI == EPI_GELU_BWD) {
+            const uint32_t z = *(const uint32_t *)(a.aux + r * a.ldaux + n);
+            *(uint32_t *)(a.out + r * a.ldo + n) = Elem<T>::pack(v0 * sc * gelu_grad(Elem<T>::lo(z), a.erf_form, sigmoidf_fast),
+                                                                 v1 * sc * gelu_grad(Elem<T>::hi(z), a.erf_form, sigmoidf_fast));
         } else {
             const uint32_t z = Elem<T>::pack(v0 * sc, v1 * sc);
             if (a.out) *(uint32_t *)(a.out + dst * a.ldo + n) = z;
@@ -385,6 +392,8 @@ __global__ __launch_bounds__(FR_THREADS) void fr_epilogue_kernel(const FwdArgs a
                 const float g = Elem<T>::lo(z), u = Elem<T>::hi(z);
                 a.aux[dst * a.ldaux + (n >> 1)] = (uint16_t)(Elem<T>::pack(u * g * sigmoidf_fast(g), 0.f) & 0xffffu);
             }
+            if constexpr (EPI == EPI_GELU)
+                *(uint32_t *)(a.aux + dst * a.ldaux + n) = Elem<T>::pack(gelu(Elem<T>::lo(z), a.erf_form, sigmoidf_fast), gelu(Elem<T>::hi(z), a.erf_form, sigmoidf_fast));
         }
     }
 }
@@ -575,6 +584,13 @@ __global__ __launch_bounds__(FR_THREADS, 4) void fr_tile_kernel(const FwdArgs a,
                     }
                     *(u32x4 *)(a.out + r * a.ldo + 2 * n) = o;
                     if (a.aux2) *(u32x2 *)(a.aux2 + r * a.ldaux2 + n) = u32x2{Elem<T>::pack(hv[0], hv[1]), Elem<T>::pack(hv[2], hv[3])};
+                } else if constexpr (EPI == EPI_GELU_BWD) {
+                    const u32x2 z = *(const u32x2 *)(a.aux + r * a.ldaux + n);
+                    float d[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        d[q] = acc[4 * g + q] * sc * gelu_grad((q & 1) ? Elem<T>::hi(z[q >> 1]) : Elem<T>::lo(z[q >> 1]), a.erf_form, sigmoidf_fast);
+                    *(u32x2 *)(a.out + r * a.ldo + n) = u32x2{Elem<T>::pack(d[0], d[1]), Elem<T>::pack(d[2], d[3])};
                 } else {
                     float v[4];
 #pragma unroll
@@ -588,6 +604,11 @@ __global__ __launch_bounds__(FR_THREADS, 4) void fr_tile_kernel(const FwdArgs a,
                     if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) {
                         const float g0 = Elem<T>::lo(z0), u0 = Elem<T>::hi(z0), g1 = Elem<T>::lo(z1), u1 = Elem<T>::hi(z1);
                         *(uint32_t *)(a.aux + dst * a.ldaux + (n >> 1)) = Elem<T>::pack(u0 * g0 * sigmoidf_fast(g0), u1 * g1 * sigmoidf_fast(g1));
+                    }
+                    if constexpr (EPI == EPI_GELU) {
+                        const float h0 = gelu(Elem<T>::lo(z0), a.erf_form, sigmoidf_fast), h1 = gelu(Elem<T>::hi(z0), a.erf_form, sigmoidf_fast);
+                        const float h2 = gelu(Elem<T>::lo(z1), a.erf_form, sigmoidf_fast), h3 = gelu(Elem<T>::hi(z1), a.erf_form, sigmoidf_fast);
+                        *(u32x2 *)(a.aux + dst * a.ldaux + n) = u32x2{Elem<T>::pack(h0, h1), Elem<T>::pack(h2, h3)};
                     }
                 }
             }
@@ -648,7 +669,7 @@ template <typename T, int EPI> int fr_launch_epi(const FwdArgs &a, int w_is_kn, 
     // one pair of rows per wave instead of four where the rows are short or the launch would have few workgroups
     const int rows_per_wg = (a.K >= 2048 && (int64_t)(a.N / FR_NT_ROWS) * a.E >= 2048) ? FR_NT_ROWS : 8;
     const dim3 grid((a.N + rows_per_wg - 1) / rows_per_wg, a.E);
-    if constexpr (EPI == XMA_ROCM_EPI_SWIGLU_BWD) {
+    if constexpr (EPI == XMA_ROCM_EPI_SWIGLU_BWD || EPI == EPI_GELU_BWD) {
         fr_nt_kernel<T, -1><<<grid, FR_THREADS, 0, st>>>(a, part, rows_per_wg);
         if ((rc = xma_check_launch("fr_nt_kernel"))) return rc;
         return fr_launch_epilogue<T, EPI>(a, part, 1, st);
@@ -661,6 +682,8 @@ template <typename T, int EPI> int fr_launch_epi(const FwdArgs &a, int w_is_kn, 
 template <typename T> int fr_launch(const FwdArgs &a, int w_is_kn, int epilogue, float *part, hipStream_t st) {
     if (epilogue == XMA_ROCM_EPI_STORE) return fr_launch_epi<T, XMA_ROCM_EPI_STORE>(a, w_is_kn, part, st);
     if (epilogue == XMA_ROCM_EPI_SWIGLU) return fr_launch_epi<T, XMA_ROCM_EPI_SWIGLU>(a, w_is_kn, part, st);
+    if (epilogue == EPI_GELU) return fr_launch_epi<T, EPI_GELU>(a, w_is_kn, part, st);
+    if (epilogue == EPI_GELU_BWD) return fr_launch_epi<T, EPI_GELU_BWD>(a, w_is_kn, part, st);
     return fr_launch_epi<T, XMA_ROCM_EPI_SWIGLU_BWD>(a, w_is_kn, part, st);
 }
 
@@ -671,6 +694,8 @@ int split_sums_epilogue(const FwdArgs &a, const float *part, int S, int epilogue
         using T = decltype(elem);
         if (epilogue == XMA_ROCM_EPI_STORE) return fr_launch_epilogue<T, XMA_ROCM_EPI_STORE>(a, part, S, st);
         if (epilogue == XMA_ROCM_EPI_SWIGLU) return fr_launch_epilogue<T, XMA_ROCM_EPI_SWIGLU>(a, part, S, st);
+        if (epilogue == EPI_GELU) return fr_launch_epilogue<T, EPI_GELU>(a, part, S, st);
+        if (epilogue == EPI_GELU_BWD) return fr_launch_epilogue<T, EPI_GELU_BWD>(a, part, S, st);
         return fr_launch_epilogue<T, XMA_ROCM_EPI_SWIGLU_BWD>(a, part, S, st);
     };
     return dtype == XMA_ROCM_BF16 ? run(__bf16{}) : run(_Float16{});
@@ -685,7 +710,7 @@ extern "C" size_t xma_rocm_scatter2scatter_few_rows_workspace_bytes(int64_t M, i
     if (fr_takes_tile(M, K, E, w_is_kn)) { // the small MFMA tile, cut along K or not
         S = fr_tile_splits(N, K, E, w_is_kn);
         if (S == 1) return mid;
-    } else if (epilogue == XMA_ROCM_EPI_SWIGLU_BWD) {
+    } else if (epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == XMA_ROCM_EPI_GELU_TANH_BWD || epilogue == XMA_ROCM_EPI_GELU_ERF_BWD) {
         S = 1; // the vector kernel's sums go to the epilogue kernel
     } else {
         return mid; // the vector kernel finishes the job itself
@@ -707,8 +732,11 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
                                                  int epilogue, int dtype, void *workspace, size_t workspace_bytes,
                                                  void *stream) {
     XMA_REQUIRE(dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16, XMA_ROCM_EUNSUPPORTED, "scatter2scatter_few_rows: dtype %d", dtype);
-    XMA_REQUIRE(epilogue >= XMA_ROCM_EPI_STORE && epilogue <= XMA_ROCM_EPI_SWIGLU_BWD, XMA_ROCM_EINVAL,
+    XMA_REQUIRE(epilogue >= XMA_ROCM_EPI_STORE && epilogue <= XMA_ROCM_EPI_GELU_ERF_BWD && epilogue != 3, XMA_ROCM_EINVAL,
                 "scatter2scatter_few_rows: epilogue %d", epilogue);
+    const int erf_form = epilogue >= XMA_ROCM_EPI_GELU_ERF ? 1 : 0;
+    const int asked = epilogue;
+    if (erf_form) epilogue -= XMA_ROCM_EPI_GELU_ERF - XMA_ROCM_EPI_GELU_TANH;
     XMA_REQUIRE(M >= 0 && M <= 65535 && N >= 8 && K >= 8 && E >= 1 && E <= 65535 && fan_out >= 1, XMA_ROCM_EINVAL,
                 "scatter2scatter_few_rows: M=%lld N=%d K=%d E=%d fan_out=%d (M and E at most 65535)", (long long)M, N, K, E, fan_out);
     XMA_REQUIRE(N % 8 == 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldo % 8 == 0 && w_expert_stride % 8 == 0,
@@ -725,6 +753,9 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
     } else if (epilogue == XMA_ROCM_EPI_SWIGLU) {
         XMA_REQUIRE(aux && al16(aux) && ldaux % 8 == 0 && N % 16 == 0 && (!out || al16(out)), XMA_ROCM_EINVAL,
                     "scatter2scatter_few_rows: SWIGLU needs aux (M, N/2), ldaux %% 8 == 0, N %% 16 == 0");
+    } else if (epilogue == EPI_GELU) {
+        XMA_REQUIRE(out && aux && al16(out) && al16(aux) && ldaux % 8 == 0 && y_grouped && !row_scale, XMA_ROCM_EINVAL,
+                    "scatter2scatter_few_rows: GELU needs out (z), aux (M, N), y_grouped and no row scale");
     } else {
         XMA_REQUIRE(out && aux && al16(out) && al16(aux) && ldaux % 8 == 0 && y_grouped && !bias, XMA_ROCM_EINVAL,
                     "scatter2scatter_few_rows: SWIGLU_BWD needs out, aux (z), y_grouped and no bias");
@@ -733,7 +764,7 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
                 "scatter2scatter_few_rows: scaled activations go with SWIGLU_BWD, 16-byte aligned rows");
     XMA_REQUIRE(!bias || (al16(bias) && bias_expert_stride % 8 == 0 && bias_expert_stride >= 0), XMA_ROCM_EINVAL,
                 "scatter2scatter_few_rows: bias (E, N) must be 16-byte aligned with an expert stride that is a multiple of 8");
-    const size_t need = xma_rocm_scatter2scatter_few_rows_workspace_bytes(M, N, K, E, w_is_kn, epilogue);
+    const size_t need = xma_rocm_scatter2scatter_few_rows_workspace_bytes(M, N, K, E, w_is_kn, asked);
     XMA_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && al16(workspace)), XMA_ROCM_EWORKSPACE,
                 "scatter2scatter_few_rows: workspace of %zu bytes, %zu needed (16-byte aligned)", workspace ? workspace_bytes : (size_t)0, need);
     FwdArgs a;
@@ -764,6 +795,7 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
     a.partial = nullptr;
     a.split_cus = 0;
     a.grid_main = 0;
+    a.erf_form = erf_form;
     hipStream_t st = (hipStream_t)stream;
     if (fr_takes_mid(a, w_is_kn ? 1 : 0, epilogue)) return xma_rocm::mid_fwd(a, w_is_kn ? 1 : 0, epilogue, dtype, (float *)workspace, st);
     if (dtype == XMA_ROCM_BF16) return fr_launch<__bf16>(a, w_is_kn ? 1 : 0, epilogue, (float *)workspace, st);

@@ -28,6 +28,7 @@ struct FwdArgs {
     float *partial;  // workspace for the K slices of the tiles of the last round, or NULL (no tile is split)
     int split_cus;   // compute units of the device = tiles per round
     int grid_main;   // workgroups that take whole tiles (an upper bound of the tile count); split_cus more follow
+    int erf_form;    // which GELU (EPI_GELU, EPI_GELU_BWD)
 };
 
 struct DwArgs {

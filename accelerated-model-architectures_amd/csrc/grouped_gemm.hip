@@ -1717,6 +1717,7 @@ static int scatter2scatter_impl(const void *X, int64_t ldx, const void *W, int64
     a.partial = nullptr;
     a.split_cus = 0;
     a.grid_main = 0;
+    a.erf_form = 0;
     if (dtype == XMA_ROCM_F32) return f32_scatter2scatter(a, w_is_kn ? 1 : 0, epilogue, (hipStream_t)stream);
     const int64_t NT = (N + BN - 1) / BN;
     const int64_t max_m_tiles = M / BM + E; // sum_e ceil(c_e / BM) <= floor(M / BM) + E

@@ -29,6 +29,8 @@ constexpr int EPI_Z_STRIDE = 128 * 2 + 16, EPI_H_STRIDE = 64 * 2 + 16;
 // Internal epilogue code beside the public XMA_ROCM_EPI_*: SWIGLU_BWD with the second output FwdArgs::aux2.  A variant of
 // its own, so that the launches without that output keep their code and register allocation unchanged.
 constexpr int EPI_SWIGLU_BWD_SCALED_ACT = 3;
+// z and h = gelu(z), both (M, N); dz = gelu'(z) d h: FwdArgs::erf_form says which GELU
+constexpr int EPI_GELU = XMA_ROCM_EPI_GELU_TANH, EPI_GELU_BWD = XMA_ROCM_EPI_GELU_TANH_BWD;
 constexpr int EPI_WAVE_BYTES = 32 * EPI_Z_STRIDE + 32 * EPI_H_STRIDE;
 // SwiGLU backward stages 32 rows of 256 pre-activation columns per wave
 constexpr int EPI_BWD_STRIDE = 256 * 2 + 16, EPI_BWD_WAVE_BYTES = 32 * EPI_BWD_STRIDE;
@@ -91,7 +93,62 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
     // lane owns row (lane & 31) of each 32-row block; quad g of tile (j, i) holds
     //      columns n0 + wp + 32 j + 8 g + 4 (lane >> 5) + {0..3}
     const int lrow = lane & 31, lhalf = lane >> 5;
-    if constexpr (EPI != XMA_ROCM_EPI_SWIGLU_BWD && EPI != EPI_SWIGLU_BWD_SCALED_ACT) {
+    if constexpr (EPI == EPI_GELU_BWD) {
+        // as the SwiGLU backward below, with z and dz as wide as d h: 32 rows of 128 columns come in and leave through the
+        // staging area of the plain store
+        if (__builtin_amdgcn_readfirstlane(n0 + wp) >= a.N) return; // this wave's columns all lie past N
+        unsigned char *stage = smem + wave * EPI_WAVE_BYTES;
+        const int piece = (n0 + wp + (lane & 15) * 8 < a.N) ? (lane & 15) : 0;
+        const int cz = n0 + wp + piece * 8;
+        // a copy per form: a branch per element keeps the elements' instructions apart (16 experts of 512 rows, K = 1024, N = 4096: 128
+        // against 112 us here, 128 against 107 in the forward; plain store 87, and a pass over the tensors 33 and 39)
+        auto blocks = [&](auto ERF) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int rbase = wq + i * 32;
+            if (rbase >= rows_valid) break; // wave-uniform
+            u32x4 zin[8];
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                int r = rbase + 4 * it + (lane >> 4);
+                if (r >= rows_valid) r = rows_valid - 1;
+                zin[it] = *(const u32x4 *)(a.aux + (row0 + r) * a.ldaux + cz);
+            }
+            int r_lane = rbase + lrow;
+            if (r_lane >= rows_valid) r_lane = rows_valid - 1;
+            float sc = 1.f;
+            if (a.scale) sc = pre ? pre->sc[i] : Elem<T>::lo((uint32_t)a.scale[a.idx[row0 + r_lane]]);
+#pragma unroll
+            for (int it = 0; it < 8; ++it) *(u32x4 *)(stage + (4 * it + (lane >> 4)) * EPI_Z_STRIDE + (lane & 15) * 16) = zin[it];
+            wave_lds_sync();
+            unsigned char *mine = stage + lrow * EPI_Z_STRIDE + lhalf * 8;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    u32x2 *zp = (u32x2 *)(mine + (j * 32 + g * 8) * 2);
+                    const u32x2 z = *zp;
+                    float d[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        d[q] = acc[j][i][4 * g + q] * sc * gelu_grad((q & 1) ? Elem<T>::hi(z[q >> 1]) : Elem<T>::lo(z[q >> 1]), ERF.value, sigmoidf_fast);
+                    *zp = u32x2{Elem<T>::pack(d[0], d[1]), Elem<T>::pack(d[2], d[3])};
+                }
+            wave_lds_sync();
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                int br = 4 * it + (lane >> 4);
+                if (rbase + br >= rows_valid) br = rows_valid - 1 - rbase;
+                *(u32x4 *)(a.out + (row0 + rbase + br) * a.ldo + cz) = *(const u32x4 *)(stage + br * EPI_Z_STRIDE + piece * 16);
+            }
+            wave_lds_sync(); // the next block overwrites the area
+        }
+        };
+        if (a.erf_form)
+            blocks(IC<1>{});
+        else
+            blocks(IC<0>{});
+    } else if constexpr (EPI != XMA_ROCM_EPI_SWIGLU_BWD && EPI != EPI_SWIGLU_BWD_SCALED_ACT) {
         // A store instruction of the accumulator layout would touch 32 rows with 16 bytes each.  Instead every
         // 32-row block goes through a wave-private LDS area and leaves as whole rows: 16 lanes x 16 bytes per row of
         // 128 columns (8 lanes per row of the 64 activation columns), i.e. full 128-byte lines.
@@ -165,6 +222,34 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                     *(u32x4 *)(out0 + d * a.ldo) = v;
                 }
             }
+            if constexpr (EPI == EPI_GELU) { // the activations of the rounded z take the same way out
+                wave_lds_sync();
+                auto activate = [&](auto ERF) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            u32x2 *zp = (u32x2 *)(z_w + (j * 32 + g * 8) * 2);
+                            const u32x2 z = *zp;
+                            float h[4];
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) h[q] = gelu((q & 1) ? Elem<T>::hi(z[q >> 1]) : Elem<T>::lo(z[q >> 1]), ERF.value, sigmoidf_fast);
+                            *zp = u32x2{Elem<T>::pack(h[0], h[1]), Elem<T>::pack(h[2], h[3])};
+                        }
+                };
+                if (a.erf_form)
+                    activate(IC<1>{});
+                else
+                    activate(IC<0>{});
+                wave_lds_sync();
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    int r = rbase + 4 * it + (lane >> 4);
+                    if (r > last) r = last;
+                    const u32x4 v = *(const u32x4 *)(stage + (r - rbase) * EPI_Z_STRIDE + z_piece * 16);
+                    *(u32x4 *)(a.aux + (row0 + r) * a.ldaux + cz) = v;
+                }
+            }
             if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) {
 #pragma unroll
                 for (int it = 0; it < 4; ++it) {
@@ -178,7 +263,9 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
             wave_lds_sync(); // the next block overwrites the area
         }
         };
-        if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) { // the layer's form: grouped rows, no scale
+        if constexpr (EPI == EPI_GELU) { // grouped rows, no scale
+            blocks(IC<0>{}, IC<1>{});
+        } else if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) { // the layer's form: grouped rows, no scale
             if (a.y_grouped && !a.scale)
                 blocks(IC<0>{}, IC<1>{});
             else if (a.y_grouped)

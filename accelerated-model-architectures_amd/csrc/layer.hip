@@ -17,6 +17,11 @@ int gemm(const xma_rocm_moe *m, int64_t few, const void *X, const void *W, int64
          int64_t ldaux, void *aux2, const void *scale, const void *bias, int64_t N, int64_t K, int64_t fan_out, int x_grouped, int y_grouped,
          int epilogue, void *stream) {
     const int64_t M = m->T * m->k, ldo = epilogue == XMA_ROCM_EPI_SWIGLU_BWD ? 2 * N : N;
+    if (epilogue >= XMA_ROCM_EPI_GELU_TANH && !few) { // no epilogue of the 256 x 256 kernels: a pass of its own
+        const int form = epilogue >= XMA_ROCM_EPI_GELU_ERF, bwd = epilogue & 1;
+        RUN(gemm(m, 0, X, W, w_es, ldw, w_is_kn, out, nullptr, 0, nullptr, scale, bias, N, K, fan_out, x_grouped, y_grouped, XMA_ROCM_EPI_STORE, stream));
+        return bwd ? xma_rocm_gelu_backward(aux, out, out, M * N, form, (int)m->dtype, stream) : xma_rocm_gelu_forward(out, aux, M * N, form, (int)m->dtype, stream);
+    }
     const int64_t *idx = (const int64_t *)m->sorted_scattered_idxs, *offs = (const int64_t *)m->expert_offsets;
     if (few)
         return xma_rocm_scatter2scatter_few_rows(X, K, W, w_es, ldw, w_is_kn, idx, offs, out, ldo, aux, ldaux, aux2, aux2 ? N : 0, scale, bias,
@@ -57,7 +62,15 @@ int check(const xma_rocm_moe *m, const char *what) {
     XMA_REQUIRE(m->x && m->w_fc && m->w_proj && m->router_weights && m->expert_ids && m->expert_offsets && m->sorted_scattered_idxs && m->z &&
                     m->expert_out,
                 XMA_ROCM_EINVAL, "%s: null buffer", what);
+    XMA_REQUIRE(m->activation == 0 || ((m->activation == 1 || m->activation == 2) && !m->recompute && m->dw2_form != 1), XMA_ROCM_EINVAL,
+                "%s: activation %lld goes without recomputation and scaled activations", what, (long long)m->activation);
     return XMA_ROCM_OK;
+}
+
+int64_t up_width(const xma_rocm_moe *m) { return m->activation ? m->I : 2 * m->I; }
+int epilogue_of(const xma_rocm_moe *m, int bwd) {
+    if (m->activation == 0) return bwd ? XMA_ROCM_EPI_SWIGLU_BWD : XMA_ROCM_EPI_SWIGLU;
+    return (m->activation == 1 ? XMA_ROCM_EPI_GELU_TANH : XMA_ROCM_EPI_GELU_ERF) + bwd;
 }
 
 } // namespace
@@ -74,8 +87,8 @@ extern "C" int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream) {
         RUN(xma_rocm_router_topk(m->logits, m->E, m->T, (int32_t)m->E, (int32_t)m->k, dtype, m->router_weights, m->expert_ids, 0, stream));
     RUN(xma_rocm_route(m->expert_ids, 0, M, (int32_t)m->E, (uint32_t *)m->counts, (int64_t *)m->expert_offsets, nullptr, nullptr,
                        (int64_t *)m->sorted_scattered_idxs, m->workspace, (size_t)m->workspace_bytes, stream));
-    RUN(gemm(m, m->few_up, m->x, m->w_fc, 2 * m->I * m->H, m->H, 0, m->z, m->h, m->I, nullptr, nullptr, m->b_fc, 2 * m->I, m->H, m->k, 0, 1,
-             XMA_ROCM_EPI_SWIGLU, stream));
+    const int64_t U = up_width(m);
+    RUN(gemm(m, m->few_up, m->x, m->w_fc, U * m->H, m->H, 0, m->z, m->h, m->I, nullptr, nullptr, m->b_fc, U, m->H, m->k, 0, 1, epilogue_of(m, 0), stream));
     RUN(down_projection(m, stream));
     return xma_rocm_combine(m->expert_out, m->H, m->router_weights, m->y, m->H, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream);
 }
@@ -101,11 +114,11 @@ extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
                     (m->dw2_form == 0 || m->dw2_operand) && (!m->d_b_fc || m->b_fc) && (!m->d_b_proj || m->b_proj),
                 XMA_ROCM_EINVAL, "moe_backward: null buffer");
     const int dtype = (int)m->dtype;
-    const int64_t M = m->T * m->k, H = m->H, I = m->I;
+    const int64_t M = m->T * m->k, H = m->H, I = m->I, U = up_width(m);
     const int64_t *idx = (const int64_t *)m->sorted_scattered_idxs, *offs = (const int64_t *)m->expert_offsets;
     // dX2 + SwiGLU', with the scaled activations for dW2 where that takes dy through the index
-    RUN(gemm(m, m->few_dx2, m->dy, m->w_proj, H * I, I, 1, m->dz, m->z, 2 * I, m->dw2_form == 1 ? m->dw2_operand : nullptr, m->router_weights,
-             nullptr, I, H, m->k, 0, 1, XMA_ROCM_EPI_SWIGLU_BWD, stream));
+    RUN(gemm(m, m->few_dx2, m->dy, m->w_proj, H * I, I, 1, m->dz, m->z, U, m->dw2_form == 1 ? m->dw2_operand : nullptr, m->router_weights,
+             nullptr, I, H, m->k, 0, 1, epilogue_of(m, 1), stream));
     if (m->dw2_form == 1) {
         RUN(dw(m, m->few_dw2, m->dy, 0, nullptr, m->dw2_operand, 1, m->d_w_proj, H, I, stream));
         if (m->d_b_proj)
@@ -118,10 +131,10 @@ extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
     } else { // the loader of the few-row kernel gathers and scales
         RUN(dw(m, m->few_dw2, m->dy, 0, m->router_weights, m->h, 1, m->d_w_proj, H, I, stream));
     }
-    RUN(dw(m, m->few_dw1, m->dz, 1, nullptr, m->x, 0, m->d_w_fc, 2 * I, H, stream));
+    RUN(dw(m, m->few_dw1, m->dz, 1, nullptr, m->x, 0, m->d_w_fc, U, H, stream));
     if (m->d_b_fc)
-        RUN(xma_rocm_expert_column_sums(m->dz, 2 * I, nullptr, 1, nullptr, offs, m->d_b_fc, 2 * I, (int32_t)(2 * I), (int32_t)m->E, dtype, stream));
-    RUN(gemm(m, m->few_dx1, m->dz, m->w_fc, 2 * I * H, H, 1, m->scattered, nullptr, 0, nullptr, nullptr, nullptr, H, 2 * I, 1, 1, 0,
+        RUN(xma_rocm_expert_column_sums(m->dz, U, nullptr, 1, nullptr, offs, m->d_b_fc, U, (int32_t)U, (int32_t)m->E, dtype, stream));
+    RUN(gemm(m, m->few_dx1, m->dz, m->w_fc, U * H, H, 1, m->scattered, nullptr, 0, nullptr, nullptr, nullptr, H, U, 1, 1, 0,
              XMA_ROCM_EPI_STORE, stream));
     return xma_rocm_combine_add(m->scattered, H, nullptr, m->d_x_addend, H, m->d_x, H, m->T, (int32_t)m->k, (int32_t)H, dtype, stream);
 }

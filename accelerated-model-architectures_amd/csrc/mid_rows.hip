@@ -626,7 +626,11 @@ template <typename T, int WT, int EPI> int mid_launch_fwd(const FwdArgs &a, floa
 }
 
 template <typename T> int mid_dispatch_fwd(const FwdArgs &a, int wt, int epi, float *part, hipStream_t st) {
-    if (wt == 0) return epi == XMA_ROCM_EPI_STORE ? mid_launch_fwd<T, 0, XMA_ROCM_EPI_STORE>(a, part, st) : mid_launch_fwd<T, 0, XMA_ROCM_EPI_SWIGLU>(a, part, st);
+    if (wt == 0) {
+        if (epi == XMA_ROCM_EPI_STORE) return mid_launch_fwd<T, 0, XMA_ROCM_EPI_STORE>(a, part, st);
+        return epi == XMA_ROCM_EPI_SWIGLU ? mid_launch_fwd<T, 0, XMA_ROCM_EPI_SWIGLU>(a, part, st) : mid_launch_fwd<T, 0, EPI_GELU>(a, part, st);
+    }
+    if (epi == EPI_GELU_BWD) return mid_launch_fwd<T, 1, EPI_GELU_BWD>(a, part, st);
     if (epi == XMA_ROCM_EPI_STORE) return mid_launch_fwd<T, 1, XMA_ROCM_EPI_STORE>(a, part, st);
     if (a.aux2) return mid_launch_fwd<T, 1, EPI_SWIGLU_BWD_SCALED_ACT>(a, part, st);
     return mid_launch_fwd<T, 1, XMA_ROCM_EPI_SWIGLU_BWD>(a, part, st);
@@ -654,7 +658,8 @@ size_t mid_fwd_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E) {
 
 bool mid_fwd_takes(const FwdArgs &a, int wt, int epi) {
     // the operand layouts the layer launches: x @ W^T and dy @ W, each with the epilogues of its own
-    if (a.E > MR_MAX_E || (wt == 0 ? epi == XMA_ROCM_EPI_SWIGLU_BWD : epi == XMA_ROCM_EPI_SWIGLU)) return false;
+    const bool bwd = epi == XMA_ROCM_EPI_SWIGLU_BWD || epi == EPI_GELU_BWD;
+    if (a.E > MR_MAX_E || (epi != XMA_ROCM_EPI_STORE && (wt == 1) != bwd)) return false;
     const int64_t x_rows = a.x_grouped ? MR_BM : (a.M + a.fan_out - 1) / a.fan_out; // 32-bit byte offsets from a tile's base
     return a.M > 0 && a.M <= 65535 && x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)MR_BN * a.ldw * 2 < ((int64_t)1 << 32);
 }
@@ -664,7 +669,11 @@ bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
     // ones (8 experts of 176 rows, K = 28672: 470 against 516 us; K = 14336, 268 against 281; 320 rows 340 against 428)
     if (K > 8192 && M > (int64_t)112 * E) return false;
     int S;
-    return mid_fwd_seconds(M, N, K, E, epilogue, &S) < 0.96 * tiles256_seconds(M, N, K, E, epilogue); // even: as it was
+    // without an epilogue of their own for GELU the 256 x 256 tiles leave it to a pass over two or three tensors
+    const bool gelu = epilogue >= XMA_ROCM_EPI_GELU_TANH;
+    const double pass = gelu ? ((epilogue & 1) ? 6.0 : 4.0) * M * N / 4.5e12 + 4e-6 : 0.;
+    const int as = gelu ? XMA_ROCM_EPI_STORE : epilogue;
+    return mid_fwd_seconds(M, N, K, E, as, &S) < 0.96 * (tiles256_seconds(M, N, K, E, as) + pass); // even: as it was
 }
 
 int mid_fwd(const FwdArgs &a, int wt, int epi, int dtype, float *part, hipStream_t st) {

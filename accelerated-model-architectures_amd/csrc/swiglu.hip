@@ -269,3 +269,60 @@ int xma_swiglu_packed_backward_elems(const void *x, int64_t ldx, const void *dy,
         swiglu_bwd_elem_kernel<float, 2><<<grid, SW_THREADS, 0, st>>>(x, ldx, x, ldx, dy, lddy, dx, lddx, dx, lddx, rows, c0, cols_out, make_fastdiv(cols_out - c0));
     return xma_check_launch("swiglu_bwd_elem_kernel (packed)");
 }
+
+// ------------------------------------------------------------------------------------------------
+// GELU of the layer's pre-activations and its gradient, for the launches whose GEMM has no epilogue for it.  HBM-bound: 2 and 3
+// elements of traffic per element, one 16-byte access per operand and thread.
+// ------------------------------------------------------------------------------------------------
+namespace {
+
+template <typename ST, int BWD>
+__global__ __launch_bounds__(SW_THREADS) void gelu_kernel(const void *__restrict__ x, const void *dy, void *y, int64_t n, int form) {
+    constexpr int V = Scalar<ST>::VEC;
+    const int64_t i = ((int64_t)blockIdx.x * SW_THREADS + threadIdx.x) * V;
+    auto one = [&](float z, float d) {
+        if (V == 4 && form == 0) { // fp32 results: through tanhf, which loses less than the sigmoid's sum and quotient
+            const float t = tanhf(0.79788456f * (z + 0.044715f * z * z * z));
+            if constexpr (BWD == 0) return 0.5f * z * (1.f + t);
+            return d * (0.5f * (1.f + t) + 0.5f * z * (1.f - t * t) * 0.79788456f * (1.f + 0.134145f * z * z));
+        }
+        return BWD ? d * gelu_grad(z, form, sigmoidf_fast) : gelu(z, form, sigmoidf_fast);
+    };
+    if (i + V <= n) {
+        const Vec<ST> z = Vec<ST>::load(x, i);
+        Vec<ST> d = z, o;
+        if constexpr (BWD != 0) d = Vec<ST>::load(dy, i);
+#pragma unroll
+        for (int q = 0; q < V; ++q) o.v[q] = one(z.v[q], d.v[q]);
+        o.store(y, i);
+    } else {
+        for (int64_t j = i; j < n; ++j) Scalar<ST>::put(y, j, one(Scalar<ST>::get(x, j), BWD ? Scalar<ST>::get(dy, j) : 0.f));
+    }
+}
+
+template <int BWD> int launch_gelu(const void *x, const void *dy, void *y, int64_t n, int form, int dtype, void *stream) {
+    XMA_REQUIRE(dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16 || dtype == XMA_ROCM_F32, XMA_ROCM_EUNSUPPORTED, "gelu: dtype %d", dtype);
+    auto al16 = [](const void *p) { return p && ((uintptr_t)p & 15) == 0; };
+    const int64_t blocks = (n + (dtype == XMA_ROCM_F32 ? 4 : 8) * SW_THREADS - 1) / ((dtype == XMA_ROCM_F32 ? 4 : 8) * SW_THREADS);
+    XMA_REQUIRE(n >= 0 && blocks < ((int64_t)1 << 31) && (form == 0 || form == 1), XMA_ROCM_EINVAL, "gelu: n=%lld form=%d", (long long)n, form);
+    if (n == 0) return XMA_ROCM_OK;
+    XMA_REQUIRE(al16(x) && al16(y) && (!BWD || al16(dy)), XMA_ROCM_EINVAL, "gelu: null or misaligned pointer");
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == XMA_ROCM_BF16)
+        gelu_kernel<__bf16, BWD><<<(unsigned)blocks, SW_THREADS, 0, st>>>(x, dy, y, n, form);
+    else if (dtype == XMA_ROCM_F16)
+        gelu_kernel<_Float16, BWD><<<(unsigned)blocks, SW_THREADS, 0, st>>>(x, dy, y, n, form);
+    else
+        gelu_kernel<float, BWD><<<(unsigned)blocks, SW_THREADS, 0, st>>>(x, dy, y, n, form);
+    return xma_check_launch("gelu_kernel");
+}
+
+} // namespace
+
+extern "C" int xma_rocm_gelu_forward(const void *x, void *y, int64_t n, int form, int dtype, void *stream) {
+    return launch_gelu<0>(x, nullptr, y, n, form, dtype, stream);
+}
+
+extern "C" int xma_rocm_gelu_backward(const void *x, const void *dy, void *dx, int64_t n, int form, int dtype, void *stream) {
+    return launch_gelu<1>(x, dy, dx, n, form, dtype, stream);
+}

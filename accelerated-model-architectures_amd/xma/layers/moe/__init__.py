@@ -108,7 +108,7 @@ class MoE(nn.Module):
         return x.view(original_shape), router_logits
 
     def _runs_as_one_call(self, kernel_backend: KernelBackend | None) -> bool:
-        """rocm backend, packed SwiGLU, and the two parts below as they are written here"""
+        """rocm backend, and the two parts below as they are written here"""
         if kernel_backend is None:
             kernel_backend = Accelerator.get_kernel_backend()
         elif kernel_backend == KernelBackend.rocm:
@@ -116,8 +116,6 @@ class MoE(nn.Module):
         cls, own = type(self), self.__dict__
         return (
             kernel_backend == KernelBackend.rocm
-            and self.is_glu
-            and getattr(self.act, "_xma_fused_activation", None) == "swiglu_packed"
             and cls._compute_experts is MoE._compute_experts
             and cls._compute_routing_weights is MoE._compute_routing_weights
             and "_compute_experts" not in own

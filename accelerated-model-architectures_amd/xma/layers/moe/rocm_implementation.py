@@ -406,12 +406,12 @@ def fused_swiglu_experts(x, w_fc, w_proj, router_weights, sorted_scattered_idxs,
 
 
 # ----------------------------------------------------------------------------------------- the layer as one call
-# A pass of a handful of tokens is as long as its host work, so the layer with packed SwiGLU runs as one autograd node, whose
+# A pass of a handful of tokens is as long as its host work, so the layer with packed SwiGLU or GELU runs as one autograd node, whose
 # forward and backward are one library call each (two around the gate's own products), on scratch that is laid out once per shape:
 # the same launches as the ops above, bit for bit.  Everything else (other activations, tracing, transforms, tensors that the
 # entry point does not describe) goes through the ops.
 _BLOCK_POINTERS = struct.Struct("29Q")
-_BLOCK_SIZES = struct.Struct("16q")
+_BLOCK_SIZES = struct.Struct("17q")
 
 
 class _Plan:
@@ -429,8 +429,11 @@ def _layout(sizes: dict[str, int]) -> tuple[dict[str, int], int]:
 
 
 @lru_cache(maxsize=4096)
-def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, b_proj: bool, save: bool, device_index: int, _limits) -> _Plan:
+def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, b_proj: bool, save: bool, device_index: int, _limits) -> _Plan:
     M, s = T * k, dtype.itemsize
+    glu = act == "swiglu_packed"
+    U = 2 * I if glu else I  # width of the up-projection
+    epi_fwd, epi_bwd = (ops.EPI_SWIGLU, ops.EPI_SWIGLU_BWD) if glu else ops.EPI_GELU[act]
     few16 = dtype != torch.float32
 
     def gemm(N, K, w_is_kn, ldw, x_span, epilogue):
@@ -443,22 +446,22 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, b_proj: bo
         return int(ops._few_rows(M, E, dtype, "dW") or (
             not scaled and ops._mid_rows_dw(M, N_out, K_in, E, dtype) and M * max(N_out, K_in) < ops.MID_ROWS_OFFSETS))
 
-    up, down = gemm(2 * I, H, 0, H, T * H, ops.EPI_SWIGLU), gemm(H, I, 0, I, M * I, ops.EPI_STORE)
-    dx2, dx1 = gemm(I, H, 1, I, T * H, ops.EPI_SWIGLU_BWD), gemm(H, 2 * I, 1, H, M * 2 * I, ops.EPI_STORE)
+    up, down = gemm(U, H, 0, H, T * H, epi_fwd), gemm(H, I, 0, I, M * I, ops.EPI_STORE)
+    dx2, dx1 = gemm(I, H, 1, I, T * H, epi_bwd), gemm(H, U, 1, H, M * U, ops.EPI_STORE)
     # the operand of dW2: see xma_rocm_moe in the library's header
-    if few16 and _scale_by_top_k(k):
+    if few16 and glu and _scale_by_top_k(k):
         dw2_form, dw2_operand = 1, M * I * s
     elif not b_proj and ops._dw_loader_scales(M, E, dtype):
         dw2_form, dw2_operand = 0, 0
     else:
         dw2_form, dw2_operand = 2, M * H * s
     keep_h = save and dw2_form != 1
-    sizes = dict(weights=M * s, ids=M * 4, offsets=E * 8, idx=M * 8, z=M * 2 * I * s)
+    sizes = dict(weights=M * s, ids=M * 4, offsets=E * 8, idx=M * 8, z=M * U * s)
     temp = dict(counts=E * 4, workspace=max(ops.route_workspace_elements(M, E) * 4, up[1], down[1]))
     (sizes if keep_h else temp)["h"] = M * I * s
     (sizes if save else temp)["out"] = M * H * s
     # the scattered rows of dX1 take the place of dW2's operand
-    back = dict(d_weights=M * s, dz=M * 2 * I * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], 256))
+    back = dict(d_weights=M * s, dz=M * U * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], 256))
     if not save:
         back |= dict(h=M * I * s, out=M * H * s)
     p = _Plan()
@@ -466,19 +469,19 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, b_proj: bo
     p.temp, p.temp_bytes = _layout(temp)
     p.back, p.back_bytes = _layout(back)
     p.recompute = not save
-    few = (up[0], down[0], dx2[0], dw(H, I, dw2_form == 0), dw(2 * I, H, False), dx1[0], dw2_form, int(not save))
-    block = _BLOCK_SIZES.size + _BLOCK_POINTERS.size
-    p.sizes_forward = _BLOCK_SIZES.pack(block, T, H, I, E, k, ops._DTYPE_CODE[dtype], *few, temp["workspace"])
-    p.sizes_backward = _BLOCK_SIZES.pack(block, T, H, I, E, k, ops._DTYPE_CODE[dtype], *few, back["workspace"])
+    few = (up[0], down[0], dx2[0], dw(H, I, dw2_form == 0), dw(U, H, False), dx1[0], dw2_form, int(not save))
+    head = (_BLOCK_SIZES.size + _BLOCK_POINTERS.size, T, H, I, E, k, ops._DTYPE_CODE[dtype], ("swiglu_packed", "tanh", "none").index(act), *few)
+    p.sizes_forward = _BLOCK_SIZES.pack(*head, temp["workspace"])
+    p.sizes_backward = _BLOCK_SIZES.pack(*head, back["workspace"])
     return p
 
 
-def _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, save, grad):
+def _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, save, grad):
     """(y, logits, kept buffer, plan); gate_weight None: the logits are given"""
     T, H = x.shape
     E, I = w_proj.size(0), w_proj.size(2)
     device = x.device
-    p = _plan(T, H, I, E, k, x.dtype, b_proj is not None, save, device.index, (ops.FEW_ROWS_MAX, *ops.FEW_ROWS_PER_EXPERT.values()))
+    p = _plan(T, H, I, E, k, x.dtype, act, b_proj is not None, save, device.index, (ops.FEW_ROWS_MAX, *ops.FEW_ROWS_PER_EXPERT.values()))
     y = torch.empty_like(x)
     if gate_weight is not None:
         logits = torch.empty(T, E, dtype=x.dtype, device=device)
@@ -508,8 +511,8 @@ class _Layer(torch.autograd.Function):
     """the whole layer: with gate_weight (logits None) -> (y, logits), with given logits -> y"""
 
     @staticmethod
-    def forward(ctx, x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, save):
-        y, logits, kept, ctx.plan = _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, save, True)
+    def forward(ctx, x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, save):
+        y, logits, kept, ctx.plan = _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, save, True)
         ctx.save_for_backward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, kept)
         ctx.set_materialize_grads(False)
         return y if gate_weight is None else (y, logits)
@@ -520,9 +523,9 @@ class _Layer(torch.autograd.Function):
         need_x, need_gate, need_logits = ctx.needs_input_grad[:3]
         if dy is None:  # nothing but the logits was used
             if d_logits_out is None:
-                return (None,) * 9
+                return (None,) * 10
             d_x = d_logits_out @ gate_weight if need_x else None
-            return d_x, _gate_weight_grad(d_logits_out, x) if need_gate else None, None, None, None, None, None, None, None
+            return d_x, _gate_weight_grad(d_logits_out, x) if need_gate else None, *(None,) * 8
         dy = dy.contiguous()
         p = ctx.plan
         scratch = torch.empty(p.back_bytes, dtype=torch.uint8, device=x.device)
@@ -550,7 +553,19 @@ class _Layer(torch.autograd.Function):
                 d_gate = _gate_weight_grad(d_logits, x)
         check(lib.xma_rocm_moe_backward(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0 if d_x_gate is None else d_x_gate.data_ptr()),
                                         stream), "xma_rocm_moe_backward")
-        return d_x, d_gate, d_logits if need_logits else None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None
+        return d_x, d_gate, d_logits if need_logits else None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None, None
+
+
+def _activation(moe) -> str | None:
+    """the layer's activation where the library has it: packed SwiGLU, or GELU in either form as a module that nothing hooks into"""
+    act = moe.act
+    if moe.is_glu:
+        return "swiglu_packed" if getattr(act, "_xma_fused_activation", None) == "swiglu_packed" else None
+    if type(act) is not torch.nn.GELU or act.approximate not in ops.EPI_GELU or torch.nn.modules.module._has_any_global_hook():
+        return None
+    if act._forward_hooks or act._forward_pre_hooks or act._backward_hooks or act._backward_pre_hooks or "forward" in act.__dict__:
+        return None
+    return act.approximate
 
 
 def _plain(t: torch.Tensor, like: torch.Tensor) -> bool:
@@ -559,17 +574,21 @@ def _plain(t: torch.Tensor, like: torch.Tensor) -> bool:
 
 
 def layer(moe, x: torch.Tensor):
-    """(y, router logits) of a layer with packed SwiGLU whose tensors the library's layer entry point describes: contiguous, one
+    """(y, router logits) of a layer with packed SwiGLU or GELU whose tensors the library's layer entry point describes: contiguous, one
     dtype and device, aligned; None for anything else, and under function transforms and forward-mode differentiation"""
     w_fc, w_proj, b_fc, b_proj = moe.c_fc.weight, moe.c_proj.weight, moe.c_fc.bias, moe.c_proj.bias
     gate, k = moe.gate, moe.top_k
     T, H = x.shape
+    act = _activation(moe)
+    if act is None:
+        return None
     if T == 0 or x.dtype not in ops._DTYPE_CODE or type(x) not in (torch.Tensor, torch.nn.Parameter) or x.data_ptr() % 16 or not x.is_contiguous():
         return None
     if not (_plain(w_fc, x) and _plain(w_proj, x)) or (b_fc is not None and not _plain(b_fc, x)) or (b_proj is not None and not _plain(b_proj, x)):
         return None
-    E, I2, _ = w_fc.shape
-    if H % 8 or I2 % 16 or w_fc.size(2) != H or w_proj.shape != (E, H, I2 // 2) or E > 16384 or T * k >= 1 << 31:
+    E, U, _ = w_fc.shape
+    I = U // 2 if act == "swiglu_packed" else U
+    if H % 8 or I % 8 or (act == "swiglu_packed" and U % 2) or w_fc.size(2) != H or w_proj.shape != (E, H, I) or E > 16384 or T * k >= 1 << 31:
         return None
     if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
         return None
@@ -581,8 +600,8 @@ def layer(moe, x: torch.Tensor):
         if logits.shape != (T, E) or not _plain(logits, x):  # a gate that casts, for one
             return moe._compute_experts(x, *router_topk(logits, k)), logits
         tensors = (x, logits, w_fc, w_proj, b_fc, b_proj)
-    save = moe.save_activations
+    save = bool(moe.save_activations) or act != "swiglu_packed"
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
-        out = _Layer.apply(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, bool(save))
+        out = _Layer.apply(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, save)
         return out if logits is None else (out, logits)
-    return _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, True, False)[:2]
+    return _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, True, False)[:2]

@@ -21,6 +21,7 @@ from .loader import check, get_library
 _DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 EPI_STORE, EPI_SWIGLU, EPI_SWIGLU_BWD = 0, 1, 2
+EPI_GELU = {"tanh": (4, 5), "none": (6, 7)}  # forward, backward; few-row entry point only
 
 
 # A step of a handful of tokens is as long as its host work: what runs once per op and argument is kept to few calls.  The
@@ -209,7 +210,7 @@ def _mid_rows_fwd(M: int, N: int, K: int, E: int, w_is_kn: int, ldw: int, x_span
     if not 0 < M <= MID_ROWS_MAX or FEW_ROWS_MAX == 0 or dtype not in (torch.bfloat16, torch.float16):
         return False
     # what the tiles cover: the layouts that the layer launches, offsets that fit
-    if epilogue != EPI_STORE and w_is_kn != (epilogue == EPI_SWIGLU_BWD):
+    if epilogue != EPI_STORE and w_is_kn != (epilogue in (EPI_SWIGLU_BWD, 5, 7)):
         return False
     if E > MID_ROWS_MAX_EXPERTS or x_span >= MID_ROWS_OFFSETS or 256 * ldw >= MID_ROWS_OFFSETS:
         return False

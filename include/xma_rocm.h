@@ -49,6 +49,11 @@ extern "C" {
 /* epilogues of xma_rocm_scatter2scatter */
 #define XMA_ROCM_EPI_STORE 0      /* out = acc (optionally * row_scale) */
 #define XMA_ROCM_EPI_SWIGLU 1     /* up-projection: out = z (pre-activation, may be NULL), aux = swiglu_packed(z) */
+/* few-row entry point only, rows in grouped order; tanh approximation or erf form */
+#define XMA_ROCM_EPI_GELU_TANH 4     /* out = z, aux (M, N) = gelu(z) */
+#define XMA_ROCM_EPI_GELU_TANH_BWD 5 /* aux (M, N) = saved z, out = dz = gelu'(z) * (acc * row_scale) */
+#define XMA_ROCM_EPI_GELU_ERF 6
+#define XMA_ROCM_EPI_GELU_ERF_BWD 7
 #define XMA_ROCM_EPI_SWIGLU_BWD 2 /* down-projection dX: aux = saved z, out = dz = swiglu_packed'(z) * (acc * row_scale) */
 
 XMA_API int xma_rocm_abi_version(void);
@@ -343,6 +348,10 @@ XMA_API int xma_rocm_router_gate_topk(const void *x, int64_t ldx, const void *ga
 XMA_API int xma_rocm_router_topk_bwd(const void *logits, int64_t ld, int64_t T, int32_t E, int32_t k, int dtype, const void *ids,
                              int ids_is_i64, const void *d_weights, void *d_logits, int64_t ldd, void *stream);
 
+/* y = gelu(x); dx = gelu'(x) * dy (dx may be dy), n elements, 16-byte aligned; form 0: tanh approximation, 1: erf */
+XMA_API int xma_rocm_gelu_forward(const void *x, void *y, int64_t n, int form, int dtype, void *stream);
+XMA_API int xma_rocm_gelu_backward(const void *x, const void *dy, void *dx, int64_t n, int form, int dtype, void *stream);
+
 /*
  * The layer as one call: the launches of the entry points above in their order, on buffers that the caller has laid out
  * (MoE.forward, xma/layers/moe/__init__.py:170-262, with packed SwiGLU, and its backward).  Everything is row-major without gaps
@@ -356,6 +365,7 @@ XMA_API int xma_rocm_router_topk_bwd(const void *logits, int64_t ld, int64_t T, 
 typedef struct xma_rocm_moe {
     int64_t size; /* sizeof(xma_rocm_moe) */
     int64_t T, H, I, E, k, dtype;
+    int64_t activation;  /* 0: packed SwiGLU; 1, 2: GELU, tanh / erf form, of an up-projection of width I (2I below reads I) */
     int64_t few_up, few_down, few_dx2, few_dw2, few_dw1, few_dx1, dw2_form, recompute, workspace_bytes;
     const void *x, *gate_weight, *w_fc, *w_proj, *b_fc, *b_proj;       /* (T,H) (E,H) (E,2I,H) (E,H,I) (E,2I) (E,H) */
     void *logits, *router_weights, *expert_ids, *counts;                /* (T,E) (T,k) int32 (T,k) uint32 (E) */

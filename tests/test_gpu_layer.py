@@ -7,6 +7,9 @@ import torch.nn as nn
 from xma.functional import swiglu_packed
 from xma.layers import MoE
 
+from .test_gpu_ops import _tol
+from .utils import nerr
+
 
 pytestmark = pytest.mark.gpu
 
@@ -16,13 +19,14 @@ class _ThroughOps(MoE):
         return super()._compute_experts(*args, **kwargs)
 
 
-def _layers(T, E, k, H, I, dtype, bias=False, save=True, seed=3):
+def _layers(T, E, k, H, I, dtype, bias=False, save=True, seed=3, act=swiglu_packed):
     torch.manual_seed(seed)
-    one = MoE(E, k, H, I, swiglu_packed, True, add_bias=bias, std=0.05)
+    glu = act is swiglu_packed
+    one = MoE(E, k, H, I, act, glu, add_bias=bias, std=0.05)
     if bias:
         nn.init.normal_(one.c_fc.bias)
         nn.init.normal_(one.c_proj.bias)
-    ops = _ThroughOps(E, k, H, I, swiglu_packed, True, add_bias=bias, std=0.05)
+    ops = _ThroughOps(E, k, H, I, act, glu, add_bias=bias, std=0.05)
     ops.load_state_dict(one.state_dict())
     one, ops = one.to("cuda", dtype), ops.to("cuda", dtype)
     one.save_activations = ops.save_activations = save
@@ -122,3 +126,30 @@ def test_two_passes_before_the_backward():
         y1.backward(dy)
         got.append([x1.grad, x2.grad, *(p.grad for p in moe.parameters())])
     _same(*got)
+
+
+@pytest.mark.parametrize("form,bias", [("tanh", False), ("tanh", True), ("none", True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", [*CASES, (5, 8, 2, 64, 2048), (700, 4, 2, 1024, 264)])
+def test_gelu_matches_the_ops(case, dtype, form, bias):
+    """GELU in the epilogues (or passes) of the library against the ops with torch's GELU between them; the gradient of the
+    pre-activations is not rounded in between here, hence agreement within the bar of the ops"""
+    from xma.layers.moe import rocm_implementation as R
+
+    T, E, k, H, I = case
+    one, ops, x, dy = _layers(T, E, k, H, I, dtype, bias, act=nn.GELU(approximate=form))
+    with torch.no_grad():
+        got = R.layer(one, x)
+        assert got is not None and R._activation(ops) == form
+        for a, b in zip(got, ops(x)):
+            assert torch.isfinite(a).all() and nerr(a, b) <= _tol(dtype)
+    for a, b in zip(_step(one, x, dy), _step(ops, x, dy)):
+        assert torch.isfinite(a).all() and nerr(a, b) <= _tol(dtype)
+
+
+def test_hooked_activation_is_called():
+    one, _, x, _ = _layers(9, 8, 2, 64, 32, torch.bfloat16, act=nn.GELU(approximate="tanh"))
+    calls = []
+    one.act.register_forward_hook(lambda *a: calls.append(1))
+    one(x)
+    assert calls
