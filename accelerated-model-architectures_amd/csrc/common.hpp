@@ -21,6 +21,10 @@ void xma_set_error(const char *fmt, ...);
 int xma_check_launch(const char *what);
 // hipFuncSetAttribute(MaxDynamicSharedMemorySize) on the first call per (kernel, device); later calls only look it up
 int xma_set_max_lds_once(const void *kernel, int bytes);
+// xma_rocm_router_gate_topk (int32 ids) and xma_rocm_route of its ids (router.hip): one launch up to 16 tokens, which needs no workspace
+int xma_router_gate_route(const void *x, int64_t ldx, const void *gate_weight, int64_t ldw, int64_t T, int32_t H, int32_t E, int32_t k,
+                          int dtype, void *logits, int64_t ldl, void *weights, void *ids, uint32_t *counts, int64_t *offs_incl,
+                          int64_t *sorted_pos, void *workspace, size_t workspace_bytes, void *stream);
 
 #define XMA_REQUIRE(cond, code, ...)   \
     do {                               \

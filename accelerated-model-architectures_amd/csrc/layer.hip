@@ -80,13 +80,15 @@ extern "C" int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream) {
     XMA_REQUIRE(m->logits && m->h && m->y && m->counts, XMA_ROCM_EINVAL, "moe_forward: null buffer");
     const int dtype = (int)m->dtype;
     const int64_t M = m->T * m->k;
-    if (m->gate_weight)
-        RUN(xma_rocm_router_gate_topk(m->x, m->H, m->gate_weight, m->H, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->logits, m->E,
-                                      m->router_weights, m->expert_ids, 0, stream));
-    else
+    if (m->gate_weight) {
+        RUN(xma_router_gate_route(m->x, m->H, m->gate_weight, m->H, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->logits, m->E,
+                                  m->router_weights, m->expert_ids, (uint32_t *)m->counts, (int64_t *)m->expert_offsets,
+                                  (int64_t *)m->sorted_scattered_idxs, m->workspace, (size_t)m->workspace_bytes, stream));
+    } else {
         RUN(xma_rocm_router_topk(m->logits, m->E, m->T, (int32_t)m->E, (int32_t)m->k, dtype, m->router_weights, m->expert_ids, 0, stream));
-    RUN(xma_rocm_route(m->expert_ids, 0, M, (int32_t)m->E, (uint32_t *)m->counts, (int64_t *)m->expert_offsets, nullptr, nullptr,
-                       (int64_t *)m->sorted_scattered_idxs, m->workspace, (size_t)m->workspace_bytes, stream));
+        RUN(xma_rocm_route(m->expert_ids, 0, M, (int32_t)m->E, (uint32_t *)m->counts, (int64_t *)m->expert_offsets, nullptr, nullptr,
+                           (int64_t *)m->sorted_scattered_idxs, m->workspace, (size_t)m->workspace_bytes, stream));
+    }
     const int64_t U = up_width(m);
     RUN(gemm(m, m->few_up, m->x, m->w_fc, U * m->H, m->H, 0, m->z, m->h, m->I, nullptr, nullptr, m->b_fc, U, m->H, m->k, 0, 1, epilogue_of(m, 0), stream));
     RUN(down_projection(m, stream));

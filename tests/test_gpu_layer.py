@@ -153,3 +153,13 @@ def test_hooked_activation_is_called():
     one.act.register_forward_hook(lambda *a: calls.append(1))
     one(x)
     assert calls
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 8, 2), (2, 1, 1), (5, 33, 3), (16, 128, 8), (16, 40, 32), (16, 96, 1), (17, 128, 8)])
+def test_routing_behind_the_gate(T, E, k):
+    """up to 16 tokens the router's kernel routes as well: bit-identical to route's own kernel, also where equal logits tie"""
+    one, ops, x, dy = _layers(T, E, k, 136, 64, torch.bfloat16)
+    with torch.no_grad():
+        for m in (one, ops):
+            m.gate.weight[E // 2 :] = m.gate.weight[E // 2].clone()
+    _same(_step(one, x, dy), _step(ops, x, dy))
