@@ -566,7 +566,10 @@ inline double tiles_about(int64_t M, int N, int E, int height) {
 // measured pairs of launches (the layers of the benchmark and six others, 100 to 4000 rows per expert): within 12 and 10 % on average.
 // On 504 pairs the launches that mid_fwd_leads chooses are 1.17 times as fast as the 256 x 256 ones, the worst of them 9 % slower.
 inline double mid_fwd_seconds(int64_t M, int N, int K, int E, int epilogue, int *best) {
-    const double tiles = tiles_about(M, N, E, MR_BM), bytes = 2.0 * (M < E ? M : E) * N * K + 2.0 * M * (N + K);
+    // Long K: one tile too many for a round of K ranges is another round of long ones (8 experts of H = 1024, K = 16384, 270 rows, where
+    // most need a third tile: 174 us in 6 ranges, 148 now), so the tiles that experts of average rows need are counted in full.
+    const double rows = (double)M / E, whole = E * ceil((rows - sqrt(rows) / 2) / MR_BM) * ((N + MR_BN - 1) / MR_BN);
+    const double some = tiles_about(M, N, E, MR_BM), tiles = K > 8192 && whole > some ? whole : some, bytes = 2.0 * (M < E ? M : E) * N * K + 2.0 * M * (N + K);
     const double epi = epilogue == XMA_ROCM_EPI_SWIGLU_BWD ? 7.7e-6 : 0.;
     const int steps = (K + MR_K - 1) / MR_K;
     double shortest = 1e30;
@@ -667,7 +670,10 @@ bool mid_fwd_takes(const FwdArgs &a, int wt, int epi) {
 bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
     // K beyond 8192 (few experts, wide layers): tiles of twice the products per byte lead as soon as experts need two of the smaller
     // ones (8 experts of 176 rows, K = 28672: 470 against 516 us; K = 14336, 268 against 281; 320 rows 340 against 428)
-    if (K > 8192 && M > (int64_t)112 * E) return false;
+    // - unless the experts' columns make at most 32 tiles, which leave most of the chip to K slices of 256 KB of sums a tile (4 experts of
+    // H = 2048, K = 16384: 180 rows 155 -> 102 us, 258 rows 153 -> 117, 600 rows 250 -> 207; of H = 1024: 120 rows 114 -> 44, 400 rows
+    // 104 -> 77; the worst of 72 pairs 7 % slower, 16 experts of H = 512, 400 rows).
+    if (K > 8192 && M > (int64_t)112 * E && (int64_t)E * ((N + MR_BN - 1) / MR_BN) > 32) return false;
     int S;
     // without an epilogue of their own for GELU the 256 x 256 tiles leave it to a pass over two or three tensors
     const bool gelu = epilogue >= XMA_ROCM_EPI_GELU_TANH;

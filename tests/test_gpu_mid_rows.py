@@ -21,6 +21,7 @@ CASES = [
     ([300, 0, 1], 200, 136),
     ([260] * 8, 1024, 512),
     ([90, 31], 4096, 256),
+    ([258, 131], 8456, 136),
     ([40 + e for e in range(70)], 136, 24),
     ([e % 37 * 7 for e in range(140)], 192, 256),
 ]
