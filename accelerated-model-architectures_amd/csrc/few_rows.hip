@@ -3,8 +3,9 @@
 // grouped_gemm.hip are built for arithmetic: with one K step per tile, or one stage of weights in flight per compute unit,
 // they move 3.3-3.8 TB/s.  Here the work is laid out for bandwidth: 16 bytes per lane, 256 contiguous bytes per row and
 // load instruction, many short workgroups per compute unit; vector FMAs for one or two rows per expert, small MFMA tiles
-// beyond.  Correct for any number of rows, but the forward-type kernels stream the weights once per 32 rows of an expert:
-// the caller picks these entry points by the number of rows per expert.
+// beyond.  Correct for any number of rows, but the forward-type kernels here stream the weights once per 32 rows of an expert:
+// the caller picks these entry points by the number of rows per expert, and they hand launches of more than 24 (weight gradient:
+// 40) rows per expert to the 128 x 256 tiles of mid_rows.hip.
 #include "mid_rows.hpp"
 
 namespace {

@@ -16,7 +16,8 @@ Differences from the reference's data flow, all of which remove HBM passes:
     wrote already scaled (then h is not kept for the backward either);
   * backward reuses the un-weighted expert outputs saved by forward instead of
     recomputing them with another GEMM (triton_implementation/__init__.py:117-128);
-  * combine and its backward are dedicated coalesced kernels, not bmm.
+  * combine and its backward are dedicated coalesced kernels, not bmm;
+  * with packed SwiGLU or GELU the layer is one autograd node (``layer``), and each direction one call of the library.
 """
 
 from __future__ import annotations

@@ -96,10 +96,10 @@ CONTINUOUS_COUNT_SET_MAX_BINS = 8192
 # The grouped GEMMs take the entry points written for the few-token regime, which stream the weights instead of tiling
 # them 256 x 256 for the matrix pipes, up to FEW_ROWS_PER_EXPERT rows per expert on average.  The limits are measured
 # cross-overs (8 experts of H = 2048, I = 8192; 64 of H = 2048, I = 1408; 128 of H = 576, I = 256): the forward-type GEMMs
-# walk an expert's rows 32 or 128 at a time (small MFMA tile; vector FMAs up to 2 rows per expert and 64 rows in all, the
-# library decides), each pass streaming the weights again, so they lead while most experts need one pass (at 128 rows
-# per expert on average uneven routing gives enough experts a second pass); the weight gradient holds a 128 x 128 tile of
-# dW in registers while it walks the rows, so it leads as long as its stores outweigh its loads.
+# walk an expert's rows 32 or, beyond 24 rows per expert, 128 at a time (vector FMAs up to 2 rows per expert and 64 rows in
+# all; the library decides), each pass streaming the weights again, so they lead while most experts need one pass (at 128 rows
+# per expert on average uneven routing gives enough experts a second pass); the weight gradient holds its tile of dW in
+# registers while it walks the rows, so it leads as long as its stores outweigh its loads.
 FEW_ROWS_PER_EXPERT = {"x @ W^T": 96, "dy @ W": 96, "dW": 128}
 FEW_ROWS_MAX = 16384  # rows in all, every form (beyond the measured range; 0 switches the few-token entry points off)
 FEW_ROWS_MAX_WORKSPACE = 256 << 20  # bytes of fp32 partial sums a forward-type launch may ask for
