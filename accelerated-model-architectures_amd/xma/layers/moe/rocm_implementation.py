@@ -591,10 +591,15 @@ def layer(moe, x: torch.Tensor):
     I = U // 2 if act == "swiglu_packed" else U
     if H % 8 or I % 8 or (act == "swiglu_packed" and U % 2) or w_fc.size(2) != H or w_proj.shape != (E, H, I) or E > 16384 or T * k >= 1 << 31:
         return None
+    # the entry point has one E, H and I for all its tensors: the ops answer a gate over fewer experts and refuse the rest
+    if moe.num_experts != E or (b_fc is not None and b_fc.shape != (E, U)) or (b_proj is not None and b_proj.shape != (E, H)):
+        return None
     if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
         return None
     gate_weight, logits = gate.weight, None
     if gate.bias is None and router_gate_topk_supported(x, gate_weight, k) and _plain(gate_weight, x):
+        if gate_weight.shape != (E, H):
+            return None
         tensors = (x, gate_weight, w_fc, w_proj, b_fc, b_proj)
     else:
         gate_weight, logits = None, gate(x)

@@ -134,6 +134,34 @@ def test_mid_rows_dispatch_rule():
     assert ops._dw_loader_scales(64 * 8, 8, bf) and not ops._dw_loader_scales(64 * 8 + 1, 8, bf)
 
 
+def test_layer_call_leaves_other_shapes_to_the_ops(monkeypatch):
+    """the layer's library call reads all its tensors by one E, H and I, so whatever has others goes through the ops (None here),
+    which check each tensor"""
+    from xma.functional import swiglu_packed
+    from xma.layers import MoE
+    from xma.layers.moe import rocm_implementation as R
+
+    monkeypatch.setattr(R, "router_gate_topk_supported", lambda x, w, k: w.dtype == torch.bfloat16)  # as on the GPU
+    reached = []
+    monkeypatch.setattr(R, "_layer_forward", lambda *a: reached.append(a) or (a[0], a[0], None, None))
+
+    def taken(**change):
+        moe = MoE(8, 2, 64, 32, swiglu_packed, True, add_bias=True, std=0.02).bfloat16()
+        for name, value in change.items():
+            part, _, field = name.partition("__")
+            setattr(getattr(moe, part) if field else moe, field or part, value)
+        n = len(reached)
+        with torch.no_grad():
+            out = R.layer(moe, torch.randn(5, 64).bfloat16())
+        assert (out is None) == (len(reached) == n)
+        return out is not None
+
+    param = lambda *shape: nn.Parameter(torch.zeros(*shape, dtype=torch.bfloat16))
+    assert taken()
+    assert not taken(gate__weight=param(6, 64)) and not taken(gate__weight=param(9, 64)) and not taken(gate__weight=param(8, 72))
+    assert not taken(c_fc__bias=param(8, 32)) and not taken(c_fc__bias=param(7, 64)) and not taken(c_proj__bias=param(8, 32))
+    assert not taken(num_experts=9) and not taken(c_proj__weight=param(7, 64, 32)) and not taken(c_fc__weight=param(8, 64, 72))
+
 
 def test_fused_router_shape_rule_matches_the_library():
     """the Python restatement of the fused gate + router kernel's coverage (evaluated under torch.compile, where a ctypes
