@@ -597,8 +597,8 @@ def layer(moe, x: torch.Tensor):
     if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
         return None
     gate_weight, logits = gate.weight, None
-    if gate.bias is None and router_gate_topk_supported(x, gate_weight, k) and _plain(gate_weight, x):
-        if gate_weight.shape != (E, H):
+    if gate.bias is None and router_gate_topk_supported(x, gate_weight, k):
+        if gate_weight.shape != (E, H) or not _plain(gate_weight, x):  # the op copies a weight that starts off a 16-byte boundary
             return None
         tensors = (x, gate_weight, w_fc, w_proj, b_fc, b_proj)
     else:

@@ -114,6 +114,17 @@ def test_what_goes_through_the_ops():
     _same(a, _step(ops, x, dy))
 
 
+@pytest.mark.parametrize("T", [40, 5000])
+def test_gates_the_entry_point_does_not_describe(T):
+    """a gate weight off a 16-byte boundary takes the router's kernel as a copy, as the ops do, and a gate over fewer experts than the
+    layer has is answered: bit for bit what the ops give"""
+    one, ops, x, dy = _layers(T, 8, 2, 64, 32, torch.bfloat16)
+    shifted = torch.empty(8 * 64 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(8, 64)
+    for weight in (shifted.copy_(one.gate.weight.detach()), one.gate.weight.detach()[:6].clone()):
+        one.gate.weight, ops.gate.weight = nn.Parameter(weight), nn.Parameter(weight)
+        _same(_step(one, x, dy), _step(ops, x, dy))
+
+
 def test_two_passes_before_the_backward():
     """each pass keeps its own buffers"""
     one, ops, x, dy = _layers(50, 8, 2, 64, 32, torch.bfloat16)

@@ -160,6 +160,7 @@ def test_layer_call_leaves_other_shapes_to_the_ops(monkeypatch):
     assert taken()
     assert not taken(gate__weight=param(6, 64)) and not taken(gate__weight=param(9, 64)) and not taken(gate__weight=param(8, 72))
     assert not taken(c_fc__bias=param(8, 32)) and not taken(c_fc__bias=param(7, 64)) and not taken(c_proj__bias=param(8, 32))
+    assert not taken(gate__weight=nn.Parameter(torch.zeros(8 * 64 + 1, dtype=torch.bfloat16)[1:].view(8, 64)))  # off a 16-byte boundary
     assert not taken(num_experts=9) and not taken(c_proj__weight=param(7, 64, 32)) and not taken(c_fc__weight=param(8, 64, 72))
 
 
