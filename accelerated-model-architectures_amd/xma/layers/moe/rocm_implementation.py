@@ -418,7 +418,7 @@ _BLOCK_SIZES = struct.Struct("17q")
 class _Plan:
     """sizes, choices and scratch layout of a layer call; a function of the shape, the options and the dispatch limits only"""
 
-    __slots__ = ("sizes_forward", "sizes_backward", "keep", "temp", "back", "keep_bytes", "temp_bytes", "back_bytes", "recompute")
+    __slots__ = ("sizes_forward", "sizes_backward", "keep", "temp", "back", "keep_bytes", "temp_bytes", "back_bytes", "recompute", "saved_shapes")
 
 
 def _layout(sizes: dict[str, int]) -> tuple[dict[str, int], int]:
@@ -470,6 +470,7 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, 
     p.temp, p.temp_bytes = _layout(temp)
     p.back, p.back_bytes = _layout(back)
     p.recompute = not save
+    p.saved_shapes = ((T, H), (E, H), (T, E), (E, U, H), (E, H, I), (E, U), (E, H), (p.keep_bytes,))
     few = (up[0], down[0], dx2[0], dw(H, I, dw2_form == 0), dw(U, H, False), dx1[0], dw2_form, int(not save))
     head = (_BLOCK_SIZES.size + _BLOCK_POINTERS.size, T, H, I, E, k, ops._DTYPE_CODE[dtype], ("swiglu_packed", "tanh", "none").index(act), *few)
     p.sizes_forward = _BLOCK_SIZES.pack(*head, temp["workspace"])
@@ -508,6 +509,20 @@ def _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, s
     return y, logits, kept, p
 
 
+def _unpacked(saved, shapes, like: torch.Tensor) -> list[torch.Tensor | None]:
+    """The saved tensors of `_Layer` as the library takes them.  Saved-tensor hooks may hand back a copy of another layout, which is
+    laid out again; one of another shape, dtype or device is refused, as the ops refuse it."""
+    out = []
+    for t, shape in zip(saved, shapes):
+        if t is not None:
+            assert t.shape == shape and t.device == like.device and (t.dtype == like.dtype or len(shape) == 1 and t.dtype == torch.uint8), \
+                "a saved tensor came back with another shape, device or dtype"
+            if not t.is_contiguous() or t.data_ptr() % 16:
+                t = t.clone(memory_format=torch.contiguous_format)
+        out.append(t)
+    return out
+
+
 class _Layer(torch.autograd.Function):
     """the whole layer: with gate_weight (logits None) -> (y, logits), with given logits -> y"""
 
@@ -520,15 +535,16 @@ class _Layer(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, d_logits_out=None):
-        x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, kept = ctx.saved_tensors
         need_x, need_gate, need_logits = ctx.needs_input_grad[:3]
         if dy is None:  # nothing but the logits was used
             if d_logits_out is None:
                 return (None,) * 10
+            x, gate_weight = ctx.saved_tensors[:2]
             d_x = d_logits_out @ gate_weight if need_x else None
             return d_x, _gate_weight_grad(d_logits_out, x) if need_gate else None, *(None,) * 8
         dy = dy.contiguous()
         p = ctx.plan
+        x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, kept = _unpacked(ctx.saved_tensors, p.saved_shapes, dy)
         scratch = torch.empty(p.back_bytes, dtype=torch.uint8, device=x.device)
         d_logits = torch.empty_like(logits, memory_format=torch.contiguous_format)
         d_x, d_w_fc, d_w_proj = torch.empty_like(x), torch.empty_like(w_fc), torch.empty_like(w_proj)

@@ -114,6 +114,26 @@ def test_what_goes_through_the_ops():
     _same(a, _step(ops, x, dy))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_saved_tensor_hooks(dtype):
+    """what hooks hand back for the saved tensors: other strides and starts give the same gradients, another dtype or device an error"""
+
+    def moved(t):  # the same values in rows further apart, or off a 16-byte boundary
+        if t.dim() == 1:
+            return torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].copy_(t)
+        return t.new_empty(*t.shape[:-1], t.shape[-1] + 8)[..., : t.shape[-1]].copy_(t)
+
+    one, _, x, dy = _layers(40, 8, 2, 64, 32, dtype, bias=True)
+    want = _step(one, x, dy)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: moved(t) if t.dtype in (dtype, torch.uint8) else t):
+        _same(_step(one, x, dy), want)
+    for wrong in (lambda t: t.cpu(), lambda t: t.double()):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, wrong):
+            y = one(x.clone().requires_grad_())[0]
+        with pytest.raises(AssertionError):
+            y.backward(dy)
+
+
 @pytest.mark.parametrize("T", [40, 5000])
 def test_gates_the_entry_point_does_not_describe(T):
     """a gate weight off a 16-byte boundary takes the router's kernel as a copy, as the ops do, and a gate over fewer experts than the

@@ -164,6 +164,25 @@ def test_layer_call_leaves_other_shapes_to_the_ops(monkeypatch):
     assert not taken(num_experts=9) and not taken(c_proj__weight=param(7, 64, 32)) and not taken(c_fc__weight=param(8, 64, 72))
 
 
+def test_layer_backward_looks_at_what_saved_tensor_hooks_return():
+    """the library reads the saved tensors by address: another layout is laid out again, another kind is refused"""
+    from xma.layers.moe import rocm_implementation as R
+
+    bf = torch.bfloat16
+    like = torch.zeros(4, 8, dtype=bf)
+    x, kept = torch.randn(4, 8).to(bf), torch.arange(64, dtype=torch.uint8)
+    wide = torch.zeros(4, 16, dtype=bf)[:, :8].copy_(x)
+    off = torch.zeros(65, dtype=torch.uint8)[1:].copy_(kept)
+    shapes = ((4, 8), (3, 8), (64,))
+    assert all(a is b for a, b in zip(R._unpacked((x, None, kept), shapes, like), (x, None, kept)))
+    for got, want in zip(R._unpacked((wide, None, off), shapes, like), (x, None, kept)):
+        assert got is want or (torch.equal(got, want) and got.is_contiguous() and got.data_ptr() % 16 == 0)
+    for bad in ((x.float(), None, kept), (x[:3], None, kept), (x, None, kept.to(bf)[:32]), (x, None, kept.int()), (x.to("meta"), None, kept),
+                (x.to(torch.uint8), None, kept), (x.half(), None, kept)):
+        with pytest.raises(AssertionError):
+            R._unpacked(bad, shapes, like)
+
+
 def test_fused_router_shape_rule_matches_the_library():
     """the Python restatement of the fused gate + router kernel's coverage (evaluated under torch.compile, where a ctypes
     call cannot be traced) against the library's own answer"""
