@@ -565,7 +565,7 @@ class _Layer(torch.autograd.Function):
             if d_logits_out is not None:  # the caller also used the returned router logits (an auxiliary loss)
                 d_logits = d_logits + d_logits_out
             if need_x:
-                d_x_gate = d_logits @ gate_weight
+                d_x_gate = (d_logits @ gate_weight).to(x.dtype)  # in an autocast region the product has another dtype
             if need_gate:
                 d_gate = _gate_weight_grad(d_logits, x)
         check(lib.xma_rocm_moe_backward(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0 if d_x_gate is None else d_x_gate.data_ptr()),

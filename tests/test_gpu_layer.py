@@ -114,6 +114,15 @@ def test_what_goes_through_the_ops():
     _same(a, _step(ops, x, dy))
 
 
+@pytest.mark.parametrize("autocast", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_backward_in_an_autocast_region(dtype, autocast):
+    """the gate's product there comes in the region's dtype; what the layer adds to d_x is its value, not its bytes"""
+    one, ops, x, dy = _layers(40, 8, 2, 64, 32, dtype)
+    with torch.autocast("cuda", dtype=autocast):
+        _same(_step(one, x, dy), _step(ops, x, dy))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_saved_tensor_hooks(dtype):
     """what hooks hand back for the saved tensors: other strides and starts give the same gradients, another dtype or device an error"""
