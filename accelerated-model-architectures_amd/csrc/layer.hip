@@ -27,14 +27,23 @@ int gemm(const xma_rocm_moe *m, int64_t few, const void *X, const void *W, int64
         return xma_rocm_scatter2scatter_few_rows(X, K, W, w_es, ldw, w_is_kn, idx, offs, out, ldo, aux, ldaux, aux2, aux2 ? N : 0, scale, bias,
                                                  bias ? N : 0, M, (int32_t)N, (int32_t)K, (int32_t)m->E, (int32_t)fan_out, x_grouped, y_grouped,
                                                  epilogue, (int)m->dtype, m->workspace, (size_t)m->workspace_bytes, stream);
-    // the 256 x 256 kernels split the last round of tiles only where they ask for a workspace
-    const size_t ws = xma_rocm_scatter2scatter_workspace_bytes(M, (int32_t)N, (int32_t)K, (int32_t)m->E);
+    // the 256 x 256 kernels split the last round of tiles where there is a workspace, and refuse one that is too small for it
     if (aux2)
         return xma_rocm_down_projection_dx_swiglu(X, K, W, w_es, ldw, idx, offs, aux, ldaux, out, ldo, aux2, N, scale, M, (int32_t)N, (int32_t)K,
-                                                  (int32_t)m->E, (int32_t)fan_out, (int)m->dtype, ws ? m->workspace : nullptr, ws, stream);
+                                                  (int32_t)m->E, (int32_t)fan_out, (int)m->dtype, m->workspace, (size_t)m->workspace_bytes, stream);
     return xma_rocm_scatter2scatter_bias(X, K, W, w_es, ldw, w_is_kn, idx, offs, out, ldo, aux, ldaux, scale, bias, bias ? N : 0, M, (int32_t)N,
                                          (int32_t)K, (int32_t)m->E, (int32_t)fan_out, x_grouped, y_grouped, epilogue, (int)m->dtype,
-                                         ws ? m->workspace : nullptr, ws, stream);
+                                         m->workspace, (size_t)m->workspace_bytes, stream);
+}
+
+// Before a pass's first launch: the workspace holds the K slices of a GEMM by the 256 x 256 kernels (0 bytes: none, and without a
+// workspace at all they split nothing).  Few-row launches and route check it themselves.
+int check_workspace(const xma_rocm_moe *m, int64_t few, int64_t N, int64_t K, const char *what) {
+    if (few || !m->workspace || m->dtype == XMA_ROCM_F32) return XMA_ROCM_OK;
+    const size_t need = xma_rocm_scatter2scatter_workspace_bytes(m->T * m->k, (int32_t)N, (int32_t)K, (int32_t)m->E);
+    XMA_REQUIRE((size_t)m->workspace_bytes >= need, XMA_ROCM_EWORKSPACE, "%s: workspace of %lld bytes, %zu needed", what,
+                (long long)m->workspace_bytes, need);
+    return XMA_ROCM_OK;
 }
 
 int dw(const xma_rocm_moe *m, int64_t few, const void *DY, int dy_grouped, const void *scale, const void *X, int x_grouped, void *DW,
@@ -59,6 +68,7 @@ int check(const xma_rocm_moe *m, const char *what) {
                     m->H < ((int64_t)1 << 30) && m->I < ((int64_t)1 << 29) && m->E <= 16384,
                 XMA_ROCM_EINVAL, "%s: T=%lld H=%lld I=%lld E=%lld k=%lld", what, (long long)m->T, (long long)m->H, (long long)m->I,
                 (long long)m->E, (long long)m->k);
+    XMA_REQUIRE(m->workspace_bytes >= 0, XMA_ROCM_EINVAL, "%s: workspace of %lld bytes", what, (long long)m->workspace_bytes);
     XMA_REQUIRE(m->x && m->w_fc && m->w_proj && m->router_weights && m->expert_ids && m->expert_offsets && m->sorted_scattered_idxs && m->z &&
                     m->expert_out,
                 XMA_ROCM_EINVAL, "%s: null buffer", what);
@@ -79,7 +89,9 @@ extern "C" int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream) {
     RUN(check(m, "moe_forward"));
     XMA_REQUIRE(m->logits && m->h && m->y && m->counts, XMA_ROCM_EINVAL, "moe_forward: null buffer");
     const int dtype = (int)m->dtype;
-    const int64_t M = m->T * m->k;
+    const int64_t M = m->T * m->k, U = up_width(m);
+    RUN(check_workspace(m, m->few_up, U, m->H, "moe_forward"));
+    RUN(check_workspace(m, m->few_down, m->H, m->I, "moe_forward"));
     if (m->gate_weight) {
         RUN(xma_router_gate_route(m->x, m->H, m->gate_weight, m->H, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->logits, m->E,
                                   m->router_weights, m->expert_ids, (uint32_t *)m->counts, (int64_t *)m->expert_offsets,
@@ -89,7 +101,6 @@ extern "C" int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream) {
         RUN(xma_rocm_route(m->expert_ids, 0, M, (int32_t)m->E, (uint32_t *)m->counts, (int64_t *)m->expert_offsets, nullptr, nullptr,
                            (int64_t *)m->sorted_scattered_idxs, m->workspace, (size_t)m->workspace_bytes, stream));
     }
-    const int64_t U = up_width(m);
     RUN(gemm(m, m->few_up, m->x, m->w_fc, U * m->H, m->H, 0, m->z, m->h, m->I, nullptr, nullptr, m->b_fc, U, m->H, m->k, 0, 1, epilogue_of(m, 0), stream));
     RUN(down_projection(m, stream));
     return xma_rocm_combine(m->expert_out, m->H, m->router_weights, m->y, m->H, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream);
@@ -101,6 +112,7 @@ extern "C" int xma_rocm_moe_backward_router(const xma_rocm_moe *m, void *stream)
     XMA_REQUIRE(m->logits && m->dy && m->d_router_weights && m->d_logits && (!m->recompute || m->h), XMA_ROCM_EINVAL,
                 "moe_backward_router: null buffer");
     const int dtype = (int)m->dtype;
+    if (m->recompute) RUN(check_workspace(m, m->few_down, m->H, m->I, "moe_backward_router"));
     if (m->recompute) { // neither was kept: h from z, the expert outputs by the down-projection
         RUN(xma_rocm_swiglu_packed_forward(m->z, 2 * m->I, m->h, m->I, m->T * m->k, (int32_t)m->I, dtype, stream));
         RUN(down_projection(m, stream));
@@ -118,6 +130,8 @@ extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
     const int dtype = (int)m->dtype;
     const int64_t M = m->T * m->k, H = m->H, I = m->I, U = up_width(m);
     const int64_t *idx = (const int64_t *)m->sorted_scattered_idxs, *offs = (const int64_t *)m->expert_offsets;
+    RUN(check_workspace(m, m->few_dx2, I, H, "moe_backward"));
+    RUN(check_workspace(m, m->few_dx1, H, U, "moe_backward"));
     // dX2 + SwiGLU', with the scaled activations for dW2 where that takes dy through the index
     RUN(gemm(m, m->few_dx2, m->dy, m->w_proj, H * I, I, 1, m->dz, m->z, U, m->dw2_form == 1 ? m->dw2_operand : nullptr, m->router_weights,
              nullptr, I, H, m->k, 0, 1, epilogue_of(m, 1), stream));

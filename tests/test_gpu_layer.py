@@ -7,7 +7,7 @@ import torch.nn as nn
 from xma.functional import swiglu_packed
 from xma.layers import MoE
 
-from .test_gpu_ops import _tol
+from .test_gpu_ops import _few_rows_limit, _tol
 from .utils import nerr
 
 
@@ -112,6 +112,39 @@ def test_what_goes_through_the_ops():
     with torch.autograd.graph.save_on_cpu():
         a = _step(one, x, dy)
     _same(a, _step(ops, x, dy))
+
+
+def test_workspace_too_small_is_refused(monkeypatch):
+    """a workspace that holds less than the K slices of the 256 x 256 kernels: each of the three entries refuses it before any launch"""
+    from xma.layers.moe import rocm_implementation as R
+    from xma.rocm import ops
+    from xma.rocm.loader import RocmLibraryError, get_library
+
+    T, E, k, H, I = 300, 4, 2, 2048, 1024
+    one, _, x, dy = _layers(T, E, k, H, I, torch.bfloat16, save=False)
+    plan = R._plan
+    short = ops.route_workspace_elements(T * k, E) * 4
+    assert get_library().xma_rocm_scatter2scatter_workspace_bytes(T * k, 2 * I, H, E) > short
+    cut = set()
+
+    def cut_plan(*args):
+        p = plan.__wrapped__(*args)
+        for name in cut:
+            setattr(p, name, getattr(p, name)[:-8] + short.to_bytes(8, "little"))
+        return p
+
+    monkeypatch.setattr(R, "_plan", cut_plan)
+    with _few_rows_limit(0):
+        cut = {"sizes_forward"}
+        with torch.no_grad(), pytest.raises(RocmLibraryError, match="xma_rocm_moe_forward failed with code -3"):
+            one(x)
+        cut = {"sizes_backward"}
+        for save, entry in ((False, "xma_rocm_moe_backward_router"), (True, "xma_rocm_moe_backward")):
+            one.save_activations = save
+            y = one(x.clone().requires_grad_())[0]
+            with pytest.raises(RocmLibraryError, match=f"{entry} failed with code -3"):
+                y.backward(dy)
+    torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("autocast", [torch.float16, torch.bfloat16])
