@@ -64,7 +64,7 @@ int down_projection(const xma_rocm_moe *m, void *stream) {
 
 int check(const xma_rocm_moe *m, const char *what) {
     XMA_REQUIRE(m && m->size == (int64_t)sizeof(xma_rocm_moe), XMA_ROCM_EINVAL, "%s: argument block of another size", what);
-    XMA_REQUIRE(m->T >= 1 && m->H >= 8 && m->I >= 8 && m->E >= 1 && m->k >= 1 && m->k <= m->E && m->T * m->k < ((int64_t)1 << 31) &&
+    XMA_REQUIRE(m->T >= 1 && m->T < ((int64_t)1 << 31) && m->H >= 8 && m->I >= 8 && m->E >= 1 && m->k >= 1 && m->k <= m->E && m->T * m->k < ((int64_t)1 << 31) &&
                     m->H < ((int64_t)1 << 30) && m->I < ((int64_t)1 << 29) && m->E <= 16384,
                 XMA_ROCM_EINVAL, "%s: T=%lld H=%lld I=%lld E=%lld k=%lld", what, (long long)m->T, (long long)m->H, (long long)m->I,
                 (long long)m->E, (long long)m->k);
@@ -127,6 +127,9 @@ extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
     XMA_REQUIRE(m->dy && m->dz && m->d_w_fc && m->d_w_proj && m->scattered && m->d_x && (m->dw2_form == 1 || m->h) &&
                     (m->dw2_form == 0 || m->dw2_operand) && (!m->d_b_fc || m->b_fc) && (!m->d_b_proj || m->b_proj),
                 XMA_ROCM_EINVAL, "moe_backward: null buffer");
+    // the column sums that make d_b_proj want dy scaled, in a copy or beside the scaled activations: the loader of form 0 keeps none
+    XMA_REQUIRE(m->dw2_form >= 0 && m->dw2_form <= 2 && !(m->dw2_form == 0 && m->d_b_proj), XMA_ROCM_EINVAL,
+                "moe_backward: dw2_form %lld%s", (long long)m->dw2_form, m->d_b_proj ? " with d_b_proj (forms 1 and 2 only)" : "");
     const int dtype = (int)m->dtype;
     const int64_t M = m->T * m->k, H = m->H, I = m->I, U = up_width(m);
     const int64_t *idx = (const int64_t *)m->sorted_scattered_idxs, *offs = (const int64_t *)m->expert_offsets;

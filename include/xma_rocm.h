@@ -359,8 +359,9 @@ XMA_API int xma_rocm_gelu_backward(const void *x, const void *dy, void *dx, int6
  * entry point for a GEMM (1) or the 256 x 256 tiles (0).  gate_weight NULL: `logits` is an input.  dw2_form: the operand of dW2,
  * 0: dy through the few-row loader, which scales it; 1: `dw2_operand` = scaled activations (M, I), written by dX2; 2:
  * `dw2_operand` = scaled grouped copy of dy (M, H).  recompute: h and expert_out are rebuilt from z by
- * xma_rocm_moe_backward_router.  d_b_fc / d_b_proj may be NULL.  M = T k.  `workspace`: the largest that any of the calls asks for
- * (route, and per GEMM its entry point's).  Argument errors as in the single calls; launches before one that is refused stand.
+ * xma_rocm_moe_backward_router.  d_b_fc / d_b_proj may be NULL; d_b_proj goes with dw2_form 1 and 2 only.  M = T k.
+ * `workspace`: the largest that any of the calls asks for (route, and per GEMM its entry point's).  Argument errors as in the single
+ * calls; launches before one that is refused stand.
  */
 typedef struct xma_rocm_moe {
     int64_t size; /* sizeof(xma_rocm_moe) */

@@ -99,6 +99,53 @@ def test_argument_errors_are_reported_before_any_launch():
     assert lib.xma_rocm_continuous_count(None, 0, 0, ctypes.c_void_p(16), 4, None, 0, None) == 0
 
 
+def test_layer_entry_points_refuse_what_they_cannot_run():
+    """xma_rocm_moe_*: every argument that has a rule of its own, before any launch"""
+    import struct
+
+    from xma.rocm import get_library
+
+    lib = get_library()
+    sizes = ("size T H I E k dtype activation few_up few_down few_dx2 few_dw2 few_dw1 few_dx1 dw2_form recompute workspace_bytes").split()
+    pointers = ("x gate_weight w_fc w_proj b_fc b_proj logits router_weights expert_ids counts expert_offsets sorted_scattered_idxs z h "
+                "expert_out y workspace dy d_router_weights d_logits dz dw2_operand scattered d_w_fc d_w_proj d_b_fc d_b_proj d_x "
+                "d_x_addend").split()
+    text = open(os.path.join(ROOT, "include", "xma_rocm.h")).read()
+    block = re.sub(r"/\*.*?\*/", "", text[text.index("typedef struct xma_rocm_moe {") : text.index("} xma_rocm_moe;")], flags=re.S)
+    assert re.findall(r"\b(\w+)[,;]", block) == sizes + pointers  # the block's fields, in order
+
+    def refused(entry, code, message, **change):
+        v = dict.fromkeys(pointers, 256) | dict(T=4, H=64, I=32, E=8, k=2, dtype=0, activation=0, dw2_form=2, recompute=0, workspace_bytes=1 << 30)
+        v |= dict(size=8 * len(sizes + pointers)) | dict.fromkeys((s for s in sizes if s.startswith("few_")), 1)
+        v |= dict(d_b_fc=0, d_b_proj=0, b_fc=0, b_proj=0) | change
+        rc = getattr(lib, "xma_rocm_moe_" + entry)(struct.pack(f"{len(sizes)}q{len(pointers)}Q", *(v[n] for n in sizes + pointers)), None)
+        assert rc == code and message in lib.xma_rocm_last_error().decode(), (entry, change, rc, lib.xma_rocm_last_error())
+
+    for entry in ("forward", "backward_router", "backward"):
+        refused(entry, -1, "another size", size=8)
+        for bad in (dict(T=0), dict(T=1 << 62, k=4), dict(H=0), dict(I=0), dict(E=0), dict(E=16385), dict(k=0), dict(k=9), dict(T=1 << 30, k=4)):
+            refused(entry, -1, "T=", **bad)
+        refused(entry, -1, "workspace of -1", workspace_bytes=-1)
+        for name in ("x", "w_fc", "w_proj", "router_weights", "expert_ids", "expert_offsets", "sorted_scattered_idxs", "z", "expert_out"):
+            refused(entry, -1, "null buffer", **{name: 0})
+        for bad in (dict(activation=3), dict(activation=-1), dict(activation=1, recompute=1), dict(activation=2, dw2_form=1)):
+            refused(entry, -1, "activation", **bad)
+    for name in ("logits", "h", "y", "counts"):
+        refused("forward", -1, "null buffer", **{name: 0})
+    for name in ("logits", "dy", "d_router_weights", "d_logits"):
+        refused("backward_router", -1, "null buffer", **{name: 0})
+    refused("backward_router", -1, "null buffer", recompute=1, h=0)
+    for name in ("dy", "dz", "d_w_fc", "d_w_proj", "scattered", "d_x", "h", "dw2_operand"):
+        refused("backward", -1, "null buffer", **{name: 0})
+    refused("backward", -1, "null buffer", d_b_fc=256)  # a bias gradient without the bias
+    refused("backward", -1, "null buffer", d_b_proj=256)
+    refused("backward", -1, "dw2_form 0 with d_b_proj", dw2_form=0, b_proj=256, d_b_proj=256)
+    refused("backward", -1, "dw2_form 3", dw2_form=3)
+    # what the single calls refuse: a workspace too small for route, or for the K ranges of a few-row launch
+    refused("forward", -2, "dtype 5", dtype=5)
+    refused("backward", -3, "scatter2scatter_few_rows: workspace", I=64, H=16384, workspace_bytes=16)
+
+
 def test_few_token_dispatch_rule():
     """which grouped GEMM forms take the kernels of the few-token regime: by rows per expert on average, per form, with a
     cap on the rows in all; fp32 never"""
