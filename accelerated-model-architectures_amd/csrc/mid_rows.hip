@@ -628,15 +628,12 @@ template <typename T, int WT, int EPI> int mid_launch_fwd(const FwdArgs &a, floa
                                __is_same(T, __bf16) ? XMA_ROCM_BF16 : XMA_ROCM_F16, st);
 }
 
-template <typename T> int mid_dispatch_fwd(const FwdArgs &a, int wt, int epi, float *part, hipStream_t st) {
-    if (wt == 0) {
-        if (epi == XMA_ROCM_EPI_STORE) return mid_launch_fwd<T, 0, XMA_ROCM_EPI_STORE>(a, part, st);
-        return epi == XMA_ROCM_EPI_SWIGLU ? mid_launch_fwd<T, 0, XMA_ROCM_EPI_SWIGLU>(a, part, st) : mid_launch_fwd<T, 0, EPI_GELU>(a, part, st);
-    }
-    if (epi == EPI_GELU_BWD) return mid_launch_fwd<T, 1, EPI_GELU_BWD>(a, part, st);
-    if (epi == XMA_ROCM_EPI_STORE) return mid_launch_fwd<T, 1, XMA_ROCM_EPI_STORE>(a, part, st);
-    if (a.aux2) return mid_launch_fwd<T, 1, EPI_SWIGLU_BWD_SCALED_ACT>(a, part, st);
-    return mid_launch_fwd<T, 1, XMA_ROCM_EPI_SWIGLU_BWD>(a, part, st);
+template <typename T, int WT> int mid_dispatch_fwd(const FwdArgs &a, int epi, float *part, hipStream_t st) {
+    if (epi == XMA_ROCM_EPI_STORE) return mid_launch_fwd<T, WT, XMA_ROCM_EPI_STORE>(a, part, st);
+    if (epi == XMA_ROCM_EPI_SWIGLU) return mid_launch_fwd<T, WT, XMA_ROCM_EPI_SWIGLU>(a, part, st);
+    if (epi == (WT ? EPI_GELU_BWD : EPI_GELU)) return mid_launch_fwd<T, WT, WT ? EPI_GELU_BWD : EPI_GELU>(a, part, st);
+    if (a.aux2) return mid_launch_fwd<T, WT, EPI_SWIGLU_BWD_SCALED_ACT>(a, part, st);
+    return mid_launch_fwd<T, WT, XMA_ROCM_EPI_SWIGLU_BWD>(a, part, st);
 }
 
 template <typename T, int GQ, int GP> int mid_launch_dw(const DwArgs &a, hipStream_t st) {
@@ -660,9 +657,10 @@ size_t mid_fwd_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E) {
 }
 
 bool mid_fwd_takes(const FwdArgs &a, int wt, int epi) {
-    // the operand layouts the layer launches: x @ W^T and dy @ W, each with the epilogues of its own
-    const bool bwd = epi == XMA_ROCM_EPI_SWIGLU_BWD || epi == EPI_GELU_BWD;
-    if (a.E > MR_MAX_E || (epi != XMA_ROCM_EPI_STORE && (wt == 1) != bwd)) return false;
+    // GELU comes in the layouts that the layer launches, x @ W^T and dy @ W.  SwiGLU also in the other two (weights stored
+    // transposed): streaming the weights once per 32 rows instead costs them, 8 experts of H = 2048, I = 8192, 96 rows each,
+    // W1 as (H, 2I), 351 us against 116, W2 as (I, H) 167 against 57.
+    if (a.E > MR_MAX_E || (epi == EPI_GELU && wt) || (epi == EPI_GELU_BWD && !wt)) return false;
     const int64_t x_rows = a.x_grouped ? MR_BM : (a.M + a.fan_out - 1) / a.fan_out; // 32-bit byte offsets from a tile's base
     return a.M > 0 && a.M <= 65535 && x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)MR_BN * a.ldw * 2 < ((int64_t)1 << 32);
 }
@@ -683,7 +681,8 @@ bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
 }
 
 int mid_fwd(const FwdArgs &a, int wt, int epi, int dtype, float *part, hipStream_t st) {
-    return dtype == XMA_ROCM_BF16 ? mid_dispatch_fwd<__bf16>(a, wt, epi, part, st) : mid_dispatch_fwd<_Float16>(a, wt, epi, part, st);
+    if (dtype == XMA_ROCM_BF16) return wt ? mid_dispatch_fwd<__bf16, 1>(a, epi, part, st) : mid_dispatch_fwd<__bf16, 0>(a, epi, part, st);
+    return wt ? mid_dispatch_fwd<_Float16, 1>(a, epi, part, st) : mid_dispatch_fwd<_Float16, 0>(a, epi, part, st);
 }
 
 bool mid_dw_takes(const DwArgs &a, int64_t M) {

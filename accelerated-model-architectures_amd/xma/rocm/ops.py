@@ -209,7 +209,7 @@ def _mid_rows_fwd(M: int, N: int, K: int, E: int, w_is_kn: int, ldw: int, x_span
     elements from X's first row to the end of its last)"""
     if not 0 < M <= MID_ROWS_MAX or FEW_ROWS_MAX == 0 or dtype not in (torch.bfloat16, torch.float16):
         return False
-    # what the tiles cover: the layouts that the layer launches, offsets that fit
+    # beyond the few-row limits: the layouts that the layer launches (where the two were compared), and offsets that fit
     if epilogue != EPI_STORE and w_is_kn != (epilogue in (EPI_SWIGLU_BWD, 5, 7)):
         return False
     if E > MID_ROWS_MAX_EXPERTS or x_span >= MID_ROWS_OFFSETS or 256 * ldw >= MID_ROWS_OFFSETS:

@@ -207,9 +207,9 @@ XMA_API int xma_rocm_down_projection_dx_swiglu(const void *dY, int64_t lddy, con
  * only.  With a handful of rows per expert the product is a stream over the weights.  W[e] as (N, K), up to 2 rows per
  * expert on average (and 64 in all), K at least 2048: vector FMAs, a wave reads two rows of W with its lanes along K.
  * Everything else: a small MFMA tile (32 rows of the expert x 128 output columns, four workgroups per compute unit), and
- * from 24 rows per expert on average 128 x 256 tiles, two workgroups per compute unit (x @ W^T with a plain store or SwiGLU,
- * dy @ W with a plain store or the SwiGLU backward, E at most 1024, operands within 32-bit byte offsets; the small tile
- * otherwise), both cut along K where N alone gives too few workgroups.
+ * from 24 rows per expert on average 128 x 256 tiles, two workgroups per compute unit (a plain store, SwiGLU or its backward in
+ * either layout of W, GELU with W as (N, K) and its backward with W as (K, N); E at most 1024, operands within 32-bit byte
+ * offsets; the small tile otherwise), both cut along K where N alone gives too few workgroups.
  * Whatever does not finish in one kernel sums through the workspace (xma_rocm_scatter2scatter_few_rows_workspace_bytes
  * bytes for the same M, N, K, num_experts, w_is_kn and epilogue; 0 = none needed, pass NULL) to a small kernel that
  * applies the bias and the epilogue with the arithmetic of the MFMA kernels.  Limits: M and E at most 65535, N * ldw

@@ -93,3 +93,42 @@ def test_mid_rows_tiles(dtype, case):
     same(lambda: ops.down_projection_dx_swiglu_scaled_act_rocm(xd, Wkd, idx, offs, zd, dz, out, wd, 1), [dz, out])
     for dy_fan, x_fan in ((0, 0), (1, 0), (0, 1)):
         same(lambda: ops.group_bwd_W_rocm(dyd, xd, idx, offs, dW.permute(0, 2, 1), None, dy_fan, x_fan), [dW])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [c for c in CASES if c[2] % 16 == 0], ids=lambda c: f"E{len(c[0])}-M{sum(c[0])}-K{c[1]}-N{c[2]}")
+def test_swiglu_of_transposed_weights(dtype, case):
+    """SwiGLU with W stored as (K, N) and its backward with W stored as (N, K), with and without the second output (which the ops
+    take in the other layout only)"""
+    from xma.rocm import ops
+    from xma.rocm.loader import check, get_library
+
+    rows, K, N = case
+    E, M = len(rows), sum(rows)
+    g = torch.Generator().manual_seed(M + N)
+    se = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))
+    ss = torch.randperm(M, generator=g)
+    idx, offs = ss.cuda(), torch.tensor(rows).cumsum(0).cuda()
+    x = torch.randn(M, K, generator=g).to(dtype)
+    Wk = (torch.randn(E, K, N, generator=g) * K**-0.5).to(dtype)
+    bias, w, z = (t.to(dtype) for t in (torch.randn(E, N, generator=g), torch.rand(M, generator=g), torch.randn(M, 2 * N, generator=g)))
+    xd, Wkd, bd, wd, zd = x.cuda(), Wk.cuda(), bias.cuda(), w.cuda(), z.cuda()
+    Wnd = Wkd.transpose(1, 2).contiguous()
+    out, h, dz, dz2, act = (torch.empty(s, dtype=dtype, device="cuda") for s in ((M, N), (M, N // 2), (M, 2 * N), (M, 2 * N), (M, N)))
+    tol = _tol(dtype)
+    want = oracle.scatter2scatter(x, Wk, se, ss, 1, False, True, None, bias=bias)
+    for (tiles256, got), ref in zip(_both(lambda: ops.up_projection_swiglu_rocm(xd, Wkd, idx, offs, out, h, 1, bd), [out, h]),
+                                    (want, oracle.swiglu_packed(want))):
+        assert torch.isfinite(got).all() and nerr(got, ref) <= tol and nerr(got, tiles256) <= tol
+    z32 = z.float().requires_grad_()
+    h32 = oracle.swiglu_packed(z32)
+    h32.backward(oracle.scatter2scatter(x, Wk, se, ss, 1, False, True, w, compute_dtype=torch.float32).float())
+    ((tiles256, got),) = _both(lambda: ops.down_projection_dx_swiglu_rocm(xd, Wnd.permute(0, 2, 1), idx, offs, zd, dz, wd, 1), [dz])
+    assert torch.isfinite(got).all() and nerr(got, z32.grad) <= tol and nerr(got, tiles256) <= tol
+    need = get_library().xma_rocm_scatter2scatter_few_rows_workspace_bytes(M, N, K, E, 0, ops.EPI_SWIGLU_BWD)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    check(get_library().xma_rocm_scatter2scatter_few_rows(
+        xd.data_ptr(), K, Wnd.data_ptr(), N * K, K, 0, idx.data_ptr(), offs.data_ptr(), dz2.data_ptr(), 2 * N, zd.data_ptr(), 2 * N,
+        act.data_ptr(), N, wd.data_ptr(), None, 0, M, N, K, E, 1, 0, 1, ops.EPI_SWIGLU_BWD, ops._code(xd), ws.data_ptr(), need, ops._stream(xd),
+    ), "xma_rocm_scatter2scatter_few_rows")
+    assert torch.equal(dz2, got) and nerr(act, h32.detach() * w.float()[ss][:, None]) <= tol
