@@ -178,7 +178,7 @@ extern "C" int xma_rocm_group_bwd_W_few_rows(const void *DY, int64_t lddy, int d
     a.dy_div = make_fastdiv((uint32_t)dy_fan_out);
     a.x_div = make_fastdiv((uint32_t)x_fan_out);
     hipStream_t st = (hipStream_t)stream;
-    if (M > (int64_t)MID_ROWS_DW_FROM * E && xma_rocm::mid_dw_takes(a, M)) return xma_rocm::mid_dw(a, dtype, st);
+    if (xma_rocm::mid_dw_leads(a, M) && xma_rocm::mid_dw_takes(a, M)) return xma_rocm::mid_dw(a, dtype, st);
     const bool wide = M > 0 && M <= (int64_t)DW_WIDE_ROWS_PER_EXPERT * E;
     const int TN = wide ? 64 : 128, TK = 16384 / TN;
     const dim3 grid((K_in + TK - 1) / TK, (N_out + TN - 1) / TN, E);

@@ -363,7 +363,8 @@ struct MidDwTile {
     int64_t row_lo;
 };
 
-template <typename T, int GQ, int GP>
+// NT = 1: the rows of dW go past L2 (a variant of its own: the compiler merges the two kinds of store into one where a branch picks).
+template <typename T, int GQ, int GP, int NT>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void mid_dw_kernel(const DwArgs a) {
     constexpr bool GATHER = GQ != 0 || GP != 0;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -520,7 +521,10 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void mid_dw_kernel(const DwArgs a)
             set_tile();
             first_items();
         }
-        // a 32-row block x 64 columns at a time through 4 KB of place 0 that belong to the wave, out as rows of 128 bytes
+        // a 32-row block x 64 columns at a time through 4 KB of place 0 that belong to the wave, out as rows of 128 bytes: past L2 (NT)
+        // where they start on 64-byte boundaries; elsewhere most lines come from two stores, which L2 has to join (40 experts of
+        // 3864 x 8136, 46 rows each: 1640 us past it, 990 through it; on the boundaries, 129 to 640 rows, 0.71 against 0.78 of the time of
+        // the 256 x 256 tiles)
         const int lrow = lane & 31, lhalf = lane >> 5;
         uint16_t *DWe = a.DW + (int64_t)done.e * a.dw_es;
         unsigned char *stage = smem + wave * 4096;
@@ -544,7 +548,13 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void mid_dw_kernel(const DwArgs a)
                 for (int it = 0; it < 4; ++it) {
                     const int r = 8 * it + (lane >> 3), o = obase + r;
                     const u32x4 v = *(const u32x4 *)(stage + r * 128 + (((lane & 7) ^ ((r >> 1) & 7)) << 4));
-                    if (o < a.N_out && cz < a.K_in) __builtin_nontemporal_store(v, (u32x4 *)(DWe + (int64_t)o * a.lddw + cz));
+                    if (o < a.N_out && cz < a.K_in) {
+                        u32x4 *at = (u32x4 *)(DWe + (int64_t)o * a.lddw + cz);
+                        if constexpr (NT != 0)
+                            __builtin_nontemporal_store(v, at);
+                        else
+                            *at = v;
+                    }
                 }
                 wave_lds_sync(); // the next block overwrites the area
             }
@@ -636,17 +646,20 @@ template <typename T, int WT> int mid_dispatch_fwd(const FwdArgs &a, int epi, fl
     return mid_launch_fwd<T, WT, XMA_ROCM_EPI_SWIGLU_BWD>(a, part, st);
 }
 
-template <typename T, int GQ, int GP> int mid_launch_dw(const DwArgs &a, hipStream_t st) {
+// whether the 128-byte pieces of dW's rows start on 64-byte boundaries
+inline int mr_whole_lines(const DwArgs &a) { return (((uintptr_t)a.DW | (uintptr_t)(a.lddw * 2) | (uintptr_t)(a.dw_es * 2)) & 63) == 0; }
+
+template <typename T, int GQ, int GP, int NT> int mid_launch_dw(const DwArgs &a, hipStream_t st) {
     const int64_t tiles = (int64_t)a.E * ((a.N_out + MR_BM - 1) / MR_BM) * ((a.K_in + MR_BN - 1) / MR_BN);
-    const int rc = gemm_set_smem(mid_dw_kernel<T, GQ, GP>, MR_SMEM_BYTES);
+    const int rc = gemm_set_smem(mid_dw_kernel<T, GQ, GP, NT>, MR_SMEM_BYTES);
     if (rc) return rc;
-    mid_dw_kernel<T, GQ, GP><<<(unsigned)(tiles + 7 < MR_RUN ? tiles + 7 : MR_RUN), GEMM_THREADS, MR_SMEM_BYTES, st>>>(a);
+    mid_dw_kernel<T, GQ, GP, NT><<<(unsigned)(tiles + 7 < MR_RUN ? tiles + 7 : MR_RUN), GEMM_THREADS, MR_SMEM_BYTES, st>>>(a);
     return xma_check_launch("mid_dw_kernel");
 }
 
-template <typename T> int mid_dispatch_dw(const DwArgs &a, hipStream_t st) {
-    if (!a.dy_grouped) return mid_launch_dw<T, 1, 0>(a, st);
-    return a.x_grouped ? mid_launch_dw<T, 0, 0>(a, st) : mid_launch_dw<T, 0, 1>(a, st);
+template <typename T, int NT> int mid_dispatch_dw(const DwArgs &a, hipStream_t st) {
+    if (!a.dy_grouped) return mid_launch_dw<T, 1, 0, NT>(a, st);
+    return a.x_grouped ? mid_launch_dw<T, 0, 0, NT>(a, st) : mid_launch_dw<T, 0, 1, NT>(a, st);
 }
 
 } // namespace
@@ -685,6 +698,14 @@ int mid_fwd(const FwdArgs &a, int wt, int epi, int dtype, float *part, hipStream
     return wt ? mid_dispatch_fwd<_Float16, 1>(a, epi, part, st) : mid_dispatch_fwd<_Float16, 0>(a, epi, part, st);
 }
 
+bool mid_dw_leads(const DwArgs &a, int64_t M) {
+    // From 40 rows per expert on in launches of two and more rounds of tiles (one and more where rows of dW start off 64-byte
+    // boundaries), from 96 in smaller ones, whose time is the latency of a tile.  Small tiles / these, us: 5 experts of 688 x 256, 58 rows
+    // each, 4.8 / 6.0; 20 of 1608 x 736, 72 rows, 1.5 rounds, 17.4 / 19.0; 89 of 600 x 832, 76 rows, 3.5 rounds, 34.5 / 25.5.
+    const int64_t tiles = (int64_t)a.E * ((a.N_out + MR_BM - 1) / MR_BM) * ((a.K_in + MR_BN - 1) / MR_BN);
+    return M > (tiles >= (mr_whole_lines(a) ? 2 : 1) * MR_RUN ? 40 : 96) * (int64_t)a.E;
+}
+
 bool mid_dw_takes(const DwArgs &a, int64_t M) {
     if (a.scale || (!a.dy_grouped && !a.x_grouped)) return false;
     const int64_t dy_rows = a.dy_grouped ? MR_K : (M + a.dy_fan_out - 1) / a.dy_fan_out, x_rows = a.x_grouped ? MR_K : (M + a.x_fan_out - 1) / a.x_fan_out;
@@ -693,7 +714,8 @@ bool mid_dw_takes(const DwArgs &a, int64_t M) {
 }
 
 int mid_dw(const DwArgs &a, int dtype, hipStream_t st) {
-    return dtype == XMA_ROCM_BF16 ? mid_dispatch_dw<__bf16>(a, st) : mid_dispatch_dw<_Float16>(a, st);
+    if (mr_whole_lines(a)) return dtype == XMA_ROCM_BF16 ? mid_dispatch_dw<__bf16, 1>(a, st) : mid_dispatch_dw<_Float16, 1>(a, st);
+    return dtype == XMA_ROCM_BF16 ? mid_dispatch_dw<__bf16, 0>(a, st) : mid_dispatch_dw<_Float16, 0>(a, st);
 }
 
 } // namespace xma_rocm

@@ -3,14 +3,16 @@
 
 #include "gemm_common.hpp"
 
-// Rows per expert on average beyond which the few-row entry points take these kernels (measured in few_rows.hip).
-constexpr int MID_ROWS_FWD_FROM = 24, MID_ROWS_DW_FROM = 40;
+// Rows per expert on average beyond which the few-row entry point takes the forward-type kernels (measured in few_rows.hip).
+constexpr int MID_ROWS_FWD_FROM = 24;
 
 namespace xma_rocm {
 
 // whether the kernels have the variant and can address the operands
 bool mid_fwd_takes(const FwdArgs &a, int w_is_kn, int epilogue);
 bool mid_dw_takes(const DwArgs &a, int64_t M);
+// whether dW is shorter with 128 x 256 tiles than with the small ones of the few-row entry point
+bool mid_dw_leads(const DwArgs &a, int64_t M);
 // whether a forward-type launch beyond the few-row regime is shorter with 128 x 256 than with 256 x 256 tiles, as far as its sizes tell
 bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue);
 // fp32 sums of the K ranges of a launch with few tiles; 0: not cut

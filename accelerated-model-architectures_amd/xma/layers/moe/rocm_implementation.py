@@ -366,7 +366,7 @@ class _FusedSwiGLUExperts(torch.autograd.Function):
             ops.down_projection_dx_swiglu_rocm(
                 grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, flat_w, top_k
             )
-            if b_proj is None and ops._dw_loader_scales(z.size(0), w_proj.size(0), z.dtype):
+            if b_proj is None and ops._dw_loader_scales(z.size(0), w_proj.size(0), z.dtype, w_proj.size(2), w_proj.size(1)):
                 # a handful of rows per expert: the weight gradient's loader gathers and scales the rows of dy itself (and
                 # rounds them like the copy would), one launch less
                 ops.group_bwd_W_rocm(grad_out, h, sorted_scattered_idxs, expert_offsets, d_w_proj, flat_w, top_k, 0)
@@ -452,7 +452,7 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, 
     # the operand of dW2: see xma_rocm_moe in the library's header
     if few16 and glu and _scale_by_top_k(k):
         dw2_form, dw2_operand = 1, M * I * s
-    elif not b_proj and ops._dw_loader_scales(M, E, dtype):
+    elif not b_proj and ops._dw_loader_scales(M, E, dtype, H, I):
         dw2_form, dw2_operand = 0, 0
     else:
         dw2_form, dw2_operand = 2, M * H * s

@@ -110,6 +110,10 @@ FEW_ROWS_MAX_WORKSPACE = 256 << 20  # bytes of fp32 partial sums a forward-type 
 # 512 rows 557 -> 440), or where it has at most one 256 x 256 tile per compute unit (8 experts of H = 512, I = 1024, 2048 rows: 49 -> 42).
 MID_ROWS_MAX = 65535  # rows in all, limit of the forward-type entry point
 MID_ROWS_PER_EXPERT_DW, MID_ROWS_FEW_TILES_DW = 640, 256
+# Rows of dW that start off 64-byte boundaries leave the 128 x 256 tiles through L2, from where they push out the operands in launches of
+# more than four rounds of 512 tiles (29 experts of 2560 x 7432, 517 rows: 768 us with the 256 x 256 tiles, 871; 102 of 1760 x 2504, 146
+# rows: 386, 426).  Up to 128 rows the small tiles are the other choice, and these lead all the same (0.70 - 0.95 of their time).
+MID_ROWS_BROKEN_LINES_DW = 2048
 
 
 @torch.library.custom_op("xma_rocm::continuous_count_set", mutates_args={"y"})
@@ -221,14 +225,19 @@ def _mid_rows_dw(M: int, N_out: int, K_in: int, E: int, dtype: torch.dtype) -> b
     """the same for the weight gradient (of operands that are not both gathered, unscaled)"""
     if M <= 0 or FEW_ROWS_MAX == 0 or dtype not in (torch.bfloat16, torch.float16) or max(E, -(-N_out // 32)) > 65535:
         return False
+    if K_in % 32 and M > 128 * E and E * -(-N_out // 128) * -(-K_in // 256) > MID_ROWS_BROKEN_LINES_DW:
+        return False
     return M <= MID_ROWS_PER_EXPERT_DW * E or E * -(-N_out // 256) * -(-K_in // 256) <= MID_ROWS_FEW_TILES_DW
 
 
-def _dw_loader_scales(M: int, E: int, dtype: torch.dtype) -> bool:
+def _dw_loader_scales(M: int, E: int, dtype: torch.dtype, N_out: int = 1 << 16, K_in: int = 1 << 16) -> bool:
     """whether dW2 gathers and scales the rows of dy in its loader, which the small tile of dW does and the larger ones do not;
     the scaled grouped copy costs a launch and pays from about 64 rows per expert on (8 experts of H = 2048, I = 8192: 64 rows 61
-    against 57 + 4 us, 96 rows 76 against 63 + 4)"""
-    return _few_rows(M, E, dtype, "dW") and M <= 64 * E
+    against 57 + 4 us, 96 rows 76 against 63 + 4), in launches of less than a round or two of 128 x 256 tiles only where those lead
+    by as much (29 experts of 616 x 512, 67 rows, 7.5 against 12.8; 10 of 608 x 536, 96 rows, 8.2 against 11.8)"""
+    tiles = E * -(-N_out // 128) * -(-K_in // 256)
+    limit = 128 if tiles < 512 else 96 if tiles < 1024 and K_in % 32 == 0 else 64
+    return _few_rows(M, E, dtype, "dW") and M <= limit * E
 
 
 def _few_rows_fwd(M: int, N: int, K: int, E: int, w_is_kn: int, ldw: int, x_span: int, dtype: torch.dtype, epilogue: int) -> bool:

@@ -254,7 +254,8 @@ XMA_API int xma_rocm_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped, i
  * fp32 sums; bf16 / fp16 only; a scaled row of DY is rounded to the operand type before it is multiplied, as a scaled
  * grouped copy would hold it).  M = rows in all (the length of the grouped order), which picks the shape of a
  * workgroup's tile of DW[e]: 64 x 256 up to 24 rows per expert on average, 128 x 128 beyond or when M <= 0 (not known), and from
- * 40 rows on 128 x 256, two workgroups per compute unit, where nothing is scaled and at most one operand is gathered.  In the
+ * 40 rows on (96 in launches of few tiles) 128 x 256, two workgroups per compute unit, where nothing is scaled and at most one
+ * operand is gathered.  In the
  * first two the expert's rows are the K dimension of the tile's MFMAs, 32 at a time: with a handful of rows per expert the launch
  * runs at the rate of a fill of DW, where xma_rocm_group_bwd_W spends a prologue, one K step and an epilogue per
  * 256 x 256 tile.  Correct for any number of rows; more rows are more passes over small operand tiles, so it leads

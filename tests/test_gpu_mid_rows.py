@@ -132,3 +132,34 @@ def test_swiglu_of_transposed_weights(dtype, case):
         act.data_ptr(), N, wd.data_ptr(), None, 0, M, N, K, E, 1, 0, 1, ops.EPI_SWIGLU_BWD, ops._code(xd), ws.data_ptr(), need, ops._stream(xd),
     ), "xma_rocm_scatter2scatter_few_rows")
     assert torch.equal(dz2, got) and nerr(act, h32.detach() * w.float()[ss][:, None]) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,N,K", [
+    ((300, 0, 64, 65, 129, 200), 1288, 2056),  # 594 tiles, rows of dW off 64-byte boundaries
+    ((0, 300, 63, 1, 128, 300), 1288, 2080),  # on them
+    (tuple(7 * e % 150 * (e % 9 != 4) for e in range(69)), 520, 776),  # 1380 tiles, more experts than a wave has lanes
+    (tuple(11 * e % 170 * (e % 7 != 2) for e in range(61)), 776, 800),  # 1708 tiles, ranked by their rows
+], ids=lambda v: str(len(v)) if isinstance(v, tuple) else str(v))
+def test_dw_walk(dtype, counts, N, K):
+    """launches of more than 512 tiles: a workgroup goes on to a second and third one, whose first items it loads while the one before
+    leaves through the ring's free place, also past experts without rows; every expert on its own against an fp32 product"""
+    from xma.rocm import ops
+
+    E, M = len(counts), sum(counts)
+    tiles = E * -(-N // 128) * -(-K // 256)
+    assert tiles > 512 and tiles % 8 and 640 * E >= M > (40 if tiles >= 1024 else 96) * E and 0 in counts
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    offs = torch.tensor(counts).cumsum(0).cuda()
+    idx = torch.randperm(M, generator=g, device="cuda")
+    x, dy = (torch.randn(M, n, generator=g, device="cuda").to(dtype) for n in (K, N))
+    for dy_fan, x_fan in ((0, 0), (1, 0), (0, 1)):
+        dW = torch.full((E, N, K), float("nan"), dtype=dtype, device="cuda")
+        ops.group_bwd_W_rocm(dy, x, idx, offs, dW.permute(0, 2, 1), None, dy_fan, x_fan)
+        gx, gdy = (x[idx] if x_fan else x), (dy[idx] if dy_fan else dy)
+        row = 0
+        for e, c in enumerate(counts):
+            want = gdy[row : row + c].float().t() @ gx[row : row + c].float()
+            err = (dW[e].float() - want).abs().max()
+            assert err <= 2.0**-8 * want.abs().max(), (e, c)  # rounding to bf16: 2^-9 of the value; fp16 is closer
+            row += c

@@ -178,6 +178,11 @@ def test_mid_rows_dispatch_rule():
     assert dw(640 * 64, 4096, 4096, 64, bf) and not dw(640 * 64 + 1, 4096, 4096, 64, bf)
     assert dw(1 << 20, 1024, 512, 8, bf) and not dw(1 << 20, 4096, 4096, 8, bf)
     assert not dw(999, 64, 64, 65536, bf) and not dw(999, 64, 64, 8, torch.float32)
+    assert dw(128 * 16, 4096, 4096 + 8, 16, bf) and not dw(129 * 16, 4096, 4096 + 8, 16, bf)  # rows off 64-byte boundaries, many rounds
+    assert dw(129 * 16, 4096, 768 + 8, 16, bf) and dw(129 * 16, 4096, 4096 + 32, 16, bf)
+    loader = ops._dw_loader_scales  # a handful of tiles: up to 128 rows per expert; a round or two of them: 96 or 64
+    assert loader(128 * 10, 10, bf, 608, 536) and not loader(129 * 10, 10, bf, 608, 536)
+    assert loader(96 * 20, 20, bf, 1608, 736) and not loader(97 * 20, 20, bf, 1608, 736) and not loader(65 * 20, 20, bf, 1608, 744)
     assert ops._dw_loader_scales(64 * 8, 8, bf) and not ops._dw_loader_scales(64 * 8 + 1, 8, bf)
 
 
