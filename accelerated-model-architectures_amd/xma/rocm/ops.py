@@ -107,9 +107,11 @@ FEW_ROWS_MAX_WORKSPACE = 256 << 20  # bytes of fp32 partial sums a forward-type 
 # 256 x 256 tiles spend their time at the tiles' edges and in a last round that is nearly empty.  Forward-type GEMMs: the library
 # compares the two by the sizes (64 experts of H = 2048, I = 1408, 256 rows, dX2 208 -> 170 us; 400 rows: equal; 16 experts, K = N = 2048,
 # 1024 rows 175 -> 150, 768 rows 112, 116 with the smaller tiles).  dW up to 640 rows per expert (64 experts, 256 rows, dW1 403 -> 269;
-# 512 rows 557 -> 440), or where it has at most one 256 x 256 tile per compute unit (8 experts of H = 512, I = 1024, 2048 rows: 49 -> 42).
+# 512 rows 557 -> 440), or where the smaller tiles are at most one per compute unit, 128 of 256 x 256 (8 experts of 512 x 1024, 2048 rows,
+# 64 tiles, 47 -> 35; of 1024 x 1024, 8192 rows, 128 tiles, 164 -> 149); beyond, two that share a unit take longer than the one
+# they replace (160 tiles, 4096 rows, 96 -> 107; 192: 107 -> 113, with 4 experts 97 -> 112; 256: 113 -> 129).
 MID_ROWS_MAX = 65535  # rows in all, limit of the forward-type entry point
-MID_ROWS_PER_EXPERT_DW, MID_ROWS_FEW_TILES_DW = 640, 256
+MID_ROWS_PER_EXPERT_DW, MID_ROWS_FEW_TILES_DW = 640, 128
 # Rows of dW that start off 64-byte boundaries leave the 128 x 256 tiles through L2, from where they push out the operands in launches of
 # more than four rounds of 512 tiles (29 experts of 2560 x 7432, 517 rows: 768 us with the 256 x 256 tiles, 871; 102 of 1760 x 2504, 146
 # rows: 386, 426).  Up to 128 rows the small tiles are the other choice, and these lead all the same (0.70 - 0.95 of their time).

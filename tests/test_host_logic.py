@@ -177,6 +177,7 @@ def test_mid_rows_dispatch_rule():
     dw = ops._mid_rows_dw
     assert dw(640 * 64, 4096, 4096, 64, bf) and not dw(640 * 64 + 1, 4096, 4096, 64, bf)
     assert dw(1 << 20, 1024, 512, 8, bf) and not dw(1 << 20, 4096, 4096, 8, bf)
+    assert dw(8192 * 8, 1024, 1024, 8, bf) and not dw(1024 * 8, 1024 + 8, 1024, 8, bf)  # at most one of the smaller tiles per compute unit
     assert not dw(999, 64, 64, 65536, bf) and not dw(999, 64, 64, 8, torch.float32)
     assert dw(128 * 16, 4096, 4096 + 8, 16, bf) and not dw(129 * 16, 4096, 4096 + 8, 16, bf)  # rows off 64-byte boundaries, many rounds
     assert dw(129 * 16, 4096, 768 + 8, 16, bf) and dw(129 * 16, 4096, 4096 + 32, 16, bf)
