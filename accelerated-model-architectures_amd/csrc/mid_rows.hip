@@ -574,7 +574,8 @@ inline double tiles_about(int64_t M, int N, int E, int height) {
 // workgroup takes 1.1 us a step, two that share one 2.1 us each, with 512 at a time, 2.4 where more wait behind them (power); the
 // sums of S > 1 ranges go through memory twice (3.3 TB/s) behind one more launch.  This and tiles256_seconds were fitted together to 336
 // measured pairs of launches (the layers of the benchmark and six others, 100 to 4000 rows per expert): within 12 and 10 % on average.
-// On 504 pairs the launches that mid_fwd_leads chooses are 1.17 times as fast as the 256 x 256 ones, the worst of them 9 % slower.
+// Of the 5302 other pairs in mid_fwd_leads it chooses 3920 launches, which are 1.40 times as fast as the 256 x 256 ones on geometric
+// average; one in twenty of them is more than 3 % slower, the worst takes 1.44 times as long.
 inline double mid_fwd_seconds(int64_t M, int N, int K, int E, int epilogue, int *best) {
     // Long K: one tile too many for a round of K ranges is another round of long ones (8 experts of H = 1024, K = 16384, 270 rows, where
     // most need a third tile: 174 us in 6 ranges, 148 now), so the tiles that experts of average rows need are counted in full.
@@ -690,7 +691,18 @@ bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
     const bool gelu = epilogue >= XMA_ROCM_EPI_GELU_TANH;
     const double pass = gelu ? ((epilogue & 1) ? 6.0 : 4.0) * M * N / 4.5e12 + 4e-6 : 0.;
     const int as = gelu ? XMA_ROCM_EPI_STORE : epilogue;
-    return mid_fwd_seconds(M, N, K, E, as, &S) < 0.96 * (tiles256_seconds(M, N, K, E, as) + pass); // even: as it was
+    // Even: as it was.  The model is one of launches of a few rounds; beyond them it flatters the smaller tiles, most where an epilogue
+    // writes a second tensor, so what they have to be ahead by grows with the rounds.  5302 pairs of launches of random layers (2 to 128
+    // experts, 97 to 8000 rows each), by epilogue, ms lost to choosing the smaller tiles where they were the slower ones, out of the ms
+    // they won: SwiGLU 6.4 of 8.1 without this -> 0.5 of 7.3, GELU 7.0 of 10.0 -> 0.4 of 9.5, store 1.9 of 18.8 -> 1.3 of 18.5, SwiGLU
+    // backward 1.4 of 15.0 -> 0.4 of 14.1; GELU backward 1.1 of 17.1 as it is.
+    const double rounds = tiles_about(M, N, E, MR_BM) / MR_RUN;
+    double even = 0.96;
+    if (gelu && !(epilogue & 1))
+        even -= rounds > 1 ? 0.15 * (rounds - 1) : 0.;
+    else if (!gelu)
+        even -= rounds > 2.5 ? (epilogue == XMA_ROCM_EPI_SWIGLU ? 0.15 : 0.04) * (rounds - 2.5) : 0.;
+    return mid_fwd_seconds(M, N, K, E, as, &S) < even * (tiles256_seconds(M, N, K, E, as) + pass);
 }
 
 int mid_fwd(const FwdArgs &a, int wt, int epi, int dtype, float *part, hipStream_t st) {
