@@ -650,7 +650,7 @@ template <typename T, int EPI> int fr_launch_epilogue(const FwdArgs &a, const fl
 }
 
 template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, float *part, hipStream_t st) {
-    const int S_max = fr_tile_splits(a.N, a.K, a.E, WT);
+    const int S_max = part ? fr_tile_splits(a.N, a.K, a.E, WT) : 1;
     const int steps_all = (a.K + st_k(WT) - 1) / st_k(WT), steps_per = (steps_all + S_max - 1) / S_max;
     const int S = (steps_all + steps_per - 1) / steps_per; // ranges that hold a step (25 steps in 6 ranges of 5: only 5 do)
     const dim3 grid((a.N + ST_N - 1) / ST_N, a.E, S);
@@ -702,22 +702,35 @@ int split_sums_epilogue(const FwdArgs &a, const float *part, int S, int epilogue
     return dtype == XMA_ROCM_BF16 ? run(__bf16{}) : run(_Float16{});
 }
 
-extern "C" size_t xma_rocm_scatter2scatter_few_rows_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E, int w_is_kn,
-                                                                    int epilogue) {
-    if (M <= 0 || N <= 0 || K <= 0 || E <= 0) return 0;
-    // (the 128 x 256 tiles may turn out not to take the launch: then it runs through the small tile, so the larger of the two)
-    const size_t mid = M > (int64_t)MID_ROWS_FWD_FROM * E ? xma_rocm::mid_fwd_workspace_bytes(M, N, K, E) : 0;
+namespace {
+
+int few_epilogue(int epilogue) { // both forms of GELU run through the same kernels
+    return epilogue >= XMA_ROCM_EPI_GELU_ERF ? epilogue - (XMA_ROCM_EPI_GELU_ERF - XMA_ROCM_EPI_GELU_TANH) : epilogue;
+}
+
+size_t few_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E, int w_is_kn, int epilogue) { // of the kernels here
     int S;
     if (fr_takes_tile(M, K, E, w_is_kn)) { // the small MFMA tile, cut along K or not
         S = fr_tile_splits(N, K, E, w_is_kn);
-        if (S == 1) return mid;
-    } else if (epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == XMA_ROCM_EPI_GELU_TANH_BWD || epilogue == XMA_ROCM_EPI_GELU_ERF_BWD) {
+        if (S == 1) return 0;
+    } else if (epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == EPI_GELU_BWD) {
         S = 1; // the vector kernel's sums go to the epilogue kernel
     } else {
-        return mid; // the vector kernel finishes the job itself
+        return 0; // the vector kernel finishes the job itself
     }
-    const size_t few = (size_t)S * (size_t)M * (size_t)N * sizeof(float);
-    return few > mid ? few : mid;
+    return (size_t)S * (size_t)M * (size_t)N * sizeof(float);
+}
+
+} // namespace
+
+extern "C" size_t xma_rocm_scatter2scatter_few_rows_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E, int w_is_kn,
+                                                                    int epilogue) {
+    if (M <= 0 || N <= 0 || K <= 0 || E <= 0) return 0;
+    // What the 128 x 256 tiles ask for where they are meant to run.  An operand beyond their 32-bit offsets, which only the launch
+    // sees, goes through the small tile, uncut where the sums of its K ranges are more than the workspace holds.
+    if (M > (int64_t)MID_ROWS_FWD_FROM * E && xma_rocm::mid_fwd_has(M, E, w_is_kn, few_epilogue(epilogue)))
+        return xma_rocm::mid_fwd_workspace_bytes(M, N, K, E);
+    return few_workspace_bytes(M, N, K, E, w_is_kn, few_epilogue(epilogue));
 }
 
 extern "C" int xma_rocm_scatter2scatter_few_rows_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
@@ -737,7 +750,7 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
                 "scatter2scatter_few_rows: epilogue %d", epilogue);
     const int erf_form = epilogue >= XMA_ROCM_EPI_GELU_ERF ? 1 : 0;
     const int asked = epilogue;
-    if (erf_form) epilogue -= XMA_ROCM_EPI_GELU_ERF - XMA_ROCM_EPI_GELU_TANH;
+    epilogue = few_epilogue(epilogue);
     XMA_REQUIRE(M >= 0 && M <= 65535 && N >= 8 && K >= 8 && E >= 1 && E <= 65535 && fan_out >= 1, XMA_ROCM_EINVAL,
                 "scatter2scatter_few_rows: M=%lld N=%d K=%d E=%d fan_out=%d (M and E at most 65535)", (long long)M, N, K, E, fan_out);
     XMA_REQUIRE(N % 8 == 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldo % 8 == 0 && w_expert_stride % 8 == 0,
@@ -798,7 +811,9 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
     a.grid_main = 0;
     a.erf_form = erf_form;
     hipStream_t st = (hipStream_t)stream;
-    if (fr_takes_mid(a, w_is_kn ? 1 : 0, epilogue)) return xma_rocm::mid_fwd(a, w_is_kn ? 1 : 0, epilogue, dtype, (float *)workspace, st);
-    if (dtype == XMA_ROCM_BF16) return fr_launch<__bf16>(a, w_is_kn ? 1 : 0, epilogue, (float *)workspace, st);
-    return fr_launch<_Float16>(a, w_is_kn ? 1 : 0, epilogue, (float *)workspace, st);
+    w_is_kn = w_is_kn ? 1 : 0;
+    if (fr_takes_mid(a, w_is_kn, epilogue)) return xma_rocm::mid_fwd(a, w_is_kn, epilogue, dtype, (float *)workspace, st);
+    float *part = workspace && al16(workspace) && workspace_bytes >= few_workspace_bytes(M, N, K, E, w_is_kn, epilogue) ? (float *)workspace : nullptr;
+    if (dtype == XMA_ROCM_BF16) return fr_launch<__bf16>(a, w_is_kn, epilogue, part, st);
+    return fr_launch<_Float16>(a, w_is_kn, epilogue, part, st);
 }

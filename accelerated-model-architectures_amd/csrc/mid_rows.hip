@@ -670,13 +670,16 @@ size_t mid_fwd_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E) {
     return S == 1 ? 0 : (size_t)S * (size_t)M * (size_t)N * sizeof(float);
 }
 
-bool mid_fwd_takes(const FwdArgs &a, int wt, int epi) {
+bool mid_fwd_has(int64_t M, int32_t E, int wt, int epi) {
     // GELU comes in the layouts that the layer launches, x @ W^T and dy @ W.  SwiGLU also in the other two (weights stored
     // transposed): streaming the weights once per 32 rows instead costs them, 8 experts of H = 2048, I = 8192, 96 rows each,
     // W1 as (H, 2I), 351 us against 116, W2 as (I, H) 167 against 57.
-    if (a.E > MR_MAX_E || (epi == EPI_GELU && wt) || (epi == EPI_GELU_BWD && !wt)) return false;
+    return M > 0 && M <= 65535 && E <= MR_MAX_E && !(epi == EPI_GELU && wt) && !(epi == EPI_GELU_BWD && !wt);
+}
+
+bool mid_fwd_takes(const FwdArgs &a, int wt, int epi) {
     const int64_t x_rows = a.x_grouped ? MR_BM : (a.M + a.fan_out - 1) / a.fan_out; // 32-bit byte offsets from a tile's base
-    return a.M > 0 && a.M <= 65535 && x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)MR_BN * a.ldw * 2 < ((int64_t)1 << 32);
+    return mid_fwd_has(a.M, a.E, wt, epi) && x_rows * a.ldx * 2 < ((int64_t)1 << 32) && (int64_t)MR_BN * a.ldw * 2 < ((int64_t)1 << 32);
 }
 
 bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {

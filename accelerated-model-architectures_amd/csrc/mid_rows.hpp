@@ -8,7 +8,8 @@ constexpr int MID_ROWS_FWD_FROM = 24;
 
 namespace xma_rocm {
 
-// whether the kernels have the variant and can address the operands
+// whether the kernels have the variant, and whether they can address the operands as well
+bool mid_fwd_has(int64_t M, int32_t E, int w_is_kn, int epilogue);
 bool mid_fwd_takes(const FwdArgs &a, int w_is_kn, int epilogue);
 bool mid_dw_takes(const DwArgs &a, int64_t M);
 // whether dW is shorter with 128 x 256 tiles than with the small ones of the few-row entry point

@@ -134,6 +134,25 @@ def test_swiglu_of_transposed_weights(dtype, case):
     assert torch.equal(dz2, got) and nerr(act, h32.detach() * w.float()[ss][:, None]) <= tol
 
 
+def test_rows_beyond_32_bit_offsets():
+    """an operand that the 128 x 256 tiles cannot address goes through the small tile, uncut: the workspace is theirs"""
+    from xma.rocm import ops
+
+    E, M, K, N = 2, 52, 8192, 64
+    far = torch.empty(M, (1 << 32) // (2 * M) // 8 * 8 + 8, dtype=torch.bfloat16, device="cuda")[:, :K]
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(M, K, generator=g).bfloat16()
+    W = (torch.randn(E, N, K, generator=g) * K**-0.5).bfloat16()
+    assert M > 24 * E and M * far.stride(0) * 2 >= 1 << 32 and ops._few_rows_workspace_bytes(M, N, K, E, 0, 0) < 16 * M * N * 4
+    far.copy_(x)
+    offs, idx = torch.tensor([30, M]).cuda(), torch.randperm(M, generator=g).cuda()
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.scatter2scatter_rocm(far, W.cuda().permute(0, 2, 1), idx, offs, out, None, 1, False, True)
+    rows = x[idx.cpu()].float()
+    want = torch.cat([rows[:30] @ W[0].float().t(), rows[30:] @ W[1].float().t()])
+    assert nerr(out, want) <= _tol(torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("counts,N,K", [
     ((300, 0, 64, 65, 129, 200), 1288, 2056),  # 594 tiles, rows of dW off 64-byte boundaries

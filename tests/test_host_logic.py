@@ -88,6 +88,11 @@ def test_argument_errors_are_reported_before_any_launch():
     assert ws(64, 16384, 2048, 8, 0, 1) == 0  # small MFMA tile, enough workgroups from N alone
     assert ws(64, 2048, 8192, 8, 0, 0) == 4 * 64 * 2048 * 4  # small MFMA tile cut into 4 ranges of K
     assert ws(0, 64, 64, 2, 1, 0) == 0
+    # beyond 24 rows per expert what the 128 x 256 tiles ask for, not the small tile's sums, which grow with M
+    assert ws(32000, 512, 2048, 8, 1, 0) == 0 and ws(2048, 8192, 1024, 4, 1, 2) == 0
+    assert ws(8198, 1024, 4096, 4, 0, 1) == 0 and ws(8198, 4096, 1024, 4, 1, 0) == 0 and ws(8000, 8192, 1024, 4, 1, 2) == 0
+    assert ws(8000, 1024, 16384, 4, 1, 0) == 2 * 8000 * 1024 * 4 and ws(258, 136, 8456, 2, 0, 0) == 8 * 258 * 136 * 4  # few tiles, long K
+    assert ws(300, 64, 16384, 2, 0, 5) == 32 * 300 * 64 * 4  # a layout that they do not have: the small tile
     dw = lib.xma_rocm_group_bwd_W_few_rows
     assert dw(p, 64, 1, 1, None, p, 64, 1, 1, p, p, p, 64 * 64, 64, 64, 64, 2, 4, 2, None) == -2  # fp32
     assert dw(p, 64, 1, 1, None, p, 60, 1, 1, p, p, p, 64 * 64, 64, 64, 64, 2, 4, 0, None) == -2  # ldx % 8
@@ -187,6 +192,9 @@ def test_mid_rows_dispatch_rule():
     loader = ops._dw_loader_scales  # a handful of tiles: up to 128 rows per expert; a round or two of them: 96 or 64
     assert loader(128 * 10, 10, bf, 608, 536) and not loader(129 * 10, 10, bf, 608, 536)
     assert loader(96 * 20, 20, bf, 1608, 736) and not loader(97 * 20, 20, bf, 1608, 736) and not loader(65 * 20, 20, bf, 1608, 744)
+    # launches that the library prefers, whose sums would not fit if the small tile made them
+    assert ops._few_rows_fwd(8198, 1024, 4096, 4, 0, 4096, 4099 * 4096, bf, glu) and ops._few_rows_fwd(8198, 4096, 1024, 4, 1, 4096, 8198 * 1024, bf, store)
+    assert ops._few_rows_fwd(8000, 8192, 1024, 4, 1, 8192, 2000 * 1024, bf, bwd) and ops._few_rows_fwd(8000, 1024, 16384, 4, 1, 1024, 8000 * 16384, bf, store)
     assert ops._dw_loader_scales(64 * 8, 8, bf) and not ops._dw_loader_scales(64 * 8 + 1, 8, bf)
 
 
