@@ -418,7 +418,7 @@ _BLOCK_SIZES = struct.Struct("17q")
 class _Plan:
     """sizes, choices and scratch layout of a layer call; a function of the shape, the options and the dispatch limits only"""
 
-    __slots__ = ("sizes_forward", "sizes_backward", "keep", "temp", "back", "keep_bytes", "temp_bytes", "back_bytes", "recompute", "saved_shapes")
+    __slots__ = ("sizes_forward", "sizes_backward", "keep", "temp", "back", "keep_bytes", "temp_bytes", "back_bytes", "saved_shapes")
 
 
 def _layout(sizes: dict[str, int]) -> tuple[dict[str, int], int]:
@@ -443,9 +443,8 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, 
             return 1, ops._few_rows_workspace_bytes(M, N, K, E, w_is_kn, epilogue)
         return 0, ops.scatter2scatter_workspace_bytes(M, N, K, E, device_index)
 
-    def dw(N_out, K_in, scaled):
-        return int(ops._few_rows(M, E, dtype, "dW") or (
-            not scaled and ops._mid_rows_dw(M, N_out, K_in, E, dtype) and M * max(N_out, K_in) < ops.MID_ROWS_OFFSETS))
+    def dw(N_out, K_in, span, scaled):
+        return int(ops._dw_few(M, N_out, K_in, E, dtype, span, scaled, False))
 
     up, down = gemm(U, H, 0, H, T * H, epi_fwd), gemm(H, I, 0, I, M * I, ops.EPI_STORE)
     dx2, dx1 = gemm(I, H, 1, I, T * H, epi_bwd), gemm(H, U, 1, H, M * U, ops.EPI_STORE)
@@ -469,9 +468,8 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, 
     p.keep, p.keep_bytes = _layout(sizes)
     p.temp, p.temp_bytes = _layout(temp)
     p.back, p.back_bytes = _layout(back)
-    p.recompute = not save
     p.saved_shapes = ((T, H), (E, H), (T, E), (E, U, H), (E, H, I), (E, U), (E, H), (p.keep_bytes,))
-    few = (up[0], down[0], dx2[0], dw(H, I, dw2_form == 0), dw(U, H, False), dx1[0], dw2_form, int(not save))
+    few = (up[0], down[0], dx2[0], dw(H, I, max((M if dw2_form == 2 else T) * H, M * I), dw2_form == 0), dw(U, H, max(M * U, T * H), False), dx1[0], dw2_form, int(not save))
     head = (_BLOCK_SIZES.size + _BLOCK_POINTERS.size, T, H, I, E, k, ops._DTYPE_CODE[dtype], ("swiglu_packed", "tanh", "none").index(act), *few)
     p.sizes_forward = _BLOCK_SIZES.pack(*head, temp["workspace"])
     p.sizes_backward = _BLOCK_SIZES.pack(*head, back["workspace"])
@@ -483,7 +481,7 @@ def _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, s
     T, H = x.shape
     E, I = w_proj.size(0), w_proj.size(2)
     device = x.device
-    p = _plan(T, H, I, E, k, x.dtype, act, b_proj is not None, save, device.index, (ops.FEW_ROWS_MAX, *ops.FEW_ROWS_PER_EXPERT.values()))
+    p = _plan(T, H, I, E, k, x.dtype, act, b_proj is not None, save, device.index, ops.dispatch_limits())
     y = torch.empty_like(x)
     if gate_weight is not None:
         logits = torch.empty(T, E, dtype=x.dtype, device=device)

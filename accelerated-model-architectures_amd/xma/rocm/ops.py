@@ -232,6 +232,19 @@ def _mid_rows_dw(M: int, N_out: int, K_in: int, E: int, dtype: torch.dtype) -> b
     return M <= MID_ROWS_PER_EXPERT_DW * E or E * -(-N_out // 256) * -(-K_in // 256) <= MID_ROWS_FEW_TILES_DW
 
 
+def _dw_few(M: int, N_out: int, K_in: int, E: int, dtype: torch.dtype, span: int, scaled: bool, both_gathered: bool) -> bool:
+    """whether a weight gradient takes the few-row entry point (span: elements of the longer of its operands, as x_span)"""
+    return _few_rows(M, E, dtype, "dW") or (
+        not scaled and not both_gathered and span < MID_ROWS_OFFSETS and _mid_rows_dw(M, N_out, K_in, E, dtype)
+    )
+
+
+def dispatch_limits() -> tuple[int, ...]:
+    """what these choices depend on besides sizes and types"""
+    return (FEW_ROWS_MAX, *FEW_ROWS_PER_EXPERT.values(), FEW_ROWS_MAX_WORKSPACE, FEW_ROWS_NT_MAX_ELEMENTS, MID_ROWS_MAX, MID_ROWS_PER_EXPERT_DW,
+            MID_ROWS_FEW_TILES_DW, MID_ROWS_BROKEN_LINES_DW, MID_ROWS_MAX_EXPERTS, MID_ROWS_OFFSETS)
+
+
 def _dw_loader_scales(M: int, E: int, dtype: torch.dtype, N_out: int = 1 << 16, K_in: int = 1 << 16) -> bool:
     """whether dW2 gathers and scales the rows of dy in its loader, which the small tile of dW does and the larger ones do not;
     the scaled grouped copy costs a launch and pays from about 64 rows per expert on (8 experts of H = 2048, I = 8192: 64 rows 61
@@ -428,10 +441,8 @@ def group_bwd_W_rocm(
     # a handful of rows per expert (the index has one entry per row): the launch is a stream of stores, not arithmetic; some
     # hundreds: the same entry point, for its 128 x 256 tiles where they cover the operands
     M = sorted_scattered_idxs.numel()
-    few = _few_rows(M, E, DW.dtype, "dW") or (
-        dy_scale is None and 0 in (dy_fan_out, x_fan_out) and _mid_rows_dw(M, N_out, K_in, E, DW.dtype)
-        and max(DY.size(0) * DY.stride(0), X.size(0) * X.stride(0)) < MID_ROWS_OFFSETS
-    )
+    few = _dw_few(M, N_out, K_in, E, DW.dtype, max(DY.size(0) * DY.stride(0), X.size(0) * X.stride(0)), dy_scale is not None,
+                  0 not in (dy_fan_out, x_fan_out))
     name = "xma_rocm_group_bwd_W_few_rows" if few else "xma_rocm_group_bwd_W"
     operands = (
         _ptr(DY), _rows(DY, "DY"), int(dy_fan_out == 0), max(dy_fan_out, 1), _ptr(dy_scale),

@@ -198,6 +198,77 @@ def test_mid_rows_dispatch_rule():
     assert ops._dw_loader_scales(64 * 8, 8, bf) and not ops._dw_loader_scales(64 * 8 + 1, 8, bf)
 
 
+def test_layer_plan_makes_the_choices_of_the_ops(monkeypatch):
+    """which entry point each GEMM of the layer's call takes, against what the single ops would do with their operands; and a plan that was
+    laid out under other dispatch limits is not used again"""
+    import random
+
+    from xma.layers.moe import rocm_implementation as R
+    from xma.rocm import ops
+
+    monkeypatch.setattr(ops, "scatter2scatter_workspace_bytes", lambda *a: 0)
+    calls = {}
+    for name in ("xma_rocm_scatter2scatter_few_rows", "xma_rocm_scatter2scatter_bias", "xma_rocm_down_projection_dx_swiglu",
+                 "xma_rocm_group_bwd_W_few_rows", "xma_rocm_group_bwd_W", "xma_rocm_group"):
+        calls[name] = lambda *a, n=name: taken.append(n) or 0
+    calls["xma_rocm_scatter2scatter_few_rows_workspace_bytes"] = lambda *a: 0
+    lib = ops.get_library()
+
+    class Library:
+        def __getattr__(self, name):
+            return calls.get(name) or getattr(lib, name)
+
+    class Device(torch.Tensor):  # a tensor without memory that passes for one on the GPU
+        is_cuda = property(lambda self: True)
+
+    new = lambda *shape, dtype: torch.empty(shape, dtype=dtype, device="meta").as_subclass(Device)
+    rng, seen = random.Random(5), set()
+    for _ in range(150):
+        E, H, I = rng.choice([2, 8, 64, 1200]), 8 * rng.randint(1, 600), 16 * rng.randint(1, 300)
+        k, dtype, act = rng.randint(1, min(E, 6)), rng.choice([torch.bfloat16, torch.bfloat16, torch.float32]), rng.choice(["swiglu_packed", "swiglu_packed", "tanh"])
+        T = max(1, int(E * 2 ** rng.uniform(0, 13)) // k)
+        M, U = T * k, 2 * I if act == "swiglu_packed" else I
+        plan = R._plan(T, H, I, E, k, dtype, act, False, True, 0, ops.dispatch_limits())
+        few = dict(zip(("up", "down", "dx2", "dw2", "dw1", "dx1", "form"), R._BLOCK_SIZES.unpack(plan.sizes_forward)[8:15]))
+        x, dy, z, h, out = new(T, H, dtype=dtype), new(T, H, dtype=dtype), new(M, U, dtype=dtype), new(M, I, dtype=dtype), new(M, H, dtype=dtype)
+        w_fc, w_proj = new(E, U, H, dtype=dtype), new(E, H, I, dtype=dtype)
+        idx, offs, w = new(M, dtype=torch.int64), new(E, dtype=torch.int64), new(M, dtype=dtype)
+        with monkeypatch.context() as m:
+            m.setattr(ops, "get_library", Library)
+            m.setattr(ops, "_stream", lambda t: 0)
+            m.setattr(ops, "_ptr", lambda t: None if t is None else 256)
+            m.setattr(ops, "_few_rows_workspace_bytes", lambda *a: lib.xma_rocm_scatter2scatter_few_rows_workspace_bytes(*a))
+            m.setattr(torch, "empty", lambda *a, **kw: None)
+            want = {}
+            for key, call in dict(
+                up=(lambda: ops.up_projection_swiglu_rocm(x, w_fc.permute(0, 2, 1), idx, offs, z, h, k)) if act == "swiglu_packed" else None,
+                down=lambda: ops.scatter2scatter_rocm(h, w_proj.permute(0, 2, 1), idx, offs, out, None, 1, True, False),
+                dx2=(lambda: ops.down_projection_dx_swiglu_rocm(dy, w_proj, idx, offs, z, z, w, k)) if act == "swiglu_packed" else None,
+                dw2={0: lambda: ops.group_bwd_W_rocm(dy, h, idx, offs, w_proj.permute(0, 2, 1), w, k, 0),
+                     1: lambda: ops.group_bwd_W_rocm(dy, h, idx, offs, w_proj.permute(0, 2, 1), None, k, 0),
+                     2: lambda: ops.group_bwd_W_rocm(out, h, idx, offs, w_proj.permute(0, 2, 1), None, 0, 0)}[few["form"]],
+                dw1=lambda: ops.group_bwd_W_rocm(z, x, idx, offs, w_fc.permute(0, 2, 1), None, 0, k),
+                dx1=lambda: ops.scatter2scatter_rocm(z, w_fc, idx, offs, out, None, 1, True, False),
+            ).items():
+                if call is None:
+                    continue
+                taken = []
+                call()
+                want[key] = int(taken[-1].endswith("few_rows"))
+        assert want == {key: few[key] for key in want}, (T, H, I, E, k, dtype, act)
+        seen |= {(key, v) for key, v in want.items()}
+    assert len(seen) == 12  # both choices of all six
+
+    R._plan.cache_clear()
+    limits = [n for n in vars(ops) if re.match(r"(FEW|MID)_ROWS_[A-Z_]+$", n)]
+    before = ops.dispatch_limits()
+    for name in limits:
+        with monkeypatch.context() as m:
+            value = getattr(ops, name)
+            m.setattr(ops, name, dict.fromkeys(value, 1) if isinstance(value, dict) else value + 1)
+            assert ops.dispatch_limits() != before, name
+
+
 def test_layer_call_leaves_other_shapes_to_the_ops(monkeypatch):
     """the layer's library call reads all its tensors by one E, H and I, so whatever has others goes through the ops (None here),
     which check each tensor"""
