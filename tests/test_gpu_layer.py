@@ -236,3 +236,44 @@ def test_routing_behind_the_gate(T, E, k):
         for m in (one, ops):
             m.gate.weight[E // 2 :] = m.gate.weight[E // 2].clone()
     _same(_step(one, x, dy), _step(ops, x, dy))
+
+
+@pytest.mark.parametrize("act", [swiglu_packed, nn.GELU(approximate="tanh")], ids=["swiglu", "gelu"])
+@pytest.mark.parametrize("T,k", [(7, 2), (300, 2), (300, 4)])  # routing inside the router's kernel; 128 x 256 tiles, both operands of dW2
+def test_side_stream_capture_and_replay(T, k, act):
+    """forward and backward of the layer as one call on another stream, and captured once and replayed on new inputs (new routing
+    included) with eager passes and synchronisations in between"""
+    from xma.layers.moe import rocm_implementation as R
+
+    one, _, sx, sdy = _layers(T, 8, k, 256, 512, torch.bfloat16, act=act)
+    assert R.layer(one, sx) is not None
+
+    def step(x, dy):
+        x = x.detach().requires_grad_()
+        for p in one.parameters():
+            p.grad = None
+        y, logits = one(x)
+        y.backward(dy)
+        return [y.detach(), logits.detach(), x.grad, *(p.grad for p in one.parameters())]
+
+    want = step(sx, sdy)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            got = step(sx, sdy)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    _same(got, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step(sx, sdy)
+    for seed in range(4):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        x, dy = (torch.randn(t.shape, device="cuda", generator=g).bfloat16() for t in (sx, sdy))
+        sx.copy_(x), sdy.copy_(dy)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [o.clone() for o in outs]
+        _same(got, step(x, dy))
+        torch.cuda.synchronize()
