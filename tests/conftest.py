@@ -23,3 +23,12 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture(params=["chosen", "256 x 256"])
+def either_tile(request, monkeypatch):
+    """the grouped GEMMs by the dispatch rule, and by the 256 x 256 kernels whatever the rule says"""
+    from xma.rocm import ops
+
+    if request.param == "256 x 256":
+        monkeypatch.setattr(ops, "FEW_ROWS_MAX", 0)

@@ -98,6 +98,7 @@ def test_moe_reference_sizes(dtype, act_name):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("act_name", ["swiglu_packed", "gelu"])
+@pytest.mark.usefixtures("either_tile")
 def test_moe_many_tokens_ragged(dtype, act_name):
     _run_case(dtype, 1500, 8, 2, 256, 384, act_name, skew=1.5, empty=(2,))
     _run_case(dtype, 777, 16, 4, 264, 136, act_name, skew=2.0, empty=(0, 15))
@@ -105,6 +106,7 @@ def test_moe_many_tokens_ragged(dtype, act_name):
 
 
 @pytest.mark.parametrize("act_name", ["swiglu_packed", "gelu"])
+@pytest.mark.usefixtures("either_tile")
 def test_moe_tiles_split_along_k(act_name):
     """Few tiles and a long K: the tiles of the only (partial) round are cut into K slices that a second kernel adds
     up, in all three epilogues (up-projection K = H, dX2 K = H, down-projection K = I, dX1 K = 2 I)."""
@@ -114,6 +116,7 @@ def test_moe_tiles_split_along_k(act_name):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("act_name", ["swiglu_packed", "glu", "gelu"])
+@pytest.mark.usefixtures("either_tile")
 def test_moe_with_expert_biases(dtype, act_name):
     """add_bias=True: Experts.bias (E, out) on both projections, as the reference's torch path applies it
     (F.linear(x[e], weight[e], bias[e]), moe/__init__.py:96-100), forward and all gradients including the two biases'

@@ -100,6 +100,7 @@ def test_scatter2scatter(dtype, case, w_kn, x_grouped, y_grouped):
             assert nerr(out, want) <= _tol(dtype), limit
 
 
+@pytest.mark.usefixtures("either_tile")
 def test_scatter2scatter_launches_outside_the_persistent_kernel():
     """Three launches that the layer itself never makes and that take the one-workgroup-per-tile kernel instead of the
     persistent one: more experts than its schedule tables hold (E = 1100, most of them empty), a row scale that starts
@@ -155,6 +156,7 @@ def test_scatter2scatter_launches_outside_the_persistent_kernel():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.usefixtures("either_tile")
 def test_scatter2scatter_bias_and_expert_column_sums(dtype):
     """The experts' bias as the first term of the grouped GEMM's sums (plain store and SwiGLU epilogues, both weight
     layouts, with and without a row scale, a tile split along K), and its gradient, the per-expert column sums of grouped
@@ -249,6 +251,7 @@ ROW_COUNT_CASES = [
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("case", ROW_COUNT_CASES)
 @pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.usefixtures("either_tile")
 def test_scatter2scatter_expert_row_counts(dtype, case, w_kn):
     from xma.layers.moe import rocm_implementation as R
 
@@ -696,6 +699,7 @@ SCALED_ACT_CASES = [
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("case", SCALED_ACT_CASES)
+@pytest.mark.usefixtures("either_tile")
 def test_down_projection_dx_swiglu_scaled_act(dtype, case):
     """dX2 + SwiGLU backward with the second output of its epilogue (xma_rocm_down_projection_dx_swiglu): dz bit-identical
     to the launch without it; scaled_act[n] = swiglu_packed(z[n]) * w[idx[n]] against the oracle's activation in fp32
@@ -813,6 +817,7 @@ def test_fp32_tiles(counts, K, N):
 
 @pytest.mark.parametrize("K", [200, 232, 328, 456, 1000])
 @pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.usefixtures("either_tile")
 def test_scatter2scatter_k_tail_of_overlapping_tiles(K, w_kn):
     """Four to sixteen K steps with a partial last one, tiles of more than 192 rows one after another on a workgroup (which load
     the next tile's first step inside their last one) and a smaller one among them: whatever lies past K in memory is NaN."""
@@ -840,6 +845,7 @@ def test_scatter2scatter_k_tail_of_overlapping_tiles(K, w_kn):
 
 @pytest.mark.parametrize("counts", [(17,) * 1000, (0,) * 400 + (16990,) + (0,) * 598 + (10,)])
 @pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.usefixtures("either_tile")
 def test_scatter2scatter_walk_refills_its_table(counts, w_kn):
     """Launches of more than 256 candidate tiles for each of 256 workgroups, (M / 256 + E) column blocks in all: a workgroup
     looks for its tiles 256 candidates at a time, and the second table holds tiles (even counts) or none (two experts with
