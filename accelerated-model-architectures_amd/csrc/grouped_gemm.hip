@@ -1647,7 +1647,6 @@ inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 } // namespace xma_rocm
 
-
 using namespace xma_rocm;
 
 static int scatter2scatter_impl(const void *X, int64_t ldx, const void *W, int64_t w_expert_stride, int64_t ldw,

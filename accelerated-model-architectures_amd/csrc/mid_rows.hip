@@ -18,7 +18,9 @@
 //
 // A load has a whole K step (two phases, 1024 cycles of the matrix pipe alone, twice that with both workgroups at work) to
 // land; 2 x 40 KB are in flight per compute unit.  Each wave loads four 1 KB pieces of an item, so the waits are vmcnt(8): the
-// two items behind the one that is waited for.  The sums run over k in the order of the 256 x 256 kernels.
+// two items behind the one that is waited for.  dW's sums run over an expert's rows from the first to the last, as in the 256 x 256
+// kernels.  Forward types add in another order than those where the launch is cut into ranges of K (one fp32 sum per range, added in
+// order), and where a column of tiles starts at a K step of its own (`turn`); both depend on the sizes only, not on the routing.
 //
 // Measured against the kernels that served these launches before (us; E experts, rows each): forward + backward GEMMs of E = 64, H =
 // 2048, I = 1408, 96 rows 933 -> 715, 256 rows 1470 -> 1240; E = 128, H = 576, I = 256, 128 rows 197 -> 143; E = 8, H = 512, I =
@@ -117,8 +119,8 @@ __device__ __forceinline__ uint32_t mr_place_after(uint32_t place, int n) {
 }
 
 // The K loop over steps 0 .. steps - 1 (> 0).  load(IC<0 | 1 | 2>, step, place) issues this wave's four pieces of Q, P0 or P1;
-// Q(0), P0(0), P1(0) and, with more than one step, Q(1) are under way, in the place `at` and those behind it.  begin(s) and mid(s) stand in front
-// of the loads of phase 1 and behind those of P1 in phase 2 (the row indices of a gathered operand); B8 and B4 are the waits at
+// Q(0), P0(0), P1(0) and, with more than one step, Q(1) are under way, in the place `at` and those behind it.  begin(s) and mid(s) stand
+// in front of the loads of phase 1 and behind those of P1 in phase 2 (the row indices of a gathered operand); wait_b() is the wait and
 // barrier B of a step with another one behind it.  NB: 32-row blocks of this wave's 64 rows that hold valid rows.
 template <typename T, int QTR, int PTR, int NB, typename Load, typename Begin, typename WaitB, typename Mid>
 __device__ __forceinline__ void mr_k_loop(f32x16 (&acc)[4][2], const unsigned char *smem, const ItemFrag<QTR> &qf,

@@ -598,8 +598,8 @@ template <typename T> __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, 
 // ROUTE: the launch is one workgroup, and what route would make of its ids - counts, inclusive offsets, the stable order by
 // expert - comes along instead of from a launch of its own.  At most 512 keys expert * 512 + position are in LDS: a thread per id counts
 // the smaller keys (where the id goes), a thread per expert those below its own and below the next expert's first key.
-// Such a pass is its launches: 7 tokens of 128 experts (H = 576, k = 8) 7.6 + 3.1 -> 9.4 us, the whole forward 35.0 -> 33.6; one token
-// of 8 experts of H = 4096, I = 14336 141.4 -> 139.1.  From 17 tokens on the ids come from several workgroups.
+// Such a pass is its launches: 7 tokens of 128 experts (H = 576, k = 8) 7.6 + 3.1 -> 9.4 us, the whole forward 35.0 -> 33.6.  From 17
+// tokens on the ids come from several workgroups.
 struct RouteOut {
     uint32_t *counts;
     int64_t *incl, *sorted_pos;
