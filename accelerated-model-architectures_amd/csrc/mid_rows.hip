@@ -576,8 +576,8 @@ inline double tiles_about(int64_t M, int N, int E, int height) {
 // workgroup takes 1.1 us a step, two that share one 2.1 us each, with 512 at a time, 2.4 where more wait behind them (power); the
 // sums of S > 1 ranges go through memory twice (3.3 TB/s) behind one more launch.  This and tiles256_seconds were fitted together to 336
 // measured pairs of launches (the layers of the benchmark and six others, 100 to 4000 rows per expert): within 12 and 10 % on average.
-// Of the 5302 other pairs in mid_fwd_leads it chooses 3920 launches, which are 1.40 times as fast as the 256 x 256 ones on geometric
-// average; one in twenty of them is more than 3 % slower, the worst takes 1.44 times as long.
+// Of the 25,500 other pairs in mid_fwd_leads that takes 17,600 launches, which are 1.46 times as fast as the 256 x 256 ones on geometric
+// average; one in thirty of them is more than 3 % slower, the worst takes 1.59 times as long (64 experts of 98 rows, K = 16640).
 inline double mid_fwd_seconds(int64_t M, int N, int K, int E, int epilogue, int *best) {
     // Long K: one tile too many for a round of K ranges is another round of long ones (8 experts of H = 1024, K = 16384, 270 rows, where
     // most need a third tile: 174 us in 6 ranges, 148 now), so the tiles that experts of average rows need are counted in full.
@@ -705,8 +705,15 @@ bool mid_fwd_leads(int64_t M, int32_t N, int32_t K, int32_t E, int epilogue) {
     double even = 0.96;
     if (gelu && !(epilogue & 1))
         even -= rounds > 1 ? 0.15 * (rounds - 1) : 0.;
-    else if (!gelu)
+    else if (!gelu) {
         even -= rounds > 2.5 ? (epilogue == XMA_ROCM_EPI_SWIGLU ? 0.15 : 0.04) * (rounds - 2.5) : 0.;
+        // Experts that need a second of the smaller tiles and fit into one of the larger, whose steps are shorter than 1.6 us then: its
+        // waves skip the blocks without rows (0.79 of the predicted time at 96 to 160 rows, 0.9 beyond 256, from K = 3072 on).  25,500
+        // pairs of random layers, 2 to 128 experts, 97 to 1400 rows each, ms lost and won by choosing the smaller tiles where they were the
+        // slower and the faster ones: 20.3 and 377 without this -> 12.1 and 370 (64 experts of 125 rows, N = 2944, K = 6272: 484, 575 us).
+        const double rows = (double)M / E, most = rows + 2.5 * sqrt(rows);
+        if (K >= 3072 && most > MR_BM && most <= 256) even -= 0.08;
+    }
     return mid_fwd_seconds(M, N, K, E, as, &S) < even * (tiles256_seconds(M, N, K, E, as) + pass);
 }
 

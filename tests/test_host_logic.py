@@ -177,6 +177,9 @@ def test_mid_rows_dispatch_rule():
     assert fwd(100 * 8, 4096, 28672, 8) and not fwd(176 * 8, 4096, 28672, 8)  # long K
     # many rounds, and an epilogue that writes a second tensor: measured 25 and 15 % slower with the smaller tiles
     assert not fwd(43320, 5328, 520, 6, epi=glu) and not fwd(3950, 15200, 2560, 25, epi=glu)
+    # long K, experts of two of the smaller tiles and one of the larger: measured 484 against 575, 333 against 379 and 450 against 573 us
+    assert not fwd(125 * 64, 2944, 6272, 64) and not fwd(134 * 128, 1344, 4096, 128) and not fwd(143 * 32, 5792, 4264, 32, epi=glu)
+    assert fwd(134 * 128, 1344, 2048, 128) and fwd(300 * 16, 1024, 4096, 16)
     assert fwd(2048, 16384, 2048, 8, epi=glu) and fwd(8198, 4096, 1024, 16, epi=4) and not fwd(32000, 4096, 1024, 16, epi=4)
     assert not fwd(65536, 512, 64, 1024) and not fwd(2000, 64, 64, 1025) and not fwd(0, 64, 64, 8)
     assert fwd(999, 64, 64, 8, kn=0, epi=glu) and not fwd(999, 64, 64, 8, kn=1, epi=glu)
