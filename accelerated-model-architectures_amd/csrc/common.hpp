@@ -26,6 +26,13 @@ int xma_router_gate_route(const void *x, int64_t ldx, const void *gate_weight, i
                           int dtype, void *logits, int64_t ldl, void *weights, void *ids, uint32_t *counts, int64_t *offs_incl,
                           int64_t *sorted_pos, void *workspace, size_t workspace_bytes, void *stream);
 
+// combine_bwd and router_topk_bwd in one launch, rows without gaps: d_sel[t, j] = d_logits[t, ids[t, j]] (router.hip)
+int xma_combine_router_bwd(const void *expert_out, const void *dy, const void *logits, const int32_t *ids, int64_t T, int32_t H, int32_t E,
+                           int32_t k, int dtype, void *d_sel, hipStream_t st);
+// what xma_rocm_gate_bwd launches in front of its last kernel, and that kernel with the sum over the k slots (gate.hip)
+int xma_gate_bwd(const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids, const void *scattered, void *d_x,
+                 void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype, void *workspace, size_t workspace_bytes, hipStream_t st);
+
 #define XMA_REQUIRE(cond, code, ...)   \
     do {                               \
         if (!(cond)) {                 \

@@ -3,6 +3,7 @@
 // All move 16 bytes per lane per access and accumulate in fp32.
 #include "common.hpp"
 #include "fp32.hpp"
+#include "row_dot.hpp"
 
 namespace {
 
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(EW_THREADS) void combine_kernel(const uint16_t *__r
     *(u32x4 *)(y + t * ldy + c) = o;
 }
 
-// one wave per (t, j): d_w[t, j] = <in[t*k + j, :], dy[t, :]>; two 16-byte chunks of each row in flight per lane
+// one wave per (t, j): d_w[t, j] = <in[t*k + j, :], dy[t, :]>
 template <typename ET>
 __global__ __launch_bounds__(EW_THREADS) void combine_bwd_kernel(const uint16_t *__restrict__ in, int64_t ld_in,
                                                                  const uint16_t *__restrict__ dy, int64_t lddy,
@@ -79,25 +80,7 @@ __global__ __launch_bounds__(EW_THREADS) void combine_bwd_kernel(const uint16_t 
     const int64_t row = (int64_t)blockIdx.x * (EW_THREADS / WAVE) + threadIdx.x / WAVE;
     if (row >= Tk) return;
     const int64_t t = (row < ((int64_t)1 << 31)) ? (int64_t)fastdiv((uint32_t)row, k_div) : row / k;
-    const uint16_t *a_row = in + row * ld_in, *b_row = dy + t * lddy;
-    float acc = 0.f;
-    auto dot = [&](const u32x4 a, const u32x4 b) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            acc += Elem<ET>::lo(a[q]) * Elem<ET>::lo(b[q]);
-            acc += Elem<ET>::hi(a[q]) * Elem<ET>::hi(b[q]);
-        }
-    };
-    int c = lane * 8;
-    for (; c + WAVE * 8 < H; c += 2 * WAVE * 8) {
-        const u32x4 a0 = load_once(a_row + c), a1 = load_once(a_row + c + WAVE * 8);
-        const u32x4 b0 = *(const u32x4 *)(b_row + c), b1 = *(const u32x4 *)(b_row + c + WAVE * 8);
-        dot(a0, b0);
-        dot(a1, b1);
-    }
-    if (c < H) dot(load_once(a_row + c), *(const u32x4 *)(b_row + c));
-#pragma unroll
-    for (int d = WAVE / 2; d > 0; d >>= 1) acc += __shfl_xor(acc, d);
+    const float acc = row_dot<ET>(in + row * ld_in, dy + t * lddy, H, lane);
     if (lane == 0) d_w[row] = (uint16_t)(Elem<ET>::pack(acc, 0.f) & 0xffffu);
 }
 

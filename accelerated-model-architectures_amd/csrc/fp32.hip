@@ -10,6 +10,7 @@
 // The MFMA "A" operand is the P fragment, so a lane owns output row (lane & 31) of a 32 x 32 block and four
 // consecutive columns per accumulator quad.
 #include "fp32.hpp"
+#include "row_dot.hpp"
 
 namespace {
 
@@ -359,13 +360,7 @@ __global__ __launch_bounds__(FTHREADS) void combine_bwd_f32_kernel(const float *
     const int64_t row = (int64_t)blockIdx.x * (FTHREADS / 64) + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int64_t t = row / k;
-    float acc = 0.f;
-    for (int c = lane * 4; c < H; c += 256) {
-        const f32x4 x = *(const f32x4 *)(in + row * ld_in + c), g = *(const f32x4 *)(dy + t * lddy + c);
-        acc += x[0] * g[0] + x[1] * g[1] + x[2] * g[2] + x[3] * g[3];
-    }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) acc += __shfl_down(acc, d);
+    const float acc = row_dot<float>(in + row * ld_in, dy + t * lddy, H, lane);
     if (lane == 0) d_w[row] = acc;
 }
 

@@ -106,35 +106,40 @@ extern "C" int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream) {
     return xma_rocm_combine(m->expert_out, m->H, m->router_weights, m->y, m->H, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream);
 }
 
+// The activations and expert outputs again where neither was kept: h from z, the expert outputs by the down-projection.
+static int recompute(const xma_rocm_moe *m, const char *what, void *stream) {
+    if (!m->recompute) return XMA_ROCM_OK;
+    RUN(check_workspace(m, m->few_down, m->H, m->I, what));
+    RUN(xma_rocm_swiglu_packed_forward(m->z, 2 * m->I, m->h, m->I, m->T * m->k, (int32_t)m->I, (int)m->dtype, stream));
+    return down_projection(m, stream);
+}
+
 // The gradient of the router's logits: what the gate's own products need before the rest of the backward.
 extern "C" int xma_rocm_moe_backward_router(const xma_rocm_moe *m, void *stream) {
     RUN(check(m, "moe_backward_router"));
     XMA_REQUIRE(m->logits && m->dy && m->d_router_weights && m->d_logits && (!m->recompute || m->h), XMA_ROCM_EINVAL,
                 "moe_backward_router: null buffer");
     const int dtype = (int)m->dtype;
-    if (m->recompute) RUN(check_workspace(m, m->few_down, m->H, m->I, "moe_backward_router"));
-    if (m->recompute) { // neither was kept: h from z, the expert outputs by the down-projection
-        RUN(xma_rocm_swiglu_packed_forward(m->z, 2 * m->I, m->h, m->I, m->T * m->k, (int32_t)m->I, dtype, stream));
-        RUN(down_projection(m, stream));
-    }
+    RUN(recompute(m, "moe_backward_router", stream));
     RUN(xma_rocm_combine_bwd(m->expert_out, m->H, m->dy, m->H, m->d_router_weights, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream));
     return xma_rocm_router_topk_bwd(m->logits, m->E, m->T, (int32_t)m->E, (int32_t)m->k, dtype, m->expert_ids, 0, m->d_router_weights, m->d_logits,
                                     m->E, stream);
 }
 
-extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
-    RUN(check(m, "moe_backward"));
+// Everything of the backward between the router's part and the sum over the k slots: `scattered` holds dX1 then.
+static int backward_experts(const xma_rocm_moe *m, const char *what, void *stream) {
+    RUN(check(m, what));
     XMA_REQUIRE(m->dy && m->dz && m->d_w_fc && m->d_w_proj && m->scattered && m->d_x && (m->dw2_form == 1 || m->h) &&
                     (m->dw2_form == 0 || m->dw2_operand) && (!m->d_b_fc || m->b_fc) && (!m->d_b_proj || m->b_proj),
-                XMA_ROCM_EINVAL, "moe_backward: null buffer");
+                XMA_ROCM_EINVAL, "%s: null buffer", what);
     // the column sums that make d_b_proj want dy scaled, in a copy or beside the scaled activations: the loader of form 0 keeps none
     XMA_REQUIRE(m->dw2_form >= 0 && m->dw2_form <= 2 && !(m->dw2_form == 0 && m->d_b_proj), XMA_ROCM_EINVAL,
-                "moe_backward: dw2_form %lld%s", (long long)m->dw2_form, m->d_b_proj ? " with d_b_proj (forms 1 and 2 only)" : "");
+                "%s: dw2_form %lld%s", what, (long long)m->dw2_form, m->d_b_proj ? " with d_b_proj (forms 1 and 2 only)" : "");
     const int dtype = (int)m->dtype;
     const int64_t M = m->T * m->k, H = m->H, I = m->I, U = up_width(m);
     const int64_t *idx = (const int64_t *)m->sorted_scattered_idxs, *offs = (const int64_t *)m->expert_offsets;
-    RUN(check_workspace(m, m->few_dx2, I, H, "moe_backward"));
-    RUN(check_workspace(m, m->few_dx1, H, U, "moe_backward"));
+    RUN(check_workspace(m, m->few_dx2, I, H, what));
+    RUN(check_workspace(m, m->few_dx1, H, U, what));
     // dX2 + SwiGLU', with the scaled activations for dW2 where that takes dy through the index
     RUN(gemm(m, m->few_dx2, m->dy, m->w_proj, H * I, I, 1, m->dz, m->z, U, m->dw2_form == 1 ? m->dw2_operand : nullptr, m->router_weights,
              nullptr, I, H, m->k, 0, 1, epilogue_of(m, 1), stream));
@@ -153,7 +158,26 @@ extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
     RUN(dw(m, m->few_dw1, m->dz, 1, nullptr, m->x, 0, m->d_w_fc, U, H, stream));
     if (m->d_b_fc)
         RUN(xma_rocm_expert_column_sums(m->dz, U, nullptr, 1, nullptr, offs, m->d_b_fc, U, (int32_t)U, (int32_t)m->E, dtype, stream));
-    RUN(gemm(m, m->few_dx1, m->dz, m->w_fc, U * H, H, 1, m->scattered, nullptr, 0, nullptr, nullptr, nullptr, H, U, 1, 1, 0,
-             XMA_ROCM_EPI_STORE, stream));
-    return xma_rocm_combine_add(m->scattered, H, nullptr, m->d_x_addend, H, m->d_x, H, m->T, (int32_t)m->k, (int32_t)H, dtype, stream);
+    return gemm(m, m->few_dx1, m->dz, m->w_fc, U * H, H, 1, m->scattered, nullptr, 0, nullptr, nullptr, nullptr, H, U, 1, 1, 0,
+                XMA_ROCM_EPI_STORE, stream);
+}
+
+extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
+    RUN(backward_experts(m, "moe_backward", stream));
+    return xma_rocm_combine_add(m->scattered, m->H, nullptr, m->d_x_addend, m->H, m->d_x, m->H, m->T, (int32_t)m->k, (int32_t)m->H, (int)m->dtype, stream);
+}
+
+extern "C" int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_weight, void *stream) {
+    RUN(check(m, "moe_backward_gated"));
+    XMA_REQUIRE(m->gate_weight && m->logits && m->dy && m->d_router_weights && m->d_x && m->scattered && (!m->recompute || m->h), XMA_ROCM_EINVAL,
+                "moe_backward_gated: null buffer");
+    const int dtype = (int)m->dtype;
+    XMA_REQUIRE(xma_rocm_gate_bwd_supported((int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype), XMA_ROCM_EUNSUPPORTED,
+                "moe_backward_gated: H=%lld E=%lld k=%lld dtype=%d", (long long)m->H, (long long)m->E, (long long)m->k, dtype);
+    RUN(recompute(m, "moe_backward_router", stream));
+    RUN(xma_combine_router_bwd(m->expert_out, m->dy, m->logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k,
+                               dtype, m->d_router_weights, (hipStream_t)stream));
+    RUN(backward_experts(m, "moe_backward", stream));
+    return xma_gate_bwd(m->x, m->H, m->gate_weight, m->d_router_weights, (const int32_t *)m->expert_ids, m->scattered, m->d_x, d_gate_weight, m->T,
+                        (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->workspace, (size_t)m->workspace_bytes, (hipStream_t)stream);
 }

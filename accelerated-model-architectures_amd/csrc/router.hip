@@ -7,6 +7,7 @@
 // remaining value, lowest index among equals" by a butterfly over the group; round r leaves its winner in lane r, so
 // the k results of a row come out of k neighbouring lanes.  HBM traffic is the logits once in, (weights, ids) once out.
 #include "common.hpp"
+#include "row_dot.hpp"
 
 namespace {
 
@@ -229,6 +230,46 @@ __global__ __launch_bounds__(RT_THREADS) void router_topk_bwd_kernel(const void 
             if (e < E) Scalar<DT>::store(d_logits, t * ldd + e, out[v]);
         }
     }
+}
+
+template <int DT> struct RowType { typedef float type; };
+template <> struct RowType<XMA_ROCM_BF16> { typedef __bf16 type; };
+template <> struct RowType<XMA_ROCM_F16> { typedef _Float16 type; };
+
+// The two kernels in front of the gate's gradients in one: the router weights' gradient d_w[t, j] = <expert_out[t k + j], dy[t]>,
+// rounded, and what router_topk_bwd_kernel makes of it, of which only the k values that are not zero leave:
+// d_sel[t, j] = d_logits[t, ids[t, j]].  A workgroup takes `tokens` tokens (at most one per wave) and deals their rows to its waves;
+// bound by the stream of expert_out, or in a launch of few tokens by its own round trips, one launch less (4 to 15 us).
+template <int DT>
+__global__ __launch_bounds__(RT_THREADS) void combine_router_bwd_kernel(const void *__restrict__ in, const void *__restrict__ dy,
+                                                                       const void *__restrict__ logits, const int32_t *__restrict__ ids,
+                                                                       int64_t T, int H, int E, int k, int tokens,
+                                                                       void *__restrict__ d_sel) {
+    typedef typename RowType<DT>::type ET;
+    constexpr int ES = sizeof(typename Scalar<DT>::type);
+    __shared__ typename Scalar<DT>::type s_dw[RT_THREADS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t t0 = (int64_t)blockIdx.x * tokens, t = t0 + wave;
+    const bool mine = wave < tokens && t < T && lane < k; // this wave's token, this lane's slot of it
+    float my_val = 0.f;
+    if (mine) {
+        int e = ids[t * k + lane];
+        e = e < 0 ? 0 : (e >= E ? E - 1 : e); // never read outside the row
+        my_val = key_value(order_key(Scalar<DT>::load(logits, t * E + e)));
+    }
+    const int rows = (int)(T - t0 < tokens ? T - t0 : tokens) * k;
+    for (int r = wave; r < rows; r += RT_THREADS / 64) {
+        const float d = row_dot<ET>((const char *)in + (t0 * k + r) * H * ES, (const char *)dy + (t0 + r / k) * H * ES, H, lane);
+        if (lane == 0) Scalar<DT>::store(s_dw, r, d);
+    }
+    __syncthreads();
+    if (wave >= tokens || t >= T) return; // uniform
+    const float my_dw = lane < k ? Scalar<DT>::load(s_dw, wave * k + lane) : 0.f;
+    const float w = group_softmax<64>(my_val, lane, k, 0);
+    const float dot = group_sum<64>(lane < k ? w * my_dw : 0.f);
+    float d = w * (my_dw - dot);
+    asm("" : "+v"(d)); // rounded to fp32 first, as in the kernel above, not by a multiplication that rounds to fp16 at once
+    if (mine) Scalar<DT>::store(d_sel, t * k + lane, d);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -893,4 +934,26 @@ extern "C" int xma_rocm_router_topk_bwd(const void *logits, int64_t ld, int64_t 
     ROUTER_DISPATCH(dtype, s, (router_topk_bwd_kernel<DT, G, VPL><<<(int)s.blocks, RT_THREADS, 0, st>>>(
                                   logits, ld, T, E, k, ids, ids_is_i64, d_weights, d_logits, ldd)));
     return xma_check_launch("router_topk_bwd_kernel");
+}
+
+int xma_combine_router_bwd(const void *expert_out, const void *dy, const void *logits, const int32_t *ids, int64_t T, int32_t H, int32_t E,
+                           int32_t k, int dtype, void *d_sel, hipStream_t st) {
+    RouterShape s;
+    if (int rc = router_shape("combine_router_bwd", T, E, k, dtype, s)) return rc;
+    XMA_REQUIRE(H >= 8 && H % 8 == 0, XMA_ROCM_EINVAL, "combine_router_bwd: H=%d (H %% 8 == 0)", H);
+    XMA_REQUIRE(T == 0 || (expert_out && dy && logits && ids && d_sel && (((uintptr_t)expert_out | (uintptr_t)dy) & 15) == 0), XMA_ROCM_EINVAL,
+                "combine_router_bwd: null or misaligned pointer");
+    if (T == 0) return XMA_ROCM_OK;
+    const int tokens = k % 4 == 0 ? 1 : k % 2 == 0 ? 2 : 4; // the rows of a workgroup are a multiple of its four waves
+    const int64_t blocks = (T + tokens - 1) / tokens;
+    XMA_REQUIRE(blocks < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "combine_router_bwd: too many rows");
+#define CALL(DT) combine_router_bwd_kernel<DT><<<(int)blocks, RT_THREADS, 0, st>>>(expert_out, dy, logits, ids, T, H, E, k, tokens, d_sel)
+    if (dtype == XMA_ROCM_BF16)
+        CALL(XMA_ROCM_BF16);
+    else if (dtype == XMA_ROCM_F16)
+        CALL(XMA_ROCM_F16);
+    else
+        CALL(XMA_ROCM_F32);
+#undef CALL
+    return xma_check_launch("combine_router_bwd_kernel");
 }

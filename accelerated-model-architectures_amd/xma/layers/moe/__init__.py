@@ -135,6 +135,8 @@ class MoE(nn.Module):
             if self.gate.bias is None and R.router_gate_topk_supported(x, self.gate.weight, self.top_k):
                 # gate GEMM, top-k, softmax, cast and int32 expert ids in one kernel: x is read once
                 return R.router_gate_topk(x, self.gate.weight, self.top_k)
+            if R.gate_without_autograd(self.gate, x, self.top_k):
+                return R.router_gate_topk(x, self.gate.weight, self.top_k)
             router_logits = self.gate(x)
             router_weights, selected_experts = R.router_topk(router_logits, self.top_k)
             return router_logits, router_weights, selected_experts

@@ -84,18 +84,23 @@ class _RouterTopK(torch.autograd.Function):
 
 
 class _RouterGateTopK(torch.autograd.Function):
-    """gate projection + top-k + fp32 softmax + cast + int32 expert ids in one kernel; backward: the router's
-    d_logits kernel, then the two skinny GEMMs of the linear layer (d_x = d_logits @ Wg, d_Wg = d_logits^T @ x) on the
-    stock GEMM.  (d_x as k gathered rows of Wg per token, which is all a row of d_logits selects when no loss hangs on the
-    logits themselves, measured slower than the dense product: 70 against 51 us at T = 32768, E = 128, H = 2048.)  Counterpart of gate(x) and xma/layers/moe/__init__.py:186-193, 256-262."""
+    """gate projection + top-k + fp32 softmax + cast + int32 expert ids in one kernel (fp32: the stock product, then the router's
+    kernel, int64 ids); backward: the router's d_logits kernel, then the two skinny products of the linear layer (d_x = d_logits @ Wg,
+    d_Wg = d_logits^T @ x) from the k values of a row of d_logits that are not zero, or, where a loss hangs on the logits themselves, on the
+    stock GEMM.  Counterpart of gate(x) and xma/layers/moe/__init__.py:186-193, 256-262."""
 
     @staticmethod
     def forward(ctx, x: torch.Tensor, gate_weight: torch.Tensor, top_k: int):
         T, E = x.size(0), gate_weight.size(0)
-        logits = torch.empty(T, E, dtype=x.dtype, device=x.device)
         weights = torch.empty(T, top_k, dtype=x.dtype, device=x.device)
-        ids = torch.empty(T, top_k, dtype=torch.int32, device=x.device)
-        ops.router_gate_topk_rocm(x, gate_weight, logits, weights, ids)
+        if x.dtype == torch.float32:
+            logits = torch.nn.functional.linear(x, gate_weight)
+            ids = torch.empty(T, top_k, dtype=torch.int64, device=x.device)
+            ops.router_topk_rocm(logits, weights, ids)
+        else:
+            logits = torch.empty(T, E, dtype=x.dtype, device=x.device)
+            ids = torch.empty(T, top_k, dtype=torch.int32, device=x.device)
+            ops.router_gate_topk_rocm(x, gate_weight, logits, weights, ids)
         ctx.save_for_backward(x, gate_weight, logits, ids)
         ctx.mark_non_differentiable(ids)
         ctx.set_materialize_grads(False)  # an output nothing depends on arrives as None in backward, not as zeros
@@ -111,11 +116,24 @@ class _RouterGateTopK(torch.autograd.Function):
         else:
             d_logits = torch.empty_like(logits)
             ops.router_topk_bwd_rocm(logits, ids, d_weights.contiguous(), d_logits)
+            if d_logits_out is None and _gate_bwd(x, gate_weight.size(0), ids.size(1)):
+                need_x, need_gate = ctx.needs_input_grad[:2]
+                d_x = torch.empty(x.shape, dtype=x.dtype, device=x.device) if need_x else None
+                d_w = torch.empty_like(gate_weight) if need_gate else None
+                if need_x or need_gate:
+                    ops.gate_bwd_rocm(x, gate_weight, d_logits.gather(1, ids.long()), ids.int(), d_x, d_w)
+                return d_x, d_w, None
             if d_logits_out is not None:  # the caller also used the returned router logits (an auxiliary loss)
                 d_logits = d_logits + d_logits_out
         d_x = d_logits @ gate_weight if ctx.needs_input_grad[0] else None
         d_w = _gate_weight_grad(d_logits, x) if ctx.needs_input_grad[1] else None
         return d_x, d_w, None
+
+
+def _gate_bwd(x: torch.Tensor, num_experts: int, top_k: int) -> bool:
+    """whether the gate's gradients come from the library's kernels, which take a row of d_logits as its k values: everywhere but in a
+    backward that is itself recorded (create_graph), where the products have to be torch's"""
+    return x.size(0) > 0 and not torch.is_grad_enabled() and ops.gate_bwd_supported(x.size(1), num_experts, top_k, x.dtype)
 
 
 def _gate_weight_grad(d_logits: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
@@ -145,6 +163,22 @@ def router_gate_topk_supported(x: torch.Tensor, gate_weight: torch.Tensor, top_k
     return x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and gate_weight.is_contiguous() and \
         gate_weight.dtype == x.dtype and gate_weight.device == x.device and gate_weight.dim() == 2 and \
         ops.router_gate_topk_supported(x.size(1), gate_weight.size(0), top_k, x.dtype)
+
+
+def gate_without_autograd(gate: torch.nn.Module, x: torch.Tensor, top_k: int) -> bool:
+    """Whether an fp32 layer takes gate(x) as `router_gate_topk` does: the stock product, but the gate's gradients by the library.  A plain
+    linear layer that nothing hooks into, outside autocast, of a shape that the gradients' kernels cover."""
+    weight = gate.weight if type(gate) is torch.nn.Linear and gate.bias is None else None
+    return (
+        type(weight) is torch.nn.Parameter and weight.dtype == x.dtype == torch.float32 and x.is_cuda and weight.device == x.device
+        and x.dim() == 2 and x.stride(1) == 1 and weight.is_contiguous() and weight.shape[1] == x.shape[1]
+        and ops.gate_bwd_supported(x.size(1), weight.size(0), top_k, x.dtype) and not torch.is_autocast_enabled("cuda") and not _hooked(gate)
+    )
+
+
+def _hooked(module: torch.nn.Module) -> bool:
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or "forward" in module.__dict__ or torch.nn.modules.module._has_any_global_hook())
 
 
 def router_topk(router_logits: torch.Tensor, top_k: int, ids_dtype: torch.dtype = torch.int64):
@@ -418,7 +452,7 @@ _BLOCK_SIZES = struct.Struct("17q")
 class _Plan:
     """sizes, choices and scratch layout of a layer call; a function of the shape, the options and the dispatch limits only"""
 
-    __slots__ = ("sizes_forward", "sizes_backward", "keep", "temp", "back", "keep_bytes", "temp_bytes", "back_bytes", "saved_shapes")
+    __slots__ = ("sizes_forward", "sizes_backward", "keep", "temp", "back", "keep_bytes", "temp_bytes", "back_bytes", "saved_shapes", "top_k")
 
 
 def _layout(sizes: dict[str, int]) -> tuple[dict[str, int], int]:
@@ -461,13 +495,15 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, 
     (sizes if keep_h else temp)["h"] = M * I * s
     (sizes if save else temp)["out"] = M * H * s
     # the scattered rows of dX1 take the place of dW2's operand
-    back = dict(d_weights=M * s, dz=M * U * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], 256))
+    gate_sums = get_library().xma_rocm_gate_bwd_workspace_bytes(T, H, E) if ops.gate_bwd_supported(H, E, k, dtype) else 0
+    back = dict(d_weights=M * s, dz=M * U * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], gate_sums, 256))
     if not save:
         back |= dict(h=M * I * s, out=M * H * s)
     p = _Plan()
     p.keep, p.keep_bytes = _layout(sizes)
     p.temp, p.temp_bytes = _layout(temp)
     p.back, p.back_bytes = _layout(back)
+    p.top_k = k
     p.saved_shapes = ((T, H), (E, H), (T, E), (E, U, H), (E, H, I), (E, U), (E, H), (p.keep_bytes,))
     few = (up[0], down[0], dx2[0], dw(H, I, max((M if dw2_form == 2 else T) * H, M * I), dw2_form == 0), dw(U, H, max(M * U, T * H), False), dx1[0], dw2_form, int(not save))
     head = (_BLOCK_SIZES.size + _BLOCK_POINTERS.size, T, H, I, E, k, ops._DTYPE_CODE[dtype], ("swiglu_packed", "tanh", "none").index(act), *few)
@@ -483,7 +519,9 @@ def _layer_forward(x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, k, act, s
     device = x.device
     p = _plan(T, H, I, E, k, x.dtype, act, b_proj is not None, save, device.index, ops.dispatch_limits())
     y = torch.empty_like(x)
-    if gate_weight is not None:
+    if gate_weight is not None and x.dtype == torch.float32:
+        logits, gate_weight = torch.nn.functional.linear(x, gate_weight), None
+    elif gate_weight is not None:
         logits = torch.empty(T, E, dtype=x.dtype, device=device)
     if grad:
         kept = torch.empty(p.keep_bytes, dtype=torch.uint8, device=device)
@@ -544,19 +582,27 @@ class _Layer(torch.autograd.Function):
         p = ctx.plan
         x, gate_weight, logits, w_fc, w_proj, b_fc, b_proj, kept = _unpacked(ctx.saved_tensors, p.saved_shapes, dy)
         scratch = torch.empty(p.back_bytes, dtype=torch.uint8, device=x.device)
-        d_logits = torch.empty_like(logits, memory_format=torch.contiguous_format)
+        gated = gate_weight is not None and d_logits_out is None and _gate_bwd(x, gate_weight.size(0), p.top_k)
+        d_logits = None if gated else torch.empty_like(logits, memory_format=torch.contiguous_format)
         d_x, d_w_fc, d_w_proj = torch.empty_like(x), torch.empty_like(w_fc), torch.empty_like(w_proj)
         d_b_fc, d_b_proj = (None if b is None else torch.empty_like(b) for b in (b_fc, b_proj))
         a, b, keep, back = kept.data_ptr(), scratch.data_ptr(), p.keep, p.back
         pointers = (
-            x.data_ptr(), 0, w_fc.data_ptr(), w_proj.data_ptr(), 0 if b_fc is None else b_fc.data_ptr(),
+            x.data_ptr(), gate_weight.data_ptr() if gated else 0, w_fc.data_ptr(), w_proj.data_ptr(), 0 if b_fc is None else b_fc.data_ptr(),
             0 if b_proj is None else b_proj.data_ptr(), logits.data_ptr(), a + keep["weights"], a + keep["ids"], 0, a + keep["offsets"],
             a + keep["idx"], a + keep["z"], b + back["h"] if "h" in back else a + keep["h"] if "h" in keep else 0,
             b + back["out"] if "out" in back else a + keep["out"], 0, b + back["workspace"], dy.data_ptr(), b + back["d_weights"],
-            d_logits.data_ptr(), b + back["dz"], b + back["scattered"], b + back["scattered"], d_w_fc.data_ptr(), d_w_proj.data_ptr(),
+            0 if gated else d_logits.data_ptr(), b + back["dz"], b + back["scattered"], b + back["scattered"], d_w_fc.data_ptr(), d_w_proj.data_ptr(),
             0 if d_b_fc is None else d_b_fc.data_ptr(), 0 if d_b_proj is None else d_b_proj.data_ptr(), d_x.data_ptr(),
         )
         lib, stream = get_library(), ops._stream(x)
+        if gated:
+            d_gate = torch.empty_like(gate_weight) if need_gate else None
+            rc = lib.xma_rocm_moe_backward_gated(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0),
+                                                 None if d_gate is None else d_gate.data_ptr(), stream)
+            if rc:  # the message begins with the part that refused
+                check(rc, "xma_rocm_" + lib.xma_rocm_last_error().decode(errors="replace").partition(":")[0])
+            return d_x, d_gate, None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None, None
         check(lib.xma_rocm_moe_backward_router(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0), stream), "xma_rocm_moe_backward_router")
         d_gate = d_x_gate = None
         if gate_weight is not None:
@@ -566,8 +612,11 @@ class _Layer(torch.autograd.Function):
                 d_x_gate = (d_logits @ gate_weight).to(x.dtype)  # in an autocast region the product has another dtype
             if need_gate:
                 d_gate = _gate_weight_grad(d_logits, x)
-        check(lib.xma_rocm_moe_backward(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0 if d_x_gate is None else d_x_gate.data_ptr()),
+        recorded = d_x_gate is not None and d_x_gate.requires_grad  # create_graph: the sum is torch's as well
+        check(lib.xma_rocm_moe_backward(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0 if d_x_gate is None or recorded else d_x_gate.data_ptr()),
                                         stream), "xma_rocm_moe_backward")
+        if recorded:
+            d_x = d_x + d_x_gate
         return d_x, d_gate, d_logits if need_logits else None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None, None
 
 
@@ -576,9 +625,7 @@ def _activation(moe) -> str | None:
     act = moe.act
     if moe.is_glu:
         return "swiglu_packed" if getattr(act, "_xma_fused_activation", None) == "swiglu_packed" else None
-    if type(act) is not torch.nn.GELU or act.approximate not in ops.EPI_GELU or torch.nn.modules.module._has_any_global_hook():
-        return None
-    if act._forward_hooks or act._forward_pre_hooks or act._backward_hooks or act._backward_pre_hooks or "forward" in act.__dict__:
+    if type(act) is not torch.nn.GELU or act.approximate not in ops.EPI_GELU or _hooked(act):
         return None
     return act.approximate
 
@@ -614,6 +661,8 @@ def layer(moe, x: torch.Tensor):
     if gate.bias is None and router_gate_topk_supported(x, gate_weight, k):
         if gate_weight.shape != (E, H) or not _plain(gate_weight, x):  # the op copies a weight that starts off a 16-byte boundary
             return None
+        tensors = (x, gate_weight, w_fc, w_proj, b_fc, b_proj)
+    elif gate_without_autograd(gate, x, k) and gate_weight.shape == (E, H) and _plain(gate_weight, x):
         tensors = (x, gate_weight, w_fc, w_proj, b_fc, b_proj)
     else:
         gate_weight, logits = None, gate(x)

@@ -82,11 +82,15 @@ SIGNATURES = {
     "xma_rocm_router_gate_topk_supported": (_int, [_i32, _i32, _i32, _int]),
     "xma_rocm_router_gate_topk": (_int, [_p, _i64, _p, _i64, _i64, _i32, _i32, _i32, _int, _p, _i64, _p, _p, _int, _p]),
     "xma_rocm_router_topk_bwd": (_int, [_p, _i64, _i64, _i32, _i32, _int, _p, _int, _p, _p, _i64, _p]),
+    "xma_rocm_gate_bwd_supported": (_int, [_i32, _i32, _i32, _int]),
+    "xma_rocm_gate_bwd_workspace_bytes": (_sz, [_i64, _i32, _i32]),
+    "xma_rocm_gate_bwd": (_int, [_p, _i64, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _int, _p, _sz, _p]),
     "xma_rocm_gelu_forward": (_int, [_p, _p, _i64, _int, _int, _p]),
     "xma_rocm_gelu_backward": (_int, [_p, _p, _p, _i64, _int, _int, _p]),
     "xma_rocm_moe_forward": (_int, [_p, _p]),
     "xma_rocm_moe_backward_router": (_int, [_p, _p]),
     "xma_rocm_moe_backward": (_int, [_p, _p]),
+    "xma_rocm_moe_backward_gated": (_int, [_p, _p, _p]),
     "xma_rocm_diag_mfma_stream": (_int, [_p, _i32, _p, _i32, _p]),
 }
 

@@ -648,6 +648,40 @@ def router_topk_bwd_rocm(logits: torch.Tensor, ids: torch.Tensor, d_weights: tor
     )
 
 
+GATE_BWD_MAX_E, GATE_BWD_MAX_K = 128, 32
+
+
+def gate_bwd_supported(H: int, E: int, k: int, dtype: torch.dtype) -> bool:
+    """whether gate_bwd_rocm covers the shape (restates xma_rocm_gate_bwd_supported, as router_gate_topk_supported does)"""
+    return dtype in _DTYPE_CODE and H >= 8 and H % 8 == 0 and 1 <= E <= GATE_BWD_MAX_E and 1 <= k <= min(E, GATE_BWD_MAX_K)
+
+
+@torch.library.custom_op("xma_rocm::gate_bwd", mutates_args={"d_x", "d_gate_weight"})
+def gate_bwd_rocm(x: torch.Tensor, gate_weight: torch.Tensor, d_selected: torch.Tensor, ids: torch.Tensor, d_x: torch.Tensor | None,
+                  d_gate_weight: torch.Tensor | None) -> None:
+    """d_x = d_logits @ gate_weight and d_gate_weight = d_logits^T @ x for d_logits that is d_selected (T, k) at the experts ids (T, k)
+    and zero elsewhere (autograd of gate(x), xma/layers/moe/__init__.py:182)"""
+    T, H = x.shape
+    E, k = gate_weight.size(0), ids.size(1)
+    assert gate_weight.shape == (E, H) and ids.shape == (T, k) and ids.dtype == torch.int32 and d_selected.shape == (T, k)
+    assert x.dtype == gate_weight.dtype == d_selected.dtype and ids.is_contiguous() and d_selected.is_contiguous() and gate_weight.is_contiguous()
+    assert d_x is None or (d_x.shape == (T, H) and d_x.is_contiguous() and d_x.dtype == x.dtype)
+    assert d_gate_weight is None or (d_gate_weight.shape == (E, H) and d_gate_weight.is_contiguous() and d_gate_weight.dtype == x.dtype)
+    lib = get_library()
+    # 16-byte pieces: what starts off such a boundary, or has rows that do, is copied
+    if x.data_ptr() % 16 or x.stride(0) * x.element_size() % 16:
+        x = x.clone(memory_format=torch.contiguous_format)
+    if gate_weight.data_ptr() % 16:
+        gate_weight = gate_weight.clone()
+    ws_bytes = lib.xma_rocm_gate_bwd_workspace_bytes(T, H, E) if d_gate_weight is not None else 0
+    workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
+    check(
+        lib.xma_rocm_gate_bwd(_ptr(x), _rows(x, "x"), _ptr(gate_weight), _ptr(d_selected), _ptr(ids), _ptr(d_x), _ptr(d_gate_weight), T, H, E, k,
+                              _code(x), _ptr(workspace), ws_bytes, _stream(x)),
+        "xma_rocm_gate_bwd",
+    )
+
+
 # ------------------------------------------------------------------------------------------------ eager fast path
 def _eager_fast_path(op):
     """The registered op when a compiler is tracing (the graph gets its node), its Python body directly otherwise: the

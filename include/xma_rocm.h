@@ -349,6 +349,19 @@ XMA_API int xma_rocm_router_gate_topk(const void *x, int64_t ldx, const void *ga
 XMA_API int xma_rocm_router_topk_bwd(const void *logits, int64_t ld, int64_t T, int32_t E, int32_t k, int dtype, const void *ids,
                              int ids_is_i64, const void *d_weights, void *d_logits, int64_t ldd, void *stream);
 
+/*
+ * Backward of the gate projection behind xma_rocm_router_topk_bwd, where nothing else hangs on the logits: with d_selected (T, k) =
+ * d_logits[t, ids[t, j]] (every other element of d_logits is zero) and ids int32 (T, k),
+ *     d_gate_weight (E, H) = d_logits^T @ x,   d_x (T, H) = d_logits @ gate_weight;
+ * either may be NULL.  Replaces the two products of autograd of gate(x), xma/layers/moe/__init__.py:182.  Row-major without gaps (x: row
+ * stride ldx), 16-byte aligned; `workspace` (for d_gate_weight) holds fp32 sums over ranges of the tokens.  E <= 128, k <= 32, H % 8 == 0.
+ */
+XMA_API int xma_rocm_gate_bwd_supported(int32_t H, int32_t E, int32_t k, int dtype);
+XMA_API size_t xma_rocm_gate_bwd_workspace_bytes(int64_t T, int32_t H, int32_t E);
+XMA_API int xma_rocm_gate_bwd(const void *x, int64_t ldx, const void *gate_weight, const void *d_selected, const int32_t *ids, void *d_x,
+                              void *d_gate_weight, int64_t T, int32_t H, int32_t E, int32_t k, int dtype, void *workspace,
+                              size_t workspace_bytes, void *stream);
+
 /* y = gelu(x); dx = gelu'(x) * dy (dx may be dy), n elements, 16-byte aligned; form 0: tanh approximation, 1: erf */
 XMA_API int xma_rocm_gelu_forward(const void *x, void *y, int64_t n, int form, int dtype, void *stream);
 XMA_API int xma_rocm_gelu_backward(const void *x, const void *dy, void *dx, int64_t n, int form, int dtype, void *stream);
@@ -384,6 +397,12 @@ XMA_API int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream);
 XMA_API int xma_rocm_moe_backward_router(const xma_rocm_moe *m, void *stream);
 /* dX2, dW2, dW1, bias gradients, dX1, sum over the k slots; behind xma_rocm_moe_backward_router */
 XMA_API int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream);
+/*
+ * The whole backward where no gradient of the logits comes from outside and xma_rocm_gate_bwd covers the gate: both of the above and the
+ * gate's two products, whose part of d_x joins the sum over the k slots.  d_router_weights receives d_selected; d_logits and d_x_addend are
+ * not used; d_gate_weight (E, H) or NULL.  `workspace` also holds xma_rocm_gate_bwd_workspace_bytes.
+ */
+XMA_API int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_weight, void *stream);
 
 /*
  * Measurement aid with no counterpart in the reference: `workgroups` workgroups of 4 waves each issue iters x 64

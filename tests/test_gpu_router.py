@@ -274,3 +274,30 @@ def test_router_gate_few_tokens(T, H, E, k):
     want_w, want_ids = oracle.routing_topk(logits, k, torch.bfloat16)
     assert torch.equal(ids.long(), want_ids)
     assert (w.float() - want_w.float()).abs().max().item() <= ULP[torch.bfloat16]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("E,k", [(1, 1), (8, 2), (31, 3), (33, 8), (64, 6), (65, 9), (128, 32)])
+@pytest.mark.parametrize("T,H", [(1, 8), (63, 128), (64, 136), (65, 120), (700, 2048), (9000, 264)])  # one range, several steps per range
+def test_gate_backward_from_the_selected_logits(dtype, T, H, E, k):
+    """d_x and d_gate_weight against the dense products in 64 bits: fp32 sums of T (k) products, then one rounding"""
+    from xma.rocm import ops
+
+    print(f"gate bwd {dtype} T={T} H={H} E={E} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + H + E)
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    x, gate, d_sel = new(T, H + 8)[:, :H], new(E, H), new(T, k)
+    ids = torch.rand(T, E, device="cuda", generator=g).argsort(1)[:, :k].int().contiguous()
+    nan = lambda *s: torch.full(s, float("nan"), device="cuda", dtype=dtype)
+    d_x, d_gate = nan(T, H), nan(E, H)
+    ops.gate_bwd_rocm(x, gate, d_sel, ids, d_x, d_gate)
+    d_x_only, d_gate_only = nan(T, H), nan(E, H)
+    ops.gate_bwd_rocm(x, gate, d_sel, ids, d_x_only, None)
+    ops.gate_bwd_rocm(x, gate, d_sel, ids, None, d_gate_only)
+    assert torch.equal(d_x, d_x_only) and torch.equal(d_gate, d_gate_only)
+    d_logits = torch.zeros(T, E, device="cuda", dtype=torch.float64).scatter_(1, ids.long(), d_sel.double())
+    unit = 2.0 ** {torch.bfloat16: -8, torch.float16: -11, torch.float32: -24}[dtype]
+    smallest = 2.0 ** {torch.bfloat16: -133, torch.float16: -24, torch.float32: -149}[dtype]
+    for got, a, b, terms in ((d_x, d_logits, gate.double(), k), (d_gate, d_logits.t().contiguous(), x.double(), T)):
+        bound = unit * (a @ b).abs() + (terms + 1) * 2.0**-24 * (a.abs() @ b.abs()) + smallest
+        assert ((got.double() - a @ b).abs() <= bound).all()
