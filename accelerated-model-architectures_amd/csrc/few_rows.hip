@@ -6,6 +6,9 @@
 // beyond.  Correct for any number of rows, but the forward-type kernels here stream the weights once per 32 rows of an expert:
 // the caller picks these entry points by the number of rows per expert, and they hand launches of more than 24 (weight gradient:
 // 40) rows per expert to the 128 x 256 tiles of mid_rows.hip.
+#include <math.h>
+
+#include "grouped_gemm_tile.hpp"
 #include "mid_rows.hpp"
 
 namespace {
@@ -425,6 +428,60 @@ __device__ __forceinline__ int st_slot(int row, int chunk) { return row * 128 + 
 // and for tiles of 256-byte rows read along the row (WT = 0): chunk 0..15, the same rotation inside each half
 __device__ __forceinline__ int st_slot_nt(int row, int chunk) { return row * 256 + ((chunk ^ (row & 7)) << 4); }
 
+// The epilogue of a small tile: acc[4 g + q] = sum of row r, column n0 + 8 g + q (n0: this lane's first column); s_idx and sc: the row's
+// scattered index and scale.
+template <typename T, int EPI>
+__device__ __forceinline__ void fr_tile_epilogue(const FwdArgs &a, const f32x16 &acc, int e, int64_t r, int64_t s_idx, float sc, int n0) {
+    const int64_t dst = a.y_grouped ? r : s_idx;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const int n = n0 + 8 * g;
+        if (n >= a.N) continue;
+        if constexpr (EPI == XMA_ROCM_EPI_SWIGLU_BWD) {
+            // d h of 4 columns -> (d gate, d up) of their 4 pairs; rows are grouped on both sides
+            const u32x4 z = *(const u32x4 *)(a.aux + r * a.ldaux + 2 * n);
+            u32x4 o;
+            float hv[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float dh = acc[4 * g + q] * sc;
+                const float gg = Elem<T>::lo(z[q]), uu = Elem<T>::hi(z[q]);
+                const float sg = sigmoidf_fast(gg), silu = gg * sg;
+                o[q] = Elem<T>::pack(dh * uu * (sg + silu * (1.f - sg)), dh * silu);
+                hv[q] = uu * silu * sc;
+            }
+            *(u32x4 *)(a.out + r * a.ldo + 2 * n) = o;
+            if (a.aux2) *(u32x2 *)(a.aux2 + r * a.ldaux2 + n) = u32x2{Elem<T>::pack(hv[0], hv[1]), Elem<T>::pack(hv[2], hv[3])};
+        } else if constexpr (EPI == EPI_GELU_BWD) {
+            const u32x2 z = *(const u32x2 *)(a.aux + r * a.ldaux + n);
+            float d[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                d[q] = acc[4 * g + q] * sc * gelu_grad((q & 1) ? Elem<T>::hi(z[q >> 1]) : Elem<T>::lo(z[q >> 1]), a.erf_form, sigmoidf_fast);
+            *(u32x2 *)(a.out + r * a.ldo + n) = u32x2{Elem<T>::pack(d[0], d[1]), Elem<T>::pack(d[2], d[3])};
+        } else {
+            float v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                v[q] = acc[4 * g + q];
+                if (a.bias) v[q] += fr_scalar<T>(a.bias, (int64_t)e * a.bias_es + n + q);
+                v[q] *= sc;
+            }
+            const uint32_t z0 = Elem<T>::pack(v[0], v[1]), z1 = Elem<T>::pack(v[2], v[3]);
+            if (a.out) *(u32x2 *)(a.out + dst * a.ldo + n) = u32x2{z0, z1};
+            if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) {
+                const float g0 = Elem<T>::lo(z0), u0 = Elem<T>::hi(z0), g1 = Elem<T>::lo(z1), u1 = Elem<T>::hi(z1);
+                *(uint32_t *)(a.aux + dst * a.ldaux + (n >> 1)) = Elem<T>::pack(u0 * g0 * sigmoidf_fast(g0), u1 * g1 * sigmoidf_fast(g1));
+            }
+            if constexpr (EPI == EPI_GELU) {
+                const float h0 = gelu(Elem<T>::lo(z0), a.erf_form, sigmoidf_fast), h1 = gelu(Elem<T>::hi(z0), a.erf_form, sigmoidf_fast);
+                const float h2 = gelu(Elem<T>::lo(z1), a.erf_form, sigmoidf_fast), h3 = gelu(Elem<T>::hi(z1), a.erf_form, sigmoidf_fast);
+                *(u32x2 *)(a.aux + dst * a.ldaux + n) = u32x2{Elem<T>::pack(h0, h1), Elem<T>::pack(h2, h3)};
+            }
+        }
+    }
+}
+
 // EPI = -1: the launch is cut along K (blockIdx.z takes `steps_per` steps) because N alone gives too few workgroups; the
 // fp32 sums go to part[blockIdx.z][M][N] and fr_epilogue_kernel finishes.
 template <typename T, int WT, int EPI>
@@ -564,64 +621,157 @@ __global__ __launch_bounds__(FR_THREADS, 4) void fr_tile_kernel(const FwdArgs a,
                 continue;
             }
             const int64_t s_idx = a.idx ? a.idx[r] : r;
-            const float sc = a.scale ? fr_scalar<T>(a.scale, s_idx) : 1.f;
-            const int64_t dst = a.y_grouped ? r : s_idx;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int n = n0 + wave * 32 + 8 * g + 4 * half; // acc[4 g + q] is column n + q of row r
-                if (n >= a.N) continue;
-                if constexpr (EPI == XMA_ROCM_EPI_SWIGLU_BWD) {
-                    // d h of 4 columns -> (d gate, d up) of their 4 pairs; rows are grouped on both sides
-                    const u32x4 z = *(const u32x4 *)(a.aux + r * a.ldaux + 2 * n);
-                    u32x4 o;
-                    float hv[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float dh = acc[4 * g + q] * sc;
-                        const float gg = Elem<T>::lo(z[q]), uu = Elem<T>::hi(z[q]);
-                        const float sg = sigmoidf_fast(gg), silu = gg * sg;
-                        o[q] = Elem<T>::pack(dh * uu * (sg + silu * (1.f - sg)), dh * silu);
-                        hv[q] = uu * silu * sc;
-                    }
-                    *(u32x4 *)(a.out + r * a.ldo + 2 * n) = o;
-                    if (a.aux2) *(u32x2 *)(a.aux2 + r * a.ldaux2 + n) = u32x2{Elem<T>::pack(hv[0], hv[1]), Elem<T>::pack(hv[2], hv[3])};
-                } else if constexpr (EPI == EPI_GELU_BWD) {
-                    const u32x2 z = *(const u32x2 *)(a.aux + r * a.ldaux + n);
-                    float d[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        d[q] = acc[4 * g + q] * sc * gelu_grad((q & 1) ? Elem<T>::hi(z[q >> 1]) : Elem<T>::lo(z[q >> 1]), a.erf_form, sigmoidf_fast);
-                    *(u32x2 *)(a.out + r * a.ldo + n) = u32x2{Elem<T>::pack(d[0], d[1]), Elem<T>::pack(d[2], d[3])};
-                } else {
-                    float v[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        v[q] = acc[4 * g + q];
-                        if (a.bias) v[q] += fr_scalar<T>(a.bias, (int64_t)e * a.bias_es + n + q);
-                        v[q] *= sc;
-                    }
-                    const uint32_t z0 = Elem<T>::pack(v[0], v[1]), z1 = Elem<T>::pack(v[2], v[3]);
-                    if (a.out) *(u32x2 *)(a.out + dst * a.ldo + n) = u32x2{z0, z1};
-                    if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) {
-                        const float g0 = Elem<T>::lo(z0), u0 = Elem<T>::hi(z0), g1 = Elem<T>::lo(z1), u1 = Elem<T>::hi(z1);
-                        *(uint32_t *)(a.aux + dst * a.ldaux + (n >> 1)) = Elem<T>::pack(u0 * g0 * sigmoidf_fast(g0), u1 * g1 * sigmoidf_fast(g1));
-                    }
-                    if constexpr (EPI == EPI_GELU) {
-                        const float h0 = gelu(Elem<T>::lo(z0), a.erf_form, sigmoidf_fast), h1 = gelu(Elem<T>::hi(z0), a.erf_form, sigmoidf_fast);
-                        const float h2 = gelu(Elem<T>::lo(z1), a.erf_form, sigmoidf_fast), h3 = gelu(Elem<T>::hi(z1), a.erf_form, sigmoidf_fast);
-                        *(u32x2 *)(a.aux + dst * a.ldaux + n) = u32x2{Elem<T>::pack(h0, h1), Elem<T>::pack(h2, h3)};
-                    }
-                }
-            }
+            fr_tile_epilogue<T, EPI>(a, acc, e, r, s_idx, a.scale ? fr_scalar<T>(a.scale, s_idx) : 1.f, n0 + wave * 32 + 4 * half);
         }
     }
+}
+
+// The same tile and sums (x @ W^T) where at most one workgroup per compute unit has work: few experts with rows, or few columns.  Four
+// workgroups of a compute unit hide each other's loads there; alone, one step at a time would wait for memory.  So here a workgroup of two
+// or four waves (64 or 128 columns) keeps four steps in flight, up to 160 KB of LDS, by LDS-DMA: 16 bytes per lane, 256 contiguous bytes per
+// row; a wave loads and reads its own 32 rows of W, the 32 rows of X are shared.  The W of the first steps is asked for before the chain
+// index -> row of X has been followed.  blockIdx.y counts the experts that have rows, so that no workgroup waits behind one without.
+// Bound by the round trips offsets -> index -> rows (narrow layers, one to a few tokens: 7 to 9 us whatever K up to 576), beyond that
+// by what one compute unit fetches, about 36 KB a us.  Against the kernels that served these launches, us, up- / down-projection: 128
+// experts of H = 576, I = 256, 1 / 7 tokens, k = 8: 8.7 -> 8.4 / 11.8 -> 10.6, 4.7 -> 4.5 / 7.8 -> 6.2; 64 of H = 2048, I = 1408, 1 token, k = 6: 19.8 ->
+// 18.4, 18.4 -> 11.2; 8 of H = 512, I = 1024, 1 to 16 tokens, k = 2: 8.0 - 9.3 -> 7.3 - 8.6, 10.6 - 11.4 in K ranges -> 8.3 uncut.
+constexpr int FD_STAGES = 4, FD_BLOCK = 32 * ST_K_NT * 2; // steps in flight; bytes of 32 rows of either operand
+__host__ __device__ constexpr int fd_stage(int waves) { return (waves + 1) * FD_BLOCK; }
+// all of this wave's pieces but the `behind` youngest have landed, and its LDS reads have returned; then meet the others
+__device__ __forceinline__ void fd_wait_and_barrier(int behind) { // uniform
+#define FD_CASE(n) \
+    case n: asm volatile("s_waitcnt vmcnt(" #n ") lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
+    switch (behind) {
+        FD_CASE(2) FD_CASE(4) FD_CASE(6) FD_CASE(8) FD_CASE(10) FD_CASE(12) FD_CASE(16) FD_CASE(20) FD_CASE(24)
+    default: asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+#undef FD_CASE
+}
+
+template <typename T, int EPI, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 1) void fr_deep_kernel(const FwdArgs a) {
+    constexpr int XP = 8 / WAVES, STAGE = fd_stage(WAVES); // pieces of X per wave and step
+    extern __shared__ __attribute__((aligned(16))) unsigned char s_deep[];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the expert: the blockIdx.y-th that has rows, 128 experts at a time
+    int e = -1, lo = 0, hi = 0;
+    for (int base = 0, left = blockIdx.y; base < a.E && e < 0; base += 2 * WAVE) {
+        int from[2], to[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int x = base + i * WAVE + lane;
+            from[i] = x < a.E && x ? (int)a.offs[x - 1] : 0;
+            to[i] = x < a.E ? (int)a.offs[x] : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint64_t some = __ballot(to[i] > from[i]);
+            const int count = __builtin_popcountll(some);
+            if (e < 0 && left < count) { // uniform
+                const int rank = __builtin_popcountll(some & (((uint64_t)1 << lane) - 1));
+                const int at = __builtin_ctzll(__ballot(to[i] > from[i] && rank == left)); // exactly one lane
+                e = base + i * WAVE + at;
+                lo = __builtin_amdgcn_readlane(from[i], at);
+                hi = __builtin_amdgcn_readlane(to[i], at);
+            }
+            left -= count;
+        }
+    }
+    if (e < 0) return; // uniform
+    const int n0 = blockIdx.x * (32 * WAVES);
+    const int steps = (a.K + ST_K_NT - 1) / ST_K_NT;
+    const int start = (int)(((unsigned)n0 / ST_N + 3u * (unsigned)e) % (unsigned)steps); // as in fr_tile_kernel
+    const int k_left = a.K - (steps - 1) * ST_K_NT; // of the last step
+    const uint32_t lds0 = xma_rocm::lds_addr_of(s_deep);
+    const uint16_t *w_base = a.W + (int64_t)e * a.w_es;
+    // instruction i of a wave: 4 rows of 256 bytes; lane = row 4 i + lane / 16, slot lane % 16 of the row, which holds chunk slot ^ (row & 7)
+    uint32_t w_off[8];
+    int chunk[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) chunk[i] = (lane & 15) ^ (4 * i + (lane >> 4));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        int n = n0 + 32 * wave + 4 * i + (lane >> 4);
+        if (n >= a.N) n = a.N - 1; // computed, never stored
+        w_off[i] = ((uint32_t)n * (uint32_t)a.ldw + 8u * chunk[i & 1]) * 2u;
+    }
+    for (int r0 = lo; r0 < hi; r0 += ST_M) {
+        uint32_t x_off[XP];
+        auto place = [&](int d) { return lds0 + (uint32_t)((d & (FD_STAGES - 1)) * STAGE); };
+        auto step_of = [&](int d) { return start + d < steps ? start + d : start + d - steps; };
+        auto piece = [&](xma_rocm::i32x4 desc, uint32_t off, int s, int i, uint32_t at) {
+            if (s == steps - 1 && 8 * chunk[i & 1] >= k_left) off = xma_rocm::BUF_OUTSIDE; // chunks past K read zeros
+            xma_rocm::lds_dma16_buf(desc, off, (uint32_t)__builtin_amdgcn_readfirstlane((int)at), 0);
+        };
+        auto load_w = [&](int d) {
+            const int s = step_of(d);
+            const xma_rocm::i32x4 desc = xma_rocm::buf_desc(w_base + s * ST_K_NT);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) piece(desc, w_off[i], s, i, place(d) + wave * FD_BLOCK + i * 1024);
+        };
+        auto load_x = [&](int d) {
+            const int s = step_of(d);
+            const xma_rocm::i32x4 desc = xma_rocm::buf_desc(a.X + s * ST_K_NT);
+#pragma unroll
+            for (int i = 0; i < XP; ++i) piece(desc, x_off[i], s, i, place(d) + WAVES * FD_BLOCK + (wave * XP + i) * 1024);
+        };
+        __syncthreads(); // the pass before no longer reads the stages
+#pragma unroll
+        for (int d = 0; d < FD_STAGES; ++d)
+            if (d < steps) load_w(d);
+        const int r = r0 + l32, rc = r < hi ? r : hi - 1;
+        const int64_t s_idx = a.idx ? a.idx[rc] : rc;
+        const float sc = a.scale ? fr_scalar<T>(a.scale, s_idx) : 1.f;
+#pragma unroll
+        for (int i = 0; i < XP; ++i) {
+            const int row = r0 + 4 * (wave * XP + i) + (lane >> 4);
+            x_off[i] = (uint32_t)fr_src_row(a, row < hi ? row : hi - 1) * (uint32_t)(2 * a.ldx) + 16u * chunk[i & 1];
+        }
+#pragma unroll
+        for (int d = 0; d < FD_STAGES; ++d)
+            if (d < steps) load_x(d);
+        f32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+        for (int d = 0; d < steps; ++d) {
+            // Pieces of this wave behind those of step d: the XP of X of each of the first four steps, whose W went out before, all 8 + XP
+            // of a later one; loads reach as far as step 3 in step 0 and step d + 2 in step d > 0, whose own load, of step d + 3, comes below.
+            int behind = 0;
+            const int last = d == 0 ? FD_STAGES - 1 : d + 2;
+            for (int j = d + 1; j <= last && j < steps; ++j) behind += j < FD_STAGES ? XP : 8 + XP;
+            fd_wait_and_barrier(behind);
+            if (d > 0 && d + FD_STAGES - 1 < steps) { // into the place of step d - 1, which every wave has read
+                load_w(d + FD_STAGES - 1);
+                load_x(d + FD_STAGES - 1);
+            }
+            const unsigned char *at = s_deep + (d & (FD_STAGES - 1)) * STAGE;
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) {
+                const int slot = st_slot_nt(l32, 2 * kk + half);
+                acc = Elem<T>::mfma(*(const u32x4 *)(at + wave * FD_BLOCK + slot), *(const u32x4 *)(at + WAVES * FD_BLOCK + slot), acc);
+            }
+        }
+        if (r < hi) fr_tile_epilogue<T, EPI>(a, acc, e, r, s_idx, sc, n0 + wave * 32 + 4 * half);
+    }
+}
+
+constexpr int FR_DEEP_K = 2048; // K ranges and their epilogue lead beyond (8 experts, K = 8192, N = 2048)
+
+// W[e] as (N, K): at most as many workgroups with work as run at the same time, counting the experts that M random choices of E hit.
+// 128 experts of H = 576, I = 256, 12 tokens, up-projection in four workgroups for each of 68 experts: 17.8 us against 12.9 with the small tile.
+inline int fr_deep_stages(int K) { const int steps = (K + ST_K_NT - 1) / ST_K_NT; return steps < FD_STAGES ? steps : FD_STAGES; }
+inline bool fr_deep_shape(int64_t M, int N, int K, int E, int w_is_kn) {
+    if (w_is_kn || K > FR_DEEP_K) return false;
+    const double experts = E * (1. - pow(1. - 1. / E, (double)M));
+    return experts * ((N + ST_N - 1) / ST_N) <= 256 * (FD_STAGES / fr_deep_stages(K));
 }
 
 // W[e] as (K, N), more than a pass or two of the vector kernel per expert, or rows of W shorter than the 4 KB a wave of
 // the vector kernel takes at a time -> the small MFMA tile (128 experts of H = 576, I = 256, 7 tokens: forward 0.036
 // instead of 0.045 ms with it; 8 experts of H = 2048, I = 8192: 0.161 instead of 0.155)
-inline bool fr_takes_tile(int64_t M, int K, int E, int w_is_kn) {
-    return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE;
+inline bool fr_takes_tile(int64_t M, int N, int K, int E, int w_is_kn) {
+    return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE || fr_deep_shape(M, N, K, E, w_is_kn);
 }
 
 // More rows than the small tile takes in one pass go to the 128 x 256 tiles of mid_rows.hip, where those have the variant.  8
@@ -650,6 +800,20 @@ template <typename T, int EPI> int fr_launch_epilogue(const FwdArgs &a, const fl
 }
 
 template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, float *part, hipStream_t st) {
+    if constexpr (WT == 0 && (EPI == XMA_ROCM_EPI_STORE || EPI == XMA_ROCM_EPI_SWIGLU || EPI == EPI_GELU)) {
+        const int64_t x_rows = a.x_grouped ? a.M : (a.M + a.fan_out - 1) / a.fan_out; // 32-bit byte offsets from its first row
+        if (fr_deep_shape(a.M, a.N, a.K, a.E, WT) && x_rows * a.ldx * 2 < ((int64_t)1 << 31)) {
+            auto run = [&](auto kernel, int waves) {
+                if (int rc = xma_set_max_lds_once((const void *)kernel, FD_STAGES * fd_stage(waves))) return rc;
+                const dim3 grid((a.N + 32 * waves - 1) / (32 * waves), (unsigned)(a.M < a.E ? a.M : a.E));
+                kernel<<<grid, 64 * waves, fr_deep_stages(a.K) * fd_stage(waves), st>>>(a);
+                return xma_check_launch("fr_deep_kernel");
+            };
+            // 64 columns where that still is at most one workgroup per compute unit (64 experts, K = 1408, N = 2048, one token 12.4 -> 11.2 us;
+            // with 264 workgroups instead of 132 18.4 -> 29.4)
+            return (a.M < a.E ? a.M : a.E) * ((a.N + 63) / 64) <= 256 ? run(fr_deep_kernel<T, EPI, 2>, 2) : run(fr_deep_kernel<T, EPI, 4>, 4);
+        }
+    }
     const int S_max = part ? fr_tile_splits(a.N, a.K, a.E, WT) : 1;
     const int steps_all = (a.K + st_k(WT) - 1) / st_k(WT), steps_per = (steps_all + S_max - 1) / S_max;
     const int S = (steps_all + steps_per - 1) / steps_per; // ranges that hold a step (25 steps in 6 ranges of 5: only 5 do)
@@ -666,7 +830,7 @@ template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, floa
 
 template <typename T, int EPI> int fr_launch_epi(const FwdArgs &a, int w_is_kn, float *part, hipStream_t st) {
     int rc;
-    if (fr_takes_tile(a.M, a.K, a.E, w_is_kn)) return w_is_kn ? fr_launch_tile<T, 1, EPI>(a, part, st) : fr_launch_tile<T, 0, EPI>(a, part, st);
+    if (fr_takes_tile(a.M, a.N, a.K, a.E, w_is_kn)) return w_is_kn ? fr_launch_tile<T, 1, EPI>(a, part, st) : fr_launch_tile<T, 0, EPI>(a, part, st);
     // one pair of rows per wave instead of four where the rows are short or the launch would have few workgroups
     const int rows_per_wg = (a.K >= 2048 && (int64_t)(a.N / FR_NT_ROWS) * a.E >= 2048) ? FR_NT_ROWS : 8;
     const dim3 grid((a.N + rows_per_wg - 1) / rows_per_wg, a.E);
@@ -710,7 +874,8 @@ int few_epilogue(int epilogue) { // both forms of GELU run through the same kern
 
 size_t few_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E, int w_is_kn, int epilogue) { // of the kernels here
     int S;
-    if (fr_takes_tile(M, K, E, w_is_kn)) { // the small MFMA tile, cut along K or not
+    if (fr_takes_tile(M, N, K, E, w_is_kn)) { // the small MFMA tile, cut along K or not
+        if (fr_deep_shape(M, N, K, E, w_is_kn)) return 0;
         S = fr_tile_splits(N, K, E, w_is_kn);
         if (S == 1) return 0;
     } else if (epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == EPI_GELU_BWD) {

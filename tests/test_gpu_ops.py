@@ -869,3 +869,48 @@ def test_scatter2scatter_walk_refills_its_table(counts, w_kn):
             err = (out[row : row + c].float() - want).abs().max() / want.abs().max()
             assert err <= 2.0**-8, e  # rounding to bf16: half a unit in the last place, 2^-9 of the value
         row += c
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "counts,K,N",
+    [  # rows per expert: one step of K and one column block; K tails and N remainders; more steps than stages; second pass of rows
+        ([1], 8, 16),
+        ([0, 2, 0, 1], 136, 144),
+        ([3, 0, 1, 1], 640, 272),
+        ([33, 0, 65], 1032, 64),
+        ([1, 32, 0, 2], 2048, 528),
+        ([0] * 63 + [1, 2] + [0] * 62 + [1, 1] + [0] * 170 + [4], 264, 80),  # experts with rows at the ends of the lists that a wave reads
+    ],
+)
+def test_forward_gemm_of_few_workgroups(dtype, counts, K, N):
+    """x @ W^T where at most one workgroup per compute unit has work: store with bias, row scale and scattered rows, and SwiGLU with gathered
+    rows, against the products in 64 bits"""
+    from xma.rocm import ops
+
+    print(f"counts={len(counts)} K={K} N={N} {dtype}", flush=True)
+    E, M = len(counts), sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    nan = lambda *s: torch.full(s, float("nan"), device="cuda", dtype=dtype)
+    offs = torch.tensor(counts, device="cuda").cumsum(0)
+    idx = torch.randperm(M, device="cuda", generator=g)
+    X, W, b, w = new(M, K), new(E, N, K), new(E, N), new(M)
+    e = torch.repeat_interleave(torch.arange(E, device="cuda"), torch.tensor(counts, device="cuda"))
+    unit = 2.0 ** {torch.bfloat16: -8, torch.float16: -11}[dtype]
+
+    def close(got, rows, scale):
+        """fp32 sums of K products and the bias, scaled, then one rounding"""
+        product = lambda f: torch.stack([f(rows[i].double()) @ f(W[e[i]].double()).t() + f(b[e[i]].double()) for i in range(M)]) * f(scale)
+        want, size = product(lambda t: t), product(torch.abs)
+        assert ((got.double() - want).abs() <= unit * want.abs() + (K + 2) * 2.0**-24 * size + 2.0**-24).all()
+
+    out = nan(M, N)
+    ops.scatter2scatter_rocm(X, W.permute(0, 2, 1), idx, offs, out, w, 1, True, False, b)
+    close(out[idx], X, w[idx].double()[:, None])
+    z, h, x = nan(M, N), nan(M, N // 2), new(M, K)
+    ops.up_projection_swiglu_rocm(x, W.permute(0, 2, 1), idx, offs, z, h, 1, b)
+    close(z, x[idx], torch.ones(M, 1, device="cuda", dtype=torch.float64))
+    gate, up = z.double()[:, ::2], z.double()[:, 1::2]
+    want = up * gate * torch.sigmoid(gate)
+    assert ((h.double() - want).abs() <= (unit + 2.0**-20) * want.abs() + 2.0**-24).all()
