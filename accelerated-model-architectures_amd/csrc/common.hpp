@@ -29,6 +29,17 @@ int xma_router_gate_route(const void *x, int64_t ldx, const void *gate_weight, i
 // combine_bwd and router_topk_bwd in one launch, rows without gaps: d_sel[t, j] = d_logits[t, ids[t, j]] (router.hip)
 int xma_combine_router_bwd(const void *expert_out, const void *dy, const void *logits, const int32_t *ids, int64_t T, int32_t H, int32_t E,
                            int32_t k, int dtype, void *d_sel, hipStream_t st);
+// the same from the products that xma_down_projection_dx_dots has left: dots (T k, parts) in fp32, summed over a row (router.hip)
+int xma_dots_router_bwd(const float *dots, int64_t parts, const void *logits, const int32_t *ids, int64_t T, int32_t E, int32_t k, int dtype,
+                        void *d_sel, hipStream_t st);
+// xma_rocm_scatter2scatter with the SWIGLU_BWD epilogue, or with scaled_act xma_rocm_down_projection_dx_swiglu, which also writes
+// dots (M, ceil(N / 128)): <d h, h> over every 128 columns before the row scale, rows in scattered order (grouped_gemm.hip)
+constexpr int64_t ROUTER_GRADIENT_MAX = ((int64_t)1 << 30) - 4; // products: 32-bit byte offsets
+int xma_down_projection_dx_dots(const void *dY, int64_t lddy, const void *W, int64_t w_expert_stride, int64_t ldw,
+                                const int64_t *sorted_scattered_idxs, const int64_t *expert_offsets, const void *z, int64_t ldz, void *dz,
+                                int64_t lddz, void *scaled_act, int64_t ld_scaled_act, const void *row_scale, int64_t M, int32_t N,
+                                int32_t K, int32_t E, int32_t fan_out, int dtype, void *workspace, size_t workspace_bytes, void *stream,
+                                float *dots);
 // what xma_rocm_gate_bwd launches in front of its last kernel, and that kernel with the sum over the k slots (gate.hip)
 int xma_gate_bwd(const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids, const void *scattered, void *d_x,
                  void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype, void *workspace, size_t workspace_bytes, hipStream_t st);

@@ -975,6 +975,8 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
     a.split_cus = 0;
     a.grid_main = 0;
     a.erf_form = erf_form;
+    a.dots = nullptr;
+    a.dots_ld = a.dots_bytes = 0;
     hipStream_t st = (hipStream_t)stream;
     w_is_kn = w_is_kn ? 1 : 0;
     if (fr_takes_mid(a, w_is_kn, epilogue)) return xma_rocm::mid_fwd(a, w_is_kn, epilogue, dtype, (float *)workspace, st);

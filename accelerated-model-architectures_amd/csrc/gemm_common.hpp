@@ -29,6 +29,10 @@ struct FwdArgs {
     int split_cus;   // compute units of the device = tiles per round
     int grid_main;   // workgroups that take whole tiles (an upper bound of the tile count); split_cus more follow
     int erf_form;    // which GELU (EPI_GELU, EPI_GELU_BWD)
+    // SWIGLU_BWD of the 256-row tiles, may be NULL: (M, dots_ld) in scattered order, <d h, h> over every 128 columns before the row
+    // scale: summed over a row, the gradient of that scale.  Wants idx.
+    float *dots;
+    uint32_t dots_ld, dots_bytes; // ceil(N / 128); of the whole
 };
 
 struct DwArgs {

@@ -1297,7 +1297,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) void grouped_gemm_persistent_kerne
                 er.sc[i] = (s_idx & 1) ? Elem<T>::hi(w) : Elem<T>::lo(w);
             }
         }
-        tile_epilogue<T, EPI>(a, acc, smem + PST_STAGING_OFF, cur.row0, cur.rows_valid, cur.n0, tid_e, -1, &er);
+        tile_epilogue<T, EPI, 4, 1>(a, acc, smem + PST_STAGING_OFF, cur.row0, cur.rows_valid, cur.n0, tid_e, -1, &er);
         };
         if (ovl)
             rest_of_tile(IC<1>{});
@@ -1566,7 +1566,7 @@ template <typename T, int WT, int EPI> int launch_fwd(const FwdArgs &a, hipStrea
     constexpr bool persistent_variant = !(WT == 1 && EPI == XMA_ROCM_EPI_SWIGLU);
     bool persistent = false;
     if constexpr (persistent_variant) {
-        if (a.E <= PST_MAX_E && cus > 0 && ((uintptr_t)a.scale & 3) == 0 && offsets_fit) {
+        if (a.E <= PST_MAX_E && cus > 0 && ((uintptr_t)a.scale & 3) == 0 && offsets_fit && row_offsets_fit(a)) {
             // whole tiles: one persistent workgroup per compute unit
             if ((rc = gemm_set_smem(grouped_gemm_persistent_kernel<T, WT, EPI>, PST_SMEM_BYTES))) return rc;
             const int launch_grid = cus < a.grid_main ? cus : a.grid_main;
@@ -1654,7 +1654,7 @@ static int scatter2scatter_impl(const void *X, int64_t ldx, const void *W, int64
                                 void *out, int64_t ldo, void *aux, int64_t ldaux, void *aux2, int64_t ldaux2,
                                 const void *row_scale, const void *bias, int64_t bias_expert_stride, int64_t M, int32_t N,
                                 int32_t K, int32_t E, int32_t fan_out, int x_grouped, int y_grouped, int epilogue, int dtype,
-                                void *workspace, size_t workspace_bytes, void *stream) {
+                                void *workspace, size_t workspace_bytes, void *stream, float *dots = nullptr) {
     XMA_REQUIRE(dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16 || dtype == XMA_ROCM_F32, XMA_ROCM_EUNSUPPORTED,
                 "scatter2scatter: dtype %d", dtype);
     XMA_REQUIRE(epilogue >= XMA_ROCM_EPI_STORE && epilogue <= XMA_ROCM_EPI_SWIGLU_BWD, XMA_ROCM_EINVAL,
@@ -1717,6 +1717,9 @@ static int scatter2scatter_impl(const void *X, int64_t ldx, const void *W, int64
     a.split_cus = 0;
     a.grid_main = 0;
     a.erf_form = 0;
+    a.dots = dots;
+    a.dots_ld = (uint32_t)((N + 127) / 128);
+    a.dots_bytes = dots ? (uint32_t)(M * a.dots_ld * 4) : 0u;
     if (dtype == XMA_ROCM_F32) return f32_scatter2scatter(a, w_is_kn ? 1 : 0, epilogue, (hipStream_t)stream);
     const int64_t NT = (N + BN - 1) / BN;
     const int64_t max_m_tiles = M / BM + E; // sum_e ceil(c_e / BM) <= floor(M / BM) + E
@@ -1773,6 +1776,46 @@ extern "C" int xma_rocm_down_projection_dx_swiglu(const void *dY, int64_t lddy, 
     return scatter2scatter_impl(dY, lddy, W, w_expert_stride, ldw, 1, sorted_scattered_idxs, expert_offsets, dz, lddz,
                                 const_cast<void *>(z), ldz, scaled_act, ld_scaled_act, row_scale, nullptr, 0, M, N, K, E,
                                 fan_out, 0, 1, XMA_ROCM_EPI_SWIGLU_BWD, dtype, workspace, workspace_bytes, stream);
+}
+
+int xma_down_projection_dx_dots(const void *dY, int64_t lddy, const void *W, int64_t w_expert_stride, int64_t ldw,
+                                const int64_t *sorted_scattered_idxs, const int64_t *expert_offsets, const void *z, int64_t ldz, void *dz,
+                                int64_t lddz, void *scaled_act, int64_t ld_scaled_act, const void *row_scale, int64_t M, int32_t N,
+                                int32_t K, int32_t E, int32_t fan_out, int dtype, void *workspace, size_t workspace_bytes, void *stream,
+                                float *dots) {
+    XMA_REQUIRE(M * ((N + 127) / 128) < ROUTER_GRADIENT_MAX, XMA_ROCM_EUNSUPPORTED, "down_projection_dx_dots: M=%lld N=%d (M ceil(N / 128) < 2^30 - 4)", (long long)M, N);
+    XMA_REQUIRE(row_scale && dots && (dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16), XMA_ROCM_EINVAL, "down_projection_dx_dots: dtype %d, row_scale and dots are required", dtype);
+    return scatter2scatter_impl(dY, lddy, W, w_expert_stride, ldw, 1, sorted_scattered_idxs, expert_offsets, dz, lddz,
+                                const_cast<void *>(z), ldz, scaled_act, ld_scaled_act, row_scale, nullptr, 0, M, N, K, E,
+                                fan_out, 0, 1, XMA_ROCM_EPI_SWIGLU_BWD, dtype, workspace, workspace_bytes, stream, dots);
+}
+
+// the K slices of the launch, then the products of rows and 128 columns
+extern "C" size_t xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E) {
+    if (M <= 0 || N <= 0 || K <= 0 || E <= 0) return 0;
+    return (fwd_workspace_bytes(M, N, K, E) + 255) / 256 * 256 + (size_t)M * ((N + 127) / 128) * sizeof(float);
+}
+
+extern "C" int xma_rocm_down_projection_dx_swiglu_router(const void *dY, int64_t lddy, const void *W, int64_t w_expert_stride,
+                                                         int64_t ldw, const int64_t *sorted_scattered_idxs,
+                                                         const int64_t *expert_offsets, const void *z, int64_t ldz, void *dz,
+                                                         int64_t lddz, void *scaled_act, int64_t ld_scaled_act,
+                                                         const void *row_scale, void *d_row_scale, int64_t M, int32_t N, int32_t K,
+                                                         int32_t E, int32_t fan_out, int dtype, void *workspace,
+                                                         size_t workspace_bytes, void *stream) {
+    XMA_REQUIRE(fan_out >= 1 && fan_out <= 32 && fan_out <= E && M >= 0 && M % fan_out == 0 && (M == 0 || d_row_scale), XMA_ROCM_EINVAL,
+                "down_projection_dx_swiglu_router: fan_out=%d E=%d M=%lld (at most 32 of the experts, M a multiple), d_row_scale is required", fan_out, E, (long long)M);
+    const size_t need = xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, N, K, E);
+    XMA_REQUIRE(M == 0 || (workspace && aligned16(workspace) && workspace_bytes >= need), XMA_ROCM_EWORKSPACE,
+                "down_projection_dx_swiglu_router: workspace of %zu bytes, %zu needed (16-byte aligned)", workspace_bytes, need);
+    if (M == 0) return XMA_ROCM_OK;
+    const int64_t parts = (N + 127) / 128;
+    float *dots = (float *)((char *)workspace + need) - M * parts;
+    const int rc = xma_down_projection_dx_dots(dY, lddy, W, w_expert_stride, ldw, sorted_scattered_idxs, expert_offsets, z, ldz, dz, lddz,
+                                               scaled_act, ld_scaled_act, row_scale, M, N, K, E, fan_out, dtype, workspace,
+                                               workspace_bytes, stream, dots);
+    if (rc) return rc;
+    return xma_dots_router_bwd(dots, parts, nullptr, nullptr, M / fan_out, E, fan_out, dtype, d_row_scale, (hipStream_t)stream);
 }
 
 #ifdef XMA_PST_TIMING

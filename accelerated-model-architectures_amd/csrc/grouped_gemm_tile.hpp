@@ -80,9 +80,41 @@ struct EpiRows {
     float sc[4];
 };
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_buffer(const void *p, uint32_t bytes) {
+    const uint64_t base = (uint64_t)p, lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
+    const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(base >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(lo | hi << 32), 0, __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+// The rows of a tile in one of its grouped matrices: 16-byte accesses at row, by 32-bit offsets from the tile's first row.  What lies past
+// the last valid row is outside the buffer: loads read zeros and stores are dropped, so no row is clamped, and an address is one addition
+// where 64-bit ones take a clamp and a product each, a fifth of the instructions of the SwiGLU backward's epilogue.  On its own that
+// gives those launches nothing (board power, and the rows' own traffic); it makes room for `dots`.
+struct RowBuffer {
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t lane_off, ld_bytes;
+    __device__ __forceinline__ RowBuffer(const uint16_t *m, int64_t ld, int64_t row0, int rows_valid, int lane_row, int col) {
+        ld_bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)(2 * ld));
+        rsrc = uniform_buffer(m + row0 * ld, (uint32_t)rows_valid * ld_bytes);
+        lane_off = mul_add_u32((uint32_t)lane_row, ld_bytes, (uint32_t)col * 2);
+    }
+    __device__ __forceinline__ u32x4 load(int row) const {
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off + (uint32_t)row * ld_bytes, 0, 0);
+    }
+    __device__ __forceinline__ void store(int row, u32x4 v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, lane_off + (uint32_t)row * ld_bytes, 0, 0);
+    }
+};
+
+// Whether the offsets of a launch's epilogue fit: 256 rows of every grouped matrix in 2^32 - 1 bytes, the scattered one in 2^32 pieces of 16.
+inline bool row_offsets_fit(const FwdArgs &a) {
+    const int64_t most = ((int64_t)1 << 23) - 1;
+    return (a.y_grouped ? a.ldo <= most : a.M * (a.ldo / 8) < ((int64_t)1 << 32)) && (!a.aux || a.ldaux <= most) && (!a.aux2 || a.ldaux2 <= most);
+}
+
 // ---- epilogue of one tile of 64 NI rows x 256 columns (2 x 2 waves of NI 32-row blocks x 128 columns); smem: staging area that no
 // wave reads operand tiles from any more
-template <typename T, int EPI, int NI = 4>
+// FIT: the launch's offsets fit (row_offsets_fit).
+template <typename T, int EPI, int NI = 4, int FIT = 0>
 __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4][NI], unsigned char *smem, int64_t row0,
                                               int rows_valid, int n0, int tid, int only_i = -1,
                                               const EpiRows *pre = nullptr) {
@@ -183,6 +215,9 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
         // need no exchange of row indices between lanes
         auto blocks = [&](auto SCALED, auto GROUPED) {
         const int last = rows_valid - 1;
+        constexpr bool buf = FIT && GROUPED.value, units = FIT && !GROUPED.value;
+        const RowBuffer out_b(a.out, a.ldo, buf ? row0 : 0, buf && write_z ? rows_valid : 0, wq + (lane >> 4), cz);
+        const RowBuffer aux_b(a.aux, a.ldaux, buf ? row0 : 0, buf ? rows_valid : 0, wq + (lane >> 3), ch);
         uint16_t *out0 = a.out + (GROUPED.value ? row0 * a.ldo : 0) + cz;
         uint16_t *aux0 = a.aux + (GROUPED.value ? row0 * a.ldaux : 0) + ch;
 #pragma unroll
@@ -212,9 +247,23 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                 }
             }
             wave_lds_sync();
-            if (write_z) {
+            if constexpr (units) {
+                // rows past the last valid one hold its sums and its place again, as everywhere here
+                const uint32_t place = (uint32_t)idx_i[i] * (uint32_t)(a.ldo >> 3);
+                if (write_z) {
+#pragma unroll
+                    for (int it = 0; it < 8; ++it) {
+                        const u32x4 v = *(const u32x4 *)(stage + (4 * it + (lane >> 4)) * EPI_Z_STRIDE + z_piece * 16);
+                        *(u32x4 *)(out0 + (int64_t)(uint32_t)__shfl((int)place, 4 * it + (lane >> 4)) * 8) = v;
+                    }
+                }
+            } else if (write_z) {
 #pragma unroll
                 for (int it = 0; it < 8; ++it) {
+                    if constexpr (buf) {
+                        out_b.store(i * 32 + 4 * it, *(const u32x4 *)(stage + (4 * it + (lane >> 4)) * EPI_Z_STRIDE + z_piece * 16));
+                        continue;
+                    }
                     int r = rbase + 4 * it + (lane >> 4);
                     if (r > last) r = last;
                     const u32x4 v = *(const u32x4 *)(stage + (r - rbase) * EPI_Z_STRIDE + z_piece * 16);
@@ -253,6 +302,10 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
             if constexpr (EPI == XMA_ROCM_EPI_SWIGLU) {
 #pragma unroll
                 for (int it = 0; it < 4; ++it) {
+                    if constexpr (buf) {
+                        aux_b.store(i * 32 + 8 * it, *(const u32x4 *)(stage + 32 * EPI_Z_STRIDE + (8 * it + (lane >> 3)) * EPI_H_STRIDE + h_piece * 16));
+                        continue;
+                    }
                     int r = rbase + 8 * it + (lane >> 3);
                     if (r > last) r = last;
                     const u32x4 v = *(const u32x4 *)(stage + 32 * EPI_Z_STRIDE + (r - rbase) * EPI_H_STRIDE + h_piece * 16);
@@ -299,17 +352,33 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
         const int piece = (2 * (n0 + wp) + (lane & 31) * 8 < 2 * a.N) ? (lane & 31) : 0; // piece 0 is inside N
         const int cz = 2 * (n0 + wp) + piece * 8; // this lane's 8 columns of z / dz on the way in and out
         float sc_i[4];
+        // The gradient of a row's scale (the router weight) is <d h, h>: a lane owns a row here and has both at hand, so it costs one
+        // multiply-add per value, an exchange between the row's two lanes and 4 bytes per row and wave.  A pass over the expert outputs
+        // that forms it as <dy, expert_out> reads k T H of them again.  Forward + backward, 262144 rows of H = 2048, I = 768: 7861 -> 7695 us;
+        // 98304 of I = 1408: 5547 -> 5510; 16384 of H = 4096, I = 14336: equal.
+        const bool dots = NI == 4 && a.dots != nullptr;
+        const int cols = a.N - (n0 + wp); // columns from here on are not the wave's: what they hold is dropped
+        // no condition on these stores either: without dots, and for the rows past the last valid one, they lie outside the buffer
+        const __amdgpu_buffer_rsrc_t dots_b = uniform_buffer(a.dots, dots ? a.dots_bytes : 0u);
+        int idx_i[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             int r = wq + i * 32 + lrow;
             if (r >= rows_valid) r = rows_valid - 1;
             sc_i[i] = 1.f;
             if (a.scale) sc_i[i] = pre ? pre->sc[i] : Elem<T>::lo((uint32_t)a.scale[a.idx[row0 + r]]);
+            if (dots) idx_i[i] = pre ? pre->idx[i] : (int)a.idx[row0 + r];
         }
+        const RowBuffer z_b(a.aux, a.ldaux, FIT ? row0 : 0, FIT ? rows_valid : 0, wq + (lane >> 5), cz);
+        const RowBuffer dz_b(a.out, a.ldo, FIT ? row0 : 0, FIT ? rows_valid : 0, wq + (lane >> 5), cz);
         u32x4 zin[16];
         auto load_block = [&](int i) {
 #pragma unroll
             for (int it = 0; it < 16; ++it) {
+                if constexpr (FIT) {
+                    zin[it] = z_b.load(i * 32 + 2 * it);
+                    continue;
+                }
                 int r = wq + i * 32 + 2 * it + (lane >> 5);
                 if (r >= rows_valid) r = rows_valid - 1;
                 zin[it] = *(const u32x4 *)(a.aux + (row0 + r) * a.ldaux + cz);
@@ -348,6 +417,7 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
             wave_lds_sync();
             const float sc = sc_i[i];
             uint32_t hs[HS.value ? 32 : 1];
+            float dot = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -355,7 +425,7 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                     u32x4 *zp = (u32x4 *)(mine + (j * 32 + g * 8) * 4);
                     const u32x4 z = *zp;
                     u32x4 o;
-                    float hv[4];
+                    float hv[4], dq = 0.f;
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         const float dh = acc[j][i][4 * g + q] * sc;
@@ -363,7 +433,9 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                         const float sg = sigmoidf_fast(gg), silu = gg * sg;
                         o[q] = Elem<T>::pack(dh * uu * (sg + silu * (1.f - sg)), dh * silu);
                         hv[q] = uu * silu * sc;
+                        if constexpr (NI == 4) dq += acc[j][i][4 * g + q] * (uu * silu);
                     }
+                    if constexpr (NI == 4) dot += (j * 32 + g * 8 < cols) ? dq : 0.f; // uniform: N is a multiple of 8
                     *zp = o;
                     if constexpr (HS.value != 0) {
                         hs[2 * (j * 4 + g)] = park(Elem<T>::pack(hv[0], hv[1]));
@@ -374,10 +446,19 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
             wave_lds_sync();
 #pragma unroll
             for (int it = 0; it < 16; ++it) {
+                if constexpr (FIT) {
+                    dz_b.store(i * 32 + 2 * it, *(const u32x4 *)(stage + (2 * it + (lane >> 5)) * EPI_BWD_STRIDE + piece * 16));
+                    continue;
+                }
                 int br = 2 * it + (lane >> 5); // row of the block; the block's first row is valid
                 if (wq + i * 32 + br >= rows_valid) br = rows_valid - 1 - (wq + i * 32);
                 const u32x4 v = *(const u32x4 *)(stage + br * EPI_BWD_STRIDE + piece * 16);
                 *(u32x4 *)(a.out + (row0 + wq + i * 32 + br) * a.ldo + cz) = v;
+            }
+            if constexpr (NI == 4) {
+                dot += __shfl_xor(dot, 32);
+                const uint32_t at = mul_add_u32((uint32_t)idx_i[i], a.dots_ld, (uint32_t)(n0 + wp) >> 7) * 4;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, dot), dots_b, wq + i * 32 + lrow < rows_valid ? at : BUF_OUTSIDE, 0, 0);
             }
             wave_lds_sync(); // the next block overwrites the area
             if constexpr (HS.value != 0) {
@@ -390,8 +471,13 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                     for (int g = 0; g < 4; ++g)
                         *(u32x2 *)(h_w + (j * 32 + g * 8) * 2) = u32x2{unpark(hs[2 * (j * 4 + g)]), unpark(hs[2 * (j * 4 + g) + 1])};
                 wave_lds_sync();
+                const RowBuffer h_b(a.aux2, a.ldaux2, FIT ? row0 : 0, FIT ? rows_valid : 0, wq + (lane >> 4), ch);
 #pragma unroll
                 for (int it = 0; it < 8; ++it) {
+                    if constexpr (FIT) {
+                        h_b.store(i * 32 + 4 * it, *(const u32x4 *)(stage + (4 * it + (lane >> 4)) * EPI_Z_STRIDE + hpiece * 16));
+                        continue;
+                    }
                     int br = 4 * it + (lane >> 4);
                     if (wq + i * 32 + br >= rows_valid) br = rows_valid - 1 - (wq + i * 32);
                     const u32x4 v = *(const u32x4 *)(stage + br * EPI_Z_STRIDE + hpiece * 16);

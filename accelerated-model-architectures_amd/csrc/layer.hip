@@ -15,7 +15,7 @@ namespace {
 // forward-type GEMM through the entry point that the caller has chosen
 int gemm(const xma_rocm_moe *m, int64_t few, const void *X, const void *W, int64_t w_es, int64_t ldw, int w_is_kn, void *out, void *aux,
          int64_t ldaux, void *aux2, const void *scale, const void *bias, int64_t N, int64_t K, int64_t fan_out, int x_grouped, int y_grouped,
-         int epilogue, void *stream) {
+         int epilogue, void *stream, float *dots = nullptr) {
     const int64_t M = m->T * m->k, ldo = epilogue == XMA_ROCM_EPI_SWIGLU_BWD ? 2 * N : N;
     if (epilogue >= XMA_ROCM_EPI_GELU_TANH && !few) { // no epilogue of the 256 x 256 kernels: a pass of its own
         const int form = epilogue >= XMA_ROCM_EPI_GELU_ERF, bwd = epilogue & 1;
@@ -27,6 +27,9 @@ int gemm(const xma_rocm_moe *m, int64_t few, const void *X, const void *W, int64
         return xma_rocm_scatter2scatter_few_rows(X, K, W, w_es, ldw, w_is_kn, idx, offs, out, ldo, aux, ldaux, aux2, aux2 ? N : 0, scale, bias,
                                                  bias ? N : 0, M, (int32_t)N, (int32_t)K, (int32_t)m->E, (int32_t)fan_out, x_grouped, y_grouped,
                                                  epilogue, (int)m->dtype, m->workspace, (size_t)m->workspace_bytes, stream);
+    if (dots)
+        return xma_down_projection_dx_dots(X, K, W, w_es, ldw, idx, offs, aux, ldaux, out, ldo, aux2, N, scale, M, (int32_t)N, (int32_t)K,
+                                           (int32_t)m->E, (int32_t)fan_out, (int)m->dtype, m->workspace, (size_t)m->workspace_bytes, stream, dots);
     // the 256 x 256 kernels split the last round of tiles where there is a workspace, and refuse one that is too small for it
     if (aux2)
         return xma_rocm_down_projection_dx_swiglu(X, K, W, w_es, ldw, idx, offs, aux, ldaux, out, ldo, aux2, N, scale, M, (int32_t)N, (int32_t)K,
@@ -106,12 +109,26 @@ extern "C" int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream) {
     return xma_rocm_combine(m->expert_out, m->H, m->router_weights, m->y, m->H, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream);
 }
 
-// The activations and expert outputs again where neither was kept: h from z, the expert outputs by the down-projection.
-static int recompute(const xma_rocm_moe *m, const char *what, void *stream) {
+// The activations and expert outputs again where neither was kept: h from z, the expert outputs by the down-projection.  Where dX2
+// leaves the router weights' gradient (`dots`), nothing reads the expert outputs, and h only dW2.
+static int recompute(const xma_rocm_moe *m, const char *what, bool dots, void *stream) {
     if (!m->recompute) return XMA_ROCM_OK;
-    RUN(check_workspace(m, m->few_down, m->H, m->I, what));
-    RUN(xma_rocm_swiglu_packed_forward(m->z, 2 * m->I, m->h, m->I, m->T * m->k, (int32_t)m->I, (int)m->dtype, stream));
-    return down_projection(m, stream);
+    if (!dots) RUN(check_workspace(m, m->few_down, m->H, m->I, what));
+    if (!dots || m->dw2_form != 1)
+        RUN(xma_rocm_swiglu_packed_forward(m->z, 2 * m->I, m->h, m->I, m->T * m->k, (int32_t)m->I, (int)m->dtype, stream));
+    return dots ? XMA_ROCM_OK : down_projection(m, stream);
+}
+
+static int64_t dots_parts(const xma_rocm_moe *m) { return (m->I + 127) / 128; }
+
+// Where dX2 by the 256 x 256 kernels leaves <d h, h> of each row and 128 columns: in the workspace, behind the K slices of that launch, if it
+// is large enough.  A bias of the down-projection would add <dy, bias> to the gradient, which <d h, h> lacks.
+static float *dots_place(const xma_rocm_moe *m) {
+    if (m->few_dx2 || m->activation || m->b_proj || m->dtype == XMA_ROCM_F32 || !m->workspace || m->k > 32) return nullptr;
+    const int64_t M = m->T * m->k, I = m->I, H = m->H, E = m->E;
+    if (M * dots_parts(m) >= ROUTER_GRADIENT_MAX) return nullptr;
+    const size_t need = xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, (int32_t)I, (int32_t)H, (int32_t)E);
+    return (size_t)m->workspace_bytes >= need ? (float *)((char *)m->workspace + need) - M * dots_parts(m) : nullptr;
 }
 
 // The gradient of the router's logits: what the gate's own products need before the rest of the backward.
@@ -120,14 +137,14 @@ extern "C" int xma_rocm_moe_backward_router(const xma_rocm_moe *m, void *stream)
     XMA_REQUIRE(m->logits && m->dy && m->d_router_weights && m->d_logits && (!m->recompute || m->h), XMA_ROCM_EINVAL,
                 "moe_backward_router: null buffer");
     const int dtype = (int)m->dtype;
-    RUN(recompute(m, "moe_backward_router", stream));
+    RUN(recompute(m, "moe_backward_router", false, stream));
     RUN(xma_rocm_combine_bwd(m->expert_out, m->H, m->dy, m->H, m->d_router_weights, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream));
     return xma_rocm_router_topk_bwd(m->logits, m->E, m->T, (int32_t)m->E, (int32_t)m->k, dtype, m->expert_ids, 0, m->d_router_weights, m->d_logits,
                                     m->E, stream);
 }
 
 // Everything of the backward between the router's part and the sum over the k slots: `scattered` holds dX1 then.
-static int backward_experts(const xma_rocm_moe *m, const char *what, void *stream) {
+static int backward_experts(const xma_rocm_moe *m, const char *what, float *dots, void *stream) {
     RUN(check(m, what));
     XMA_REQUIRE(m->dy && m->dz && m->d_w_fc && m->d_w_proj && m->scattered && m->d_x && (m->dw2_form == 1 || m->h) &&
                     (m->dw2_form == 0 || m->dw2_operand) && (!m->d_b_fc || m->b_fc) && (!m->d_b_proj || m->b_proj),
@@ -142,7 +159,10 @@ static int backward_experts(const xma_rocm_moe *m, const char *what, void *strea
     RUN(check_workspace(m, m->few_dx1, H, U, what));
     // dX2 + SwiGLU', with the scaled activations for dW2 where that takes dy through the index
     RUN(gemm(m, m->few_dx2, m->dy, m->w_proj, H * I, I, 1, m->dz, m->z, U, m->dw2_form == 1 ? m->dw2_operand : nullptr, m->router_weights,
-             nullptr, I, H, m->k, 0, 1, epilogue_of(m, 1), stream));
+             nullptr, I, H, m->k, 0, 1, epilogue_of(m, 1), stream, dots));
+    if (dots) // before dX1, whose K slices take their place
+        RUN(xma_dots_router_bwd(dots, dots_parts(m), m->logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->E, (int32_t)m->k, dtype,
+                                m->d_router_weights, (hipStream_t)stream));
     if (m->dw2_form == 1) {
         RUN(dw(m, m->few_dw2, m->dy, 0, nullptr, m->dw2_operand, 1, m->d_w_proj, H, I, stream));
         if (m->d_b_proj)
@@ -163,7 +183,7 @@ static int backward_experts(const xma_rocm_moe *m, const char *what, void *strea
 }
 
 extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
-    RUN(backward_experts(m, "moe_backward", stream));
+    RUN(backward_experts(m, "moe_backward", nullptr, stream));
     return xma_rocm_combine_add(m->scattered, m->H, nullptr, m->d_x_addend, m->H, m->d_x, m->H, m->T, (int32_t)m->k, (int32_t)m->H, (int)m->dtype, stream);
 }
 
@@ -174,10 +194,12 @@ extern "C" int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_w
     const int dtype = (int)m->dtype;
     XMA_REQUIRE(xma_rocm_gate_bwd_supported((int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype), XMA_ROCM_EUNSUPPORTED,
                 "moe_backward_gated: H=%lld E=%lld k=%lld dtype=%d", (long long)m->H, (long long)m->E, (long long)m->k, dtype);
-    RUN(recompute(m, "moe_backward_router", stream));
-    RUN(xma_combine_router_bwd(m->expert_out, m->dy, m->logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k,
-                               dtype, m->d_router_weights, (hipStream_t)stream));
-    RUN(backward_experts(m, "moe_backward", stream));
+    float *const dots = dots_place(m);
+    RUN(recompute(m, "moe_backward_router", dots != nullptr, stream));
+    if (!dots)
+        RUN(xma_combine_router_bwd(m->expert_out, m->dy, m->logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k,
+                                   dtype, m->d_router_weights, (hipStream_t)stream));
+    RUN(backward_experts(m, "moe_backward", dots, stream));
     return xma_gate_bwd(m->x, m->H, m->gate_weight, m->d_router_weights, (const int32_t *)m->expert_ids, m->scattered, m->d_x, d_gate_weight, m->T,
                         (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->workspace, (size_t)m->workspace_bytes, (hipStream_t)stream);
 }

@@ -272,6 +272,41 @@ __global__ __launch_bounds__(RT_THREADS) void combine_router_bwd_kernel(const vo
     if (mine) Scalar<DT>::store(d_sel, t * k + lane, d);
 }
 
+// The same behind a dX2 launch that has left <d h, h> of every row and 128 columns (dots, T k rows of `parts`): a wave takes a token, 64 / P
+// lanes of it a slot (P = k rounded up to a power of two).  Without logits it leaves d_w itself.  A few MB: 7 us where the
+// pass over expert_out takes 34 (16384 rows of H = 4096, 112 parts), 15 where it takes 216 (262144 of 2048, 6 parts).
+template <int DT>
+__global__ __launch_bounds__(RT_THREADS) void dots_router_bwd_kernel(const float *__restrict__ dots, int64_t parts,
+                                                                    const void *__restrict__ logits, const int32_t *__restrict__ ids,
+                                                                    int64_t T, int E, int k, int lanes, void *__restrict__ d_sel) {
+    const int lane = threadIdx.x & 63;
+    const int64_t t = (int64_t)blockIdx.x * (RT_THREADS / 64) + (threadIdx.x >> 6);
+    if (t >= T) return; // uniform
+    float my_val = 0.f;
+    if (logits && lane < k) {
+        int e = ids[t * k + lane];
+        e = e < 0 ? 0 : (e >= E ? E - 1 : e); // never read outside the row
+        my_val = key_value(order_key(Scalar<DT>::load(logits, t * E + e)));
+    }
+    const int slot = lane / lanes, q = lane % lanes;
+    float sum = 0.f;
+    if (slot < k)
+        for (int64_t p = q; p < parts; p += lanes) sum += dots[(t * k + slot) * parts + p];
+    for (int d = lanes / 2; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+    typedef Elem<typename RowType<DT>::type> El;
+    const uint32_t rounded = El::pack(__shfl(sum, lane * lanes & 63), 0.f) & 0xffffu;
+    const float my_dw = El::lo(rounded);
+    if (!logits) {
+        if (lane < k) ((uint16_t *)d_sel)[t * k + lane] = (uint16_t)rounded;
+        return;
+    }
+    const float w = group_softmax<64>(my_val, lane, k, 0);
+    const float dot = group_sum<64>(lane < k ? w * my_dw : 0.f);
+    float d = w * (my_dw - dot);
+    asm("" : "+v"(d)); // rounded to fp32 first
+    if (lane < k) Scalar<DT>::store(d_sel, t * k + lane, d);
+}
+
 // ------------------------------------------------------------------------------------------------
 // Gate projection fused with the router: logits = x @ Wg^T (fp32 accumulation, rounded to the activation dtype as the
 // stock linear layer does), then top-k, fp32 softmax and expert ids from the rounded logits, in one kernel
@@ -956,4 +991,22 @@ int xma_combine_router_bwd(const void *expert_out, const void *dy, const void *l
         CALL(XMA_ROCM_F32);
 #undef CALL
     return xma_check_launch("combine_router_bwd_kernel");
+}
+
+int xma_dots_router_bwd(const float *dots, int64_t parts, const void *logits, const int32_t *ids, int64_t T, int32_t E, int32_t k, int dtype,
+                        void *d_sel, hipStream_t st) {
+    RouterShape s;
+    if (int rc = router_shape("dots_router_bwd", T, E, k, dtype, s)) return rc;
+    XMA_REQUIRE(parts >= 1 && k <= 64 && (dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16) && (T == 0 || (dots && (ids || !logits) && d_sel)),
+                XMA_ROCM_EINVAL, "dots_router_bwd: parts=%lld k=%d dtype=%d or a null pointer", (long long)parts, k, dtype);
+    if (T == 0) return XMA_ROCM_OK;
+    int lanes = 64;
+    while (lanes * k > 64) lanes >>= 1;
+    const int64_t blocks = (T + RT_THREADS / 64 - 1) / (RT_THREADS / 64);
+    XMA_REQUIRE(blocks < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "dots_router_bwd: too many rows");
+    if (dtype == XMA_ROCM_BF16)
+        dots_router_bwd_kernel<XMA_ROCM_BF16><<<(int)blocks, RT_THREADS, 0, st>>>(dots, parts, logits, ids, T, E, k, lanes, d_sel);
+    else
+        dots_router_bwd_kernel<XMA_ROCM_F16><<<(int)blocks, RT_THREADS, 0, st>>>(dots, parts, logits, ids, T, E, k, lanes, d_sel);
+    return xma_check_launch("dots_router_bwd_kernel");
 }

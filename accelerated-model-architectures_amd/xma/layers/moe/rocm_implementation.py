@@ -380,7 +380,8 @@ class _FusedSwiGLUExperts(torch.autograd.Function):
             expert_out = torch.empty(z.size(0), w_proj.size(-1), device=z.device, dtype=z.dtype)
             ops.scatter2scatter_rocm(h, w_proj, sorted_scattered_idxs, expert_offsets, expert_out, None, 1, True, False, b_proj)
         d_router_weights = torch.empty_like(router_weights)
-        ops.combine_bwd_rocm(expert_out, grad_out, d_router_weights)
+        if b_proj is not None:  # <dy, bias> is part of the gradient: it comes from the expert outputs
+            ops.combine_bwd_rocm(expert_out, grad_out, d_router_weights)
 
         dz = torch.empty_like(z)
         d_w_proj = _empty_dw_like(w_proj)
@@ -390,16 +391,28 @@ class _FusedSwiGLUExperts(torch.autograd.Function):
             # w_n h_n (T*k, I), and dW2 takes dy unscaled through the index - instead of a scaled, grouped copy of dy
             # (T*k, H) written by `group` and read back by the GEMM
             scaled_h = torch.empty(z.size(0), z.size(1) // 2, dtype=z.dtype, device=z.device)
-            ops.down_projection_dx_swiglu_scaled_act_rocm(
-                grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, scaled_h, flat_w, top_k
-            )
+            if b_proj is None:
+                ops.down_projection_dx_swiglu_router_rocm(
+                    grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, scaled_h, flat_w, expert_out,
+                    d_router_weights, top_k
+                )
+            else:
+                ops.down_projection_dx_swiglu_scaled_act_rocm(
+                    grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, scaled_h, flat_w, top_k
+                )
             ops.group_bwd_W_rocm(grad_out, scaled_h, sorted_scattered_idxs, expert_offsets, d_w_proj, None, top_k, 0)
             if b_proj is not None:
                 d_b_proj = _bias_grad(grad_out, sorted_scattered_idxs, expert_offsets, b_proj, flat_w, top_k)
         else:
-            ops.down_projection_dx_swiglu_rocm(
-                grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, flat_w, top_k
-            )
+            if b_proj is None:
+                ops.down_projection_dx_swiglu_router_rocm(
+                    grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, None, flat_w, expert_out,
+                    d_router_weights, top_k
+                )
+            else:
+                ops.down_projection_dx_swiglu_rocm(
+                    grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, flat_w, top_k
+                )
             if b_proj is None and ops._dw_loader_scales(z.size(0), w_proj.size(0), z.dtype, w_proj.size(2), w_proj.size(1)):
                 # a handful of rows per expert: the weight gradient's loader gathers and scales the rows of dy itself (and
                 # rounds them like the copy would), one launch less
@@ -496,7 +509,9 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, 
     (sizes if save else temp)["out"] = M * H * s
     # the scattered rows of dX1 take the place of dW2's operand
     gate_sums = get_library().xma_rocm_gate_bwd_workspace_bytes(T, H, E) if ops.gate_bwd_supported(H, E, k, dtype) else 0
-    back = dict(d_weights=M * s, dz=M * U * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], gate_sums, 256))
+    # dX2 by the 256 x 256 kernels leaves the router weights' gradient behind its K slices
+    dots = ops.router_gradient_workspace_bytes(M, I, H, E, device_index) if glu and not b_proj and ops.dx2_leaves_router_gradient(dx2[0], M, I, k, dtype) else 0
+    back = dict(d_weights=M * s, dz=M * U * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], gate_sums, dots, 256))
     if not save:
         back |= dict(h=M * I * s, out=M * H * s)
     p = _Plan()

@@ -55,6 +55,12 @@ SIGNATURES = {
         [_p, _i64, _p, _i64, _i64, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _i32, _int,
          _p, _sz, _p],
     ),
+    "xma_rocm_down_projection_dx_swiglu_router_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32]),
+    "xma_rocm_down_projection_dx_swiglu_router": (
+        _int,
+        [_p, _i64, _p, _i64, _i64, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _i32, _i32, _i32, _i32, _int,
+         _p, _sz, _p],
+    ),
     "xma_rocm_group_bwd_W": (
         _int,
         [_p, _i64, _int, _i32, _p, _p, _i64, _int, _i32, _p, _p, _p, _i64, _i64, _i32, _i32, _i32, _int, _p],

@@ -416,6 +416,63 @@ def down_projection_dx_swiglu_scaled_act_rocm(
     )
 
 
+@lru_cache(maxsize=4096)
+def router_gradient_workspace_bytes(M: int, N: int, K: int, E: int, device_index: int) -> int:
+    """scratch of dX2 by the 256 x 256 kernels with the router weights' gradient; depends on the shape and the device only"""
+    with torch.cuda.device(device_index):
+        return get_library().xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, N, K, E)
+
+
+def dx2_leaves_router_gradient(few: int, M: int, N: int, k: int, dtype: torch.dtype) -> bool:
+    """whether dX2 + SwiGLU' also forms the gradient of the router weights: where the 256 x 256 kernels take it (few == 0) and 32-bit
+    offsets reach its products"""
+    return not few and k <= 32 and M * -(-N // 128) < (1 << 30) - 4 and dtype in (torch.bfloat16, torch.float16)
+
+
+@torch.library.custom_op("xma_rocm::down_projection_dx_swiglu_router", mutates_args={"dz", "scaled_act", "d_row_scale"})
+def down_projection_dx_swiglu_router_rocm(
+    dY: torch.Tensor,
+    W: torch.Tensor,
+    sorted_scattered_idxs: torch.Tensor,
+    expert_offsets: torch.Tensor,
+    z: torch.Tensor,
+    dz: torch.Tensor,
+    scaled_act: torch.Tensor | None,
+    row_scale: torch.Tensor,
+    expert_out: torch.Tensor,
+    d_row_scale: torch.Tensor,
+    FAN_OUT: int,
+) -> None:
+    """down_projection_dx_swiglu[_scaled_act] and combine_bwd of a down-projection without a bias: d_row_scale (T, k) from dX2's own
+    products where the 256 x 256 kernels take it, from expert_out otherwise"""
+    M = sorted_scattered_idxs.numel()
+    E, K, N = W.shape
+    assert dY.size(1) == K and dY.size(0) * FAN_OUT == M and d_row_scale.shape == (dY.size(0), FAN_OUT)
+    w_is_kn, w_es, ldw = _weight_layout(W)
+    few = _few_rows_fwd(M, N, K, E, w_is_kn, ldw, dY.size(0) * dY.stride(0), dY.dtype, EPI_SWIGLU_BWD)
+    if M == 0 or w_is_kn != 1 or not dx2_leaves_router_gradient(few, M, N, FAN_OUT, dY.dtype):
+        combine_bwd_rocm(expert_out, dY, d_row_scale)
+        if scaled_act is None:
+            down_projection_dx_swiglu_rocm(dY, W, sorted_scattered_idxs, expert_offsets, z, dz, row_scale, FAN_OUT)
+        else:
+            down_projection_dx_swiglu_scaled_act_rocm(dY, W, sorted_scattered_idxs, expert_offsets, z, dz, scaled_act, row_scale, FAN_OUT)
+        return
+    assert z.shape == (M, 2 * N) and dz.shape == (M, 2 * N) and (scaled_act is None or scaled_act.shape == (M, N) and scaled_act.dtype == dY.dtype)
+    assert W.dtype == dY.dtype == z.dtype == dz.dtype == row_scale.dtype == d_row_scale.dtype and row_scale.is_contiguous() and d_row_scale.is_contiguous()
+    assert sorted_scattered_idxs.dtype == torch.int64 and sorted_scattered_idxs.is_contiguous()
+    assert expert_offsets.dtype == torch.int64 and expert_offsets.is_contiguous() and expert_offsets.numel() == E
+    ws_bytes = router_gradient_workspace_bytes(M, N, K, E, dY.device.index or 0)
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dY.device)
+    check(
+        get_library().xma_rocm_down_projection_dx_swiglu_router(
+            _ptr(dY), _rows(dY, "dY"), _ptr(W), w_es, ldw, _ptr(sorted_scattered_idxs), _ptr(expert_offsets),
+            _ptr(z), _rows(z, "z"), _ptr(dz), _rows(dz, "dz"), _ptr(scaled_act), 0 if scaled_act is None else _rows(scaled_act, "scaled_act"),
+            _ptr(row_scale), _ptr(d_row_scale), M, N, K, E, FAN_OUT, _code(dY), _ptr(workspace), ws_bytes, _stream(dY),
+        ),
+        "xma_rocm_down_projection_dx_swiglu_router",
+    )
+
+
 @torch.library.custom_op("xma_rocm::group_bwd_W", mutates_args={"DW"})
 def group_bwd_W_rocm(
     DY: torch.Tensor,

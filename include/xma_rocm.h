@@ -200,6 +200,19 @@ XMA_API int xma_rocm_down_projection_dx_swiglu(const void *dY, int64_t lddy, con
                                                const void *row_scale, int64_t M, int32_t N, int32_t K, int32_t num_experts,
                                                int32_t fan_out, int dtype, void *workspace, size_t workspace_bytes,
                                                void *stream);
+/*
+ * The same, scaled_act optional, with the gradient of the row scale (combine backward of a down-projection without a bias): d_row_scale
+ * (M / fan_out, fan_out) = <(dY @ B_e)[n], swiglu_packed(z[n])> at idx[n], formed where both are at hand instead of from the expert
+ * outputs.  row_scale and workspace required; fan_out <= 32.
+ */
+XMA_API size_t xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t num_experts);
+XMA_API int xma_rocm_down_projection_dx_swiglu_router(const void *dY, int64_t lddy, const void *W, int64_t w_expert_stride,
+                                                      int64_t ldw, const int64_t *sorted_scattered_idxs,
+                                                      const int64_t *expert_offsets, const void *z, int64_t ldz, void *dz,
+                                                      int64_t lddz, void *scaled_act, int64_t ld_scaled_act,
+                                                      const void *row_scale, void *d_row_scale, int64_t M, int32_t N, int32_t K,
+                                                      int32_t num_experts, int32_t fan_out, int dtype, void *workspace,
+                                                      size_t workspace_bytes, void *stream);
 
 /*
  * xma_rocm_scatter2scatter_bias / xma_rocm_down_projection_dx_swiglu for the few-token regime: the same arguments
@@ -400,7 +413,9 @@ XMA_API int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream);
 /*
  * The whole backward where no gradient of the logits comes from outside and xma_rocm_gate_bwd covers the gate: both of the above and the
  * gate's two products, whose part of d_x joins the sum over the k slots.  d_router_weights receives d_selected; d_logits and d_x_addend are
- * not used; d_gate_weight (E, H) or NULL.  `workspace` also holds xma_rocm_gate_bwd_workspace_bytes.
+ * not used; d_gate_weight (E, H) or NULL.  `workspace` also holds xma_rocm_gate_bwd_workspace_bytes.  A bf16 / fp16 SwiGLU layer with few_dx2 = 0
+ * and no b_proj forms the router weights' gradient in dX2 instead of from expert_out, if `workspace` holds
+ * xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, I, H, E).
  */
 XMA_API int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_weight, void *stream);
 

@@ -745,6 +745,48 @@ def test_down_projection_dx_swiglu_scaled_act(dtype, case):
             assert nerr(dw[e], want_dw[e]) <= 2 * _tol(dtype), e  # two roundings (w h, then the sum) against (w dy, h)
 
 
+@pytest.mark.parametrize("scaled_act", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [*SCALED_ACT_CASES, ((40, 0, 33, 3), 4, 64, 8), ((700, 1, 257, 66), 32, 128, 264)])
+def test_router_gradient_from_dx2(dtype, case, scaled_act):
+    """d_w[t, j] = <dy[t] @ W2[e], swiglu_packed(z)> by the 256 x 256 kernels, which do not read the expert outputs, against 64 bits: fp32
+    sums of H and of I products, an activation of a few 2^-21, one rounding; the other outputs as without it"""
+    from xma.rocm import ops
+
+    counts, k, H, I = case
+    E = max(len(counts), k)
+    counts = (*counts, *[0] * (E - len(counts)))
+    counts = (counts[0] - sum(counts) % k + k, *counts[1:])
+    print(f"router gradient counts={counts} k={k} H={H} I={I} {dtype} scaled_act={scaled_act}", flush=True)
+    _, _, ss, offs = _routing_with_counts(counts, k, 21)
+    M = sum(counts)
+    g = torch.Generator().manual_seed(22)
+    new = lambda *s: torch.randn(*s, generator=g).to(dtype).cuda()
+    dy, W2, z, w, ss, offs = new(M // k, H), new(E, H, I), new(M, 2 * I), torch.rand(M, generator=g).to(dtype).cuda(), ss.cuda(), offs.cuda()
+    nan = lambda *s: torch.full(s, float("nan"), dtype=dtype, device="cuda")
+    dz, dz0, act, act0, d_w = nan(M, 2 * I), nan(M, 2 * I), nan(M, I), nan(M, I), nan(M // k, k)
+    with _few_rows_limit(0):
+        ops.down_projection_dx_swiglu_router_rocm(dy, W2, ss, offs, z, dz, act if scaled_act else None, w, nan(M, H), d_w, k)
+        if scaled_act:
+            ops.down_projection_dx_swiglu_scaled_act_rocm(dy, W2, ss, offs, z, dz0, act0, w, k)
+            assert torch.equal(act, act0)
+        else:
+            ops.down_projection_dx_swiglu_rocm(dy, W2, ss, offs, z, dz0, w, k)
+    assert torch.equal(dz, dz0)
+    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).tolist()
+    gate, up = z.double()[:, ::2], z.double()[:, 1::2]
+    h = up * gate * torch.sigmoid(gate)
+    want, size = torch.empty(M, dtype=torch.float64, device="cuda"), torch.empty(M, dtype=torch.float64, device="cuda")
+    for e in set(expert):
+        rows = torch.tensor([i for i, x in enumerate(expert) if x == e], device="cuda")
+        a, b = dy.double()[ss[rows] // k], W2[e].double()
+        want[ss[rows]] = ((a @ b) * h[rows]).sum(1)
+        size[ss[rows]] = ((a.abs() @ b.abs()) * h[rows].abs()).sum(1)
+    unit, smallest = (2.0**-8, 2.0**-133) if dtype == torch.bfloat16 else (2.0**-11, 2.0**-24)
+    bound = unit * want.abs() + ((H + I + 8) * 2.0**-24 + 2.0**-18) * size + smallest
+    assert ((d_w.view(-1).double() - want).abs() <= bound).all()
+
+
 def test_scatter2scatter_with_and_without_workspace():
     """The same launch through the C ABI with the scratch for splitting the last round of tiles along K and without
     it (every tile by one workgroup): both within tolerance of the oracle; the workspace query and its error code."""
