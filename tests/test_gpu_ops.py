@@ -219,6 +219,30 @@ def test_expert_column_sums_block_sizes(dtype, counts, N):
     assert nerr(got, want) <= _tol(dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("counts,N", [((0, 1, 255, 256, 257, 1025), 136), ((15, 17, 63, 0, 64, 65), 264), ((4,) * 511 + (40,), 256), ((5, 3), 8)])
+def test_expert_column_sums_whole_pieces(dtype, counts, N):
+    """rows of whole 16-byte pieces: grouped, further apart than they are long, and gathered and scaled; a start off 16 bytes takes the
+    other kernel.  Against 64 bits: fp32 sums of the rows and one rounding"""
+    from xma.rocm import ops
+
+    print(f"column sums of pieces E={len(counts)} N={N} {dtype}", flush=True)
+    _, _, ss, offs = _routing_with_counts(counts, 2, 3)
+    g, M = torch.Generator().manual_seed(5), sum(counts)
+    wide, scale = torch.randn(M, N + 24, generator=g).to(dtype).cuda(), torch.rand(M, generator=g).to(dtype).cuda()
+    ss, offs = ss.cuda(), offs.cuda()
+    unit, smallest = {torch.bfloat16: (2.0**-8, 0.0), torch.float16: (2.0**-11, 2.0**-24), torch.float32: (2.0**-24, 0.0)}[dtype]
+    for A in (wide[:, :N].contiguous(), wide[:, 16 : 16 + N], wide[:, 4 : 4 + N]):
+        for gathered in (False, True):
+            got = torch.full((len(counts), N), float("nan"), dtype=dtype, device="cuda")
+            src = A[: M // 2] if gathered else A
+            ops.expert_column_sums_rocm(src, ss if gathered else None, offs, got, scale if gathered else None, 2 if gathered else 1)
+            rows = src.double()[ss // 2] * scale.double()[ss][:, None] if gathered else src.double()
+            want = torch.stack([a.sum(0) for a in rows.split(counts)])
+            size = torch.stack([a.abs().sum(0) for a in rows.split(counts)])
+            assert ((got.double() - want).abs() <= unit * want.abs() + (max(counts) + 1) * 2.0**-24 * size + smallest).all()
+
+
 def _routing_with_counts(counts, k, seed):
     """a routing whose experts own exactly `counts` rows (sum divisible by k): the slots are dealt out at random"""
     g = torch.Generator().manual_seed(seed)
