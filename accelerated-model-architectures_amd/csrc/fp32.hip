@@ -9,6 +9,8 @@
 //   dW           :  Q = dY columns (out features), P = X columns (in features), K = tokens of the expert
 // The MFMA "A" operand is the P fragment, so a lane owns output row (lane & 31) of a 32 x 32 block and four
 // consecutive columns per accumulator quad.
+#include <math.h>
+
 #include "fp32.hpp"
 #include "row_dot.hpp"
 
@@ -38,6 +40,11 @@ struct TileRegs {
 
 // ---- operand tile loaders: DIM "rows" x BK k per tile, two float4 per thread
 template <int TB> __device__ __forceinline__ void load_kcontig(TileRegs &r, const float *row_ptr, int k0, int K, int tid) {
+    if (k0 + Tile<TB>::BK <= K) { // uniform: loads under a per-lane condition sit in branches of their own
+#pragma unroll
+        for (int h = 0; h < 2; ++h) r.v[h] = *(const f32x4 *)(row_ptr + k0 + Tile<TB>::kc(tid, h));
+        return;
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int k = k0 + Tile<TB>::kc(tid, h);
@@ -84,6 +91,34 @@ __device__ __forceinline__ void mma_tiles(const float *sP, const float *sQ, f32x
     }
 }
 
+// The K loop.  LDS holds two steps, so a step has one barrier: the next one's operands go into the other place in front of this one's MFMAs,
+// which cover them, and their registers are loaded again for the step after.  us, against two barriers and one place: x @ W^T of 16 experts of
+// 250 rows, K = 2048, N = 1024 208 -> 184, 8 of 1000, K = 2048, N = 512 168 -> 150 (small tile); 8 of 2000, K = 2048, N = 512, dy @ W 303 ->
+// 284 (large).
+template <int TB, typename Load, typename Store, typename Multiply>
+__device__ __forceinline__ void walk_k(int KT, Load load, Store store, Multiply multiply) {
+    constexpr int SETS = Tile<TB>::SETS;
+#pragma unroll
+    for (int s = 0; s < SETS; ++s)
+        if (s < KT) load(s, s);
+    if (KT > 0) store(0, 0);
+    if (SETS < KT) load(0, SETS);
+    __syncthreads();
+    for (int kt0 = 0; kt0 < KT; kt0 += SETS) {
+#pragma unroll
+        for (int s = 0; s < SETS; ++s) {
+            const int kt = kt0 + s;
+            if (kt >= KT) break; // uniform
+            if (kt + 1 < KT) {
+                store((s + 1) % SETS, kt + 1); // everybody has read what was there before the last barrier
+                if (kt + 1 + SETS < KT) load((s + 1) % SETS, kt + 1 + SETS);
+            }
+            multiply(kt);
+            __syncthreads();
+        }
+    }
+}
+
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
 // ------------------------------------------------------------------------------------------------ forward / dX
@@ -91,8 +126,8 @@ template <int WT, int EPI, int TB>
 __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
     typedef Tile<TB> T;
     extern __shared__ int s_pre[]; // [E + 1]
-    __shared__ __attribute__((aligned(16))) float sQ[T::BK * T::LD];
-    __shared__ __attribute__((aligned(16))) float sP[T::BK * T::LD];
+    __shared__ __attribute__((aligned(16))) float sQ[2][T::BK * T::LD];
+    __shared__ __attribute__((aligned(16))) float sP[2][T::BK * T::LD];
     __shared__ int s_sched[2];
     const float *X = (const float *)a.X, *W = (const float *)a.W, *scale = (const float *)a.scale;
     float *out = (float *)a.out, *aux = (float *)a.aux;
@@ -159,6 +194,9 @@ __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
     auto load_p = [&](TileRegs &r, int k0) {
         if (WT == 0) {
             load_kcontig<TB>(r, p_row, k0, a.K, tid);
+        } else if (k0 + T::BK <= a.K) { // uniform
+#pragma unroll
+            for (int h = 0; h < 2; ++h) r.v[h] = *(const f32x4 *)(We + (int64_t)(k0 + T::ks(tid, h)) * a.ldw + p_col);
         } else {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -189,30 +227,18 @@ __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
     }
     const int KT = (a.K + T::BK - 1) / T::BK;
     TileRegs rq[T::SETS], rp[T::SETS]; // the next SETS steps
-#pragma unroll
-    for (int s = 0; s < T::SETS; ++s) {
-        load_kcontig<TB>(rq[s], q_row, s * T::BK, a.K, tid); // zeros past K
-        load_p(rp[s], s * T::BK);
-    }
-    for (int kt0 = 0; kt0 < KT; kt0 += T::SETS) {
-#pragma unroll
-        for (int s = 0; s < T::SETS; ++s) {
-            const int kt = kt0 + s;
-            if (kt >= KT) break; // uniform
-            __syncthreads();     // the previous step's fragments have been read
-            store_kcontig<TB>(sQ, rq[s], tid);
-            if (WT == 0)
-                store_kcontig<TB>(sP, rp[s], tid);
-            else
-                store_kstrided<TB>(sP, rp[s], tid);
-            __syncthreads();
-            if (kt + T::SETS < KT) { // these loads fly while this step (and the next) multiplies
-                load_kcontig<TB>(rq[s], q_row, (kt + T::SETS) * T::BK, a.K, tid);
-                load_p(rp[s], (kt + T::SETS) * T::BK);
-            }
-            mma_tiles<TB>(sP, sQ, acc, wp, wq, lane);
-        }
-    }
+    auto load = [&](int s, int kt) {
+        load_kcontig<TB>(rq[s], q_row, kt * T::BK, a.K, tid); // zeros past K
+        load_p(rp[s], kt * T::BK);
+    };
+    auto store = [&](int s, int kt) {
+        store_kcontig<TB>(sQ[kt & 1], rq[s], tid);
+        if (WT == 0)
+            store_kcontig<TB>(sP[kt & 1], rp[s], tid);
+        else
+            store_kstrided<TB>(sP[kt & 1], rp[s], tid);
+    };
+    walk_k<TB>(KT, load, store, [&](int kt) { mma_tiles<TB>(sP[kt & 1], sQ[kt & 1], acc, wp, wq, lane); });
 
     // epilogue: lane owns row (lane & 31) of each 32-row block, 4 consecutive columns per quad
     const int lrow = lane & 31, lhalf = lane >> 5;
@@ -262,8 +288,8 @@ __global__ __launch_bounds__(FTHREADS) void gemm_f32_kernel(const FwdArgs a) {
 // ------------------------------------------------------------------------------------------------ dW
 template <int TB> __global__ __launch_bounds__(FTHREADS) void dw_f32_kernel(const DwArgs a) {
     typedef Tile<TB> T;
-    __shared__ __attribute__((aligned(16))) float sQ[T::BK * T::LD];
-    __shared__ __attribute__((aligned(16))) float sP[T::BK * T::LD];
+    __shared__ __attribute__((aligned(16))) float sQ[2][T::BK * T::LD];
+    __shared__ __attribute__((aligned(16))) float sP[2][T::BK * T::LD];
     const float *DY = (const float *)a.DY, *X = (const float *)a.X, *scale = (const float *)a.scale;
     float *DW = (float *)a.DW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -277,46 +303,49 @@ template <int TB> __global__ __launch_bounds__(FTHREADS) void dw_f32_kernel(cons
     if (q_col >= a.N_out) q_col = a.N_out - 4; // masked at the store
     if (p_col >= a.K_in) p_col = a.K_in - 4;
 
-    // k-rows are tokens of the expert: a thread takes two rows of a step, through the index if the
-    // operand is in scattered order; dY may carry a per-token scale
-    auto load_tiles = [&](TileRegs &rq, TileRegs &rp, int k0) {
+    // k-rows are tokens of the expert: a thread takes two rows of a step, through the index if the operand is in scattered order; dY may
+    // carry a per-token scale.  The indices of a step are fetched with the operands of the one before it in the same registers, so that
+    // no load waits for another in front of the MFMAs.
+    const bool gathers = !a.dy_grouped || !a.x_grouped || scale;
+    TileRegs rq[T::SETS], rp[T::SETS];
+    uint32_t idx[T::SETS][2];
+    float scales[T::SETS][2];
+    auto load_idx = [&](int s, int kt) {
+        if (!gathers) return; // uniform
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int k = k0 + T::ks(tid, h);
-            rq.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-            rp.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (k < rows) {
-                const int64_t n = row_lo + k;
-                int64_t sidx = 0;
-                if (!a.dy_grouped || !a.x_grouped || scale) sidx = a.idx[n];
-                const int64_t dsrc = a.dy_grouped ? n : (int64_t)fastdiv((uint32_t)sidx, a.dy_div);
-                const int64_t xsrc = a.x_grouped ? n : (int64_t)fastdiv((uint32_t)sidx, a.x_div);
-                rq.v[h] = *(const f32x4 *)(DY + dsrc * a.lddy + q_col);
-                if (scale) rq.v[h] *= scale[sidx];
-                rp.v[h] = *(const f32x4 *)(X + xsrc * a.ldx + p_col);
-            }
+            const int k = kt * T::BK + T::ks(tid, h);
+            idx[s][h] = (uint32_t)a.idx[row_lo + (k < rows ? k : rows - 1)];
         }
+    };
+    auto load = [&](int s, int kt) {
+        if (kt == s) load_idx(s, kt); // of the first step in these registers; uniform
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = kt * T::BK + T::ks(tid, h), at = k < rows ? k : rows - 1; // past the last row: zeros, below
+            const int64_t n = row_lo + at;
+            const int64_t dsrc = a.dy_grouped ? n : (int64_t)fastdiv(idx[s][h], a.dy_div);
+            const int64_t xsrc = a.x_grouped ? n : (int64_t)fastdiv(idx[s][h], a.x_div);
+            rq[s].v[h] = *(const f32x4 *)(DY + dsrc * a.lddy + q_col);
+            rp[s].v[h] = *(const f32x4 *)(X + xsrc * a.ldx + p_col);
+            if (scale) scales[s][h] = scale[idx[s][h]];
+        }
+        if (kt + T::SETS < KT) load_idx(s, kt + T::SETS);
+    };
+    auto store = [&](int s, int kt) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (scale) rq[s].v[h] *= scales[s][h];
+            if (kt * T::BK + T::BK > rows && kt * T::BK + T::ks(tid, h) >= rows) rq[s].v[h] = rp[s].v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        store_kstrided<TB>(sQ[kt & 1], rq[s], tid);
+        store_kstrided<TB>(sP[kt & 1], rp[s], tid);
     };
 
     f32x16 acc[TB][TB];
     zero_acc<TB>(acc);
     const int wq = (wave & 1) * 32 * TB, wp = (wave >> 1) * 32 * TB;
-    TileRegs rq[T::SETS], rp[T::SETS];
-#pragma unroll
-    for (int s = 0; s < T::SETS; ++s) load_tiles(rq[s], rp[s], s * T::BK); // zeros past the expert's rows
-    for (int kt0 = 0; kt0 < KT; kt0 += T::SETS) {
-#pragma unroll
-        for (int s = 0; s < T::SETS; ++s) {
-            const int kt = kt0 + s;
-            if (kt >= KT) break; // uniform
-            __syncthreads();
-            store_kstrided<TB>(sQ, rq[s], tid);
-            store_kstrided<TB>(sP, rp[s], tid);
-            __syncthreads();
-            if (kt + T::SETS < KT) load_tiles(rq[s], rp[s], (kt + T::SETS) * T::BK);
-            mma_tiles<TB>(sP, sQ, acc, wp, wq, lane);
-        }
-    }
+    walk_k<TB>(KT, load, store, [&](int kt) { mma_tiles<TB>(sP[kt & 1], sQ[kt & 1], acc, wp, wq, lane); });
     // every element of DW[e] is written, zeros for an expert without tokens
     const int lrow = lane & 31, lhalf = lane >> 5;
     float *DWe = DW + (int64_t)e * a.dw_es;
@@ -422,22 +451,34 @@ template <int WT, int TB> int launch_gemm(const FwdArgs &a, int epi, int grid, s
     return xma_check_launch("gemm_f32_kernel");
 }
 
-// Which tile: a launch is bound by the matrix pipes of the compute units that have a tile.  The small one pays where the large
-// one is mostly padding, up to 64 rows per expert on average, and where the large ones leave compute units idle, below two
-// per unit.  Results are bit-identical.  Measured, large / small tile in us (x @ W^T; dy @ W).  Padding: 64 experts of
-// K = 1024, N = 2048, 30 rows each 302 / 184; 285 / 178, 64 rows 287 / 188; 288 / 186, 70 rows 292 / 291; 288 / 288.  Tiles:
-// 128 of them 45 / 30; 45 / 28, 256 48 / 49; 47 / 46, 384 78 / 69; 80 / 69, 512 80 / 85; 81 / 85 (K = 512) and 163 / 184;
-// 157 / 179 (64 experts of 128 rows, K = 1024), 1024 156 / 170; 150 / 164, 2048 297 / 322; 290 / 322.
-constexpr int64_t F32_SMALL_ROWS = 64, F32_SMALL_TILES = 512;
-// dW: the reduction is the expert's rows.  64 large tiles 476 / 194, 256 125 / 97, 384 655 / 553, 2560 72 / 80, 4096 1150 / 1378.
+// Which tile.  The small one pays where the large ones leave compute units idle, below two per unit, and where they are padding by more
+// than the small one's extra traffic through LDS is worth: an expert of random load ends in half a tile on average, of 128 rows or of 64.
+// Results are bit-identical.  Large / small tile in us (x @ W^T; dy @ W).  Rows: 64 experts of K = 1024, N = 2048, 30 rows each 287 / 162;
+// 286 / 166, 90 rows (one large tile or two) 303 / 325; 296 / 339; 128 of K = 576, N = 512, 125 rows 128 / 114; 127 / 116, 250 rows 212 /
+// 199; 207 / 202, 500 rows 379 / 378; 367 / 372, 1000 rows 689 / 706; 677 / 710; 30 of K = 400, N = 1200, 300 rows 122 / 99; 121 / 102; 16 of
+// K = 1024, N = 4096, 250 rows 352 / 326; 350 / 340.  Tiles: 8 experts of K = 2048, N = 512, 256 tiles 168 / 150; 174 / 155, 512 of them 293 /
+// 295; 284 / 299, of K = 512, N = 2048, 4096 tiles 563 / 602; 558 / 622.
+constexpr int64_t F32_SMALL_TILES = 512;
+constexpr double F32_SMALL_WORSE = 1.04;
+// dW: the reduction is the expert's rows.  8 experts of 500 rows, 256 tiles 62 / 52, 512 tiles 96 / 109; 1000 x 2048 x 2048 4 experts 309 / 343;
+// 128 of 576 x 512, 500 rows 413 / 427; padded by a fifth, 30 of 1200 x 400, 300 rows 141 / 116, 700 rows 285 / 251.
 constexpr int F32_SMALL_TILES_DW = 512;
+constexpr double F32_SMALL_WORSE_DW = 1.12;
 inline int64_t f32_tiles(int64_t m, int64_t n, int dim) { return ((m + dim - 1) / dim) * ((n + dim - 1) / dim); }
+inline double f32_padded(int64_t n, int dim) { return (double)((n + dim - 1) / dim * dim); }
+// rows that tiles of `dim` multiply for an expert of about `rows` (within two standard deviations of a random load)
+inline double f32_padded_load(double rows, int dim) {
+    const double lo = ceil((rows - 2 * sqrt(rows)) / dim), hi = ceil((rows + 2 * sqrt(rows)) / dim);
+    return dim * (lo == hi ? hi : rows / dim + 0.5);
+}
 
 } // namespace
 
 int f32_scatter2scatter(const FwdArgs &a, int w_is_kn, int epilogue, hipStream_t st) {
     const int64_t rows = (a.M + a.E - 1) / a.E; // of an expert, on average
-    const bool small = rows <= F32_SMALL_ROWS || a.E * f32_tiles(rows, a.N, 128) < F32_SMALL_TILES;
+    const double load = (double)a.M / a.E;
+    const bool small = a.E * f32_tiles(rows, a.N, 128) < F32_SMALL_TILES ||
+                       F32_SMALL_WORSE * f32_padded_load(load, 64) * f32_padded(a.N, 64) < f32_padded_load(load, 128) * f32_padded(a.N, 128);
     const int dim = small ? 64 : 128;
     const int64_t grid = (a.M / dim + a.E) * ((a.N + dim - 1) / dim); // sum_e ceil(c_e / dim) <= floor(M / dim) + E
     XMA_REQUIRE(grid < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "scatter2scatter (fp32): grid too large");
@@ -448,7 +489,8 @@ int f32_scatter2scatter(const FwdArgs &a, int w_is_kn, int epilogue, hipStream_t
 }
 
 int f32_group_bwd_W(const DwArgs &a, hipStream_t st) {
-    const bool small = a.E * f32_tiles(a.N_out, a.K_in, 128) < F32_SMALL_TILES_DW;
+    const bool small = a.E * f32_tiles(a.N_out, a.K_in, 128) < F32_SMALL_TILES_DW ||
+                       F32_SMALL_WORSE_DW * f32_padded(a.N_out, 64) * f32_padded(a.K_in, 64) < f32_padded(a.N_out, 128) * f32_padded(a.K_in, 128);
     const int64_t grid = a.E * f32_tiles(a.N_out, a.K_in, small ? 64 : 128);
     XMA_REQUIRE(grid < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "group_bwd_W (fp32): grid too large");
     if (small)

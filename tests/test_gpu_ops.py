@@ -243,6 +243,45 @@ def test_expert_column_sums_whole_pieces(dtype, counts, N):
             assert ((got.double() - want).abs() <= unit * want.abs() + (max(counts) + 1) * 2.0**-24 * size + smallest).all()
 
 
+@pytest.mark.parametrize("E,N", [(3, 72), (64, 1024)])  # small and large tiles
+@pytest.mark.parametrize("K", [8, 16, 24, 32, 40, 72, 136])
+def test_fp32_k_steps(E, N, K):
+    """fp32 GEMMs whose K, and for dW whose rows per expert (none, one, around the steps of 16 and 32), make none to several K steps with and
+    without a remainder, rows gathered and grouped: against 64 bits, fp32 sums of K (rows) products"""
+    from xma.rocm import ops
+
+    print(f"fp32 K steps E={E} N={N} K={K}", flush=True)
+    edges = (0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 97)
+    counts = [90 + (i % 5) for i in range(E)] if E == 64 else [33, 0, 65]
+    if E == 64:
+        counts[: len(edges)] = edges
+        counts[20] += 90 * 64 - sum(counts)
+    counts[-1] += sum(counts) % 2
+    _, _, ss, offs = _routing_with_counts(tuple(counts), 2, 7)
+    g, M = torch.Generator().manual_seed(9), sum(counts)
+    X, Xt, DY, W, w = (torch.randn(*n, generator=g).cuda() for n in ((M, K), (M // 2, K), (M, N), (E, N, K), (M,)))
+    ss, offs, nan = ss.cuda(), offs.cuda(), lambda *n: torch.full(n, float("nan"), device="cuda")
+    starts = [0, *offs.tolist()]
+    for gathered in (False, True):
+        rows = Xt.double()[ss // 2] if gathered else X.double()
+        src, fan = (Xt, 2) if gathered else (X, 1)
+        for weight in (W.permute(0, 2, 1), W.permute(0, 2, 1).contiguous()):
+            out, want, size = nan(M, N), torch.empty(M, N, dtype=torch.float64, device="cuda"), torch.empty(M, N, dtype=torch.float64, device="cuda")
+            ops.scatter2scatter_rocm(src, weight, ss, offs, out, None, fan, not gathered, True)
+            for e in range(E):
+                part = slice(starts[e], starts[e + 1])
+                want[part], size[part] = rows[part] @ W[e].double().t(), rows[part].abs() @ W[e].double().t().abs()
+            assert ((out.double() - want).abs() <= (K + 1) * 2.0**-24 * size).all()
+        for scale in (None, w):
+            dw = nan(E, N, K)
+            ops.group_bwd_W_rocm(DY, src, ss, offs, dw.permute(0, 2, 1), scale, 0, fan if gathered else 0)
+            dy = DY.double() if scale is None else (DY * w[ss][:, None]).double()  # rounded to fp32, as the loader does
+            for e in range(E):
+                part = slice(starts[e], starts[e + 1])
+                want, size = dy[part].t() @ rows[part], dy[part].t().abs() @ rows[part].abs()
+                assert ((dw[e].double() - want).abs() <= (counts[e] + 1) * 2.0**-24 * size).all(), e
+
+
 def _routing_with_counts(counts, k, seed):
     """a routing whose experts own exactly `counts` rows (sum divisible by k): the slots are dealt out at random"""
     g = torch.Generator().manual_seed(seed)
