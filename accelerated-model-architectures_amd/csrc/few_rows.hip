@@ -761,8 +761,8 @@ constexpr int FR_DEEP_K = 2048; // K ranges and their epilogue lead beyond (8 ex
 // W[e] as (N, K): at most as many workgroups with work as run at the same time, counting the experts that M random choices of E hit.
 // 128 experts of H = 576, I = 256, 12 tokens, up-projection in four workgroups for each of 68 experts: 17.8 us against 12.9 with the small tile.
 inline int fr_deep_stages(int K) { const int steps = (K + ST_K_NT - 1) / ST_K_NT; return steps < FD_STAGES ? steps : FD_STAGES; }
-inline bool fr_deep_shape(int64_t M, int N, int K, int E, int w_is_kn) {
-    if (w_is_kn || K > FR_DEEP_K) return false;
+inline bool fr_deep_shape(int64_t M, int N, int K, int E, int w_is_kn, int epilogue) {
+    if (w_is_kn || K > FR_DEEP_K || epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == EPI_GELU_BWD) return false; // those have no such kernel
     const double experts = E * (1. - pow(1. - 1. / E, (double)M));
     return experts * ((N + ST_N - 1) / ST_N) <= 256 * (FD_STAGES / fr_deep_stages(K));
 }
@@ -770,8 +770,9 @@ inline bool fr_deep_shape(int64_t M, int N, int K, int E, int w_is_kn) {
 // W[e] as (K, N), more than a pass or two of the vector kernel per expert, or rows of W shorter than the 4 KB a wave of
 // the vector kernel takes at a time -> the small MFMA tile (128 experts of H = 576, I = 256, 7 tokens: forward 0.036
 // instead of 0.045 ms with it; 8 experts of H = 2048, I = 8192: 0.161 instead of 0.155)
-inline bool fr_takes_tile(int64_t M, int N, int K, int E, int w_is_kn) {
-    return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE || fr_deep_shape(M, N, K, E, w_is_kn);
+inline bool fr_takes_tile(int64_t M, int N, int K, int E, int w_is_kn, int epilogue) {
+    return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE ||
+           fr_deep_shape(M, N, K, E, w_is_kn, epilogue);
 }
 
 // More rows than the small tile takes in one pass go to the 128 x 256 tiles of mid_rows.hip, where those have the variant.  8
@@ -802,7 +803,7 @@ template <typename T, int EPI> int fr_launch_epilogue(const FwdArgs &a, const fl
 template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, float *part, hipStream_t st) {
     if constexpr (WT == 0 && (EPI == XMA_ROCM_EPI_STORE || EPI == XMA_ROCM_EPI_SWIGLU || EPI == EPI_GELU)) {
         const int64_t x_rows = a.x_grouped ? a.M : (a.M + a.fan_out - 1) / a.fan_out; // 32-bit byte offsets from its first row
-        if (fr_deep_shape(a.M, a.N, a.K, a.E, WT) && x_rows * a.ldx * 2 < ((int64_t)1 << 31)) {
+        if (fr_deep_shape(a.M, a.N, a.K, a.E, WT, EPI) && x_rows * a.ldx * 2 < ((int64_t)1 << 31)) {
             auto run = [&](auto kernel, int waves) {
                 if (int rc = xma_set_max_lds_once((const void *)kernel, FD_STAGES * fd_stage(waves))) return rc;
                 const dim3 grid((a.N + 32 * waves - 1) / (32 * waves), (unsigned)(a.M < a.E ? a.M : a.E));
@@ -830,7 +831,7 @@ template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, floa
 
 template <typename T, int EPI> int fr_launch_epi(const FwdArgs &a, int w_is_kn, float *part, hipStream_t st) {
     int rc;
-    if (fr_takes_tile(a.M, a.N, a.K, a.E, w_is_kn)) return w_is_kn ? fr_launch_tile<T, 1, EPI>(a, part, st) : fr_launch_tile<T, 0, EPI>(a, part, st);
+    if (fr_takes_tile(a.M, a.N, a.K, a.E, w_is_kn, EPI)) return w_is_kn ? fr_launch_tile<T, 1, EPI>(a, part, st) : fr_launch_tile<T, 0, EPI>(a, part, st);
     // one pair of rows per wave instead of four where the rows are short or the launch would have few workgroups
     const int rows_per_wg = (a.K >= 2048 && (int64_t)(a.N / FR_NT_ROWS) * a.E >= 2048) ? FR_NT_ROWS : 8;
     const dim3 grid((a.N + rows_per_wg - 1) / rows_per_wg, a.E);
@@ -874,8 +875,8 @@ int few_epilogue(int epilogue) { // both forms of GELU run through the same kern
 
 size_t few_workspace_bytes(int64_t M, int32_t N, int32_t K, int32_t E, int w_is_kn, int epilogue) { // of the kernels here
     int S;
-    if (fr_takes_tile(M, N, K, E, w_is_kn)) { // the small MFMA tile, cut along K or not
-        if (fr_deep_shape(M, N, K, E, w_is_kn)) return 0;
+    if (fr_takes_tile(M, N, K, E, w_is_kn, epilogue)) { // the small MFMA tile, cut along K or not
+        if (fr_deep_shape(M, N, K, E, w_is_kn, epilogue)) return 0;
         S = fr_tile_splits(N, K, E, w_is_kn);
         if (S == 1) return 0;
     } else if (epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == EPI_GELU_BWD) {
