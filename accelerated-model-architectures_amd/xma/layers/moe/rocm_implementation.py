@@ -510,7 +510,7 @@ def _plan(T: int, H: int, I: int, E: int, k: int, dtype: torch.dtype, act: str, 
     # the scattered rows of dX1 take the place of dW2's operand
     gate_sums = get_library().xma_rocm_gate_bwd_workspace_bytes(T, H, E) if ops.gate_bwd_supported(H, E, k, dtype) else 0
     # dX2 by the 256 x 256 kernels leaves the router weights' gradient behind its K slices
-    dots = ops.router_gradient_workspace_bytes(M, I, H, E, device_index) if glu and not b_proj and ops.dx2_leaves_router_gradient(dx2[0], M, I, k, dtype) else 0
+    dots = ops.router_gradient_workspace_bytes(M, I, dx2[1]) if glu and not b_proj and ops.dx2_leaves_router_gradient(dx2[0], M, I, k, dtype) else 0
     back = dict(d_weights=M * s, dz=M * U * s, scattered=max(M * H * s, dw2_operand), workspace=max(down[1], dx2[1], dx1[1], gate_sums, dots, 256))
     if not save:
         back |= dict(h=M * I * s, out=M * H * s)

@@ -416,11 +416,10 @@ def down_projection_dx_swiglu_scaled_act_rocm(
     )
 
 
-@lru_cache(maxsize=4096)
-def router_gradient_workspace_bytes(M: int, N: int, K: int, E: int, device_index: int) -> int:
-    """scratch of dX2 by the 256 x 256 kernels with the router weights' gradient; depends on the shape and the device only"""
-    with torch.cuda.device(device_index):
-        return get_library().xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, N, K, E)
+def router_gradient_workspace_bytes(M: int, N: int, slices: int) -> int:
+    """scratch of dX2 by the 256 x 256 kernels with the router weights' gradient (slices: what the launch asks for without it); restates
+    xma_rocm_down_projection_dx_swiglu_router_workspace_bytes"""
+    return -(-slices // 256) * 256 + M * -(-N // 128) * 4
 
 
 def dx2_leaves_router_gradient(few: int, M: int, N: int, k: int, dtype: torch.dtype) -> bool:
@@ -461,7 +460,7 @@ def down_projection_dx_swiglu_router_rocm(
     assert W.dtype == dY.dtype == z.dtype == dz.dtype == row_scale.dtype == d_row_scale.dtype and row_scale.is_contiguous() and d_row_scale.is_contiguous()
     assert sorted_scattered_idxs.dtype == torch.int64 and sorted_scattered_idxs.is_contiguous()
     assert expert_offsets.dtype == torch.int64 and expert_offsets.is_contiguous() and expert_offsets.numel() == E
-    ws_bytes = router_gradient_workspace_bytes(M, N, K, E, dY.device.index or 0)
+    ws_bytes = router_gradient_workspace_bytes(M, N, scatter2scatter_workspace_bytes(M, N, K, E, dY.device.index or 0))
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dY.device)
     check(
         get_library().xma_rocm_down_projection_dx_swiglu_router(
