@@ -981,7 +981,9 @@ extern "C" int xma_rocm_scatter2scatter_few_rows(const void *X, int64_t ldx, con
     hipStream_t st = (hipStream_t)stream;
     w_is_kn = w_is_kn ? 1 : 0;
     if (fr_takes_mid(a, w_is_kn, epilogue)) return xma_rocm::mid_fwd(a, w_is_kn, epilogue, dtype, (float *)workspace, st);
-    float *part = workspace && al16(workspace) && workspace_bytes >= few_workspace_bytes(M, N, K, E, w_is_kn, epilogue) ? (float *)workspace : nullptr;
+    // nullptr where nothing was asked for: a launch whose X only the small tile reaches, in a shape that fr_deep_kernel takes uncut, is uncut too
+    const size_t sums = few_workspace_bytes(M, N, K, E, w_is_kn, epilogue);
+    float *part = sums && workspace && al16(workspace) && workspace_bytes >= sums ? (float *)workspace : nullptr;
     if (dtype == XMA_ROCM_BF16) return fr_launch<__bf16>(a, w_is_kn, epilogue, part, st);
     return fr_launch<_Float16>(a, w_is_kn, epilogue, part, st);
 }

@@ -1019,3 +1019,26 @@ def test_forward_gemm_of_few_workgroups(dtype, counts, K, N):
     gate, up = z.double()[:, ::2], z.double()[:, 1::2]
     want = up * gate * torch.sigmoid(gate)
     assert ((h.double() - want).abs() <= (unit + 2.0**-20) * want.abs() + 2.0**-24).all()
+
+
+def test_few_rows_beyond_32_bit_offsets_leaves_the_workspace_alone():
+    """rows of X that only the small tile's 64-bit addresses reach, in a shape whose usual kernel asks for no workspace: a workspace of
+    another purpose stays as it is (the small tile would cut this K in two ranges and leave their sums there)"""
+    from xma.rocm.loader import get_library
+
+    lib, (M, N, K, E), ldx = get_library(), (5, 512, 1024, 4), 1 << 28
+    assert lib.xma_rocm_scatter2scatter_few_rows_workspace_bytes(M, N, K, E, 0, 0) == 0
+    print("few rows, X beyond 2 GiB", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    X = torch.empty((M - 1) * ldx + K, dtype=torch.bfloat16, device="cuda").as_strided((M, K), (ldx, 1))
+    X.copy_(torch.randn(M, K, device="cuda", generator=g))
+    W = torch.randn(E, N, K, device="cuda", generator=g).bfloat16()
+    counts, out = torch.tensor([2, 0, 2, 1]), torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    offs, space = counts.cumsum(0).cuda(), torch.full((1 << 20,), 171, dtype=torch.uint8, device="cuda")
+    rc = lib.xma_rocm_scatter2scatter_few_rows(
+        X.data_ptr(), ldx, W.data_ptr(), N * K, K, 0, None, offs.data_ptr(), out.data_ptr(), N, None, 0, None, 0, None, None, 0, M, N, K, E, 1, 1, 1,
+        0, 0, space.data_ptr(), 16, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and (space == 171).all()
+    w = W[torch.repeat_interleave(torch.arange(E), counts).cuda()].double()
+    want, size = (w * X.double()[:, None]).sum(2), (w.abs() * X.double().abs()[:, None]).sum(2)
+    assert ((out.double() - want).abs() <= 2.0**-8 * want.abs() + (K + 1) * 2.0**-24 * size).all()  # fp32 sums of K products, one rounding
