@@ -119,7 +119,7 @@ class _RouterGateTopK(torch.autograd.Function):
             if d_logits_out is None and _gate_bwd(x, gate_weight.size(0), ids.size(1)):
                 need_x, need_gate = ctx.needs_input_grad[:2]
                 d_x = torch.empty(x.shape, dtype=x.dtype, device=x.device) if need_x else None
-                d_w = torch.empty_like(gate_weight) if need_gate else None
+                d_w = torch.empty_like(gate_weight, memory_format=torch.contiguous_format) if need_gate else None
                 if need_x or need_gate:
                     ops.gate_bwd_rocm(x, gate_weight, d_logits.gather(1, ids.long()), ids.int(), d_x, d_w)
                 return d_x, d_w, None

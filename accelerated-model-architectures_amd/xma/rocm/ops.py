@@ -720,15 +720,16 @@ def gate_bwd_rocm(x: torch.Tensor, gate_weight: torch.Tensor, d_selected: torch.
     T, H = x.shape
     E, k = gate_weight.size(0), ids.size(1)
     assert gate_weight.shape == (E, H) and ids.shape == (T, k) and ids.dtype == torch.int32 and d_selected.shape == (T, k)
-    assert x.dtype == gate_weight.dtype == d_selected.dtype and ids.is_contiguous() and d_selected.is_contiguous() and gate_weight.is_contiguous()
+    assert x.dtype == gate_weight.dtype == d_selected.dtype and ids.is_contiguous() and d_selected.is_contiguous()
     assert d_x is None or (d_x.shape == (T, H) and d_x.is_contiguous() and d_x.dtype == x.dtype)
     assert d_gate_weight is None or (d_gate_weight.shape == (E, H) and d_gate_weight.is_contiguous() and d_gate_weight.dtype == x.dtype)
     lib = get_library()
-    # 16-byte pieces: what starts off such a boundary, or has rows that do, is copied
-    if x.data_ptr() % 16 or x.stride(0) * x.element_size() % 16:
+    # 16-byte pieces of rows behind one another: what starts off such a boundary, has rows that do, rows that overlap (an expanded one) or
+    # columns that are apart is copied
+    if x.data_ptr() % 16 or x.stride(0) * x.element_size() % 16 or x.stride(1) != 1 or x.stride(0) < H:
         x = x.clone(memory_format=torch.contiguous_format)
-    if gate_weight.data_ptr() % 16:
-        gate_weight = gate_weight.clone()
+    if gate_weight.data_ptr() % 16 or not gate_weight.is_contiguous():
+        gate_weight = gate_weight.clone(memory_format=torch.contiguous_format)
     ws_bytes = lib.xma_rocm_gate_bwd_workspace_bytes(T, H, E) if d_gate_weight is not None else 0
     workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
     check(

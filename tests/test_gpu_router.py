@@ -301,3 +301,60 @@ def test_gate_backward_from_the_selected_logits(dtype, T, H, E, k):
     for got, a, b, terms in ((d_x, d_logits, gate.double(), k), (d_gate, d_logits.t().contiguous(), x.double(), T)):
         bound = unit * (a @ b).abs() + (terms + 1) * 2.0**-24 * (a.abs() @ b.abs()) + smallest
         assert ((got.double() - a @ b).abs() <= bound).all()
+
+
+_T, _H, _E, _K = 40, 64, 8, 2
+LAYOUTS = {  # of x: what torch's own product takes
+    "one row expanded": lambda new: new(1, _H).expand(_T, _H),
+    "overlapping rows": lambda new: new(_T * 16 + _H).as_strided((_T, _H), (16, 1)),
+    "columns apart": lambda new: new(_T, _H, 2)[..., 0],
+    "rows off 16 bytes": lambda new: new(_T, _H + 1)[:, :_H],
+    "one row without a stride": lambda new: new(_H).as_strided((1, _H), (0, 1)),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_gate_backward_of_any_layout(dtype, layout):
+    """x and the gate's weight in other layouts, as a saved-tensor hook may hand them back: bit for bit what copies without gaps give"""
+    from xma.rocm import ops
+
+    g = torch.Generator(device="cuda").manual_seed(4)
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    x, gate = LAYOUTS[layout](new), new(_E, _H, 2)[..., 1]
+    T = x.size(0)
+    ids = torch.rand(T, _E, device="cuda", generator=g).argsort(1)[:, :_K].int().contiguous()
+    d_sel, got = new(T, _K), []
+    for a, b in ((x, gate), (x.contiguous(), gate.contiguous())):
+        d_x, d_gate = (torch.full(s, float("nan"), device="cuda", dtype=dtype) for s in ((T, _H), (_E, _H)))
+        ops.gate_bwd_rocm(a, b, d_sel, ids, d_x, d_gate)
+        got.append((d_x, d_gate))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_fp32_gate_of_any_layout(layout):
+    """the routing part of an fp32 layer, which computes gate(x) itself, takes the x that gate(x) takes: forward, and the gradients against
+    the products in 64 bits (d_logits to a few units of fp32, sums of k and T products)"""
+    from xma.functional import swiglu_packed
+    from xma.layers import MoE
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    moe = MoE(_E, _K, _H, 32, swiglu_packed, True, add_bias=False, std=0.3).cuda()
+    x = LAYOUTS[layout](new).detach().requires_grad_()
+    if layout == "columns apart":  # reaches the backward through a hook only
+        x = x.detach().contiguous().requires_grad_()
+        apart = lambda t: t if t.shape[-1] != _H else t.new_empty(*t.shape, 2)[..., 0].copy_(t)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, apart):
+            logits, w, ids = moe._compute_routing_weights(x)
+    else:
+        logits, w, ids = moe._compute_routing_weights(x)
+    dw = new(x.size(0), _K)
+    got = torch.autograd.grad(w, [x, moe.gate.weight], dw)
+    w, dw = w.double(), dw.double()
+    d = torch.zeros(x.size(0), _E, device="cuda", dtype=torch.float64).scatter_(1, ids.long(), w * (dw - (w * dw).sum(1, keepdim=True)))
+    err = torch.zeros_like(d).scatter_(1, ids.long(), w * (dw.abs() + (w * dw).abs().sum(1, keepdim=True)) * 8 * 2.0**-24)
+    for a, p, q, e, terms in zip(got, (d, d.t()), (moe.gate.weight.double(), x.double()), (err, err.t()), (_K, x.size(0))):
+        bound = (p.abs() @ q.abs()) * (terms + 1) * 2.0**-24 + e @ q.abs()
+        assert ((a.double() - p @ q).abs() <= bound).all()
