@@ -1042,3 +1042,24 @@ def test_few_rows_beyond_32_bit_offsets_leaves_the_workspace_alone():
     w = W[torch.repeat_interleave(torch.arange(E), counts).cuda()].double()
     want, size = (w * X.double()[:, None]).sum(2), (w.abs() * X.double().abs()[:, None]).sum(2)
     assert ((out.double() - want).abs() <= 2.0**-8 * want.abs() + (K + 1) * 2.0**-24 * size).all()  # fp32 sums of K products, one rounding
+
+
+@pytest.mark.parametrize("rows,N", [(1, 8), (800, 128)])  # small and large tiles
+@pytest.mark.parametrize("E", [7677, 7678, 8192])  # around the table's size from which a workgroup asks for more than 64 KB of LDS; the most
+def test_fp32_gemm_of_many_experts(E, rows, N):
+    """both orders of the weights, as many experts as the fp32 kernels take; every 97th expert and the last against 64 bits"""
+    from xma.rocm import ops
+
+    print(f"fp32 E={E} rows={rows} N={N}", flush=True)
+    K, M = 8, E * rows
+    g = torch.Generator(device="cuda").manual_seed(E)
+    X, W = torch.randn(M, K, device="cuda", generator=g), torch.randn(E, N, K, device="cuda", generator=g)
+    offs = torch.arange(1, E + 1, device="cuda") * rows
+    idx = torch.arange(M, device="cuda")
+    for weight in (W.permute(0, 2, 1), W.permute(0, 2, 1).contiguous()):
+        out = torch.full((M, N), float("nan"), device="cuda")
+        ops.scatter2scatter_rocm(X, weight, idx, offs, out, None, 1, True, True)
+        assert torch.isfinite(out).all()
+        for e in [*range(0, E, 97), E - 1]:
+            x, w = X[e * rows : (e + 1) * rows].double(), W[e].double().t()
+            assert ((out[e * rows : (e + 1) * rows].double() - x @ w).abs() <= (K + 1) * 2.0**-24 * (x.abs() @ w.abs())).all(), e
