@@ -1803,8 +1803,8 @@ extern "C" int xma_rocm_down_projection_dx_swiglu_router(const void *dY, int64_t
                                                          const void *row_scale, void *d_row_scale, int64_t M, int32_t N, int32_t K,
                                                          int32_t E, int32_t fan_out, int dtype, void *workspace,
                                                          size_t workspace_bytes, void *stream) {
-    XMA_REQUIRE(fan_out >= 1 && fan_out <= 32 && fan_out <= E && M >= 0 && M % fan_out == 0 && (M == 0 || d_row_scale), XMA_ROCM_EINVAL,
-                "down_projection_dx_swiglu_router: fan_out=%d E=%d M=%lld (at most 32 of the experts, M a multiple), d_row_scale is required", fan_out, E, (long long)M);
+    XMA_REQUIRE(fan_out >= 1 && fan_out <= 32 && M >= 0 && M % fan_out == 0 && (M == 0 || d_row_scale), XMA_ROCM_EINVAL,
+                "down_projection_dx_swiglu_router: fan_out=%d M=%lld (at most 32, M a multiple), d_row_scale is required", fan_out, (long long)M);
     const size_t need = xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, N, K, E);
     XMA_REQUIRE(M == 0 || (workspace && aligned16(workspace) && workspace_bytes >= need), XMA_ROCM_EWORKSPACE,
                 "down_projection_dx_swiglu_router: workspace of %zu bytes, %zu needed (16-byte aligned)", workspace_bytes, need);

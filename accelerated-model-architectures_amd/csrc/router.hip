@@ -996,8 +996,9 @@ int xma_combine_router_bwd(const void *expert_out, const void *dy, const void *l
 int xma_dots_router_bwd(const float *dots, int64_t parts, const void *logits, const int32_t *ids, int64_t T, int32_t E, int32_t k, int dtype,
                         void *d_sel, hipStream_t st) {
     RouterShape s;
-    if (int rc = router_shape("dots_router_bwd", T, E, k, dtype, s)) return rc;
-    XMA_REQUIRE(parts >= 1 && k <= 64 && (dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16) && (T == 0 || (dots && (ids || !logits) && d_sel)),
+    if (logits) // the sums alone know no experts
+        if (int rc = router_shape("dots_router_bwd", T, E, k, dtype, s)) return rc;
+    XMA_REQUIRE(parts >= 1 && k >= 1 && k <= 64 && (dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16) && (T == 0 || (dots && (ids || !logits) && d_sel)),
                 XMA_ROCM_EINVAL, "dots_router_bwd: parts=%lld k=%d dtype=%d or a null pointer", (long long)parts, k, dtype);
     if (T == 0) return XMA_ROCM_OK;
     int lanes = 64;

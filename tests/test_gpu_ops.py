@@ -850,6 +850,28 @@ def test_router_gradient_from_dx2(dtype, case, scaled_act):
     assert ((d_w.view(-1).double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("E,k,M,H,I", [(2, 5, 600, 64, 136), (4096, 2, 20000, 64, 16)])  # more slots than experts; more experts than route counts
+def test_router_gradient_knows_no_number_of_experts(E, k, M, H, I):
+    """the ids of a caller's own, in the same bounds as above; the pass over the expert outputs that it replaces takes them as well"""
+    from xma.rocm import ops
+
+    print(f"router gradient E={E} k={k} M={M}", flush=True)
+    g = torch.Generator().manual_seed(23)
+    expert, ss = torch.randint(0, E, (M,), generator=g).sort().values.cuda(), torch.randperm(M, generator=g).cuda()
+    offs = torch.bincount(expert, minlength=E).cumsum(0)
+    new = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()
+    dy, W2, z, w = new(M // k, H), new(E, H, I), new(M, 2 * I), torch.rand(M, generator=g).bfloat16().cuda()
+    dz, d_w = torch.empty_like(z), torch.full((M // k, k), float("nan"), dtype=torch.bfloat16, device="cuda")
+    with _few_rows_limit(0):
+        ops.down_projection_dx_swiglu_router_rocm(dy, W2, ss, offs, z, dz, None, w, new(M, H), d_w, k)
+    gate, up = z.double()[:, ::2], z.double()[:, 1::2]
+    h, a, b = up * gate * torch.sigmoid(gate), dy.double()[ss // k][:, :, None], W2.double()[expert]
+    want, size = torch.empty(2, M, dtype=torch.float64, device="cuda")
+    want[ss], size[ss] = ((a * b).sum(1) * h).sum(1), ((a.abs() * b.abs()).sum(1) * h.abs()).sum(1)
+    bound = 2.0**-8 * want.abs() + ((H + I + 8) * 2.0**-24 + 2.0**-18) * size + 2.0**-133
+    assert ((d_w.view(-1).double() - want).abs() <= bound).all()
+
+
 def test_scatter2scatter_with_and_without_workspace():
     """The same launch through the C ABI with the scratch for splitting the last round of tiles along K and without
     it (every tile by one workgroup): both within tolerance of the oracle; the workspace query and its error code."""

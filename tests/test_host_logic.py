@@ -104,6 +104,36 @@ def test_argument_errors_are_reported_before_any_launch():
     assert lib.xma_rocm_continuous_count(None, 0, 0, ctypes.c_void_p(16), 4, None, 0, None) == 0
 
 
+def test_router_gradient_entry_point_arguments():
+    """xma_rocm_down_projection_dx_swiglu_router knows slots and rows, not how many experts there are: more slots than experts (ids that
+    repeat) and more experts than route counts are taken; the rest is refused before any launch"""
+    from xma.rocm import get_library, ops
+
+    lib, p = get_library(), ctypes.c_void_p(1 << 20)
+
+    def call(M=8, N=64, K=64, E=4, k=2, dtype=0, d_w=p, scale=p, space=p, short=0):
+        need = lib.xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, N, K, E)
+        return lib.xma_rocm_down_projection_dx_swiglu_router(p, K, p, K * N, N, p, p, p, 2 * N, p, 2 * N, None, 0, scale, d_w, M, N, K, E, k,
+                                                             dtype, space, need - short, None)
+
+    assert call(M=0, E=2, k=4) == 0 and call(M=0, E=4096) == 0 and call(M=0, k=32, d_w=None) == 0
+    for bad in (dict(k=0), dict(k=33, M=66), dict(M=7), dict(M=-2), dict(d_w=None), dict(scale=None), dict(dtype=2)):
+        assert call(**bad) == -1, bad
+    assert call(short=1) == -3 and call(space=None) == -3 and call(space=ctypes.c_void_p((1 << 20) + 8)) == -3
+    assert call(M=1 << 24, N=1 << 13, space=p) == -2  # products beyond 32-bit offsets
+    # what Python restates
+    for M, N, K, E in ((8, 64, 64, 4), (1000, 1032, 256, 8), (4096, 768, 2048, 128), (20000, 16, 64, 4096)):
+        slices = lib.xma_rocm_scatter2scatter_workspace_bytes(M, N, K, E)
+        assert ops.router_gradient_workspace_bytes(M, N, slices) == lib.xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, N, K, E)
+    takes = ops.dx2_leaves_router_gradient
+    assert takes(0, 8, 64, 32, torch.bfloat16) and takes(0, 8, 64, 2, torch.float16)
+    assert not takes(1, 8, 64, 2, torch.bfloat16) and not takes(0, 8, 64, 33, torch.bfloat16) and not takes(0, 8, 64, 2, torch.float32)
+    assert takes(0, (1 << 30) - 5, 128, 1, torch.bfloat16) and not takes(0, (1 << 30) - 4, 128, 1, torch.bfloat16)
+    for H, E, k, dtype in ((8, 1, 1, 0), (64, 128, 32, 2), (64, 128, 33, 0), (64, 129, 2, 0), (12, 8, 2, 0), (64, 8, 9, 1), (0, 8, 2, 0), (64, 8, 0, 2)):
+        name = (torch.bfloat16, torch.float16, torch.float32)[dtype]
+        assert ops.gate_bwd_supported(H, E, k, name) == bool(lib.xma_rocm_gate_bwd_supported(H, E, k, dtype)), (H, E, k, dtype)
+
+
 def test_layer_entry_points_refuse_what_they_cannot_run():
     """xma_rocm_moe_*: every argument that has a rule of its own, before any launch"""
     import struct
