@@ -40,7 +40,10 @@ int xma_down_projection_dx_dots(const void *dY, int64_t lddy, const void *W, int
                                 int64_t lddz, void *scaled_act, int64_t ld_scaled_act, const void *row_scale, int64_t M, int32_t N,
                                 int32_t K, int32_t E, int32_t fan_out, int dtype, void *workspace, size_t workspace_bytes, void *stream,
                                 float *dots);
-// what xma_rocm_gate_bwd launches in front of its last kernel, and that kernel with the sum over the k slots (gate.hip)
+// xma_rocm_gate_bwd, whose last kernel also sums the k slots of `scattered` (may be NULL); every rule of its arguments, without a launch (gate.hip)
+int xma_gate_bwd_check(const char *what, const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids,
+                       const void *scattered, const void *d_x, const void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype,
+                       const void *workspace, size_t workspace_bytes);
 int xma_gate_bwd(const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids, const void *scattered, void *d_x,
                  void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype, void *workspace, size_t workspace_bytes, hipStream_t st);
 

@@ -303,19 +303,25 @@ extern "C" size_t xma_rocm_gate_bwd_workspace_bytes(int64_t T, int32_t H, int32_
     return (size_t)gate_ranges(T, H).count * (size_t)E * (size_t)H * sizeof(float);
 }
 
-int xma_gate_bwd(const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids, const void *scattered, void *d_x,
-                 void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype, void *workspace, size_t workspace_bytes, hipStream_t st) {
-    XMA_REQUIRE(xma_rocm_gate_bwd_supported(H, E, k, dtype), XMA_ROCM_EUNSUPPORTED, "gate_bwd: H=%d E=%d k=%d dtype=%d", H, E, k, dtype);
+int xma_gate_bwd_check(const char *what, const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids,
+                       const void *scattered, const void *d_x, const void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype,
+                       const void *workspace, size_t workspace_bytes) {
+    XMA_REQUIRE(xma_rocm_gate_bwd_supported(H, E, k, dtype), XMA_ROCM_EUNSUPPORTED, "%s: H=%d E=%d k=%d dtype=%d", what, H, E, k, dtype);
     const int es = dtype == XMA_ROCM_F32 ? 4 : 2;
-    XMA_REQUIRE(T >= 1 && T * k < ((int64_t)1 << 31) && ldx >= H && ldx * es % 16 == 0, XMA_ROCM_EINVAL, "gate_bwd: T=%lld ldx=%lld",
+    XMA_REQUIRE(T >= 1 && T * k < ((int64_t)1 << 31) && ldx >= H && ldx * es % 16 == 0, XMA_ROCM_EINVAL, "%s: T=%lld ldx=%lld", what,
                 (long long)T, (long long)ldx);
     const uintptr_t all = (uintptr_t)x | (uintptr_t)gate_weight | (uintptr_t)scattered | (uintptr_t)d_x | (uintptr_t)d_gate | (uintptr_t)workspace;
     XMA_REQUIRE(d_sel && ids && (d_x || d_gate) && (!d_x || gate_weight) && (!d_gate || (x && workspace)) && (all & 15) == 0, XMA_ROCM_EINVAL,
-                "gate_bwd: null or misaligned pointer");
-    if (d_gate) {
-        const size_t need = xma_rocm_gate_bwd_workspace_bytes(T, H, E);
-        XMA_REQUIRE(workspace_bytes >= need, XMA_ROCM_EWORKSPACE, "gate_bwd: workspace of %zu bytes, %zu needed", workspace_bytes, need);
-    }
+                "%s: null or misaligned pointer", what);
+    const size_t need = d_gate ? xma_rocm_gate_bwd_workspace_bytes(T, H, E) : 0;
+    XMA_REQUIRE(workspace_bytes >= need, XMA_ROCM_EWORKSPACE, "%s: workspace of %zu bytes, %zu needed", what, workspace_bytes, need);
+    return XMA_ROCM_OK;
+}
+
+int xma_gate_bwd(const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids, const void *scattered, void *d_x,
+                 void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype, void *workspace, size_t workspace_bytes, hipStream_t st) {
+    if (int rc = xma_gate_bwd_check("gate_bwd", x, ldx, gate_weight, d_sel, ids, scattered, d_x, d_gate, T, H, E, k, dtype, workspace, workspace_bytes))
+        return rc;
     float *sums = (float *)workspace;
     if (dtype == XMA_ROCM_BF16) return gate_bwd<__bf16>(x, ldx, gate_weight, d_sel, ids, scattered, d_x, d_gate, T, H, E, k, sums, st);
     if (dtype == XMA_ROCM_F16) return gate_bwd<_Float16>(x, ldx, gate_weight, d_sel, ids, scattered, d_x, d_gate, T, H, E, k, sums, st);

@@ -109,11 +109,13 @@ extern "C" int xma_rocm_moe_forward(const xma_rocm_moe *m, void *stream) {
     return xma_rocm_combine(m->expert_out, m->H, m->router_weights, m->y, m->H, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream);
 }
 
+static int check_recompute(const xma_rocm_moe *m, const char *what, bool dots) {
+    return m->recompute && !dots ? check_workspace(m, m->few_down, m->H, m->I, what) : XMA_ROCM_OK;
+}
 // The activations and expert outputs again where neither was kept: h from z, the expert outputs by the down-projection.  Where dX2
 // leaves the router weights' gradient (`dots`), nothing reads the expert outputs, and h only dW2.
-static int recompute(const xma_rocm_moe *m, const char *what, bool dots, void *stream) {
+static int recompute(const xma_rocm_moe *m, bool dots, void *stream) {
     if (!m->recompute) return XMA_ROCM_OK;
-    if (!dots) RUN(check_workspace(m, m->few_down, m->H, m->I, what));
     if (!dots || m->dw2_form != 1)
         RUN(xma_rocm_swiglu_packed_forward(m->z, 2 * m->I, m->h, m->I, m->T * m->k, (int32_t)m->I, (int)m->dtype, stream));
     return dots ? XMA_ROCM_OK : down_projection(m, stream);
@@ -137,26 +139,30 @@ extern "C" int xma_rocm_moe_backward_router(const xma_rocm_moe *m, void *stream)
     XMA_REQUIRE(m->logits && m->dy && m->d_router_weights && m->d_logits && (!m->recompute || m->h), XMA_ROCM_EINVAL,
                 "moe_backward_router: null buffer");
     const int dtype = (int)m->dtype;
-    RUN(recompute(m, "moe_backward_router", false, stream));
+    RUN(check_recompute(m, "moe_backward_router", false));
+    RUN(recompute(m, false, stream));
     RUN(xma_rocm_combine_bwd(m->expert_out, m->H, m->dy, m->H, m->d_router_weights, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream));
     return xma_rocm_router_topk_bwd(m->logits, m->E, m->T, (int32_t)m->E, (int32_t)m->k, dtype, m->expert_ids, 0, m->d_router_weights, m->d_logits,
                                     m->E, stream);
 }
 
-// Everything of the backward between the router's part and the sum over the k slots: `scattered` holds dX1 then.
-static int backward_experts(const xma_rocm_moe *m, const char *what, float *dots, void *stream) {
-    RUN(check(m, what));
+// What the part below asks of its arguments, before the first launch.
+static int check_experts(const xma_rocm_moe *m, const char *what) {
     XMA_REQUIRE(m->dy && m->dz && m->d_w_fc && m->d_w_proj && m->scattered && m->d_x && (m->dw2_form == 1 || m->h) &&
                     (m->dw2_form == 0 || m->dw2_operand) && (!m->d_b_fc || m->b_fc) && (!m->d_b_proj || m->b_proj),
                 XMA_ROCM_EINVAL, "%s: null buffer", what);
     // the column sums that make d_b_proj want dy scaled, in a copy or beside the scaled activations: the loader of form 0 keeps none
     XMA_REQUIRE(m->dw2_form >= 0 && m->dw2_form <= 2 && !(m->dw2_form == 0 && m->d_b_proj), XMA_ROCM_EINVAL,
                 "%s: dw2_form %lld%s", what, (long long)m->dw2_form, m->d_b_proj ? " with d_b_proj (forms 1 and 2 only)" : "");
+    RUN(check_workspace(m, m->few_dx2, m->I, m->H, what));
+    return check_workspace(m, m->few_dx1, m->H, up_width(m), what);
+}
+
+// Everything of the backward between the router's part and the sum over the k slots: `scattered` holds dX1 then.
+static int backward_experts(const xma_rocm_moe *m, float *dots, void *stream) {
     const int dtype = (int)m->dtype;
     const int64_t M = m->T * m->k, H = m->H, I = m->I, U = up_width(m);
     const int64_t *idx = (const int64_t *)m->sorted_scattered_idxs, *offs = (const int64_t *)m->expert_offsets;
-    RUN(check_workspace(m, m->few_dx2, I, H, what));
-    RUN(check_workspace(m, m->few_dx1, H, U, what));
     // dX2 + SwiGLU', with the scaled activations for dW2 where that takes dy through the index
     RUN(gemm(m, m->few_dx2, m->dy, m->w_proj, H * I, I, 1, m->dz, m->z, U, m->dw2_form == 1 ? m->dw2_operand : nullptr, m->router_weights,
              nullptr, I, H, m->k, 0, 1, epilogue_of(m, 1), stream, dots));
@@ -183,7 +189,9 @@ static int backward_experts(const xma_rocm_moe *m, const char *what, float *dots
 }
 
 extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
-    RUN(backward_experts(m, "moe_backward", nullptr, stream));
+    RUN(check(m, "moe_backward"));
+    RUN(check_experts(m, "moe_backward"));
+    RUN(backward_experts(m, nullptr, stream));
     return xma_rocm_combine_add(m->scattered, m->H, nullptr, m->d_x_addend, m->H, m->d_x, m->H, m->T, (int32_t)m->k, (int32_t)m->H, (int)m->dtype, stream);
 }
 
@@ -195,11 +203,15 @@ extern "C" int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_w
     XMA_REQUIRE(xma_rocm_gate_bwd_supported((int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype), XMA_ROCM_EUNSUPPORTED,
                 "moe_backward_gated: H=%lld E=%lld k=%lld dtype=%d", (long long)m->H, (long long)m->E, (long long)m->k, dtype);
     float *const dots = dots_place(m);
-    RUN(recompute(m, "moe_backward_router", dots != nullptr, stream));
+    RUN(check_recompute(m, "moe_backward_gated, as moe_backward_router", dots != nullptr));
+    RUN(check_experts(m, "moe_backward_gated, as moe_backward"));
+    RUN(xma_gate_bwd_check("moe_backward_gated", m->x, m->H, m->gate_weight, m->d_router_weights, (const int32_t *)m->expert_ids, m->scattered, m->d_x,
+                           d_gate_weight, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->workspace, (size_t)m->workspace_bytes));
+    RUN(recompute(m, dots != nullptr, stream));
     if (!dots)
         RUN(xma_combine_router_bwd(m->expert_out, m->dy, m->logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k,
                                    dtype, m->d_router_weights, (hipStream_t)stream));
-    RUN(backward_experts(m, "moe_backward", dots, stream));
+    RUN(backward_experts(m, dots, stream));
     return xma_gate_bwd(m->x, m->H, m->gate_weight, m->d_router_weights, (const int32_t *)m->expert_ids, m->scattered, m->d_x, d_gate_weight, m->T,
                         (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->workspace, (size_t)m->workspace_bytes, (hipStream_t)stream);
 }

@@ -615,8 +615,9 @@ class _Layer(torch.autograd.Function):
             d_gate = torch.empty_like(gate_weight) if need_gate else None
             rc = lib.xma_rocm_moe_backward_gated(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0),
                                                  None if d_gate is None else d_gate.data_ptr(), stream)
-            if rc:  # the message begins with the part that refused
-                check(rc, "xma_rocm_" + lib.xma_rocm_last_error().decode(errors="replace").partition(":")[0])
+            if rc:  # the message of a part that it shares with another entry begins with both names
+                part = lib.xma_rocm_last_error().decode(errors="replace").partition(":")[0].partition(", as ")[2]
+                check(rc, "xma_rocm_moe_backward_gated" + (", as xma_rocm_" + part if part else ""))
             return d_x, d_gate, None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None, None
         check(lib.xma_rocm_moe_backward_router(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0), stream), "xma_rocm_moe_backward_router")
         d_gate = d_x_gate = None

@@ -181,6 +181,49 @@ def test_layer_entry_points_refuse_what_they_cannot_run():
     refused("backward", -3, "scatter2scatter_few_rows: workspace", I=64, H=16384, workspace_bytes=16)
 
 
+def test_gated_backward_refuses_before_any_launch():
+    """xma_rocm_moe_backward_gated: every argument that has a rule of its own, under its own name; what its parts share with the other two
+    entries under both (the K slices of its GEMMs take a device to be counted: tests/test_gpu_layer.py)"""
+    import struct
+
+    from xma.rocm import get_library
+
+    lib = get_library()
+    text = open(os.path.join(ROOT, "include", "xma_rocm.h")).read()
+    block = re.sub(r"/\*.*?\*/", "", text[text.index("typedef struct xma_rocm_moe {") : text.index("} xma_rocm_moe;")], flags=re.S)
+    names = re.findall(r"\b(\w+)[,;]", block)
+    sizes = names[: names.index("x")]
+    base = dict.fromkeys(names, 256) | dict(size=8 * len(names), T=4, H=64, I=32, E=8, k=2, dtype=0, activation=0, dw2_form=2, recompute=0)
+    base |= dict(workspace_bytes=1 << 30, d_b_fc=0, d_b_proj=0, b_fc=0, b_proj=0) | dict.fromkeys((s for s in sizes if s.startswith("few_")), 1)
+
+    def refused(code, message, d_gate=256, **change):
+        v = base | change
+        rc = lib.xma_rocm_moe_backward_gated(struct.pack(f"{len(sizes)}q{len(names) - len(sizes)}Q", *(v[n] for n in names)), d_gate, None)
+        assert rc == code and lib.xma_rocm_last_error().decode().startswith(message), (change, rc, lib.xma_rocm_last_error())
+
+    own, experts, router = "moe_backward_gated: ", "moe_backward_gated, as moe_backward: ", "moe_backward_gated, as moe_backward_router: "
+    refused(-1, own + "argument block", size=8)
+    for bad in (dict(T=0), dict(H=0), dict(E=16385), dict(k=9)):
+        refused(-1, own + "T=", **bad)
+    refused(-1, own + "workspace of -1", workspace_bytes=-1)
+    for name in ("x", "z", "expert_out", "gate_weight", "logits", "dy", "d_router_weights", "d_x", "scattered"):
+        refused(-1, own + "null buffer", **{name: 0})
+    refused(-1, own + "null buffer", recompute=1, h=0)
+    refused(-1, own + "activation", activation=3)
+    for bad in (dict(H=68), dict(E=129), dict(k=33, E=64), dict(dtype=5)):
+        refused(-2, own + "H=", **bad)
+    for name in ("dz", "d_w_fc", "d_w_proj", "h", "dw2_operand"):
+        refused(-1, experts + "null buffer", **{name: 0})
+    refused(-1, experts + "null buffer", d_b_fc=256)
+    refused(-1, experts + "dw2_form 3", dw2_form=3)
+    refused(-1, experts + "dw2_form 0 with d_b_proj", dw2_form=0, b_proj=256, d_b_proj=256)
+    refused(-1, own + "null or misaligned", workspace=0)
+    for bad in (dict(x=264), dict(gate_weight=264), dict(d_x=264), dict(scattered=264), dict(workspace=264), dict(d_gate=264)):
+        refused(-1, own + "null or misaligned", **bad)
+    need = lib.xma_rocm_gate_bwd_workspace_bytes(4, 64, 8)
+    refused(-3, own + f"workspace of {need - 1} bytes, {need} needed", workspace_bytes=need - 1)
+
+
 def test_few_token_dispatch_rule():
     """which grouped GEMM forms take the kernels of the few-token regime: by rows per expert on average, per form, with a
     cap on the rows in all; fp32 never"""
