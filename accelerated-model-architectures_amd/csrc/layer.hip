@@ -158,8 +158,9 @@ static int check_experts(const xma_rocm_moe *m, const char *what) {
     return check_workspace(m, m->few_dx1, m->H, up_width(m), what);
 }
 
-// Everything of the backward between the router's part and the sum over the k slots: `scattered` holds dX1 then.
-static int backward_experts(const xma_rocm_moe *m, float *dots, void *stream) {
+// Everything of the backward between the router's part and the sum over the k slots: `scattered` holds dX1 then.  With `dots`, d_router_weights
+// too: the router weights' gradient or, with logits, that of the selected logits.
+static int backward_experts(const xma_rocm_moe *m, float *dots, const void *logits, void *stream) {
     const int dtype = (int)m->dtype;
     const int64_t M = m->T * m->k, H = m->H, I = m->I, U = up_width(m);
     const int64_t *idx = (const int64_t *)m->sorted_scattered_idxs, *offs = (const int64_t *)m->expert_offsets;
@@ -167,7 +168,7 @@ static int backward_experts(const xma_rocm_moe *m, float *dots, void *stream) {
     RUN(gemm(m, m->few_dx2, m->dy, m->w_proj, H * I, I, 1, m->dz, m->z, U, m->dw2_form == 1 ? m->dw2_operand : nullptr, m->router_weights,
              nullptr, I, H, m->k, 0, 1, epilogue_of(m, 1), stream, dots));
     if (dots) // before dX1, whose K slices take their place
-        RUN(xma_dots_router_bwd(dots, dots_parts(m), m->logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->E, (int32_t)m->k, dtype,
+        RUN(xma_dots_router_bwd(dots, dots_parts(m), logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->E, (int32_t)m->k, dtype,
                                 m->d_router_weights, (hipStream_t)stream));
     if (m->dw2_form == 1) {
         RUN(dw(m, m->few_dw2, m->dy, 0, nullptr, m->dw2_operand, 1, m->d_w_proj, H, I, stream));
@@ -191,8 +192,26 @@ static int backward_experts(const xma_rocm_moe *m, float *dots, void *stream) {
 extern "C" int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream) {
     RUN(check(m, "moe_backward"));
     RUN(check_experts(m, "moe_backward"));
-    RUN(backward_experts(m, nullptr, stream));
+    RUN(backward_experts(m, nullptr, nullptr, stream));
     return xma_rocm_combine_add(m->scattered, m->H, nullptr, m->d_x_addend, m->H, m->d_x, m->H, m->T, (int32_t)m->k, (int32_t)m->H, (int)m->dtype, stream);
+}
+
+// The order of the launches is that of the ops: whether the router weights' gradient comes from dX2 does not depend on what else hangs on
+// the logits, and d_logits waits for it.
+extern "C" int xma_rocm_moe_backward_logits(const xma_rocm_moe *m, void *stream) {
+    RUN(check(m, "moe_backward_logits"));
+    XMA_REQUIRE(m->logits && m->dy && m->d_router_weights && m->d_logits && (!m->recompute || m->h), XMA_ROCM_EINVAL,
+                "moe_backward_logits: null buffer");
+    const int dtype = (int)m->dtype;
+    float *const dots = dots_place(m);
+    RUN(check_recompute(m, "moe_backward_logits, as moe_backward_router", dots != nullptr));
+    RUN(check_experts(m, "moe_backward_logits, as moe_backward"));
+    RUN(recompute(m, dots != nullptr, stream));
+    if (!dots)
+        RUN(xma_rocm_combine_bwd(m->expert_out, m->H, m->dy, m->H, m->d_router_weights, m->T, (int32_t)m->k, (int32_t)m->H, dtype, stream));
+    RUN(backward_experts(m, dots, nullptr, stream));
+    return xma_rocm_router_topk_bwd(m->logits, m->E, m->T, (int32_t)m->E, (int32_t)m->k, dtype, m->expert_ids, 0, m->d_router_weights, m->d_logits,
+                                    m->E, stream);
 }
 
 extern "C" int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_weight, void *stream) {
@@ -211,7 +230,7 @@ extern "C" int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_w
     if (!dots)
         RUN(xma_combine_router_bwd(m->expert_out, m->dy, m->logits, (const int32_t *)m->expert_ids, m->T, (int32_t)m->H, (int32_t)m->E, (int32_t)m->k,
                                    dtype, m->d_router_weights, (hipStream_t)stream));
-    RUN(backward_experts(m, dots, stream));
+    RUN(backward_experts(m, dots, m->logits, stream));
     return xma_gate_bwd(m->x, m->H, m->gate_weight, m->d_router_weights, (const int32_t *)m->expert_ids, m->scattered, m->d_x, d_gate_weight, m->T,
                         (int32_t)m->H, (int32_t)m->E, (int32_t)m->k, dtype, m->workspace, (size_t)m->workspace_bytes, (hipStream_t)stream);
 }

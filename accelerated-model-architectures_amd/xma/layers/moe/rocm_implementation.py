@@ -455,7 +455,7 @@ def fused_swiglu_experts(x, w_fc, w_proj, router_weights, sorted_scattered_idxs,
 
 # ----------------------------------------------------------------------------------------- the layer as one call
 # A pass of a handful of tokens is as long as its host work, so the layer with packed SwiGLU or GELU runs as one autograd node, whose
-# forward and backward are one library call each (two around the gate's own products), on scratch that is laid out once per shape:
+# forward and backward are one library call each (and the last sum another behind gate products of torch's), on scratch that is laid out once per shape:
 # the same launches as the ops above, bit for bit.  Everything else (other activations, tracing, transforms, tensors that the
 # entry point does not describe) goes through the ops.
 _BLOCK_POINTERS = struct.Struct("29Q")
@@ -574,6 +574,13 @@ def _unpacked(saved, shapes, like: torch.Tensor) -> list[torch.Tensor | None]:
     return out
 
 
+def _check_backward(rc: int, entry: str) -> None:
+    """raises what the entry refused; the message of a rule that it shares with another entry begins with both names"""
+    if rc:
+        part = get_library().xma_rocm_last_error().decode(errors="replace").partition(":")[0].partition(", as ")[2]
+        check(rc, entry + (", as xma_rocm_" + part if part else ""))
+
+
 class _Layer(torch.autograd.Function):
     """the whole layer: with gate_weight (logits None) -> (y, logits), with given logits -> y"""
 
@@ -613,13 +620,10 @@ class _Layer(torch.autograd.Function):
         lib, stream = get_library(), ops._stream(x)
         if gated:
             d_gate = torch.empty_like(gate_weight) if need_gate else None
-            rc = lib.xma_rocm_moe_backward_gated(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0),
-                                                 None if d_gate is None else d_gate.data_ptr(), stream)
-            if rc:  # the message of a part that it shares with another entry begins with both names
-                part = lib.xma_rocm_last_error().decode(errors="replace").partition(":")[0].partition(", as ")[2]
-                check(rc, "xma_rocm_moe_backward_gated" + (", as xma_rocm_" + part if part else ""))
+            _check_backward(lib.xma_rocm_moe_backward_gated(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0),
+                                                            None if d_gate is None else d_gate.data_ptr(), stream), "xma_rocm_moe_backward_gated")
             return d_x, d_gate, None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None, None
-        check(lib.xma_rocm_moe_backward_router(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0), stream), "xma_rocm_moe_backward_router")
+        _check_backward(lib.xma_rocm_moe_backward_logits(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0), stream), "xma_rocm_moe_backward_logits")
         d_gate = d_x_gate = None
         if gate_weight is not None:
             if d_logits_out is not None:  # the caller also used the returned router logits (an auxiliary loss)
@@ -629,8 +633,9 @@ class _Layer(torch.autograd.Function):
             if need_gate:
                 d_gate = _gate_weight_grad(d_logits, x)
         recorded = d_x_gate is not None and d_x_gate.requires_grad  # create_graph: the sum is torch's as well
-        check(lib.xma_rocm_moe_backward(p.sizes_backward + _BLOCK_POINTERS.pack(*pointers, 0 if d_x_gate is None or recorded else d_x_gate.data_ptr()),
-                                        stream), "xma_rocm_moe_backward")
+        T, H = x.shape
+        check(lib.xma_rocm_combine_add(b + back["scattered"], H, None, None if d_x_gate is None or recorded else d_x_gate.data_ptr(), H,
+                                       d_x.data_ptr(), H, T, p.top_k, H, ops._DTYPE_CODE[x.dtype], stream), "xma_rocm_combine_add")
         if recorded:
             d_x = d_x + d_x_gate
         return d_x, d_gate, d_logits if need_logits else None, d_w_fc, d_w_proj, d_b_fc, d_b_proj, None, None, None

@@ -96,6 +96,7 @@ SIGNATURES = {
     "xma_rocm_moe_forward": (_int, [_p, _p]),
     "xma_rocm_moe_backward_router": (_int, [_p, _p]),
     "xma_rocm_moe_backward": (_int, [_p, _p]),
+    "xma_rocm_moe_backward_logits": (_int, [_p, _p]),
     "xma_rocm_moe_backward_gated": (_int, [_p, _p, _p]),
     "xma_rocm_diag_mfma_stream": (_int, [_p, _i32, _p, _i32, _p]),
 }

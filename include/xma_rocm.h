@@ -411,11 +411,16 @@ XMA_API int xma_rocm_moe_backward_router(const xma_rocm_moe *m, void *stream);
 /* dX2, dW2, dW1, bias gradients, dX1, sum over the k slots; behind xma_rocm_moe_backward_router */
 XMA_API int xma_rocm_moe_backward(const xma_rocm_moe *m, void *stream);
 /*
- * The whole backward where no gradient of the logits comes from outside and xma_rocm_gate_bwd covers the gate: both of the above and the
+ * Both of the above in one, for a caller that forms the gate's products: d_logits (without what comes from outside) and, in `scattered`, dX1,
+ * whose k slots xma_rocm_combine_add sums into d_x together with the gate's part; d_x_addend is not used.  A bf16 / fp16 SwiGLU layer with
+ * few_dx2 = 0 and no b_proj forms the router weights' gradient in dX2 instead of from expert_out, which it does not read then, if `workspace`
+ * holds xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, I, H, E).
+ */
+XMA_API int xma_rocm_moe_backward_logits(const xma_rocm_moe *m, void *stream);
+/*
+ * The whole backward where no gradient of the logits comes from outside and xma_rocm_gate_bwd covers the gate: the above with the
  * gate's two products, whose part of d_x joins the sum over the k slots.  d_router_weights receives d_selected; d_logits and d_x_addend are
- * not used; d_gate_weight (E, H) or NULL.  `workspace` also holds xma_rocm_gate_bwd_workspace_bytes.  A bf16 / fp16 SwiGLU layer with few_dx2 = 0
- * and no b_proj forms the router weights' gradient in dX2 instead of from expert_out, if `workspace` holds
- * xma_rocm_down_projection_dx_swiglu_router_workspace_bytes(M, I, H, E).
+ * not used; d_gate_weight (E, H) or NULL.  `workspace` also holds xma_rocm_gate_bwd_workspace_bytes.
  */
 XMA_API int xma_rocm_moe_backward_gated(const xma_rocm_moe *m, void *d_gate_weight, void *stream);
 

@@ -1,5 +1,7 @@
 """The layer as one autograd node against the same layer through the single ops: same launches, so bit for bit."""
 
+import contextlib
+
 import pytest
 import torch
 import torch.nn as nn
@@ -277,3 +279,85 @@ def test_side_stream_capture_and_replay(T, k, act):
         got = [o.clone() for o in outs]
         _same(got, step(x, dy))
         torch.cuda.synchronize()
+
+
+def _biased_gate(moe, bias):
+    gate = nn.Linear(moe.gate.in_features, moe.gate.out_features).to("cuda", moe.gate.weight.dtype)
+    with torch.no_grad():
+        gate.weight.copy_(moe.gate.weight)
+        gate.bias.copy_(bias)
+    moe.gate = gate
+
+
+LARGE_TILES = [  # T, E, k, H, I through the 256 x 256 tiles: both forms of dW2's operand, parts of a row's products that end anywhere
+    (33, 8, 2, 64, 40),
+    (300, 8, 2, 136, 72),
+    (500, 8, 5, 128, 264),
+    (300, 160, 2, 64, 136),  # more experts than the gate's kernels take
+    (40, 8, 8, 64, 128),
+]
+
+
+def _takes_large_tiles(moe, T, dtype):
+    from xma.layers.moe import rocm_implementation as R
+    from xma.rocm import ops
+
+    E, H, I = moe.c_proj.weight.shape
+    sizes = R._plan(T, H, I, E, moe.top_k, dtype, "swiglu_packed", moe.c_proj.bias is not None, bool(moe.save_activations), 0, ops.dispatch_limits())
+    return R._BLOCK_SIZES.unpack(sizes.sizes_backward)[10] == 0
+
+
+@pytest.mark.parametrize("bias,save", [(False, True), (False, False), (True, True), (True, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [*LARGE_TILES, (32768, 8, 2, 256, 768)])  # the last by the dispatch's own rule
+def test_one_call_matches_the_ops_by_large_tiles(case, dtype, bias, save):
+    """there dX2 leaves the gradient of the router weights, whatever else hangs on the logits: with and without an auxiliary loss, a gate
+    with a bias, biases of the experts (whose gradient comes from the expert outputs)"""
+    T, E, k, H, I = case
+    print(f"layer by large tiles {case} {dtype} bias={bias} save={save}", flush=True)
+    one, ops, x, dy = _layers(T, E, k, H, I, dtype, bias, save)
+    with _few_rows_limit(0) if T < 1000 else contextlib.nullcontext():
+        assert _takes_large_tiles(one, T, dtype)
+        for aux in (0.0, 0.1):
+            _same(_step(one, x, dy, aux), _step(ops, x, dy, aux))
+        gate_bias = torch.randn(E, device="cuda").to(dtype)
+        for moe in (one, ops):
+            _biased_gate(moe, gate_bias)
+        _same(_step(one, x, dy, 0.1), _step(ops, x, dy, 0.1))
+
+
+@pytest.mark.parametrize("aux", [0.0, 0.1])
+@pytest.mark.parametrize("save", [True, False])
+@pytest.mark.parametrize("k", [2, 4])
+def test_large_tiles_capture_and_replay(k, save, aux):
+    """the same backward captured once and replayed on new inputs, with eager passes and synchronisations in between"""
+    one, _, sx, sdy = _layers(300, 8, k, 136, 264, torch.bfloat16, save=save)
+
+    def step(x, dy):
+        x = x.detach().requires_grad_()
+        y, logits = one(x)
+        outs, grads = ([y, logits], [dy, aux * logits.detach()]) if aux else ([y], [dy])
+        return [t.detach() for t in (y, logits, *torch.autograd.grad(outs, [x, *one.parameters()], grads))]
+
+    print(f"large tiles captured k={k} save={save} aux={aux}", flush=True)
+    with _few_rows_limit(0):
+        assert _takes_large_tiles(one, 300, torch.bfloat16)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(3):
+                step(sx, sdy)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs = step(sx, sdy)
+        for seed in range(4):
+            g = torch.Generator(device="cuda").manual_seed(seed)
+            x, dy = (torch.randn(t.shape, device="cuda", generator=g).bfloat16() for t in (sx, sdy))
+            sx.copy_(x), sdy.copy_(dy)
+            graph.replay()
+            torch.cuda.synchronize()
+            got = [o.clone() for o in outs]
+            _same(got, step(x, dy))
+            torch.cuda.synchronize()

@@ -181,8 +181,8 @@ def test_layer_entry_points_refuse_what_they_cannot_run():
     refused("backward", -3, "scatter2scatter_few_rows: workspace", I=64, H=16384, workspace_bytes=16)
 
 
-def test_gated_backward_refuses_before_any_launch():
-    """xma_rocm_moe_backward_gated: every argument that has a rule of its own, under its own name; what its parts share with the other two
+def test_whole_backward_refuses_before_any_launch():
+    """xma_rocm_moe_backward_gated and _logits: every argument that has a rule of its own, under its own name; what its parts share with the other two
     entries under both (the K slices of its GEMMs take a device to be counted: tests/test_gpu_layer.py)"""
     import struct
 
@@ -198,25 +198,28 @@ def test_gated_backward_refuses_before_any_launch():
 
     def refused(code, message, d_gate=256, **change):
         v = base | change
-        rc = lib.xma_rocm_moe_backward_gated(struct.pack(f"{len(sizes)}q{len(names) - len(sizes)}Q", *(v[n] for n in names)), d_gate, None)
+        block = struct.pack(f"{len(sizes)}q{len(names) - len(sizes)}Q", *(v[n] for n in names))
+        rc = lib.xma_rocm_moe_backward_gated(block, d_gate, None) if gated else lib.xma_rocm_moe_backward_logits(block, None)
         assert rc == code and lib.xma_rocm_last_error().decode().startswith(message), (change, rc, lib.xma_rocm_last_error())
 
-    own, experts, router = "moe_backward_gated: ", "moe_backward_gated, as moe_backward: ", "moe_backward_gated, as moe_backward_router: "
-    refused(-1, own + "argument block", size=8)
-    for bad in (dict(T=0), dict(H=0), dict(E=16385), dict(k=9)):
-        refused(-1, own + "T=", **bad)
-    refused(-1, own + "workspace of -1", workspace_bytes=-1)
-    for name in ("x", "z", "expert_out", "gate_weight", "logits", "dy", "d_router_weights", "d_x", "scattered"):
-        refused(-1, own + "null buffer", **{name: 0})
-    refused(-1, own + "null buffer", recompute=1, h=0)
-    refused(-1, own + "activation", activation=3)
+    for gated in (False, True):
+        entry = "moe_backward_" + ("gated" if gated else "logits")
+        own, experts = entry + ": ", entry + ", as moe_backward: "
+        refused(-1, own + "argument block", size=8)
+        for bad in (dict(T=0), dict(H=0), dict(E=16385), dict(k=9)):
+            refused(-1, own + "T=", **bad)
+        refused(-1, own + "workspace of -1", workspace_bytes=-1)
+        for name in ("x", "z", "expert_out", "logits", "dy", "d_router_weights", *(("gate_weight", "d_x", "scattered") if gated else ("d_logits",))):
+            refused(-1, own + "null buffer", **{name: 0})
+        refused(-1, own + "null buffer", recompute=1, h=0)
+        refused(-1, own + "activation", activation=3)
+        for name in ("dz", "d_w_fc", "d_w_proj", "h", "dw2_operand", *(() if gated else ("d_x", "scattered"))):
+            refused(-1, experts + "null buffer", **{name: 0})
+        refused(-1, experts + "null buffer", d_b_fc=256)
+        refused(-1, experts + "dw2_form 3", dw2_form=3)
+        refused(-1, experts + "dw2_form 0 with d_b_proj", dw2_form=0, b_proj=256, d_b_proj=256)
     for bad in (dict(H=68), dict(E=129), dict(k=33, E=64), dict(dtype=5)):
         refused(-2, own + "H=", **bad)
-    for name in ("dz", "d_w_fc", "d_w_proj", "h", "dw2_operand"):
-        refused(-1, experts + "null buffer", **{name: 0})
-    refused(-1, experts + "null buffer", d_b_fc=256)
-    refused(-1, experts + "dw2_form 3", dw2_form=3)
-    refused(-1, experts + "dw2_form 0 with d_b_proj", dw2_form=0, b_proj=256, d_b_proj=256)
     refused(-1, own + "null or misaligned", workspace=0)
     for bad in (dict(x=264), dict(gate_weight=264), dict(d_x=264), dict(scattered=264), dict(workspace=264), dict(d_gate=264)):
         refused(-1, own + "null or misaligned", **bad)
