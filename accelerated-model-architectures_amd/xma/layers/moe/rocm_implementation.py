@@ -338,9 +338,9 @@ class _FusedSwiGLUExperts(torch.autograd.Function):
     """Whole expert computation with packed SwiGLU in the GEMM epilogues:
     forward  up-projection (+ bias, SwiGLU) -> down-projection (+ bias, scattered) -> combine
     backward combine' -> dX2 (+ SwiGLU') -> dW2, dW1 (and the bias gradients) -> dX1 (scattered) -> k-way sum.
-    save_activations = False keeps x and the pre-activations z only: the backward then recomputes h = swiglu_packed(z)
-    and the expert outputs (one more down-projection GEMM), as the reference's backward recomputes its expert outputs
-    (triton_implementation/__init__.py:117-128)."""
+    save_activations = False keeps x and the pre-activations z only: the backward then recomputes what it reads of h = swiglu_packed(z)
+    and the expert outputs (one more down-projection GEMM, except where dX2 leaves the router weights' gradient), as the reference's
+    backward recomputes its expert outputs (triton_implementation/__init__.py:117-128)."""
 
     @staticmethod
     def forward(ctx, x, w_fc, w_proj, router_weights, sorted_scattered_idxs, expert_offsets, b_fc=None, b_proj=None,
@@ -373,10 +373,11 @@ class _FusedSwiGLUExperts(torch.autograd.Function):
         flat_w = router_weights.view(-1)
         scaled_act_path = _scale_activations_for_dw2(top_k, grad_out)
 
-        if expert_out.numel() == 0 and z.numel() != 0:  # not kept: recomputed from z
-            if h.numel() == 0:
-                h = torch.empty(z.size(0), z.size(1) // 2, dtype=z.dtype, device=z.device)
-                ops.swiglu_packed_forward_rocm(z, h)
+        recomputed = expert_out.numel() == 0 and z.numel() != 0  # from z: what reads them, and the op below may not
+        if recomputed and h.numel() == 0 and (b_proj is not None or not scaled_act_path):
+            h = torch.empty(z.size(0), z.size(1) // 2, dtype=z.dtype, device=z.device)
+            ops.swiglu_packed_forward_rocm(z, h)
+        if recomputed and b_proj is not None:
             expert_out = torch.empty(z.size(0), w_proj.size(-1), device=z.device, dtype=z.dtype)
             ops.scatter2scatter_rocm(h, w_proj, sorted_scattered_idxs, expert_offsets, expert_out, None, 1, True, False, b_proj)
         d_router_weights = torch.empty_like(router_weights)
@@ -407,7 +408,7 @@ class _FusedSwiGLUExperts(torch.autograd.Function):
             if b_proj is None:
                 ops.down_projection_dx_swiglu_router_rocm(
                     grad_out, w_proj.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, z, dz, None, flat_w, expert_out,
-                    d_router_weights, top_k
+                    d_router_weights, top_k, h
                 )
             else:
                 ops.down_projection_dx_swiglu_rocm(
@@ -447,8 +448,8 @@ def down_projection_experts(x, expert_weights, k, sorted_expert_idxs, sorted_sca
 def fused_swiglu_experts(x, w_fc, w_proj, router_weights, sorted_scattered_idxs, expert_offsets, b_fc=None, b_proj=None,
                          save_activations=True):
     """save_activations = False: the backward recomputes h and the expert outputs instead of keeping them, which frees
-    T k (H + I) elements per layer between forward and backward (Mixtral-shaped layer: 604 MB of 1.5 GB) for one more
-    down-projection GEMM."""
+    T k (H + I) elements per layer between forward and backward (Mixtral-shaped layer: 604 MB of 1.5 GB) for h again and, unless
+    the 256 x 256 tiles take dX2 of a layer without a down-projection bias, one more down-projection GEMM."""
     return _FusedSwiGLUExperts.apply(x, w_fc, w_proj, router_weights, sorted_scattered_idxs, expert_offsets, b_fc, b_proj,
                                      save_activations)
 

@@ -441,15 +441,23 @@ def down_projection_dx_swiglu_router_rocm(
     expert_out: torch.Tensor,
     d_row_scale: torch.Tensor,
     FAN_OUT: int,
+    h: torch.Tensor | None = None,
 ) -> None:
     """down_projection_dx_swiglu[_scaled_act] and combine_bwd of a down-projection without a bias: d_row_scale (T, k) from dX2's own
-    products where the 256 x 256 kernels take it, from expert_out otherwise"""
+    products where the 256 x 256 kernels take it, from expert_out otherwise, which an empty one leaves to be computed again from z (or
+    from h = swiglu_packed(z) where the caller has it)"""
     M = sorted_scattered_idxs.numel()
     E, K, N = W.shape
     assert dY.size(1) == K and dY.size(0) * FAN_OUT == M and d_row_scale.shape == (dY.size(0), FAN_OUT)
     w_is_kn, w_es, ldw = _weight_layout(W)
     few = _few_rows_fwd(M, N, K, E, w_is_kn, ldw, dY.size(0) * dY.stride(0), dY.dtype, EPI_SWIGLU_BWD)
     if M == 0 or w_is_kn != 1 or not dx2_leaves_router_gradient(few, M, N, FAN_OUT, dY.dtype):
+        if expert_out.numel() == 0 and M != 0:
+            if h is None:
+                h = torch.empty(M, N, dtype=z.dtype, device=z.device)
+                swiglu_packed_forward_rocm(z, h)
+            expert_out = torch.empty(M, K, dtype=z.dtype, device=z.device)
+            scatter2scatter_rocm(h, W.permute(0, 2, 1), sorted_scattered_idxs, expert_offsets, expert_out, None, 1, True, False)
         combine_bwd_rocm(expert_out, dY, d_row_scale)
         if scaled_act is None:
             down_projection_dx_swiglu_rocm(dY, W, sorted_scattered_idxs, expert_offsets, z, dz, row_scale, FAN_OUT)

@@ -361,3 +361,19 @@ def test_large_tiles_capture_and_replay(k, save, aux):
             got = [o.clone() for o in outs]
             _same(got, step(x, dy))
             torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("k,bias,large,again", [(2, False, True, 0), (5, False, True, 0), (2, True, True, 1), (2, False, False, 1), (5, False, False, 1)])
+def test_what_the_ops_compute_again(monkeypatch, k, bias, large, again):
+    """save_activations = False: the down-projection is repeated only where something reads the expert outputs (a bias there, few-row
+    launches), with the gradients of a layer that keeps them either way"""
+    from xma.rocm import ops as rocm_ops
+
+    _, ops, x, dy = _layers(300, 8, k, 136, 72, torch.bfloat16, bias, save=False)
+    calls, one = [], rocm_ops.scatter2scatter_rocm
+    monkeypatch.setattr(rocm_ops, "scatter2scatter_rocm", lambda *a: calls.append(1) or one(*a))
+    with _few_rows_limit(0) if large else contextlib.nullcontext():
+        got = _step(ops, x, dy)
+        assert len(calls) == 2 + again  # the down-projection, dX1
+        ops.save_activations = True
+        _same(got, _step(ops, x, dy))
