@@ -756,32 +756,6 @@ __global__ __launch_bounds__(64 * WAVES, 1) void fr_deep_kernel(const FwdArgs a)
     }
 }
 
-constexpr int FR_DEEP_K = 2048; // K ranges and their epilogue lead beyond (8 experts, K = 8192, N = 2048)
-
-// W[e] as (N, K): at most as many workgroups with work as run at the same time, counting the experts that M random choices of E hit.
-// 128 experts of H = 576, I = 256, 12 tokens, up-projection in four workgroups for each of 68 experts: 17.8 us against 12.9 with the small tile.
-inline int fr_deep_stages(int K) { const int steps = (K + ST_K_NT - 1) / ST_K_NT; return steps < FD_STAGES ? steps : FD_STAGES; }
-inline bool fr_deep_shape(int64_t M, int N, int K, int E, int w_is_kn, int epilogue) {
-    if (w_is_kn || K > FR_DEEP_K || epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == EPI_GELU_BWD) return false; // those have no such kernel
-    const double experts = E * (1. - pow(1. - 1. / E, (double)M));
-    return experts * ((N + ST_N - 1) / ST_N) <= 256 * (FD_STAGES / fr_deep_stages(K));
-}
-
-// W[e] as (K, N), more than a pass or two of the vector kernel per expert, or rows of W shorter than the 4 KB a wave of
-// the vector kernel takes at a time -> the small MFMA tile (128 experts of H = 576, I = 256, 7 tokens: forward 0.036
-// instead of 0.045 ms with it; 8 experts of H = 2048, I = 8192: 0.161 instead of 0.155)
-inline bool fr_takes_tile(int64_t M, int N, int K, int E, int w_is_kn, int epilogue) {
-    return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE ||
-           fr_deep_shape(M, N, K, E, w_is_kn, epilogue);
-}
-
-// More rows than the small tile takes in one pass go to the 128 x 256 tiles of mid_rows.hip, where those have the variant.  8
-// experts of H = 2048, I = 8192, 32 rows each, up- / down-projection: 132 -> 102 / 61 -> 55 us against a small tile of 128 rows that
-// stood here; 128 experts of H = 2048, I = 768, 64 rows: 190 -> 166 / 103 -> 90.
-inline bool fr_takes_mid(const FwdArgs &a, int w_is_kn, int epilogue) {
-    return a.M > (int64_t)MID_ROWS_FWD_FROM * a.E && xma_rocm::mid_fwd_takes(a, w_is_kn, epilogue);
-}
-
 // K ranges of the small MFMA tile: enough workgroups for two per compute unit of a 256-CU device, ranges of at least 512
 // columns of K.  Measured (8 experts, 16 rows each, down-projection / dX1 / dX2): 1024 workgroups 61 / 99 / 57 us, 512
 // 52 / 91 / 46, 256 55 / 137 / 46: beyond two per compute unit the partial sums and their kernel cost more than the
@@ -792,6 +766,49 @@ inline int fr_tile_splits(int N, int K, int E, int w_is_kn) {
     int S = (int)((512 + wgs - 1) / wgs);
     if (S > steps / min_steps) S = steps / min_steps;
     return S < 1 ? 1 : S;
+}
+
+// W[e] as (K, N), more than a pass or two of the vector kernel per expert, or rows of W shorter than the 4 KB a wave of
+// the vector kernel takes at a time -> an MFMA tile (128 experts of H = 576, I = 256, 7 tokens: forward 0.036
+// instead of 0.045 ms with it; 8 experts of H = 2048, I = 8192: 0.161 instead of 0.155)
+inline bool fr_beyond_vector(int64_t M, int K, int E, int w_is_kn) {
+    return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE;
+}
+
+// Where the kernel with four K steps in flight takes x @ W^T.  Measured against the kernel that takes the launch otherwise, us with the weights in
+// the Infinity Cache / behind a read of 512 MB, over 4545 launches of 1 to 128 experts, 1 to 96 tokens, K = 64 to 2048, N = 128 to 4096: 0.985 / 0.923
+// of the time over all of them, 0.978 / 0.89 over its own, 99 in 100 within 1.17 / 1.03.
+//  * As many workgroups with work as run at the same time, counting the experts that M random choices of E hit, with a margin unless there cannot be
+//    more: 64 experts, K = 2048, N = 2816, 12 rows (242 expected, up to 264) 29 / 34 -> 38 / 47.
+//  * It walks K alone, at 0.9 us a step.  Instead of three or four K ranges, or of the vector kernel, only in launches of half the compute
+//    units, where those stream more than they wait: 2 experts, K = 2048, N = 1024, one row 4.6 / 10 -> 14 / 18; up to 32 workgroups
+//    in three ranges (K = 1536) 9 / 14 -> 13 / 16, in four (K = 2048) 9 / 14 -> 15 / 18; from 112 workgroups on 0.9 - 1.1 / 0.9 - 1.05.  Of two ranges:
+//    down-projections 1.0 / 0.9, SwiGLU launches of up to 64 workgroups (K = 1024) 8.9 / 13.8 -> 9.9 / 13.6.
+//  * With four waves where most experts have rows only for K between 512 and 1024: there 1.03 / 0.93, below (K <= 512) 1.12 / 1.00, above 1.04 / 1.00.
+//    Where most have none the small tile starts a workgroup for each of them: 0.87 / 0.85.
+constexpr int FR_DEEP_K = 2048, FR_DEEP_LONG_FROM = 112;
+inline int fr_deep_stages(int K) { const int steps = (K + ST_K_NT - 1) / ST_K_NT; return steps < FD_STAGES ? steps : FD_STAGES; }
+// two waves, 64 columns, where that still is at most one workgroup per compute unit, or four (64 experts, K = 1408, N = 2048, one
+// token 12.4 -> 11.2 us; with 264 workgroups instead of 132 18.4 -> 29.4)
+inline bool fr_deep_two_waves(int64_t M, int N, int E) { return (M < E ? M : E) * ((N + 63) / 64) <= 256; }
+inline bool fr_deep_shape(int64_t M, int N, int K, int E, int w_is_kn, int epilogue) {
+    if (w_is_kn || K > FR_DEEP_K || epilogue == XMA_ROCM_EPI_SWIGLU_BWD || epilogue == EPI_GELU_BWD) return false; // those have no such kernel
+    const double experts = E * (1. - pow(1. - 1. / E, (double)M)), columns = (N + ST_N - 1) / ST_N, workgroups = experts * columns;
+    const double at_once = 256 * (FD_STAGES / fr_deep_stages(K)), most = (double)(M < E ? M : E) * columns;
+    if (workgroups > (most > at_once ? at_once * 15 / 16 : at_once)) return false;
+    if ((fr_tile_splits(N, K, E, 0) >= 3 || !fr_beyond_vector(M, K, E, 0)) && workgroups < FR_DEEP_LONG_FROM) return false;
+    return fr_deep_two_waves(M, N, E) || 2 * experts < E || (K > 4 * ST_K_NT && K < 8 * ST_K_NT);
+}
+
+inline bool fr_takes_tile(int64_t M, int N, int K, int E, int w_is_kn, int epilogue) {
+    return fr_beyond_vector(M, K, E, w_is_kn) || fr_deep_shape(M, N, K, E, w_is_kn, epilogue);
+}
+
+// More rows than the small tile takes in one pass go to the 128 x 256 tiles of mid_rows.hip, where those have the variant.  8
+// experts of H = 2048, I = 8192, 32 rows each, up- / down-projection: 132 -> 102 / 61 -> 55 us against a small tile of 128 rows that
+// stood here; 128 experts of H = 2048, I = 768, 64 rows: 190 -> 166 / 103 -> 90.
+inline bool fr_takes_mid(const FwdArgs &a, int w_is_kn, int epilogue) {
+    return a.M > (int64_t)MID_ROWS_FWD_FROM * a.E && xma_rocm::mid_fwd_takes(a, w_is_kn, epilogue);
 }
 
 template <typename T, int EPI> int fr_launch_epilogue(const FwdArgs &a, const float *part, int S, hipStream_t st) {
@@ -810,9 +827,7 @@ template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, floa
                 kernel<<<grid, 64 * waves, fr_deep_stages(a.K) * fd_stage(waves), st>>>(a);
                 return xma_check_launch("fr_deep_kernel");
             };
-            // 64 columns where that still is at most one workgroup per compute unit (64 experts, K = 1408, N = 2048, one token 12.4 -> 11.2 us;
-            // with 264 workgroups instead of 132 18.4 -> 29.4)
-            return (a.M < a.E ? a.M : a.E) * ((a.N + 63) / 64) <= 256 ? run(fr_deep_kernel<T, EPI, 2>, 2) : run(fr_deep_kernel<T, EPI, 4>, 4);
+            return fr_deep_two_waves(a.M, a.N, a.E) ? run(fr_deep_kernel<T, EPI, 2>, 2) : run(fr_deep_kernel<T, EPI, 4>, 4);
         }
     }
     const int S_max = part ? fr_tile_splits(a.N, a.K, a.E, WT) : 1;

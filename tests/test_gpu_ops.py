@@ -1043,6 +1043,53 @@ def test_forward_gemm_of_few_workgroups(dtype, counts, K, N):
     assert ((h.double() - want).abs() <= (unit + 2.0**-20) * want.abs() + 2.0**-24).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "counts,K,N",
+    [  # four waves, 128 columns: more steps than stages, K tails and N remainders; a second pass of rows
+        ([1 if e % 5 == 0 else 0 for e in range(60)], 1032, 1424),
+        ([0] * 20 + [33] + [0] * 20 + [1, 2, 34], 520, 2064),
+        ([3, 9, 1, 40, 5, 0, 2, 4], 776, 3600),  # rows for most experts
+        ([1 if e % 11 == 5 else 0 for e in range(64)], 2048, 2832),  # 16 steps, in the place of the vector kernel
+        # two waves, as many steps
+        ([0] * 30 + [1, 1, 1] + [0] * 30 + [1], 2040, 4048),
+    ],
+)
+def test_forward_gemm_of_four_k_steps_in_flight(dtype, counts, K, N):
+    """the forms of that kernel which the launches above do not reach: rows gathered from tokens (fan_out 2) with SwiGLU, and both forms of
+    GELU, against the products in 64 bits"""
+    from xma.rocm import ops
+
+    print(f"four steps in flight E={len(counts)} K={K} N={N} {dtype}", flush=True)
+    counts = [*counts[:-1], counts[-1] + sum(counts) % 2]
+    E, M = len(counts), sum(counts)
+    assert ops._few_rows_fwd(M, N, K, E, 0, K, M * K, dtype, ops.EPI_SWIGLU) and ops._few_rows_workspace_bytes(M, N, K, E, 0, ops.EPI_SWIGLU) == 0
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    nan = lambda *s: torch.full(s, float("nan"), device="cuda", dtype=dtype)
+    offs, idx = torch.tensor(counts, device="cuda").cumsum(0), torch.randperm(M, device="cuda", generator=g)
+    X, W, b = new(M // 2, K), new(E, N, K) * 0.05, new(E, N)
+    e = torch.repeat_interleave(torch.arange(E, device="cuda"), torch.tensor(counts, device="cuda")).tolist()
+    unit = 2.0 ** {torch.bfloat16: -8, torch.float16: -11}[dtype]
+    product = lambda f: torch.stack([f(X[idx[i] // 2].double()) @ f(W[e[i]].double()).t() + f(b[e[i]].double()) for i in range(M)])
+    want, size = product(lambda t: t), product(torch.abs)
+
+    def near(z):
+        return ((z.double() - want).abs() <= unit * want.abs() + (K + 2) * 2.0**-24 * size + 2.0**-24).all()
+
+    z, h = nan(M, N), nan(M, N // 2)
+    ops.up_projection_swiglu_rocm(X, W.permute(0, 2, 1), idx, offs, z, h, 2, b)
+    gate, up = z.double()[:, ::2], z.double()[:, 1::2]
+    act = up * gate * torch.sigmoid(gate)
+    assert near(z) and ((h.double() - act).abs() <= (unit + 2.0**-20) * act.abs() + 2.0**-24).all()
+    for form, (epi, _) in ops.EPI_GELU.items():
+        z, h = nan(M, N), nan(M, N)
+        ops._scatter2scatter(X, W.permute(0, 2, 1), idx, offs, z, h, None, 2, False, True, epi, M, N, K, b)
+        act = torch.nn.functional.gelu(z.double(), approximate=form)
+        # a few units of fp32 of the argument, whose own size is that of z
+        assert near(z) and ((h.double() - act).abs() <= unit * act.abs() + 2.0**-18 * (1 + z.double().abs())).all()
+
+
 def test_few_rows_beyond_32_bit_offsets_leaves_the_workspace_alone():
     """rows of X that only the small tile's 64-bit addresses reach, in a shape whose usual kernel asks for no workspace: a workspace of
     another purpose stays as it is (the small tile would cut this K in two ranges and leave their sums there)"""

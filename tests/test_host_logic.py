@@ -242,6 +242,21 @@ def test_few_token_dispatch_rule():
     assert ops._few_rows(14, 8, torch.float16, "dy @ W")
 
 
+def test_which_few_row_launches_are_cut_along_k():
+    """the kernel with four K steps in flight cuts nothing, so the workspace says which launches of x @ W^T it takes among those that the
+    small tile would cut: not where that makes three or four K ranges of few workgroups (measured 9 -> 15 us, 4 experts of 64 rows)"""
+    from xma.rocm import get_library
+
+    need = lambda M, N, K, E, epi=0: get_library().xma_rocm_scatter2scatter_few_rows_workspace_bytes(M, N, K, E, 0, epi)
+    for epi in (0, 1):
+        assert need(64, 512, 2048, 4, epi) == 4 * 64 * 512 * 4 and need(16, 512, 1536, 4, epi) == 3 * 16 * 512 * 4
+        assert need(64, 512, 1408, 4, epi) == 0 and need(32, 1024, 1024, 8, epi) == 0  # two ranges against none
+        assert need(16, 4096, 2048, 4, epi) == 0  # half of the compute units have work
+        # four waves with rows for most experts: only K between 512 and 1024, which the small tile would not cut either
+        assert need(128, 1024, 1024, 32, epi) == 2 * 128 * 1024 * 4 and need(128, 1024, 1016, 32, epi) == 0
+    assert need(64, 512, 8192, 8) and need(12, 2816, 2048, 64) == 0  # K beyond; the vector kernel
+
+
 def test_mid_rows_dispatch_rule():
     """which launches beyond the few-token limits take the few-row entry points for their 128 x 256 tiles"""
     from xma.rocm import ops
