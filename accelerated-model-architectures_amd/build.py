@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT_DIR = os.path.join(HERE, "xma", "rocm")
 LIB = os.path.join(OUT_DIR, "libxma_rocm.so")
-SOURCES = ["api.hip", "routing.hip", "elementwise.hip", "grouped_gemm.hip", "mid_rows.hip", "grouped_gemm_staged.hip", "fp32.hip", "router.hip", "gate.hip", "swiglu.hip", "bias.hip", "few_rows.hip", "layer.hip", "diagnostics.hip"]
+SOURCES = ["grouped_gemm.hip", "grouped_gemm_f16.hip", "mid_rows.hip", "api.hip", "routing.hip", "elementwise.hip", "grouped_gemm_staged.hip", "fp32.hip", "router.hip", "gate.hip", "swiglu.hip", "bias.hip", "few_rows.hip", "layer.hip", "diagnostics.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -41,7 +41,7 @@ FLAGS = [
 # the destination of such a load before the wait, or if a loop of MFMAs without an inner loop accesses scratch memory (spills;
 # those outside such loops are reported with the kernel's registers).  It also says so if the compiler is not the version the
 # kernels were written and measured with.
-CHECK_ISA = {"grouped_gemm.hip": re.compile(r"grouped_gemm"), "mid_rows.hip": re.compile(r"mid_\w+_kernel")}
+CHECK_ISA = {"grouped_gemm.hip": re.compile(r"grouped_gemm"), "grouped_gemm_f16.hip": re.compile(r"grouped_gemm"), "mid_rows.hip": re.compile(r"mid_\w+_kernel")}
 TESTED_HIPCC = "7.2"
 USAGE_REPORT = os.path.join(HERE, "build", "kernel_resource_usage.txt")
 

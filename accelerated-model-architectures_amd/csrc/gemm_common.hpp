@@ -61,5 +61,9 @@ __device__ __forceinline__ int xcd_remap(int bid, int grid) {
 // Raises a kernel's dynamic-LDS limit; the attribute belongs to (kernel, device) and is set on the first launch only.
 template <typename K> inline int gemm_set_smem(K kernel, int bytes) { return xma_set_max_lds_once((const void *)kernel, bytes); }
 
+// the 256 x 256 kernels for fp16 (grouped_gemm_f16.hip)
+int grouped_fwd_f16(const FwdArgs &a, int wt, int epi, hipStream_t st);
+int grouped_dw_f16(const DwArgs &a, int grid, hipStream_t st);
+
 // dW with a per-token scale on dY (register-staged loader, grouped_gemm_staged.hip)
 int launch_dw_scaled(const DwArgs &a, int dtype, int grid, hipStream_t st);

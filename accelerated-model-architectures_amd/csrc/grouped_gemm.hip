@@ -1649,6 +1649,11 @@ inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 using namespace xma_rocm;
 
+#ifdef XMA_GROUPED_GEMM_F16 // the kernels for fp16 are a translation unit of their own (grouped_gemm_f16.hip), without the entry points
+int grouped_fwd_f16(const FwdArgs &a, int wt, int epi, hipStream_t st) { return dispatch_fwd<_Float16>(a, wt, epi, st); }
+int grouped_dw_f16(const DwArgs &a, int grid, hipStream_t st) { return dispatch_dw<_Float16>(a, grid, st); }
+#else
+
 static int scatter2scatter_impl(const void *X, int64_t ldx, const void *W, int64_t w_expert_stride, int64_t ldw,
                                 int w_is_kn, const int64_t *sorted_scattered_idxs, const int64_t *expert_offsets,
                                 void *out, int64_t ldo, void *aux, int64_t ldaux, void *aux2, int64_t ldaux2,
@@ -1737,7 +1742,7 @@ static int scatter2scatter_impl(const void *X, int64_t ldx, const void *W, int64
     }
     hipStream_t st = (hipStream_t)stream;
     if (dtype == XMA_ROCM_BF16) return dispatch_fwd<__bf16>(a, w_is_kn ? 1 : 0, epilogue, st);
-    return dispatch_fwd<_Float16>(a, w_is_kn ? 1 : 0, epilogue, st);
+    return grouped_fwd_f16(a, w_is_kn ? 1 : 0, epilogue, st);
 }
 
 extern "C" int xma_rocm_scatter2scatter(const void *X, int64_t ldx, const void *W, int64_t w_expert_stride, int64_t ldw,
@@ -1894,5 +1899,6 @@ extern "C" int xma_rocm_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped
     if (dtype == XMA_ROCM_F32) return f32_group_bwd_W(a, st);
     if (dy_scale) return launch_dw_scaled(a, dtype, (int)grid, st);
     if (dtype == XMA_ROCM_BF16) return dispatch_dw<__bf16>(a, (int)grid, st);
-    return dispatch_dw<_Float16>(a, (int)grid, st);
+    return grouped_dw_f16(a, (int)grid, st);
 }
+#endif
