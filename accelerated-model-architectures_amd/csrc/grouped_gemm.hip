@@ -481,7 +481,7 @@ constexpr int ROLE_TILES = 0, ROLE_SLICES = 1, ROLE_FIXUP = 2;
 // the kernel of the K slices.  Its SwiGLU-backward instantiations also walk several tiles per workgroup (one workgroup
 // per compute unit), the others run one workgroup per tile.
 __host__ __device__ constexpr bool fwd_persistent(int epi, int role) {
-    return role == ROLE_TILES && (epi == XMA_ROCM_EPI_SWIGLU_BWD || epi == EPI_SWIGLU_BWD_SCALED_ACT);
+    return role == ROLE_TILES && epi_swiglu_bwd(epi);
 }
 template <int ROLE>
 __device__ __forceinline__ bool locate_tile(const FwdArgs &a, unsigned char *smem, int *s_sched, TileSched &ts,
@@ -1612,6 +1612,7 @@ template <typename T> int dispatch_fwd(const FwdArgs &a, int wt, int epi, hipStr
     }
     if (epi == XMA_ROCM_EPI_STORE) return launch_fwd<T, 1, XMA_ROCM_EPI_STORE>(a, st);
     if (epi == XMA_ROCM_EPI_SWIGLU) return launch_fwd<T, 1, XMA_ROCM_EPI_SWIGLU>(a, st);
+    if (a.dots) return a.aux2 ? launch_fwd<T, 1, EPI_SWIGLU_BWD_SCALED_ACT_DOTS>(a, st) : launch_fwd<T, 1, EPI_SWIGLU_BWD_DOTS>(a, st);
     if (a.aux2) return launch_fwd<T, 1, EPI_SWIGLU_BWD_SCALED_ACT>(a, st);
     return launch_fwd<T, 1, XMA_ROCM_EPI_SWIGLU_BWD>(a, st);
 }

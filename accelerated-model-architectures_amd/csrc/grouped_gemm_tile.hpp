@@ -29,6 +29,13 @@ constexpr int EPI_Z_STRIDE = 128 * 2 + 16, EPI_H_STRIDE = 64 * 2 + 16;
 // Internal epilogue code beside the public XMA_ROCM_EPI_*: SWIGLU_BWD with the second output FwdArgs::aux2.  A variant of
 // its own, so that the launches without that output keep their code and register allocation unchanged.
 constexpr int EPI_SWIGLU_BWD_SCALED_ACT = 3;
+// And both of them with the gradient of the row scale, FwdArgs::dots (256-row tiles).  Compiled into the launches that do not ask for it, its
+// arithmetic made them 1.00 - 1.03 times as long as the kernel ahead of it, without it they are 0.95 - 1.00 (262144 rows of H = 2048, I = 768
+// 897 -> 904 us with it, 911 -> 893 without, in turn on two boxes; 24000 of H = 512, I = 1032 68.8 -> 69.8, 70.0 -> 66.2).
+constexpr int EPI_SWIGLU_BWD_DOTS = 8, EPI_SWIGLU_BWD_SCALED_ACT_DOTS = 9;
+__host__ __device__ constexpr bool epi_dots(int epi) { return epi == EPI_SWIGLU_BWD_DOTS || epi == EPI_SWIGLU_BWD_SCALED_ACT_DOTS; }
+__host__ __device__ constexpr bool epi_scaled_act(int epi) { return epi == EPI_SWIGLU_BWD_SCALED_ACT || epi == EPI_SWIGLU_BWD_SCALED_ACT_DOTS; }
+__host__ __device__ constexpr bool epi_swiglu_bwd(int epi) { return epi == XMA_ROCM_EPI_SWIGLU_BWD || epi_scaled_act(epi) || epi_dots(epi); }
 // z and h = gelu(z), both (M, N); dz = gelu'(z) d h: FwdArgs::erf_form says which GELU
 constexpr int EPI_GELU = XMA_ROCM_EPI_GELU_TANH, EPI_GELU_BWD = XMA_ROCM_EPI_GELU_TANH_BWD;
 constexpr int EPI_WAVE_BYTES = 32 * EPI_Z_STRIDE + 32 * EPI_H_STRIDE;
@@ -180,7 +187,7 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
             blocks(IC<1>{});
         else
             blocks(IC<0>{});
-    } else if constexpr (EPI != XMA_ROCM_EPI_SWIGLU_BWD && EPI != EPI_SWIGLU_BWD_SCALED_ACT) {
+    } else if constexpr (!epi_swiglu_bwd(EPI)) {
         // A store instruction of the accumulator layout would touch 32 rows with 16 bytes each.  Instead every
         // 32-row block goes through a wave-private LDS area and leaves as whole rows: 16 lanes x 16 bytes per row of
         // 128 columns (8 lanes per row of the 64 activation columns), i.e. full 128-byte lines.
@@ -341,9 +348,9 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
         unsigned char *stage = smem + wave * EPI_BWD_WAVE_BYTES;
         unsigned char *row_io = stage + (lane >> 5) * EPI_BWD_STRIDE + (lane & 31) * 16; // + 2 it rows (way in)
         unsigned char *mine = stage + lrow * EPI_BWD_STRIDE + lhalf * 16;                // + (32 j + 8 g) * 4 bytes
-        // Loads and stores of this epilogue are unconditional: a lane whose row or column lies outside the tile's valid
-        // part repeats the access of a lane inside it (same address, and for stores the same data, read from the same place
-        // of the staging area).  Memory operations under a per-lane condition sit in branches, and the compiler then waits
+        // Loads and stores of this epilogue are unconditional: a lane whose column lies outside the tile's valid part, and without FIT one
+        // whose row does, repeats the access of a lane inside it (same address, and for stores the same data, read from the same place
+        // of the staging area); with FIT a row outside lies outside the buffer.  Memory operations under a per-lane condition sit in branches, and the compiler then waits
         // for all of them (vmcnt(0)) where it would otherwise count: every block would wait for the stores of the one
         // before it to complete before it could bring its own rows of z into LDS.
         // this wave's 128 columns lie past N: nothing to do, and nothing in here joins other waves (the value is uniform;
@@ -356,9 +363,10 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
         // multiply-add per value, an exchange between the row's two lanes and 4 bytes per row and wave.  A pass over the expert outputs
         // that forms it as <dy, expert_out> reads k T H of them again.  Forward + backward, 262144 rows of H = 2048, I = 768: 7861 -> 7695 us;
         // 98304 of I = 1408: 5547 -> 5510; 16384 of H = 4096, I = 14336: equal.
-        const bool dots = NI == 4 && a.dots != nullptr;
+        constexpr bool dots = epi_dots(EPI);
+        static_assert(!dots || NI == 4, "the 256-row tiles only");
         const int cols = a.N - (n0 + wp); // columns from here on are not the wave's: what they hold is dropped
-        // no condition on these stores either: without dots, and for the rows past the last valid one, they lie outside the buffer
+        // no condition on these stores either: for the rows past the last valid one they lie outside the buffer
         const __amdgpu_buffer_rsrc_t dots_b = uniform_buffer(a.dots, dots ? a.dots_bytes : 0u);
         int idx_i[4] = {0, 0, 0, 0};
 #pragma unroll
@@ -433,9 +441,9 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                         const float sg = sigmoidf_fast(gg), silu = gg * sg;
                         o[q] = Elem<T>::pack(dh * uu * (sg + silu * (1.f - sg)), dh * silu);
                         hv[q] = uu * silu * sc;
-                        if constexpr (NI == 4) dq += acc[j][i][4 * g + q] * (uu * silu);
+                        if constexpr (dots) dq += acc[j][i][4 * g + q] * (uu * silu);
                     }
-                    if constexpr (NI == 4) dot += (j * 32 + g * 8 < cols) ? dq : 0.f; // uniform: N is a multiple of 8
+                    if constexpr (dots) dot += (j * 32 + g * 8 < cols) ? dq : 0.f; // uniform: N is a multiple of 8
                     *zp = o;
                     if constexpr (HS.value != 0) {
                         hs[2 * (j * 4 + g)] = park(Elem<T>::pack(hv[0], hv[1]));
@@ -455,7 +463,7 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
                 const u32x4 v = *(const u32x4 *)(stage + br * EPI_BWD_STRIDE + piece * 16);
                 *(u32x4 *)(a.out + (row0 + wq + i * 32 + br) * a.ldo + cz) = v;
             }
-            if constexpr (NI == 4) {
+            if constexpr (dots) {
                 dot += __shfl_xor(dot, 32);
                 const uint32_t at = mul_add_u32((uint32_t)idx_i[i], a.dots_ld, (uint32_t)(n0 + wp) >> 7) * 4;
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, dot), dots_b, wq + i * 32 + lrow < rows_valid ? at : BUF_OUTSIDE, 0, 0);
@@ -487,7 +495,7 @@ __device__ __forceinline__ void tile_epilogue(const FwdArgs &a, f32x16 (&acc)[4]
             }
         }
         };
-        blocks(IC<(EPI == EPI_SWIGLU_BWD_SCALED_ACT) ? 1 : 0>{});
+        blocks(IC<epi_scaled_act(EPI) ? 1 : 0>{});
     }
 }
 
