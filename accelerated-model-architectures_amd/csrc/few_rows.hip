@@ -775,18 +775,23 @@ inline bool fr_beyond_vector(int64_t M, int K, int E, int w_is_kn) {
     return w_is_kn || M > (int64_t)FR_NT_VALU_ROWS_PER_EXPERT * E || M > FR_NT_VALU_ROWS || K < FR_NT_PIECE;
 }
 
-// Where the kernel with four K steps in flight takes x @ W^T.  Measured against the kernel that takes the launch otherwise, us with the weights in
-// the Infinity Cache / behind a read of 512 MB, over 4545 launches of 1 to 128 experts, 1 to 96 tokens, K = 64 to 2048, N = 128 to 4096: 0.985 / 0.923
-// of the time over all of them, 0.978 / 0.89 over its own, 99 in 100 within 1.17 / 1.03.
+// Rows of W per workgroup of the vector kernel: one pair per wave instead of four where the rows are short or the launch would have few workgroups
+inline int fr_nt_rows(int N, int K, int E) { return K >= FR_NT_PIECE && (int64_t)(N / FR_NT_ROWS) * E >= 2048 ? FR_NT_ROWS : 8; }
+
+// Where the kernel with four K steps in flight takes x @ W^T.  Measured against the kernel that takes the launch otherwise, time with the weights in
+// the Infinity Cache / from HBM, uneven loads (logits with a spread of 1.5 between experts) as often as even ones, 4 to 128 experts, 1 to 1500
+// rows, K = 256 to 2048, N = 128 to 4800; 567 launches that it takes 0.82 / 0.93, 99 in 100 within 1.06 / 1.16; 453 that this rule leaves 0.99 / 1.09.
 //  * As many workgroups with work as run at the same time, counting the experts that M random choices of E hit, with a margin unless there cannot be
-//    more: 64 experts, K = 2048, N = 2816, 12 rows (242 expected, up to 264) 29 / 34 -> 38 / 47.
-//  * It walks K alone, at 0.9 us a step.  Instead of three or four K ranges, or of the vector kernel, only in launches of half the compute
-//    units, where those stream more than they wait: 2 experts, K = 2048, N = 1024, one row 4.6 / 10 -> 14 / 18; up to 32 workgroups
-//    in three ranges (K = 1536) 9 / 14 -> 13 / 16, in four (K = 2048) 9 / 14 -> 15 / 18; from 112 workgroups on 0.9 - 1.1 / 0.9 - 1.05.  Of two ranges:
-//    down-projections 1.0 / 0.9, SwiGLU launches of up to 64 workgroups (K = 1024) 8.9 / 13.8 -> 9.9 / 13.6.
+//    more: 64 experts, K = 2048, N = 2816, 12 rows (242 expected, up to 264) 29 / 34 -> 38 / 47 us.
+//  * It walks K alone, at 0.9 us a step for every 32 rows of an expert.  Never instead of three or four K ranges: 1.13 / 1.15, and where one expert has
+//    most rows (60 experts, K = 2048, N = 168, 1254 rows, 215 of them one expert's) 45 -> 82.  Of two ranges 0.87 / 0.98 up to eight rows per expert on
+//    average (beyond, uneven loads 1.0 - 1.17), but SwiGLU and GELU from 32 workgroups on: below 0.93 / 1.09.
+//  * The vector kernel is slow where its workgroups take 32 rows of W each and some expert has two rows of X or more: 0.81 / 0.91 there, with no more
+//    workgroups than run at once (16 experts, N = 4720, 7 rows, up to 259 of them: 29 / 34 -> 38 / 52) and less than half as many rows as experts
+//    (beyond, 0.87 / 1.1 for even loads).  Where they take 8, 1.07 / 1.19.
 //  * With four waves where most experts have rows only for K between 512 and 1024: there 1.03 / 0.93, below (K <= 512) 1.12 / 1.00, above 1.04 / 1.00.
 //    Where most have none the small tile starts a workgroup for each of them: 0.87 / 0.85.
-constexpr int FR_DEEP_K = 2048, FR_DEEP_LONG_FROM = 112;
+constexpr int FR_DEEP_K = 2048, FR_DEEP_ROWS_PER_EXPERT_OF_TWO_RANGES = 8, FR_DEEP_ACTIVATION_FROM = 32;
 inline int fr_deep_stages(int K) { const int steps = (K + ST_K_NT - 1) / ST_K_NT; return steps < FD_STAGES ? steps : FD_STAGES; }
 // two waves, 64 columns, where that still is at most one workgroup per compute unit, or four (64 experts, K = 1408, N = 2048, one
 // token 12.4 -> 11.2 us; with 264 workgroups instead of 132 18.4 -> 29.4)
@@ -796,7 +801,13 @@ inline bool fr_deep_shape(int64_t M, int N, int K, int E, int w_is_kn, int epilo
     const double experts = E * (1. - pow(1. - 1. / E, (double)M)), columns = (N + ST_N - 1) / ST_N, workgroups = experts * columns;
     const double at_once = 256 * (FD_STAGES / fr_deep_stages(K)), most = (double)(M < E ? M : E) * columns;
     if (workgroups > (most > at_once ? at_once * 15 / 16 : at_once)) return false;
-    if ((fr_tile_splits(N, K, E, 0) >= 3 || !fr_beyond_vector(M, K, E, 0)) && workgroups < FR_DEEP_LONG_FROM) return false;
+    const int ranges = fr_tile_splits(N, K, E, 0);
+    if (!fr_beyond_vector(M, K, E, 0)) {
+        if (fr_nt_rows(N, K, E) < FR_NT_ROWS || most > at_once || 2 * M >= E) return false;
+    } else if (ranges > 2 || (ranges == 2 && (M > (int64_t)FR_DEEP_ROWS_PER_EXPERT_OF_TWO_RANGES * E ||
+                                              (epilogue != XMA_ROCM_EPI_STORE && workgroups < FR_DEEP_ACTIVATION_FROM)))) {
+        return false;
+    }
     return fr_deep_two_waves(M, N, E) || 2 * experts < E || (K > 4 * ST_K_NT && K < 8 * ST_K_NT);
 }
 
@@ -847,8 +858,7 @@ template <typename T, int WT, int EPI> int fr_launch_tile(const FwdArgs &a, floa
 template <typename T, int EPI> int fr_launch_epi(const FwdArgs &a, int w_is_kn, float *part, hipStream_t st) {
     int rc;
     if (fr_takes_tile(a.M, a.N, a.K, a.E, w_is_kn, EPI)) return w_is_kn ? fr_launch_tile<T, 1, EPI>(a, part, st) : fr_launch_tile<T, 0, EPI>(a, part, st);
-    // one pair of rows per wave instead of four where the rows are short or the launch would have few workgroups
-    const int rows_per_wg = (a.K >= 2048 && (int64_t)(a.N / FR_NT_ROWS) * a.E >= 2048) ? FR_NT_ROWS : 8;
+    const int rows_per_wg = fr_nt_rows(a.N, a.K, a.E);
     const dim3 grid((a.N + rows_per_wg - 1) / rows_per_wg, a.E);
     if constexpr (EPI == XMA_ROCM_EPI_SWIGLU_BWD || EPI == EPI_GELU_BWD) {
         fr_nt_kernel<T, -1><<<grid, FR_THREADS, 0, st>>>(a, part, rows_per_wg);

@@ -1048,11 +1048,12 @@ def test_forward_gemm_of_few_workgroups(dtype, counts, K, N):
     "counts,K,N",
     [  # four waves, 128 columns: more steps than stages, K tails and N remainders; a second pass of rows
         ([1 if e % 5 == 0 else 0 for e in range(60)], 1032, 1424),
-        ([0] * 20 + [33] + [0] * 20 + [1, 2, 34], 520, 2064),
+        ([0] * 20 + [33] + [0] * 20 + [1, 2, 34], 520, 720),
         ([3, 9, 1, 40, 5, 0, 2, 4], 776, 3600),  # rows for most experts
         ([1 if e % 11 == 5 else 0 for e in range(64)], 2048, 2832),  # 16 steps, in the place of the vector kernel
-        # two waves, as many steps
+        # two waves, as many steps; a second pass of rows
         ([0] * 30 + [1, 1, 1] + [0] * 30 + [1], 2040, 4048),
+        ([0] * 20 + [33] + [0] * 20 + [1, 2, 34], 776, 272),
     ],
 )
 def test_forward_gemm_of_four_k_steps_in_flight(dtype, counts, K, N):

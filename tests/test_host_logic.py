@@ -244,14 +244,17 @@ def test_few_token_dispatch_rule():
 
 def test_which_few_row_launches_are_cut_along_k():
     """the kernel with four K steps in flight cuts nothing, so the workspace says which launches of x @ W^T it takes among those that the
-    small tile would cut: not where that makes three or four K ranges of few workgroups (measured 9 -> 15 us, 4 experts of 64 rows)"""
+    small tile would cut: not where that makes three or four K ranges, nor of two where one expert may have several times 32 rows (measured
+    45 -> 82 us), nor with an activation behind fewer than 32 workgroups"""
     from xma.rocm import get_library
 
     need = lambda M, N, K, E, epi=0: get_library().xma_rocm_scatter2scatter_few_rows_workspace_bytes(M, N, K, E, 0, epi)
     for epi in (0, 1):
         assert need(64, 512, 2048, 4, epi) == 4 * 64 * 512 * 4 and need(16, 512, 1536, 4, epi) == 3 * 16 * 512 * 4
-        assert need(64, 512, 1408, 4, epi) == 0 and need(32, 1024, 1024, 8, epi) == 0  # two ranges against none
-        assert need(16, 4096, 2048, 4, epi) == 0  # half of the compute units have work
+        assert need(16, 4096, 2048, 4, epi) == 4 * 16 * 4096 * 4 and need(1008, 320, 2000, 45, epi) == 4 * 1008 * 320 * 4
+        # two ranges: up to eight rows per expert
+        assert need(64, 1024, 1024, 8, epi) == 0 and need(65, 1024, 1024, 8, epi) == 2 * 65 * 1024 * 4
+        assert need(32, 512, 1408, 4, epi) == epi * 2 * 32 * 512 * 4
         # four waves with rows for most experts: only K between 512 and 1024, which the small tile would not cut either
         assert need(128, 1024, 1024, 32, epi) == 2 * 128 * 1024 * 4 and need(128, 1024, 1016, 32, epi) == 0
     assert need(64, 512, 8192, 8) and need(12, 2816, 2048, 64) == 0  # K beyond; the vector kernel
