@@ -95,7 +95,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_buffer(const void *p, 
 // The rows of a tile in one of its grouped matrices: 16-byte accesses at row, by 32-bit offsets from the tile's first row.  What lies past
 // the last valid row is outside the buffer: loads read zeros and stores are dropped, so no row is clamped, and an address is one addition
 // where 64-bit ones take a clamp and a product each, a fifth of the instructions of the SwiGLU backward's epilogue.  On its own that
-// gives those launches nothing (board power, and the rows' own traffic); it makes room for `dots`.
+// gives those launches nothing (the epilogue's vector ALU is busy for 0.6 of it either way); it makes room for `dots`.
 struct RowBuffer {
     __amdgpu_buffer_rsrc_t rsrc;
     uint32_t lane_off, ld_bytes;

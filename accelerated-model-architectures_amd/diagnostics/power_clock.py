@@ -1,7 +1,7 @@
 """Board power while a kernel runs in a loop: the MFMA-only stream, the grouped GEMMs of the Mixtral-shaped layer and the
 stock dense GEMM of the same sizes.
 
-    python accelerated-model-architectures_amd/diagnostics/power_clock.py        (on the GPU box)
+    python accelerated-model-architectures_amd/diagnostics/power_clock.py        (on the MI355X)
 
 Each kernel is launched back to back for a few seconds while a thread samples the board's power sensor
 (/sys/class/drm/card*/device/hwmon/hwmon*/power1_input, microwatts) every 20 ms; the first third of the samples is

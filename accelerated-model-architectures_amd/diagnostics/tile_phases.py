@@ -1,7 +1,7 @@
 """Where a tile of the persistent grouped GEMM kernel spends its time, in shader cycles and microseconds.
 
     python accelerated-model-architectures_amd/build.py --timing       (here, no GPU needed)
-    python accelerated-model-architectures_amd/diagnostics/tile_phases.py [c3] [c4] [c5]    (on the GPU box)
+    python accelerated-model-architectures_amd/diagnostics/tile_phases.py [c3] [c4] [c5]    (on the MI355X)
 
 The timing build of the library (xma/rocm/libxma_rocm_timing.so, grouped_gemm.hip compiled with -DXMA_PST_TIMING) makes
 thread 0 of every workgroup read the 100 MHz real-time counter and the shader clock counter at six points of each of its
