@@ -40,6 +40,10 @@ int xma_down_projection_dx_dots(const void *dY, int64_t lddy, const void *W, int
                                 int64_t lddz, void *scaled_act, int64_t ld_scaled_act, const void *row_scale, int64_t M, int32_t N,
                                 int32_t K, int32_t E, int32_t fan_out, int dtype, void *workspace, size_t workspace_bytes, void *stream,
                                 float *dots);
+// xma_rocm_group_bwd_W with the number of rows in all, by which fp32 launches pick their tile; 0: not known (grouped_gemm.hip)
+int xma_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped, int32_t dy_fan_out, const void *dy_scale, const void *X, int64_t ldx, int x_grouped,
+                    int32_t x_fan_out, const int64_t *sorted_scattered_idxs, const int64_t *expert_offsets, void *DW, int64_t dw_expert_stride,
+                    int64_t lddw, int32_t N_out, int32_t K_in, int32_t E, int64_t M, int dtype, void *stream);
 // xma_rocm_gate_bwd, whose last kernel also sums the k slots of `scattered` (may be NULL); every rule of its arguments, without a launch (gate.hip)
 int xma_gate_bwd_check(const char *what, const void *x, int64_t ldx, const void *gate_weight, const void *d_sel, const int32_t *ids,
                        const void *scattered, const void *d_x, const void *d_gate, int64_t T, int32_t H, int32_t E, int32_t k, int dtype,

@@ -9,9 +9,8 @@
 //   dW           :  Q = dY columns (out features), P = X columns (in features), K = tokens of the expert
 // The MFMA "A" operand is the P fragment, so a lane owns output row (lane & 31) of a 32 x 32 block and four
 // consecutive columns per accumulator quad.
-#include <math.h>
-
 #include "fp32.hpp"
+#include "fp32_tiles.hpp"
 #include "row_dot.hpp"
 
 namespace {
@@ -24,7 +23,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // is 2048 cycles of matrix pipe behind one step's loads.  The small one has 1024 and keeps the loads of two steps in
 // flight: its launches have one or two workgroups per compute unit, so nothing else covers the latency.
 template <int TB> struct Tile {
-    static constexpr int DIM = 64 * TB, BK = 32 / TB, SETS = 3 - TB;
+    static constexpr int DIM = 64 * TB, BK = f32_tile_step(64 * TB), SETS = 3 - TB;
     static constexpr int LD = DIM + 4; // floats per k-row of an LDS tile [BK][DIM + 4]: 16-byte aligned rows, conflict-free columns
     // K-contiguous source ([row][k]): 2 or 4 neighbouring threads share a row, two float4 per thread
     static __device__ __forceinline__ int row(int tid) { return TB == 2 ? tid >> 1 : tid >> 2; }
@@ -454,34 +453,10 @@ template <int WT, int TB> int launch_gemm(const FwdArgs &a, int epi, int grid, h
     return run(gemm_f32_kernel<WT, XMA_ROCM_EPI_SWIGLU_BWD, TB>);
 }
 
-// Which tile.  The small one pays where the large ones leave compute units idle, below two per unit, and where they are padding by more
-// than the small one's extra traffic through LDS is worth: an expert of random load ends in half a tile on average, of 128 rows or of 64.
-// Results are bit-identical.  Large / small tile in us (x @ W^T; dy @ W).  Rows: 64 experts of K = 1024, N = 2048, 30 rows each 287 / 162;
-// 286 / 166, 90 rows (one large tile or two) 303 / 325; 296 / 339; 128 of K = 576, N = 512, 125 rows 128 / 114; 127 / 116, 250 rows 212 /
-// 199; 207 / 202, 500 rows 379 / 378; 367 / 372, 1000 rows 689 / 706; 677 / 710; 30 of K = 400, N = 1200, 300 rows 122 / 99; 121 / 102; 16 of
-// K = 1024, N = 4096, 250 rows 352 / 326; 350 / 340.  Tiles: 8 experts of K = 2048, N = 512, 256 tiles 168 / 150; 174 / 155, 512 of them 293 /
-// 295; 284 / 299, of K = 512, N = 2048, 4096 tiles 563 / 602; 558 / 622.
-constexpr int64_t F32_SMALL_TILES = 512;
-constexpr double F32_SMALL_WORSE = 1.04;
-// dW: the reduction is the expert's rows.  8 experts of 500 rows, 256 tiles 62 / 52, 512 tiles 96 / 109; 1000 x 2048 x 2048 4 experts 309 / 343;
-// 128 of 576 x 512, 500 rows 413 / 427; padded by a fifth, 30 of 1200 x 400, 300 rows 141 / 116, 700 rows 285 / 251.
-constexpr int F32_SMALL_TILES_DW = 512;
-constexpr double F32_SMALL_WORSE_DW = 1.12;
-inline int64_t f32_tiles(int64_t m, int64_t n, int dim) { return ((m + dim - 1) / dim) * ((n + dim - 1) / dim); }
-inline double f32_padded(int64_t n, int dim) { return (double)((n + dim - 1) / dim * dim); }
-// rows that tiles of `dim` multiply for an expert of about `rows` (within two standard deviations of a random load)
-inline double f32_padded_load(double rows, int dim) {
-    const double lo = ceil((rows - 2 * sqrt(rows)) / dim), hi = ceil((rows + 2 * sqrt(rows)) / dim);
-    return dim * (lo == hi ? hi : rows / dim + 0.5);
-}
-
 } // namespace
 
 int f32_scatter2scatter(const FwdArgs &a, int w_is_kn, int epilogue, hipStream_t st) {
-    const int64_t rows = (a.M + a.E - 1) / a.E; // of an expert, on average
-    const double load = (double)a.M / a.E;
-    const bool small = a.E * f32_tiles(rows, a.N, 128) < F32_SMALL_TILES ||
-                       F32_SMALL_WORSE * f32_padded_load(load, 64) * f32_padded(a.N, 64) < f32_padded_load(load, 128) * f32_padded(a.N, 128);
+    const bool small = f32_small_tile(a.M, a.N, a.K, a.E);
     const int dim = small ? 64 : 128;
     const int64_t grid = (a.M / dim + a.E) * ((a.N + dim - 1) / dim); // sum_e ceil(c_e / dim) <= floor(M / dim) + E
     XMA_REQUIRE(grid < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "scatter2scatter (fp32): grid too large");
@@ -490,9 +465,8 @@ int f32_scatter2scatter(const FwdArgs &a, int w_is_kn, int epilogue, hipStream_t
     return w_is_kn ? launch_gemm<1, 2>(a, epilogue, (int)grid, st) : launch_gemm<0, 2>(a, epilogue, (int)grid, st);
 }
 
-int f32_group_bwd_W(const DwArgs &a, hipStream_t st) {
-    const bool small = a.E * f32_tiles(a.N_out, a.K_in, 128) < F32_SMALL_TILES_DW ||
-                       F32_SMALL_WORSE_DW * f32_padded(a.N_out, 64) * f32_padded(a.K_in, 64) < f32_padded(a.N_out, 128) * f32_padded(a.K_in, 128);
+int f32_group_bwd_W(const DwArgs &a, int64_t M, hipStream_t st) {
+    const bool small = f32_small_tile_dw(M, a.N_out, a.K_in, a.E);
     const int64_t grid = a.E * f32_tiles(a.N_out, a.K_in, small ? 64 : 128);
     XMA_REQUIRE(grid < ((int64_t)1 << 31), XMA_ROCM_EUNSUPPORTED, "group_bwd_W (fp32): grid too large");
     if (small)

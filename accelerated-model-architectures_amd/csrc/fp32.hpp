@@ -6,7 +6,7 @@
 #include "gemm_common.hpp"
 
 int f32_scatter2scatter(const FwdArgs &a, int w_is_kn, int epilogue, hipStream_t st);
-int f32_group_bwd_W(const DwArgs &a, hipStream_t st);
+int f32_group_bwd_W(const DwArgs &a, int64_t M, hipStream_t st); // M rows in all, 0: not known
 int f32_combine(const void *in, int64_t ld_in, const void *w, const void *addend, int64_t ld_add, void *y, int64_t ldy, int64_t T, int k, int H, hipStream_t st);
 int f32_combine_bwd(const void *in, int64_t ld_in, const void *dy, int64_t lddy, void *d_w, int64_t T, int k, int H,
                     hipStream_t st);

@@ -1855,11 +1855,9 @@ extern "C" size_t xma_rocm_scatter2scatter_workspace_bytes(int64_t M, int32_t N,
     return fwd_workspace_bytes(M, N, K, E);
 }
 
-extern "C" int xma_rocm_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped, int32_t dy_fan_out,
-                                    const void *dy_scale, const void *X, int64_t ldx, int x_grouped, int32_t x_fan_out,
-                                    const int64_t *sorted_scattered_idxs, const int64_t *expert_offsets, void *DW,
-                                    int64_t dw_expert_stride, int64_t lddw, int32_t N_out, int32_t K_in, int32_t E,
-                                    int dtype, void *stream) {
+int xma_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped, int32_t dy_fan_out, const void *dy_scale, const void *X, int64_t ldx, int x_grouped,
+                    int32_t x_fan_out, const int64_t *sorted_scattered_idxs, const int64_t *expert_offsets, void *DW, int64_t dw_expert_stride,
+                    int64_t lddw, int32_t N_out, int32_t K_in, int32_t E, int64_t M, int dtype, void *stream) {
     XMA_REQUIRE(dtype == XMA_ROCM_BF16 || dtype == XMA_ROCM_F16 || dtype == XMA_ROCM_F32, XMA_ROCM_EUNSUPPORTED,
                 "group_bwd_W: dtype %d", dtype);
     XMA_REQUIRE(N_out >= 8 && K_in >= 8 && E >= 1 && dy_fan_out >= 1 && x_fan_out >= 1, XMA_ROCM_EINVAL,
@@ -1897,9 +1895,18 @@ extern "C" int xma_rocm_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped
     hipStream_t st = (hipStream_t)stream;
     a.dy_div = make_fastdiv((uint32_t)dy_fan_out);
     a.x_div = make_fastdiv((uint32_t)x_fan_out);
-    if (dtype == XMA_ROCM_F32) return f32_group_bwd_W(a, st);
+    if (dtype == XMA_ROCM_F32) return f32_group_bwd_W(a, M, st);
     if (dy_scale) return launch_dw_scaled(a, dtype, (int)grid, st);
     if (dtype == XMA_ROCM_BF16) return dispatch_dw<__bf16>(a, (int)grid, st);
     return grouped_dw_f16(a, (int)grid, st);
+}
+
+extern "C" int xma_rocm_group_bwd_W(const void *DY, int64_t lddy, int dy_grouped, int32_t dy_fan_out,
+                                    const void *dy_scale, const void *X, int64_t ldx, int x_grouped, int32_t x_fan_out,
+                                    const int64_t *sorted_scattered_idxs, const int64_t *expert_offsets, void *DW,
+                                    int64_t dw_expert_stride, int64_t lddw, int32_t N_out, int32_t K_in, int32_t E,
+                                    int dtype, void *stream) {
+    return xma_group_bwd_W(DY, lddy, dy_grouped, dy_fan_out, dy_scale, X, ldx, x_grouped, x_fan_out, sorted_scattered_idxs, expert_offsets, DW,
+                           dw_expert_stride, lddw, N_out, K_in, E, 0, dtype, stream);
 }
 #endif

@@ -56,8 +56,8 @@ int dw(const xma_rocm_moe *m, int64_t few, const void *DY, int dy_grouped, const
     if (few)
         return xma_rocm_group_bwd_W_few_rows(DY, N_out, dy_grouped, dy_fan, scale, X, K_in, x_grouped, x_fan, idx, offs, DW, N_out * K_in, K_in,
                                              (int32_t)N_out, (int32_t)K_in, (int32_t)m->E, m->T * m->k, (int)m->dtype, stream);
-    return xma_rocm_group_bwd_W(DY, N_out, dy_grouped, dy_fan, scale, X, K_in, x_grouped, x_fan, idx, offs, DW, N_out * K_in, K_in,
-                                (int32_t)N_out, (int32_t)K_in, (int32_t)m->E, (int)m->dtype, stream);
+    return xma_group_bwd_W(DY, N_out, dy_grouped, dy_fan, scale, X, K_in, x_grouped, x_fan, idx, offs, DW, N_out * K_in, K_in, (int32_t)N_out,
+                           (int32_t)K_in, (int32_t)m->E, m->T * m->k, (int)m->dtype, stream);
 }
 
 int down_projection(const xma_rocm_moe *m, void *stream) {
